@@ -536,7 +536,7 @@ __global__ __launch_bounds__(512) void attention_bwd_scores_kernel(
 
 hipError_t launch_attention_backward_scores(const AttentionArgs &p, hipStream_t st)
 {
-    dim3 grid(8u * (unsigned)p.sched_wgs * (unsigned)((p.batches + 7) / 8)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
     const size_t lds = (size_t)p.sched_waves * at_bwd_lds_per_wave(p.head_dim);
 #define BSA_AT_ARGS (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, \
                     (const half_t *)p.out, (const float *)p.lse, (half_t *)p.p_out, (half_t *)p.ds_out, (half_t *)p.dq_out, (float *)p.delta, \
@@ -747,7 +747,7 @@ __global__ __launch_bounds__(512) void attention_bwd_dkdv_kernel(
 
 hipError_t launch_attention_backward_dkdv(const AttentionArgs &p, hipStream_t st)
 {
-    dim3 grid(8u * (unsigned)p.sched_wgs * (unsigned)((p.batches + 7) / 8)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
     const size_t lds = (size_t)p.sched_waves * at_bwd_col_lds_per_wave(64);
 #define BSA_AT_ARGS (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, \
                     (const float *)p.lse, (const float *)p.delta, (half_t *)p.dk_out, (half_t *)p.dv_out, \
@@ -773,7 +773,7 @@ hipError_t launch_attention_backward_dkdv(const AttentionArgs &p, hipStream_t st
 
 hipError_t launch_attention_forward(const AttentionArgs &p, hipStream_t st)
 {
-    dim3 grid(8u * (unsigned)p.sched_wgs * (unsigned)((p.batches + 7) / 8)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
     AtSplitWorkspace ws;
     ws.tile_slots = p.tile_slots;
     ws.split_groups = p.split_groups;

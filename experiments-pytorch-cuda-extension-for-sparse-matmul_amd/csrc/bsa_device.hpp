@@ -93,32 +93,60 @@ struct DescWindow {
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63u); }
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
-// Workgroup -> (batch, schedule workgroup).  Hardware deals consecutive
-// workgroup ids round-robin to the 8 XCDs, each with its own 4 MB L2; batch b
-// is pinned to XCD b % 8 so that its dense operand is fetched into one L2 only.
-// The grid holds 8 * n_swg * ceil(batches / 8) workgroups.
+// Workgroup -> (batch, schedule workgroup).  Hardware deals consecutive workgroup ids round-robin to the 8 XCDs,
+// each with its own 4 MB L2.  Batches are taken eight at a time, batch b on XCD b % 8, so that a batch's dense
+// operand is fetched into one L2 only; what is left over (batches % 8) is taken four, two and one at a time with the
+// workgroups of a batch dealt to 2, 4 or 8 XCDs in turn: a remainder batch costs a second copy of its operand in
+// another L2, but pinned to one XCD it left the other seven without work (a launch of 1 batch ran on 32 of 256
+// compute units).  Dealing them in turn keeps a schedule that lists long work first even over the XCDs.
+// The grid holds grid_workgroups() workgroups, a multiple of 8 whatever the batches, so that a second grid dimension
+// keeps the assignment.  Measured, 4096 tokens, causal local-4 + stride-8 mask, head dim 64, fused attention forward:
+// 16.4 / 17.3 / 21.5 us at 1 / 2 / 9 batches pinned, 13.0 / 13.2 / 19.7 us dealt; a training step of a 2048 x 2048
+// block-sparse bf16 weight on 4 x 1056 tokens 279 us pinned, 183 us dealt.  Multiples of 8 are mapped as before.
+__host__ __device__ __forceinline__ int remainder_per_xcd(int n_swg, int m) { return (n_swg * m + 7) >> 3; }
+__host__ __forceinline__ unsigned grid_workgroups(int n_swg, int batches)
+{
+    unsigned per_xcd = (unsigned)n_swg * (unsigned)(batches >> 3);
+    for (int m = 4; m >= 1; m >>= 1)
+        if (batches & m) per_xcd += (unsigned)remainder_per_xcd(n_swg, m);
+    return 8u * per_xcd;
+}
 __device__ __forceinline__ bool map_workgroup(int n_swg, int batches, int &batch, int &swg)
 {
-    int w = (int)blockIdx.x;
+    const int w = (int)blockIdx.x, x = w & 7;
     int t = w >> 3;
-    batch = (w & 7) + 8 * (t / n_swg);
-    swg = t % n_swg;
-    return batch < batches;
+    const int whole = n_swg * (batches >> 3);
+    if (t < whole) {
+        batch = x + 8 * (t / n_swg);
+        swg = t % n_swg;
+        return true;
+    }
+    t -= whole;
+    int base = batches & ~7;
+#pragma unroll
+    for (int m = 4; m >= 1; m >>= 1) {
+        if (batches & m) {
+            const int n = remainder_per_xcd(n_swg, m);
+            if (t < n) {
+                batch = base + (x & (m - 1));
+                swg = t * (8 / m) + x / m;
+                return swg < n_swg;
+            }
+            t -= n;
+            base += m;
+        }
+    }
+    return false;
 }
 
-// The same grid for kernels without a dense operand (the softmax reads and writes every byte
-// once, so there is nothing to keep in an L2): schedule order first, i.e. workgroup s of every
-// batch entry is dispatched before workgroup s + 1 of any.  A schedule lists long work first, and
-// in batch-major order the long rows of the last batch entries would start near the end of the
-// launch and finish on an empty machine.
-__device__ __forceinline__ bool map_workgroup_schedule_major(int n_swg, int batches, int &batch, int &swg)
+// The mapping for kernels without a dense operand (the softmax reads and writes every byte once, so there is nothing
+// to keep in an L2): schedule order first, i.e. workgroup s of every batch entry is dispatched before workgroup s + 1
+// of any.  A schedule lists long work first, and in batch-major order the long rows of the last batch entries would
+// start near the end of the launch and finish on an empty machine.  The grid holds n_swg * batches workgroups.
+__device__ __forceinline__ void map_workgroup_schedule_major(int batches, int &batch, int &swg)
 {
-    int w = (int)blockIdx.x;
-    int t = w >> 3;
-    const int nb8 = (batches + 7) >> 3;
-    batch = (w & 7) + 8 * (t % nb8);
-    swg = t / nb8;
-    return batch < batches;
+    batch = (int)blockIdx.x % batches;
+    swg = (int)blockIdx.x / batches;
 }
 
 // Orders the LDS traffic of ONE wavefront: what its lanes wrote before is

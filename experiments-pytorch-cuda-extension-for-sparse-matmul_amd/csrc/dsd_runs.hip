@@ -372,7 +372,7 @@ static hipError_t launch_runs(Kernel kernel, const RunsArgs &p, hipStream_t st)
     if (lds > RUN_LDS_MAX) return hipErrorInvalidValue;
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return err;
-    dim3 grid(8u * (unsigned)p.n_runs * (unsigned)((p.batches + 7) / 8), (unsigned)(p.N / 64)), block(64 * p.waves);
+    dim3 grid(grid_workgroups(p.n_runs, p.batches), (unsigned)(p.N / 64)), block(64 * p.waves);
     const RunRecord *runs = reinterpret_cast<const RunRecord *>(p.sched);
     const unsigned char *pair_byte = reinterpret_cast<const unsigned char *>(p.sched) + (size_t)p.mask_rows * sizeof(RunRecord);
     kernel<<<grid, block, lds, st>>>((const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, (const BlockDesc *)p.blocks,

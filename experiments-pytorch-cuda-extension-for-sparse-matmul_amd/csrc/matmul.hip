@@ -1025,14 +1025,13 @@ __global__ __launch_bounds__(512) void gw_f32_tiled_kernel(
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-static inline unsigned grid_x(int n_swg, int batches) { return 8u * (unsigned)n_swg * (unsigned)((batches + 7) / 8); }
 static inline const SchedGroup *sched_groups(const MatmulArgs &p) { return (const SchedGroup *)p.sched; }
 static inline const SchedEntry *sched_slots(const MatmulArgs &p) { return (const SchedEntry *)p.sched + p.groups; }
 
 template <bool A_KC, bool B_KC, bool BF>
 static hipError_t launch_sdd_f16(const MatmulArgs &p, hipStream_t st)
 {
-    dim3 grid(grid_x(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
     size_t lds = (size_t)p.sched_waves * SDD_LDS_PER_WAVE;
 #define BSA_SDD_ARGS (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, (const BlockDesc *)p.blocks, \
                      sched_slots(p), p.sched_wgs, p.batches, p.nnz, p.M, p.N, p.K
@@ -1050,7 +1049,7 @@ static hipError_t launch_sdd_f16(const MatmulArgs &p, hipStream_t st)
 template <bool A_KC, bool B_KC>
 static hipError_t launch_sdd_f32(const MatmulArgs &p, hipStream_t st)
 {
-    dim3 grid(grid_x(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
 #define BSA_SDD_ARGS (const float *)p.a, (const float *)p.b, (float *)p.c, (const BlockDesc *)p.blocks, \
                      sched_slots(p), p.sched_wgs, p.batches, p.nnz, p.M, p.N, p.K
     const int kbs = p.K / BS;
@@ -1097,7 +1096,7 @@ template <bool S_KC, bool D_KC, bool DSD>
 static hipError_t launch_gw_t(int dtype, const void *sp, const void *dn, const MatmulArgs &p,
                               int DN, int KT, int XT, hipStream_t st)
 {
-    dim3 grid(grid_x(p.sched_wgs, p.batches), (unsigned)((DN + 63) / 64)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches), (unsigned)((DN + 63) / 64)), block(64 * p.sched_waves);
     size_t lds = (size_t)p.sched_waves * GW_LDS_PER_WAVE;
     // workspace: counters of every (batch, strip, split group), then the partial tiles
     SplitWorkspace ws;
@@ -1137,7 +1136,7 @@ static hipError_t launch_gw_t(int dtype, const void *sp, const void *dn, const M
 
 hipError_t launch_dsd_block64(int dtype, const Block64Args &p, hipStream_t st)
 {
-    dim3 grid(grid_x(p.sched_wgs, p.batches), (unsigned)(p.N / 64)), block(64 * p.sched_waves);
+    dim3 grid(grid_workgroups(p.sched_wgs, p.batches), (unsigned)(p.N / 64)), block(64 * p.sched_waves);
     const size_t lds = (size_t)p.sched_waves * GW64_LDS_PER_WAVE;
     const SchedEntry *slots = (const SchedEntry *)p.sched + p.coarse_rows;
     hipError_t err = hipSuccess;

@@ -487,7 +487,7 @@ __device__ __forceinline__ void softmax_fwd_sliced(const T *__restrict__ xb, T *
 template <typename T, int CB, int CBS>
 __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void softmax_fwd_kernel(
     const T *__restrict__ x, T *__restrict__ y, const BlockDesc *__restrict__ blocks,
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, int nnz,
+    const SchedEntry *__restrict__ sched, int batches, int nnz,
     float scale2 /* scale * log2(e) */, int causal)
 {
     typedef Chunk<T> C;
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_
     __shared__ float2 stats[SM_MAX_WAVES][BS];
 
     int batch, swg;
-    if (!map_workgroup_schedule_major(n_swg, batches, batch, swg)) return;
+    map_workgroup_schedule_major(batches, batch, swg);
     const int w = wave_id(), l = lane_id();
     const int W = (int)(blockDim.x >> 6);
     const SchedEntry e = sched[swg * W + w];
@@ -810,7 +810,7 @@ template <typename T, int CB, int CBS>
 __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void softmax_bwd_kernel(
     const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx,
     const BlockDesc *__restrict__ blocks, const SchedEntry *__restrict__ sched,
-    int n_swg, int batches, int nnz, float scale)
+    int batches, int nnz, float scale)
 {
     typedef Chunk<T> C;
     constexpr int NQ = C::NQ, EPC = C::EPC, LPR = C::LPR;
@@ -819,7 +819,7 @@ __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_
     __shared__ float dots[SM_MAX_WAVES][BS];
 
     int batch, swg;
-    if (!map_workgroup_schedule_major(n_swg, batches, batch, swg)) return;
+    map_workgroup_schedule_major(batches, batch, swg);
     const int w = wave_id(), l = lane_id();
     const int W = (int)(blockDim.x >> 6);
     const SchedEntry e = sched[swg * W + w];
@@ -960,42 +960,41 @@ __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-static inline unsigned grid_x(int n_swg, int batches) { return 8u * (unsigned)n_swg * (unsigned)((batches + 7) / 8); }
 
 hipError_t launch_softmax_forward(int dtype, const SoftmaxArgs &p, hipStream_t st)
 {
-    dim3 grid(grid_x(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
+    dim3 grid((unsigned)p.sched_wgs * (unsigned)p.batches), block(64 * p.sched_waves);
     const float scale2 = p.scale * 1.4426950408889634f;
     if (dtype == BSA_F16)
         softmax_fwd_kernel<half_t, 4, 48><<<grid, block, 0, st>>>(
             (const half_t *)p.x, (half_t *)p.out, (const BlockDesc *)p.blocks,
-            (const SchedEntry *)p.sched + p.groups, p.sched_wgs, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
     else if (dtype == BSA_BF16)
         softmax_fwd_kernel<bf16_t, 4, 48><<<grid, block, 0, st>>>(
             (const bf16_t *)p.x, (bf16_t *)p.out, (const BlockDesc *)p.blocks,
-            (const SchedEntry *)p.sched + p.groups, p.sched_wgs, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
     else
         softmax_fwd_kernel<float, 2, 24><<<grid, block, 0, st>>>(
             (const float *)p.x, (float *)p.out, (const BlockDesc *)p.blocks,
-            (const SchedEntry *)p.sched + p.groups, p.sched_wgs, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
     return hipGetLastError();
 }
 
 hipError_t launch_softmax_backward(int dtype, const SoftmaxArgs &p, hipStream_t st)
 {
-    dim3 grid(grid_x(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
+    dim3 grid((unsigned)p.sched_wgs * (unsigned)p.batches), block(64 * p.sched_waves);
     if (dtype == BSA_F16)
         softmax_bwd_kernel<half_t, 2, 24><<<grid, block, 0, st>>>(
             (const half_t *)p.x, (const half_t *)p.dy, (half_t *)p.out, (const BlockDesc *)p.blocks,
-            (const SchedEntry *)p.sched + p.groups, p.sched_wgs, p.batches, p.nnz, p.scale);
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, p.scale);
     else if (dtype == BSA_BF16)
         softmax_bwd_kernel<bf16_t, 2, 24><<<grid, block, 0, st>>>(
             (const bf16_t *)p.x, (const bf16_t *)p.dy, (bf16_t *)p.out, (const BlockDesc *)p.blocks,
-            (const SchedEntry *)p.sched + p.groups, p.sched_wgs, p.batches, p.nnz, p.scale);
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, p.scale);
     else
         softmax_bwd_kernel<float, 1, 24><<<grid, block, 0, st>>>(
             (const float *)p.x, (const float *)p.dy, (float *)p.out, (const BlockDesc *)p.blocks,
-            (const SchedEntry *)p.sched + p.groups, p.sched_wgs, p.batches, p.nnz, p.scale);
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, p.scale);
     return hipGetLastError();
 }
 
