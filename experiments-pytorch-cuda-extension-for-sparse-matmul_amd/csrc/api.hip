@@ -520,7 +520,7 @@ int bsa_attention_backward_scores(int dtype, const void *q, const void *k, const
     return check_launch(bsa::launch_attention_backward_scores(p, (hipStream_t)stream), who);
 }
 
-int bsa_attention_backward(int dtype, const void *q, const void *k, const void *v, const void *dout,
+static int attention_backward(const char *who, int dtype, const void *q, const void *k, const void *v, const void *dout,
                            const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
                            float *delta_ws,
                            const int32_t *row_blocks, const int32_t *row_offsets,
@@ -533,14 +533,15 @@ int bsa_attention_backward(int dtype, const void *q, const void *k, const void *
                            int mask_rows, int mask_cols, int nnz, int batches, int head_dim,
                            float scale, int causal, void *stream)
 {
-    const char *who = "bsa_attention_backward";
     int rc = check_attention(who, dtype, head_dim, row_blocks, row_offsets, row_sched, row_sched_wgs, row_sched_waves,
                              mask_rows, mask_cols, nnz, batches);
     if (rc) return rc;
-    if (head_dim != 64) return fail(BSA_ERR_UNSUPPORTED, "%s: head_dim 64 is built, got %d", who, head_dim);
     if (!col_offsets || (!col_blocks && nnz > 0)) return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
     rc = check_schedule(col_sched, col_sched_wgs, col_sched_waves, batches, who);
     if (rc) return rc;
+    if (head_dim == 128 && col_sched_waves > bsa::AT_COLUMN_WAVES_128)
+        return fail(BSA_ERR_INVALID, "%s: the column schedule has %d waves per workgroup, at most %d at head_dim 128", who,
+                    col_sched_waves, bsa::AT_COLUMN_WAVES_128);
     if (!q || !k || !v || !dout || !out || !lse || !dq_out || !dk_out || !dv_out || !delta_ws)
         return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
     rc = check_split_workspace(who, row_tile_slots, row_split_groups);
@@ -576,6 +577,50 @@ int bsa_attention_backward(int dtype, const void *q, const void *k, const void *
     p.dk_out = dk_out;
     p.dv_out = dv_out;
     return check_launch(bsa::launch_attention_backward_dkdv(p, (hipStream_t)stream), who);
+}
+
+int bsa_attention_backward(int dtype, const void *q, const void *k, const void *v, const void *dout,
+                           const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
+                           float *delta_ws,
+                           const int32_t *row_blocks, const int32_t *row_offsets,
+                           const int32_t *row_sched, int row_sched_wgs, int row_sched_waves,
+                           int row_tile_slots, int row_split_groups,
+                           const int32_t *col_blocks, const int32_t *col_offsets,
+                           const int32_t *col_sched, int col_sched_wgs, int col_sched_waves,
+                           int col_tile_slots, int col_split_groups,
+                           void *workspace, size_t workspace_bytes,
+                           int mask_rows, int mask_cols, int nnz, int batches, int head_dim,
+                           float scale, int causal, void *stream)
+{
+    if (head_dim == 128)
+        return fail(BSA_ERR_UNSUPPORTED,
+                    "bsa_attention_backward: head_dim 64 is built, got %d (bsa_attention_gradients takes both)",
+                    head_dim);
+    return attention_backward("bsa_attention_backward", dtype, q, k, v, dout, out, lse, dq_out, dk_out, dv_out,
+                              delta_ws, row_blocks, row_offsets, row_sched, row_sched_wgs, row_sched_waves,
+                              row_tile_slots, row_split_groups, col_blocks, col_offsets, col_sched, col_sched_wgs, col_sched_waves, col_tile_slots,
+                              col_split_groups, workspace, workspace_bytes, mask_rows, mask_cols, nnz,
+                              batches, head_dim, scale, causal, stream);
+}
+
+int bsa_attention_gradients(int dtype, const void *q, const void *k, const void *v, const void *dout,
+                            const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
+                            float *delta_ws,
+                            const int32_t *row_blocks, const int32_t *row_offsets,
+                            const int32_t *row_sched, int row_sched_wgs, int row_sched_waves,
+                            int row_tile_slots, int row_split_groups,
+                            const int32_t *col_blocks, const int32_t *col_offsets,
+                            const int32_t *col_sched, int col_sched_wgs, int col_sched_waves,
+                            int col_tile_slots, int col_split_groups,
+                            void *workspace, size_t workspace_bytes,
+                            int mask_rows, int mask_cols, int nnz, int batches, int head_dim,
+                            float scale, int causal, void *stream)
+{
+    return attention_backward("bsa_attention_gradients", dtype, q, k, v, dout, out, lse, dq_out, dk_out, dv_out,
+                              delta_ws, row_blocks, row_offsets, row_sched, row_sched_wgs, row_sched_waves,
+                              row_tile_slots, row_split_groups, col_blocks, col_offsets, col_sched, col_sched_wgs, col_sched_waves, col_tile_slots,
+                              col_split_groups, workspace, workspace_bytes, mask_rows, mask_cols, nnz,
+                              batches, head_dim, scale, causal, stream);
 }
 
 }  // extern "C"

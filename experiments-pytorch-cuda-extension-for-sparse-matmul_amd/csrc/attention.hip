@@ -1,5 +1,5 @@
-// Fused block-sparse attention forward for gfx950: out = softmax(scale * q k^T, over the stored
-// blocks of a row, causal if asked) v, without the scores ever leaving the chip.
+// Fused block-sparse attention for gfx950: out = softmax(scale * q k^T, over the stored
+// blocks of a row, causal if asked) v, without the scores ever leaving the chip, and its gradients.
 //
 // The reference computes this as three launches with the scores written and read twice in between
 // (SDD sparse/native/sparse_smm_gpu.cu:22-95, softmax sparse_softmax.cu:113-155, DSD
@@ -9,32 +9,37 @@
 // One wavefront walks a chunk of the blocks (r, c) of block row r:
 //   S^T = K_c Q_r^T        32 keys x 32 queries, 4 MFMAs over head dim 64; Q_r stays in registers
 //   online softmax          a lane holds ONE query column of S^T (16 keys; the other 16 sit in lane
-//                           l ^ 32), so max, sum and the rescaling factor are per-lane scalars and
-//                           one cross-lane exchange per block
+//                           l ^ 32), so reference point, sum and the rescaling factor are per-lane scalars
 //   O^T += V_c^T P^T        the probabilities go from the accumulators of the first product straight
 //                           into the operand registers of the second: accumulator value v of lane
-//                           half h is key 8 (v / 4) + 4 h + v % 4, and V_c is parked in LDS with
-//                           its rows exchanged to match (put_strip_swapped_addr).  No LDS round
-//                           trip, no shuffle.
+//                           half h is key 8 (v / 4) + 4 h + v % 4, and V_c is read from LDS in that
+//                           order of rows.  No LDS round trip, no shuffle.
 // The waves of a row (a team of the schedule) merge their (max, sum, O^T) through LDS.
+//
+// What bounds it.  A wave has one block in work: about 1750 clocks beside three other waves of its SIMD (LDS operands
+// 500, products 200, exponentials 600, the rest scalar), so a SIMD finishes one per 440, of which the vector ALU is busy
+// about 390; a wave also spends 6000 clocks before its first block (schedule slot, block columns, first tiles: three
+// dependent round trips) and 3000 behind its last.  K and V go straight to LDS, each tile requested as soon as the
+// operands of the one before sit in registers, and have arrived when they are wanted (45 and 80 clocks of waiting per
+// block); with every request served from one address the launch takes as long.  Against tiles that pass through
+// registers, a maximum per block and 8-byte result pieces (us, before -> after): 3 x 5 heads of 2976 tokens, 1053 blocks
+// a head 20.1 -> 14.7; 48 heads of 8192 tokens, 2526 blocks 98 -> 82; 16 heads of 4096 tokens, 1530 blocks 23.1 -> 17.6,
+// at head dim 128 41.9 -> 35.3.  Panels of four block rows sharing the tiles of a workgroup (half the L2 traffic, a
+// barrier per column) took 18.7 / 84 / 21.5: the rows of a panel wait for one another.
+#include <cmath>
+
 #include "bsa_device.hpp"
 #include "lds_tiles.hpp"
+#include "attention_tiles.hpp"
 #include "bsa_internal.hpp"
 #include "../../include/bsa.h"
 
 namespace bsa {
 
-// per wave: K tiles (HD / 32 of 2 KB) + V strips (HD / 64 of 4 KB), reused for the O^T partial of the
+// per wave: the K tile and the V tile (64 HD bytes each), reused for the O^T partial of the
 // team merge (HD x 32 floats: the same size), + row stats
-constexpr int at_lds_per_wave(int hd) { return 128 * hd + 512; }
-constexpr float AT_LAZY = 8.f;                // log2 of the growth of a row maximum that forces a rescale
-
-__device__ __forceinline__ float at_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-__device__ __forceinline__ float at_lane_xor32(float x)
-{
-    return __int_as_float(__builtin_amdgcn_ds_bpermute((lane_id() ^ 32) << 2, __float_as_int(x)));
-}
-__device__ __forceinline__ float at_finite_or_zero(float m) { return m == -__builtin_inff() ? 0.f : m; }
+constexpr int at_lds_per_wave(int hd) { return 128 * hd + 256; }
+constexpr float AT_LAZY_SUM = 256.f;          // probabilities stay below it (fp16 holds them) until the reference point moves
 
 // Split rows of the forward walk: a block row longer than one workgroup's share is cut into parts
 // that run in different workgroups.  Every part parks (O^T, max, sum) of its 32 queries in the
@@ -42,16 +47,6 @@ __device__ __forceinline__ float at_finite_or_zero(float m) { return m == -__bui
 // (so the result does not depend on arrival order), resets the counter and stores the row.  Parked
 // values are published and consumed with park_store / split_publish / split_consume / park_load
 // (bsa_device.hpp: release and acquire at agent scope).
-struct AtSplitWorkspace {
-    int *counters;     // [batches][split_groups], zero between launches
-    float *tiles;      // [batches][tile_slots][at_split_tile_floats(head dim)]
-    int tile_slots, split_groups;
-};
-constexpr int at_split_tile_floats(int hd) { return 32 * hd + 2 * WAVE; }   // O^T, then every lane's max and sum
-static size_t at_split_counter_bytes(int split_groups, int batches)
-{
-    return (((size_t)split_groups * batches * sizeof(int)) + 255) / 256 * 256;
-}
 size_t attention_workspace_bytes(int tile_slots, int split_groups, int batches, int head_dim)
 {
     if (tile_slots <= 0 || split_groups <= 0) return 0;
@@ -59,33 +54,6 @@ size_t attention_workspace_bytes(int tile_slots, int split_groups, int batches, 
            (size_t)tile_slots * batches * at_split_tile_floats(head_dim) * sizeof(float);
 }
 
-// The backward walks split a group the same way, but their parts only add up (the row statistics are
-// known): a part parks NT accumulator tiles, bumps the counter, and the last to arrive sums in part order.
-template <int NT>
-__device__ __forceinline__ void at_park(const f16v (&acc)[NT], float *dst)
-{
-    const int l = lane_id();
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            park_store(dst + (t * 16 + i) * WAVE + l, acc[t][i]);
-}
-template <int NT>
-__device__ __forceinline__ void at_sum_parts(f16v (&acc)[NT], const float *first, int stride, int parts)
-{
-    const int l = lane_id();
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = f16v{0};
-    for (int p = 0; p < parts; ++p) {
-        const float *src = first + (size_t)p * stride;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                acc[t][i] += park_load(src + (t * 16 + i) * WAVE + l);
-    }
-}
 // workspace of the two backward walks: [row counters | row tiles of 32 hd floats | column counters | column
 // tiles of 2 x 32 hd floats (dv^T, dk^T)]
 static size_t at_bwd_region_bytes(int tile_slots, int split_groups, int batches, int tile_floats)
@@ -101,13 +69,14 @@ size_t attention_backward_workspace_bytes(int row_tile_slots, int row_split_grou
 }
 
 template <int HD, bool BF>
-__global__ __launch_bounds__(512) void attention_fwd_f16_kernel(
+__global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attention_fwd_f16_kernel(
     const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
     half_t *__restrict__ out, float *__restrict__ lse, const BlockDesc *__restrict__ blocks,
     const SchedGroup *__restrict__ sched_groups, const SchedEntry *__restrict__ sched, AtSplitWorkspace ws,
     int n_swg, int batches, int rows_q, int rows_k, float scale2 /* scale * log2(e) */, int causal)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int KS = HD / 16, KT = HD / 32, LDS_PER_WAVE = at_lds_per_wave(HD), STAT_OFF = 128 * HD;
     int batch, swg;
     if (!map_workgroup(n_swg, batches, batch, swg)) return;
     const int w = wave_id(), l = lane_id();
@@ -115,175 +84,132 @@ __global__ __launch_bounds__(512) void attention_fwd_f16_kernel(
     const SchedEntry e = sched[swg * W + w];
     const bool active = e.group >= 0;
     const int r = e.group;
-    const int qq = l & 31, h = l >> 5;          // query column of this lane, lane half
+    const int qq = l & 31, h = l >> 5;           // query column of this lane, lane half
     const float NEG_INF = -__builtin_inff();
 
-    constexpr int AT_HEAD = HD, AT_LDS_PER_WAVE = at_lds_per_wave(HD);
-    constexpr int KT = HD / 32, VS = HD / 64;   // 32-wide K tiles, 64-wide V strips
-    unsigned char *my_lds = lds_raw + (size_t)w * AT_LDS_PER_WAVE;
-    half_t *tile_k = reinterpret_cast<half_t *>(my_lds);                 // KT [key][32 d] tiles
-    half_t *tile_v = reinterpret_cast<half_t *>(my_lds + 2048 * KT);     // VS [key][64 n] strips, rows exchanged
-    const half_t *kb = k + (size_t)batch * rows_k * AT_HEAD;
-    const half_t *vb = v + (size_t)batch * rows_k * AT_HEAD;
+    unsigned char *tile_k = lds_raw + (size_t)w * LDS_PER_WAVE, *tile_v = tile_k + 64 * HD;
+    const TileReader rd(tile_k);
+    constexpr unsigned K_TILE = 0, V_TILE = 64 * HD;
+    const TileRequests<HD> kreq(k + (size_t)batch * rows_k * HD, tile_k), vreq(v + (size_t)batch * rows_k * HD, tile_v);
 
-    // Q_r as the column operand of S^T: lane (qq, h) holds d = 16 s + 8 h .. + 7 of query qq
-    h8 qop[AT_HEAD / 16];
-    if (active) {
-        const half_t *qrow = q + ((size_t)batch * rows_q + BS * r + qq) * AT_HEAD + 8 * h;
-#pragma unroll
-        for (int s = 0; s < AT_HEAD / 16; ++s) qop[s] = as_h8(ldg16(qrow + 16 * s));
-    }
+    // reference point of the query (both lane halves agree), minus it (0 while nothing was seen), this half's sum;
+    // unseen: some query of the wave has no reference point yet
+    float m = NEG_INF, minus_m = 0.f, lsum = 0.f;
+    bool unseen = true;
+    RowTile<HD> oacc;
+    clear<HD>(oacc);
 
-    struct Frag { uint4 kk[KT][2], vv[VS][4]; };   // K_c as 32 x 32 tiles (d slices), V_c as 4 KB strips (n slices)
-    DescWindow win;
-    auto load = [&](int p, Frag &f) {
-        const int c = win.get(p).col();
-#pragma unroll
-        for (int dt = 0; dt < KT; ++dt) ldg_tile32(kb + (size_t)(BS * c) * AT_HEAD + 32 * dt, AT_HEAD, f.kk[dt]);
-        const half_t *vs = vb + (size_t)(BS * c) * AT_HEAD;
-#pragma unroll
-        for (int u = 0; u < VS; ++u)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int piece = l + 64 * t;               // key row piece / 8, 16-byte piece % 8 of the 128-byte strip row
-                f.vv[u][t] = ldg16(vs + (size_t)(piece >> 3) * AT_HEAD + 64 * u + 8 * (piece & 7));
-            }
-    };
-
-    float m = NEG_INF, lsum = 0.f;               // running max of the query (both lane halves agree), this half's sum
-    f16v oacc[KT];                               // O^T: lane = query column, values = head dims 32 t + 8 (v / 4) + 4 h + v % 4
-#pragma unroll
-    for (int t = 0; t < KT; ++t) oacc[t] = f16v{0};
-
-    // registers -> staging tiles; the registers are free for the next block's loads afterwards
-    auto stage = [&](const Frag &f) {
-        wave_lds_fence();
-#pragma unroll
-        for (int dt = 0; dt < KT; ++dt) lds_put_kc<false>(tile_k + dt * BS2, f.kk[dt]);
-#pragma unroll
-        for (int u = 0; u < VS; ++u) lds_put_strip_swapped(tile_v + u * 2048, f.vv[u]);
-        wave_lds_fence();
-    };
-    auto step = [&](int c) {
-        f16v sacc = {0};
-#pragma unroll
-        for (int dt = 0; dt < KT; ++dt)
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                sacc = mfma_16<BF>(lds_get_kc(tile_k + dt * BS2, s), qop[2 * dt + s], sacc);
-
-        // Row maximum of the scaled scores.  Off the diagonal nothing is masked and the scale is
-        // folded into the exponent (one fused multiply-add per score); the diagonal block of a
-        // causal launch takes the explicit route.
-        float bm;
-        const bool masked = causal && c >= r;
-        float mul = scale2;                      // what is still to be applied to sacc in the exponent
-        if (masked) {
-            bm = NEG_INF;
-            mul = 1.f;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int key = 8 * (i >> 2) + 4 * h + (i & 3);
-                sacc[i] = (c > r || key > qq) ? NEG_INF : sacc[i] * scale2;
-                bm = fmaxf(bm, sacc[i]);
-            }
-        } else {
-            float hi = sacc[0], lo = sacc[0];
-#pragma unroll
-            for (int i = 1; i < 16; ++i) {
-                hi = fmaxf(hi, sacc[i]);
-                if (scale2 < 0.f) lo = fminf(lo, sacc[i]);     // uniform: a negative scale turns the order round
-            }
-            bm = scale2 < 0.f ? lo * scale2 : hi * scale2;
-        }
-        bm = fmaxf(bm, at_lane_xor32(bm));
-        // Lazy rescaling: the reference point m only moves when some row's maximum has grown by
-        // more than 2^AT_LAZY since it was set, so the 32 multiplies of O^T (and the branch is
-        // uniform) are skipped for most blocks; until then probabilities may reach 2^AT_LAZY,
-        // which fp16 holds without loss of relative precision.
-        if (__builtin_amdgcn_ballot_w64(bm > m + AT_LAZY) != 0ull) {
-            const float m_new = fmaxf(m, bm);
-            const float alpha = at_exp2(at_finite_or_zero(m) - at_finite_or_zero(m_new));
-            const float keep = m == NEG_INF ? 0.f : alpha;      // nothing accumulated so far
-            m = m_new;
-            lsum *= keep;
-#pragma unroll
-            for (int t = 0; t < KT; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) oacc[t][i] *= keep;
-        }
-        const float mm = at_finite_or_zero(m);
-        float psum = 0.f;
-        h8 pop[2];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const float pv = at_exp2(__builtin_fmaf(sacc[i], mul, -mm));
-            psum += pv;
-            pop[i >> 3][i & 7] = narrow_16<BF>(pv);
-        }
-        lsum += psum;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                oacc[t] = mfma_16<BF>(lds_get_strip<false>(tile_v + (t / 2) * 2048, 32 * (t % 2), s), pop[s], oacc[t]);
-    };
-
-    // One block in flight: its tiles are requested as soon as the previous block's have been copied
-    // to LDS, so the loads run under the previous block's products and softmax.  (A second set of
-    // load registers costs an occupancy step, which measured worse than the shorter prefetch.)
-    if (active) {
-        Frag fr;
+    if (active && e.begin < e.end) {
+        DescWindow win;
+        h8 qop[KS];
+        // Q_r waits for nothing but the schedule slot: it goes through the V tile (4 requests of whole lines; read
+        // straight into operand layout every request would touch 32 lines) beside the load of the block columns.
+        TileRequests<HD>(q + (size_t)batch * rows_q * HD, tile_v).issue(r);
         for (int seg = e.begin; seg < e.end; seg += WAVE) {
             const int seg_end = seg + WAVE < e.end ? seg + WAVE : e.end;
             win.fetch(blocks, seg, seg_end);
-            load(seg, fr);
+            kreq.issue(win.get(seg).col());
+            if (seg == e.begin) {
+                tile_wait<TileRequests<HD>::N>();
+#pragma unroll
+                for (int s = 0; s < KS; ++s) qop[s] = rd.rows(V_TILE, s);
+                lds_reads_done();
+            }
+            vreq.issue(win.get(seg).col());
             for (int p = seg; p < seg_end; ++p) {
-                stage(fr);
-                if (p + 1 < seg_end) load(p + 1, fr);
-                step(win.get(p).col());
+                const int c = win.get(p).col();
+                const bool last = p + 1 == seg_end;
+                // A stage is a single buffer: K of the next block is requested as soon as this block's operands sit in
+                // registers, V likewise, so each has the other half of the block's work to arrive in.
+                tile_wait<TileRequests<HD>::N>();            // everything but V
+                h8 kop[KS];
+#pragma unroll
+                for (int s = 0; s < KS; ++s) kop[s] = rd.rows(K_TILE, s);
+                lds_reads_done();
+                if (!last) kreq.issue(win.get(p + 1).col());
+                f16v sacc = {0};                 // keys 8 (v / 4) + 4 h + v % 4 of query qq
+#pragma unroll
+                for (int s = 0; s < KS; ++s) sacc = mfma_16<BF>(kop[s], qop[s], sacc);
+                float mul = scale2;              // what is still to be applied to sacc in the exponent
+                if (causal && c >= r) {          // -inf only once scaled, whatever the scale's sign
+                    mul = 1.f;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        sacc[v] = c > r || 8 * (v >> 2) + 4 * h + (v & 3) > qq ? NEG_INF : sacc[v] * scale2;
+                }
+                float psum;
+                h8 pop[2];
+                auto exponentials = [&]() {
+                    psum = 0.f;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const float pv = at_exp2(__builtin_fmaf(sacc[v], mul, minus_m));
+                        psum += pv;
+                        pop[v >> 3][v & 7] = narrow_16<BF>(pv);
+                    }
+                };
+                // There is no maximum per block: the reference point of a row is the maximum of its first visible block
+                // and moves only when a block's sum of exponentials exceeds AT_LAZY_SUM.
+                bool move = unseen;
+                if (!move) {
+                    exponentials();
+                    move = __builtin_amdgcn_ballot_w64(!(psum <= AT_LAZY_SUM)) != 0ull;
+                }
+                if (move) {
+                    float bm = sacc[0] * mul;
+#pragma unroll
+                    for (int v = 1; v < 16; ++v) bm = fmaxf(bm, sacc[v] * mul);
+                    const float m_new = fmaxf(m, fmaxf(bm, at_lane_xor32(bm)));
+                    const float keep = m == NEG_INF ? 0.f : at_exp2(m - at_finite_or_zero(m_new));   // nothing accumulated so far: 0
+                    m = m_new;
+                    minus_m = -at_finite_or_zero(m_new);
+                    lsum *= keep;
+                    each<HD>(oacc, [&](float x, int) { return x * keep; });
+                    unseen = __builtin_amdgcn_ballot_w64(m == NEG_INF) != 0ull;
+                    exponentials();
+                }
+                lsum += psum;
+                if (last) tile_wait<0>();
+                else tile_wait<TileRequests<HD>::N>();       // everything but the next K
+                h8 vop[KT][2];
+#pragma unroll
+                for (int t = 0; t < KT; ++t)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) vop[t][s] = rd.columns(V_TILE, t, s);
+                lds_reads_done();
+                if (!last) vreq.issue(win.get(p + 1).col());
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int t = 0; t < KT; ++t) oacc[t] = mfma_16<BF>(vop[t][s], pop[s], oacc[t]);
             }
         }
+        lsum += at_lane_xor32(lsum);             // both halves used the same reference point
     }
-    lsum += at_lane_xor32(lsum);                 // both halves used the same max
 
-    // team merge: every wave but the leader parks (max, sum, O^T); the leader rescales and adds
+    // team merge: every wave but the leader parks (max, sum) per query and O^T; the leader rescales and adds
     const int slot0 = e.first_wave(), nw = e.team_waves();
     const bool leader = active && w == slot0;
-    constexpr int STAT_OFF = 128 * HD;                                // behind the HD x 32 floats of O^T
-    float *park = reinterpret_cast<float *>(my_lds);
-    float2 *stat = reinterpret_cast<float2 *>(my_lds + STAT_OFF);     // 32 (max, sum)
     if (active && !leader) {
         wave_lds_fence();
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) park[(t * 16 + i) * WAVE + l] = oacc[t][i];
-        if (h == 0) stat[qq] = make_float2(m, lsum);
+        each<HD>(oacc, [&](float x, int at) { return reinterpret_cast<float *>(tile_k)[at] = x; });
+        if (h == 0) reinterpret_cast<float2 *>(tile_k + STAT_OFF)[qq] = make_float2(m, lsum);
     }
     __syncthreads();
     if (!leader) return;
     if (nw > 1) {
+        auto stat = [&](int o) { return reinterpret_cast<const float2 *>(tile_k + o * LDS_PER_WAVE + STAT_OFF)[qq]; };
         float M = m;
-        for (int o = 1; o < nw; ++o)
-            M = fmaxf(M, reinterpret_cast<const float2 *>(lds_raw + (size_t)(w + o) * AT_LDS_PER_WAVE + STAT_OFF)[qq].x);
-        const float MM = at_finite_or_zero(M);
-        const float mine = at_exp2(m - MM);
-        lsum *= mine;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) oacc[t][i] *= mine;
+        for (int o = 1; o < nw; ++o) M = fmaxf(M, stat(o).x);
+        const float MM = at_finite_or_zero(M), own = at_exp2(m - MM);
+        lsum *= own;
+        each<HD>(oacc, [&](float x, int) { return x * own; });
         for (int o = 1; o < nw; ++o) {
-            const unsigned char *other = lds_raw + (size_t)(w + o) * AT_LDS_PER_WAVE;
-            const float2 st = reinterpret_cast<const float2 *>(other + STAT_OFF)[qq];
+            const float2 st = stat(o);
             const float f = at_exp2(st.x - MM);
             lsum += st.y * f;
-            const float *op = reinterpret_cast<const float *>(other);
-#pragma unroll
-            for (int t = 0; t < KT; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) oacc[t][i] += op[(t * 16 + i) * WAVE + l] * f;
+            const float *src = reinterpret_cast<const float *>(tile_k + o * LDS_PER_WAVE);
+            each<HD>(oacc, [&](float x, int at) { return x + src[at] * f; });
         }
         m = M;                                   // the sums are relative to the team's reference point now
     }
@@ -292,86 +218,64 @@ __global__ __launch_bounds__(512) void attention_fwd_f16_kernel(
         const SchedGroup sg = sched_groups[r];
         float *tile0 = ws.tiles + ((size_t)batch * ws.tile_slots + sg.tile_slot) * TILE;
         float *mine = tile0 + (size_t)e.part() * TILE;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                park_store(mine + (t * 16 + i) * WAVE + l, oacc[t][i]);
+        park_part<HD>(oacc, mine);
         park_store(mine + 32 * HD + l, m);
         park_store(mine + 32 * HD + WAVE + l, lsum);
         int *counter = ws.counters + (size_t)batch * ws.split_groups + sg.split_index;
         const int parts = e.parts();
         if (split_publish(counter) != parts - 1) return;
         split_consume();
-        float M = NEG_INF;
-        for (int p = 0; p < parts; ++p)
-            M = fmaxf(M, park_load(tile0 + (size_t)p * TILE + 32 * HD + l));
-        const float MM = at_finite_or_zero(M);
+        m = NEG_INF;
+        for (int j = 0; j < parts; ++j) m = fmaxf(m, park_load(tile0 + (size_t)j * TILE + 32 * HD + l));
+        const float MM = at_finite_or_zero(m);
         lsum = 0.f;
-#pragma unroll
-        for (int t = 0; t < KT; ++t) oacc[t] = f16v{0};
-        for (int p = 0; p < parts; ++p) {
-            const float *src = tile0 + (size_t)p * TILE;
+        clear<HD>(oacc);
+        for (int j = 0; j < parts; ++j) {
+            const float *src = tile0 + (size_t)j * TILE;
             const float f = at_exp2(park_load(src + 32 * HD + l) - MM);
             lsum += park_load(src + 32 * HD + WAVE + l) * f;
-#pragma unroll
-            for (int t = 0; t < KT; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    oacc[t][i] += park_load(src + (t * 16 + i) * WAVE + l) * f;
+            each<HD>(oacc, [&](float x, int at) { return x + park_load(src + at) * f; });
         }
-        m = M;
         split_reset(counter);
     }
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    // log2 of the row's sum of exponentials of the scaled scores (what the backward pass needs to
-    // rebuild the probabilities); +inf for a row that sees nothing, so that they come out as zeros
-    if (lse != nullptr && h == 0)
-        lse[(size_t)batch * rows_q + BS * r + qq] = lsum > 0.f ? at_finite_or_zero(m) + __builtin_amdgcn_logf(lsum)
-                                                               : __builtin_inff();
-    half_t *orow = out + ((size_t)batch * rows_q + BS * r + qq) * AT_HEAD + 4 * h;
-#pragma unroll
-    for (int t = 0; t < KT; ++t) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            h4 o;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = narrow_16<BF>(oacc[t][4 * g + j] * inv);
-            *reinterpret_cast<h4 *>(orow + 32 * t + 8 * g) = o;
-        }
-    }
+    // log2 of the row's sum of exponentials of the scaled scores (what the backward pass needs to rebuild the
+    // probabilities); +inf for a row that sees nothing, so that they come out as zeros
+    const size_t row0 = (size_t)batch * rows_q + (size_t)BS * r;
+    if (lse != nullptr && h == 0) lse[row0 + qq] = lsum > 0.f ? at_finite_or_zero(m) + __builtin_amdgcn_logf(lsum) : __builtin_inff();
+    store_rows<HD, BF>(oacc, lsum > 0.f ? 1.f / lsum : 0.f, tile_k, out + row0 * HD);
 }
 
 // ---------------------------------------------------------------------------
-// Backward, first half: the probabilities P and the score gradients dS of every stored block, and
-// dq, in one launch, from q, k, v, dO, O and the row statistics of the forward pass:
+// Backward, the walk over the ROWS: dq, and (STACKS) the probabilities P and the score gradients dS of every stored
+// block, from q, k, v, dO, O and the row statistics of the forward pass:
 //   P  = exp2(scale2 * q k^T - lse)                         (no second softmax pass: lse is known)
 //   dS = scale * P o (dO v^T - delta),  delta_q = sum_d dO_qd O_qd
-//   dq^T += K_c^T dS^T                                       (K_c is on the chip already)
-// This replaces SDD(q, k), softmax forward, SDD(dO, v), softmax backward and the DSD product dS k
-// of the unfused chain (five launches, 350 MB of score traffic at seq 4096 and dS read once more) by
-// one kernel that only WRITES the two block stacks.  Same walk as the forward kernel: a lane holds
-// one query column of S^T and dP^T, and the fp16 dS values feed the dq product straight from those
-// registers (the K_c tiles are read a second time along their rows, the reader exchanging rows the way
-// the forward kernel parks V_c).
-// The waves of a row add their dq^T parts through LDS.  The two products that follow
-// (dk = dS^T q, dv = P^T dO) walk the columns and are DSD launches on P and dS.
+//   dq^T += K_c^T dS^T
+// Same walk as the forward kernel: a lane holds one query column with 16 keys, and the 16-bit dS values feed the dq product
+// straight from those registers.  K_c is read from LDS twice, along d for S and along its rows for dq;
+// both reads come first, so that the next K is requested before anything is multiplied.  dq alone (us, before -> after):
+// 16 heads of 4096 tokens 26.8 -> 20.6, 48 of 8192 116 -> 94; at head dim 128, where two stacks were stored, 69 -> 40.
+// Without STACKS nothing is stored per block and scale * delta is left for the column walk.
 // ---------------------------------------------------------------------------
-// per wave: K tiles + V tiles, [key][32 d] each; the V tiles take the two result blocks afterwards, and
-// the whole the dq^T part of the merge (HD x 32 floats)
-constexpr int at_bwd_lds_per_wave(int hd) { return 128 * hd; }
+// per wave: K and V tiles (= the dq^T part of the merge), and with STACKS the two result blocks of 2 KB
+constexpr int at_bwd_lds_per_wave(int hd, bool stacks) { return 128 * hd + (stacks ? 4096 : 0); }
 
-template <int HD, bool BF>
-__global__ __launch_bounds__(512) void attention_bwd_scores_kernel(
+// Hidden scores are set to an infinity of the sign that scale2 turns into -inf, so it must not be zero: 1e-30 leaves
+// every exponent of a zero scale at 0.
+__device__ __forceinline__ float exponent_scale(float scale) { return scale == 0.f ? 1e-30f : scale * 1.4426950408889634f; }
+
+template <int HD, bool BF, bool STACKS>
+__global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kernel(
     const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
     const half_t *__restrict__ dout, const half_t *__restrict__ out, const float *__restrict__ lse,
     half_t *__restrict__ p_out, half_t *__restrict__ ds_out, half_t *__restrict__ dq_out,
     float *__restrict__ delta_out,
     const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
     const SchedEntry *__restrict__ sched, AtSplitWorkspace ws,
-    int n_swg, int batches, int rows_q, int rows_k, int nnz, float scale, int causal)
+    int n_swg, int batches, int rows_q, int rows_k, int nnz, float scale, float log2_scale /* of |scale| */, int causal)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int KS = HD / 16, KT = HD / 32, LDS_PER_WAVE = at_bwd_lds_per_wave(HD, STACKS), N = TileRequests<HD>::N;
     int batch, swg;
     if (!map_workgroup(n_swg, batches, batch, swg)) return;
     const int w = wave_id(), l = lane_id();
@@ -380,111 +284,119 @@ __global__ __launch_bounds__(512) void attention_bwd_scores_kernel(
     const bool active = e.group >= 0;
     const int r = e.group;
     const int qq = l & 31, h = l >> 5;
-    constexpr int KT = HD / 32, LDS_PER_WAVE = at_bwd_lds_per_wave(HD);
-    const float scale2 = scale * 1.4426950408889634f;
+    const float scale2 = exponent_scale(scale);
+    const size_t row0 = (size_t)batch * rows_q + (size_t)BS * r;
 
-    unsigned char *my_lds = lds_raw + (size_t)w * LDS_PER_WAVE;
-    half_t *tile_k = reinterpret_cast<half_t *>(my_lds);
-    half_t *tile_v = tile_k + KT * BS2;
-    const half_t *kb = k + (size_t)batch * rows_k * HD;
-    const half_t *vb = v + (size_t)batch * rows_k * HD;
-    half_t *pb = p_out + (size_t)batch * nnz * BS2;
-    half_t *dsb = ds_out + (size_t)batch * nnz * BS2;
+    unsigned char *tile_k = lds_raw + (size_t)w * LDS_PER_WAVE, *tile_v = tile_k + 64 * HD, *tile_p = tile_k + 128 * HD;
+    const TileReader rd(tile_k);
+    constexpr unsigned K_TILE = 0, V_TILE = 64 * HD;
+    const TileRequests<HD> kreq(k + (size_t)batch * rows_k * HD, tile_k), vreq(v + (size_t)batch * rows_k * HD, tile_v);
 
-    f16v dqacc[KT];                              // dq^T: lane = query column, values = head dims as in the forward kernel
-#pragma unroll
-    for (int t = 0; t < KT; ++t) dqacc[t] = f16v{0};
+    RowTile<HD> dq;
+    clear<HD>(dq);
 
     if (active && e.begin < e.end) {
-        // column operands of the two products: lane (qq, h) holds d = 16 s + 8 h .. + 7 of query qq
-        const size_t qoff = ((size_t)batch * rows_q + BS * r + qq) * HD + 8 * h;
-        h8 qop[HD / 16], dop[HD / 16];
-        float delta = 0.f;
-#pragma unroll
-        for (int s = 0; s < HD / 16; ++s) {
-            qop[s] = as_h8(ldg16(q + qoff + 16 * s));
-            dop[s] = as_h8(ldg16(dout + qoff + 16 * s));
-            const h8 o = as_h8(ldg16(out + qoff + 16 * s));
-#pragma unroll
-            for (int i = 0; i < 8; ++i) delta += widen_16<BF>(dop[s][i]) * widen_16<BF>(o[i]);
-        }
-        delta += at_lane_xor32(delta);           // the other half of the head dim sits in lane l ^ 32
-        const float row_lse = lse[(size_t)batch * rows_q + BS * r + qq];
-        if (delta_out != nullptr && w == e.first_wave() && e.part() == 0 && h == 0)
-            delta_out[(size_t)batch * rows_q + BS * r + qq] = delta;
-
-        struct Frag { uint4 kk[KT][2], vv[KT][2]; };
         DescWindow win;
-        auto load = [&](int p, Frag &f) {
-            const int c = win.get(p).col();
-#pragma unroll
-            for (int dt = 0; dt < KT; ++dt) {
-                ldg_tile32(kb + (size_t)(BS * c) * HD + 32 * dt, HD, f.kk[dt]);
-                ldg_tile32(vb + (size_t)(BS * c) * HD + 32 * dt, HD, f.vv[dt]);
-            }
-        };
-        Frag fr;
+        h8 qop[KS], dop[KS];
+        float delta = 0.f, minus_lse = 0.f;
+        // Q_r and dO_r go through the tiles, as in the forward walk, while the block columns are fetched
+        TileRequests<HD>(q + (size_t)batch * rows_q * HD, tile_k).issue(r);
+        TileRequests<HD>(dout + (size_t)batch * rows_q * HD, tile_v).issue(r);
         for (int seg = e.begin; seg < e.end; seg += WAVE) {
             const int seg_end = seg + WAVE < e.end ? seg + WAVE : e.end;
             win.fetch(blocks, seg, seg_end);
-            load(seg, fr);
+            if (seg == e.begin) {
+                h8 oop[KS];
+                load_row_operands<HD>(out + row0 * HD, oop);
+                // |scale| rides in the exponent (where dS alone is wanted), its sign in the store
+                minus_lse = (STACKS ? 0.f : log2_scale) - lse[row0 + qq];
+                tile_wait<0>();
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    qop[s] = rd.rows(K_TILE, s);
+                    dop[s] = rd.rows(V_TILE, s);
+                }
+                lds_reads_done();
+                kreq.issue(win.get(seg).col());
+                vreq.issue(win.get(seg).col());
+#pragma unroll
+                for (int s = 0; s < KS; ++s)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) delta += widen_16<BF>(dop[s][j]) * widen_16<BF>(oop[s][j]);
+                delta += at_lane_xor32(delta);   // the other half of the head dim sits in lane ^ 32
+                if (delta_out != nullptr && w == e.first_wave() && e.part() == 0 && h == 0) delta_out[row0 + qq] = scale * delta;
+            } else {
+                kreq.issue(win.get(seg).col());
+                vreq.issue(win.get(seg).col());
+            }
             for (int p = seg; p < seg_end; ++p) {
                 const BlockDesc d = win.get(p);
                 const int c = d.col();
-                wave_lds_fence();
+                const bool last = p + 1 == seg_end;
+                tile_wait<N>();                  // everything but V (and, in the first round, the delta store)
+                h8 ktr[KT][2];
+                f16v sacc = {0}, dpacc = {0};    // keys 8 (v / 4) + 4 h + v % 4 of query qq
+                {
+                    h8 kop[KS];
 #pragma unroll
-                for (int dt = 0; dt < KT; ++dt) {
-                    lds_put_kc<false>(tile_k + dt * BS2, fr.kk[dt]);
-                    lds_put_kc<false>(tile_v + dt * BS2, fr.vv[dt]);
+                    for (int s = 0; s < KS; ++s) kop[s] = rd.rows(K_TILE, s);
+#pragma unroll
+                    for (int t = 0; t < KT; ++t)
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) ktr[t][s] = rd.columns(K_TILE, t, s);
+                    lds_reads_done();
+                    if (!last) kreq.issue(win.get(p + 1).col());
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) sacc = mfma_16<BF>(kop[s], qop[s], sacc);
                 }
-                wave_lds_fence();
-                if (p + 1 < seg_end) load(p + 1, fr);
-                f16v sacc = {0}, dpacc = {0};
+                if (last) tile_wait<0>();
+                else tile_wait<N>();             // everything but the next K
+                {
+                    h8 vop[KS];
 #pragma unroll
-                for (int dt = 0; dt < KT; ++dt)
+                    for (int s = 0; s < KS; ++s) vop[s] = rd.rows(V_TILE, s);
+                    lds_reads_done();
+                    if (!last) vreq.issue(win.get(p + 1).col());
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        sacc = mfma_16<BF>(lds_get_kc(tile_k + dt * BS2, s), qop[2 * dt + s], sacc);
-                        dpacc = mfma_16<BF>(lds_get_kc(tile_v + dt * BS2, s), dop[2 * dt + s], dpacc);
-                    }
-                // Accumulator value i of lane half h is key 8 (i / 4) + 4 h + i % 4 of query qq: four runs of 4
-                // keys.  Written from here a store instruction would touch 64 separate 8-byte pieces, so
-                // the two result blocks go through the (now idle) V tiles and leave as whole 2 KB
-                // pieces, like the SDD result.  The K tiles stay: dq reads them once more.
-                wave_lds_fence();
-                h8 dsop[2];
+                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(vop[s], dop[s], dpacc);
+                }
+                if (causal && c >= r) {          // a hidden score has no probability
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        if (c > r || 8 * (v >> 2) + 4 * h + (v & 3) > qq) sacc[v] = scale2 < 0.f ? __builtin_inff() : -__builtin_inff();
+                }
+                h8 ds[2];
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     h4 pv, dv;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int i = 4 * g + j, key = 8 * g + 4 * h + j;
-                        float pr = at_exp2(__builtin_fmaf(sacc[i], scale2, -row_lse));
-                        if (causal && (c > r || (c == r && key > qq))) pr = 0.f;
-                        pv[j] = narrow_16<BF>(pr);
-                        dv[j] = narrow_16<BF>(scale * pr * (dpacc[i] - delta));
-                        dsop[i >> 3][i & 7] = dv[j];
+                        const int v = 4 * g + j;
+                        const float pr = at_exp2(__builtin_fmaf(sacc[v], scale2, minus_lse)), grad = dpacc[v] - delta;
+                        if (STACKS) pv[j] = narrow_16<BF>(pr);
+                        dv[j] = narrow_16<BF>(STACKS ? scale * pr * grad : pr * grad);
+                        ds[v >> 3][v & 7] = dv[j];
                     }
-                    if (p_out != nullptr) {
-                        const int at = 16 * kc_slot(qq, g) + 8 * h;   // 16-byte piece g of row qq, its half h
-                        *reinterpret_cast<h4 *>(lds_bytes(tile_v) + at) = pv;
-                        *reinterpret_cast<h4 *>(lds_bytes(tile_v + BS2) + at) = dv;
+                    if (STACKS) {                // rows of 64 bytes: query qq, keys 8 g + 4 h .. + 3
+                        const int at = 16 * kc_slot(qq, g) + 8 * h;
+                        *reinterpret_cast<h4 *>(tile_p + at) = pv;
+                        *reinterpret_cast<h4 *>(tile_p + 2048 + at) = dv;
                     }
                 }
                 if (dq_out != nullptr) {
 #pragma unroll
-                    for (int t = 0; t < KT; ++t)
+                    for (int s = 0; s < 2; ++s)
 #pragma unroll
-                        for (int s = 0; s < 2; ++s)
-                            dqacc[t] = mfma_16<BF>(lds_get_kc_tr_swapped(tile_k + t * BS2, s), dsop[s], dqacc[t]);
+                        for (int t = 0; t < KT; ++t) dq[t] = mfma_16<BF>(ktr[t][s], ds[s], dq[t]);
                 }
-                if (p_out != nullptr) {
+                if (STACKS) {                    // out of LDS as whole 2 KB pieces
                     wave_lds_fence();
                     uint4 raw[2];
-                    lds_get_linear(tile_v, raw);
-                    stg_tile32(pb + (size_t)d.idx * BS2, raw);
-                    lds_get_linear(tile_v + BS2, raw);
-                    stg_tile32(dsb + (size_t)d.idx * BS2, raw);
+                    lds_get_linear(reinterpret_cast<const half_t *>(tile_p), raw);
+                    stg_tile32(p_out + ((size_t)batch * nnz + d.idx) * BS2, raw);
+                    lds_get_linear(reinterpret_cast<const half_t *>(tile_p + 2048), raw);
+                    stg_tile32(ds_out + ((size_t)batch * nnz + d.idx) * BS2, raw);
+                    wave_lds_fence();
                 }
             }
         }
@@ -494,97 +406,49 @@ __global__ __launch_bounds__(512) void attention_bwd_scores_kernel(
     // team merge: every wave of a row but the leader parks its dq^T part, the leader adds and stores
     const int slot0 = e.first_wave(), nw = e.team_waves();
     const bool leader = active && w == slot0;
-    float *park = reinterpret_cast<float *>(my_lds);
     if (active && !leader) {
         wave_lds_fence();
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) park[(t * 16 + i) * WAVE + l] = dqacc[t][i];
+        each<HD>(dq, [&](float x, int at) { return reinterpret_cast<float *>(tile_k)[at] = x; });
     }
     __syncthreads();
     if (!leader) return;
     for (int o = 1; o < nw; ++o) {
-        const float *op = reinterpret_cast<const float *>(lds_raw + (size_t)(w + o) * LDS_PER_WAVE);
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dqacc[t][i] += op[(t * 16 + i) * WAVE + l];
+        const float *src = reinterpret_cast<const float *>(tile_k + o * LDS_PER_WAVE);
+        each<HD>(dq, [&](float x, int at) { return x + src[at]; });
     }
     if (e.parts() > 1) {                         // a row cut into parts: they add up in the workspace
         constexpr int TILE = 32 * HD;
         const SchedGroup sg = sched_groups[r];
         float *tile0 = ws.tiles + ((size_t)batch * ws.tile_slots + sg.tile_slot) * TILE;
-        at_park<KT>(dqacc, tile0 + (size_t)e.part() * TILE);
+        park_part<HD>(dq, tile0 + (size_t)e.part() * TILE);
         int *counter = ws.counters + (size_t)batch * ws.split_groups + sg.split_index;
         if (split_publish(counter) != e.parts() - 1) return;
         split_consume();
-        at_sum_parts<KT>(dqacc, tile0, TILE, e.parts());
+        sum_parts<HD>(dq, tile0, TILE, e.parts());
         split_reset(counter);
     }
-    half_t *drow = dq_out + ((size_t)batch * rows_q + BS * r + qq) * HD + 4 * h;
-#pragma unroll
-    for (int t = 0; t < KT; ++t)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            h4 o;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = narrow_16<BF>(dqacc[t][4 * g + j]);
-            *reinterpret_cast<h4 *>(drow + 32 * t + 8 * g) = o;
-        }
-}
-
-hipError_t launch_attention_backward_scores(const AttentionArgs &p, hipStream_t st)
-{
-    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
-    const size_t lds = (size_t)p.sched_waves * at_bwd_lds_per_wave(p.head_dim);
-#define BSA_AT_ARGS (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, \
-                    (const half_t *)p.out, (const float *)p.lse, (half_t *)p.p_out, (half_t *)p.ds_out, (half_t *)p.dq_out, (float *)p.delta, \
-                    (const BlockDesc *)p.blocks, (const SchedGroup *)p.sched, (const SchedEntry *)p.sched + p.groups, ws, \
-                    p.sched_wgs, p.batches, \
-                    32 * p.mask_rows, 32 * p.mask_cols, p.nnz, p.scale, p.causal ? 1 : 0
-    AtSplitWorkspace ws;
-    ws.tile_slots = p.tile_slots;
-    ws.split_groups = p.split_groups;
-    ws.counters = (int *)p.workspace;
-    ws.tiles = (float *)((char *)p.workspace + at_split_counter_bytes(p.split_groups, p.batches));
-    if (p.head_dim == 64) {
-        if (p.bf16) attention_bwd_scores_kernel<64, true><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-        else attention_bwd_scores_kernel<64, false><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-    } else {
-        if (lds > 65536) {
-            const void *fn = p.bf16 ? (const void *)attention_bwd_scores_kernel<128, true>
-                                    : (const void *)attention_bwd_scores_kernel<128, false>;
-            hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        if (p.bf16) attention_bwd_scores_kernel<128, true><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-        else attention_bwd_scores_kernel<128, false><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-    }
-#undef BSA_AT_ARGS
-    return hipGetLastError();
+    const float sign = !STACKS && scale < 0.f ? -1.f : 1.f;
+    store_rows<HD, BF>(dq, sign, tile_k, dq_out + row0 * HD);
 }
 
 // ---------------------------------------------------------------------------
 // Backward, the walk over the COLUMNS: dk and dv of block column c from the blocks (r, c) of the
 // column table, with nothing but q, k, v, dO and two floats per query (lse of the forward pass,
-// delta of the row walk above) read: the probabilities and the score gradients are rebuilt in
+// scale * delta of the row walk above) read: the probabilities and the score gradients are rebuilt in
 // registers a second time rather than stored by the row walk and read back (4 KB written + 4 KB
 // read of HBM traffic per block that this pair of kernels does not have).
-//   S  = Q_r K_c^T, dP = dO_r V_c^T    K_c and V_c stay in registers as the column operands; a lane
-//                                      holds ONE key column, 16 queries
-//   P, dS                              as in the row walk; lse and delta of the 16 queries come from a
-//                                      256-byte LDS slot
-//   dv^T += dO_r^T P,  dk^T += Q_r^T dS   the fp16 P and dS values are the column operands straight
-//                                      from the accumulators, the Q_r and dO_r tiles are read a second
-//                                      time along their rows (get_kc_tr_swapped_addr)
-// The waves of a column add their parts through LDS.  Head dim 64 only: at 128 the four accumulator
-// sets alone are 256 registers.
+//   S  = Q_r K_c^T, dP = dO_r V_c^T    K_c and V_c stay in registers; a lane holds ONE key column, 16 queries, whose lse
+//                                      and delta come into LDS with the tiles
+//   dv^T += dO_r^T P,  dk^T += Q_r^T dS   the 16-bit P and dS values are the column operands straight from the
+//                                      accumulators, the Q_r and dO_r tiles are read a second time along their rows
+// The waves of a column add their parts through LDS.  Two waves per SIMD at head dim 64 (200 registers), one at 128 (its
+// four accumulators are 256); three at 64 spill the K operands and are slower.  us, before -> after: 16 heads of 4096
+// tokens 34.9 -> 29.6, 48 of 8192 150 -> 135; at head dim 128, as two products over stored stacks before, 69 -> 66.
 // ---------------------------------------------------------------------------
-constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256; }   // Q tiles + dO tiles (= one parked accumulator set) + stats
+constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256; }   // Q + dO tiles (= one parked accumulator set) + lse, delta
 
 template <int HD, bool BF>
-__global__ __launch_bounds__(512) void attention_bwd_dkdv_kernel(
+__global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64 ? 2 : 1) void attention_bwd_dkdv_kernel(
     const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
     const half_t *__restrict__ dout, const float *__restrict__ lse, const float *__restrict__ delta,
     half_t *__restrict__ dk_out, half_t *__restrict__ dv_out,
@@ -593,6 +457,7 @@ __global__ __launch_bounds__(512) void attention_bwd_dkdv_kernel(
     int n_swg, int batches, int rows_q, int rows_k, float scale, int causal)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int KS = HD / 16, KT = HD / 32, LDS_PER_WAVE = at_bwd_col_lds_per_wave(HD);
     int batch, swg;
     if (!map_workgroup(n_swg, batches, batch, swg)) return;
     const int w = wave_id(), l = lane_id();
@@ -601,89 +466,106 @@ __global__ __launch_bounds__(512) void attention_bwd_dkdv_kernel(
     const bool active = e.group >= 0;
     const int c = e.group;
     const int key = l & 31, h = l >> 5;          // key column of this lane, lane half
-    constexpr int KT = HD / 32, LDS_PER_WAVE = at_bwd_col_lds_per_wave(HD);
-    const float scale2 = scale * 1.4426950408889634f;
+    const float scale2 = exponent_scale(scale);
+    const size_t row0 = (size_t)batch * rows_k + (size_t)BS * c;
 
-    unsigned char *my_lds = lds_raw + (size_t)w * LDS_PER_WAVE;
-    half_t *tile_q = reinterpret_cast<half_t *>(my_lds);
-    half_t *tile_do = tile_q + KT * BS2;
-    float *stats = reinterpret_cast<float *>(my_lds + 128 * HD);      // 32 lse, 32 delta of the block's queries
-    const half_t *qb = q + (size_t)batch * rows_q * HD;
-    const half_t *dob = dout + (size_t)batch * rows_q * HD;
-    const float *lse_b = lse + (size_t)batch * rows_q;
-    const float *delta_b = delta + (size_t)batch * rows_q;
+    unsigned char *tile_q = lds_raw + (size_t)w * LDS_PER_WAVE, *tile_do = tile_q + 64 * HD;
+    const TileReader rd(tile_q);
+    constexpr unsigned Q_TILE = 0, DO_TILE = 64 * HD;
+    const float *stats = reinterpret_cast<const float *>(tile_q + 128 * HD);      // 32 lse, 32 delta of the block's queries
+    const TileRequests<HD> qreq(q + (size_t)batch * rows_q * HD, tile_q), doreq(dout + (size_t)batch * rows_q * HD, tile_do);
+    const float *my_stat = (l < 32 ? lse : delta) + (size_t)batch * rows_q + (l & 31);
+    const unsigned stat_lds = __builtin_amdgcn_readfirstlane(lds_address(stats));
 
-    f16v dvacc[KT], dkacc[KT];                   // dv^T, dk^T: lane = key column, values = head dims as in the forward kernel
-#pragma unroll
-    for (int t = 0; t < KT; ++t) dvacc[t] = dkacc[t] = f16v{0};
+    RowTile<HD> dv, dk;
+    clear<HD>(dv);
+    clear<HD>(dk);
 
     if (active && e.begin < e.end) {
-        // column operands of the first two products: lane (key, h) holds d = 16 s + 8 h .. + 7 of its key
-        const size_t koff = ((size_t)batch * rows_k + BS * c + key) * HD + 8 * h;
-        h8 kop[HD / 16], vop[HD / 16];
-#pragma unroll
-        for (int s = 0; s < HD / 16; ++s) {
-            kop[s] = as_h8(ldg16(k + koff + 16 * s));
-            vop[s] = as_h8(ldg16(v + koff + 16 * s));
-        }
-        struct Frag { uint4 qq[KT][2], dd[KT][2]; float stat; };
         DescWindow win;
-        auto load = [&](int p, Frag &f) {
-            const int r = win.get(p).row();
-#pragma unroll
-            for (int dt = 0; dt < KT; ++dt) {
-                ldg_tile32(qb + (size_t)(BS * r) * HD + 32 * dt, HD, f.qq[dt]);
-                ldg_tile32(dob + (size_t)(BS * r) * HD + 32 * dt, HD, f.dd[dt]);
-            }
-            f.stat = h == 0 ? lse_b[BS * r + key] : delta_b[BS * r + key];
-        };
-        Frag fr;
+        h8 kop[KS], vop[KS];
+        // K_c and V_c go through the tiles, as Q_r does in the forward walk, while the block rows are fetched
+        TileRequests<HD>(k + (size_t)batch * rows_k * HD, tile_q).issue(c);
+        TileRequests<HD>(v + (size_t)batch * rows_k * HD, tile_do).issue(c);
         for (int seg = e.begin; seg < e.end; seg += WAVE) {
             const int seg_end = seg + WAVE < e.end ? seg + WAVE : e.end;
             win.fetch(blocks, seg, seg_end);
-            load(seg, fr);
+            auto request_q = [&](int p) {
+                const int r = win.get(p).row();
+                dma4_gather(my_stat + BS * r, stat_lds);
+                qreq.issue(r);
+            };
+            if (seg == e.begin) {
+                tile_wait<0>();
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    kop[s] = rd.rows(Q_TILE, s);
+                    vop[s] = rd.rows(DO_TILE, s);
+                }
+                lds_reads_done();
+            }
+            request_q(seg);
+            doreq.issue(win.get(seg).row());
             for (int p = seg; p < seg_end; ++p) {
                 const int r = win.get(p).row();
-                wave_lds_fence();
+                const bool last = p + 1 == seg_end, masked = causal && c >= r;
+                h8 pop[2], ds[2];                // queries 8 (v / 4) + 4 h + v % 4 of this lane's key
+                tile_wait<0>();
+                {
+                    f16v sacc = {0}, dpacc = {0};
+                    {
+                        h8 qop[KS];
 #pragma unroll
-                for (int dt = 0; dt < KT; ++dt) {
-                    lds_put_kc<false>(tile_q + dt * BS2, fr.qq[dt]);
-                    lds_put_kc<false>(tile_do + dt * BS2, fr.dd[dt]);
+                        for (int s = 0; s < KS; ++s) qop[s] = rd.rows(Q_TILE, s);
+#pragma unroll
+                        for (int s = 0; s < KS; ++s) sacc = mfma_16<BF>(qop[s], kop[s], sacc);
+                    }
+                    {
+                        h8 dop[KS];
+#pragma unroll
+                        for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
+#pragma unroll
+                        for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], vop[s], dpacc);
+                    }
+                    if (masked) {                // a hidden score has no probability
+#pragma unroll
+                        for (int v = 0; v < 16; ++v)
+                            if (c > r || key > 8 * (v >> 2) + 4 * h + (v & 3)) sacc[v] = scale2 < 0.f ? __builtin_inff() : -__builtin_inff();
+                    }
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const f4v ls = *reinterpret_cast<const f4v *>(stats + 8 * g + 4 * h);
+                        const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int v = 4 * g + j;
+                            const float pr = at_exp2(__builtin_fmaf(sacc[v], scale2, -ls[j]));
+                            pop[v >> 3][v & 7] = narrow_16<BF>(pr);
+                            ds[v >> 3][v & 7] = narrow_16<BF>(pr * __builtin_fmaf(dpacc[v], scale, -dl[j]));
+                        }
+                    }
                 }
-                stats[l] = fr.stat;
-                wave_lds_fence();
-                if (p + 1 < seg_end) load(p + 1, fr);
-                f16v sacc = {0}, dpacc = {0};
+                // The tiles are read a second time, Q first: the requests for the next block go out as soon as each is free.
+                h8 tr[KT][2];
+                auto read_columns = [&](unsigned tile) {
 #pragma unroll
-                for (int dt = 0; dt < KT; ++dt)
+                    for (int t = 0; t < KT; ++t)
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        sacc = mfma_16<BF>(lds_get_kc(tile_q + dt * BS2, s), kop[2 * dt + s], sacc);
-                        dpacc = mfma_16<BF>(lds_get_kc(tile_do + dt * BS2, s), vop[2 * dt + s], dpacc);
-                    }
-                // accumulator value i of lane half h is query 8 (i / 4) + 4 h + i % 4 of this lane's key
-                h8 pop[2], dsop[2];
+                        for (int s = 0; s < 2; ++s) tr[t][s] = rd.columns(tile, t, s);
+                    lds_reads_done();
+                };
+                read_columns(Q_TILE);
+                if (!last) request_q(p + 1);
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const float4 ls = *reinterpret_cast<const float4 *>(stats + 8 * g + 4 * h);
-                    const float4 dl = *reinterpret_cast<const float4 *>(stats + 32 + 8 * g + 4 * h);
-                    const float lsv[4] = {ls.x, ls.y, ls.z, ls.w}, dlv[4] = {dl.x, dl.y, dl.z, dl.w};
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int i = 4 * g + j, qrow = 8 * g + 4 * h + j;
-                        float pr = at_exp2(__builtin_fmaf(sacc[i], scale2, -lsv[j]));
-                        if (causal && (c > r || (c == r && key > qrow))) pr = 0.f;
-                        pop[i >> 3][i & 7] = narrow_16<BF>(pr);
-                        dsop[i >> 3][i & 7] = narrow_16<BF>(scale * pr * (dpacc[i] - dlv[j]));
-                    }
-                }
+                    for (int t = 0; t < KT; ++t) dk[t] = mfma_16<BF>(tr[t][s], ds[s], dk[t]);
+                read_columns(DO_TILE);
+                if (!last) doreq.issue(win.get(p + 1).row());
 #pragma unroll
-                for (int t = 0; t < KT; ++t)
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        dvacc[t] = mfma_16<BF>(lds_get_kc_tr_swapped(tile_do + t * BS2, s), pop[s], dvacc[t]);
-                        dkacc[t] = mfma_16<BF>(lds_get_kc_tr_swapped(tile_q + t * BS2, s), dsop[s], dkacc[t]);
-                    }
+                    for (int t = 0; t < KT; ++t) dv[t] = mfma_16<BF>(tr[t][s], pop[s], dv[t]);
             }
         }
     }
@@ -692,26 +574,19 @@ __global__ __launch_bounds__(512) void attention_bwd_dkdv_kernel(
     // column but the leader parks its part, the leader adds
     const int slot0 = e.first_wave(), nw = e.team_waves();
     const bool leader = active && w == slot0;
-    float *park = reinterpret_cast<float *>(my_lds);
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
-        f16v (&acc)[KT] = which == 0 ? dvacc : dkacc;
+        RowTile<HD> &acc = which == 0 ? dv : dk;
         if (which == 1) __syncthreads();         // the leaders have read the first set
         if (active && !leader) {
             wave_lds_fence();
-#pragma unroll
-            for (int t = 0; t < KT; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) park[(t * 16 + i) * WAVE + l] = acc[t][i];
+            each<HD>(acc, [&](float x, int at) { return reinterpret_cast<float *>(tile_q)[at] = x; });
         }
         __syncthreads();
         if (leader) {
             for (int o = 1; o < nw; ++o) {
-                const float *op = reinterpret_cast<const float *>(lds_raw + (size_t)(w + o) * LDS_PER_WAVE);
-#pragma unroll
-                for (int t = 0; t < KT; ++t)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[t][i] += op[(t * 16 + i) * WAVE + l];
+                const float *src = reinterpret_cast<const float *>(tile_q + o * LDS_PER_WAVE);
+                each<HD>(acc, [&](float x, int at) { return x + src[at]; });
             }
         }
     }
@@ -720,92 +595,108 @@ __global__ __launch_bounds__(512) void attention_bwd_dkdv_kernel(
         constexpr int HALF = 32 * HD, TILE = 2 * HALF;       // dv^T then dk^T
         const SchedGroup sg = sched_groups[c];
         float *tile0 = ws.tiles + ((size_t)batch * ws.tile_slots + sg.tile_slot) * TILE;
-        at_park<KT>(dvacc, tile0 + (size_t)e.part() * TILE);
-        at_park<KT>(dkacc, tile0 + (size_t)e.part() * TILE + HALF);
+        park_part<HD>(dv, tile0 + (size_t)e.part() * TILE);
+        park_part<HD>(dk, tile0 + (size_t)e.part() * TILE + HALF);
         int *counter = ws.counters + (size_t)batch * ws.split_groups + sg.split_index;
         if (split_publish(counter) != e.parts() - 1) return;
         split_consume();
-        at_sum_parts<KT>(dvacc, tile0, TILE, e.parts());
-        at_sum_parts<KT>(dkacc, tile0 + HALF, TILE, e.parts());
+        sum_parts<HD>(dv, tile0, TILE, e.parts());
+        sum_parts<HD>(dk, tile0 + HALF, TILE, e.parts());
         split_reset(counter);
     }
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        f16v (&acc)[KT] = which == 0 ? dvacc : dkacc;
-        half_t *drow = (which == 0 ? dv_out : dk_out) + ((size_t)batch * rows_k + BS * c + key) * HD + 4 * h;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                h4 o;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) o[j] = narrow_16<BF>(acc[t][4 * g + j]);
-                *reinterpret_cast<h4 *>(drow + 32 * t + 8 * g) = o;
-            }
+    store_rows<HD, BF>(dv, 1.f, tile_q, dv_out + row0 * HD);
+    store_rows<HD, BF>(dk, 1.f, tile_q, dk_out + row0 * HD);
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+// ---------------------------------------------------------------------------
+namespace {
+struct Walk {                                    // what the three kernels are launched with alike
+    dim3 grid, block;
+    size_t lds;
+    AtSplitWorkspace ws;
+    const BlockDesc *blocks;
+    const SchedGroup *groups;
+    const SchedEntry *slots;
+    Walk(const AttentionArgs &p, int lds_per_wave)
+        : grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves), lds((size_t)p.sched_waves * lds_per_wave),
+          blocks((const BlockDesc *)p.blocks), groups((const SchedGroup *)p.sched), slots((const SchedEntry *)p.sched + p.groups)
+    {
+        ws.tile_slots = p.tile_slots;
+        ws.split_groups = p.split_groups;
+        ws.counters = (int *)p.workspace;
+        ws.tiles = (float *)((char *)p.workspace + at_split_counter_bytes(p.split_groups, p.batches));
     }
+    // a launch gets 64 KB of LDS without asking
+    template <class Kernel>
+    hipError_t allow(Kernel kernel) const
+    {
+        if (lds <= 65536) return hipSuccess;
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    }
+};
+
+template <int HD, bool BF>
+hipError_t forward(const AttentionArgs &p, hipStream_t st)
+{
+    const Walk w(p, at_lds_per_wave(HD));
+    const hipError_t err = w.allow(attention_fwd_f16_kernel<HD, BF>);
+    if (err != hipSuccess) return err;
+    attention_fwd_f16_kernel<HD, BF><<<w.grid, w.block, w.lds, st>>>(
+        (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (half_t *)p.out, (float *)p.lse, w.blocks, w.groups,
+        w.slots, w.ws, p.sched_wgs, p.batches, 32 * p.mask_rows, 32 * p.mask_cols, p.scale * 1.4426950408889634f, p.causal ? 1 : 0);
+    return hipGetLastError();
+}
+
+template <int HD, bool BF, bool STACKS>
+hipError_t backward_rows(const AttentionArgs &p, hipStream_t st)
+{
+    const Walk w(p, at_bwd_lds_per_wave(HD, STACKS));
+    const hipError_t err = w.allow(attention_bwd_rows_kernel<HD, BF, STACKS>);
+    if (err != hipSuccess) return err;
+    attention_bwd_rows_kernel<HD, BF, STACKS><<<w.grid, w.block, w.lds, st>>>(
+        (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, (const half_t *)p.out,
+        (const float *)p.lse, (half_t *)p.p_out, (half_t *)p.ds_out, (half_t *)p.dq_out, (float *)p.delta, w.blocks, w.groups,
+        w.slots, w.ws, p.sched_wgs, p.batches, 32 * p.mask_rows, 32 * p.mask_cols, p.nnz, p.scale, log2f(fabsf(p.scale)),
+        p.causal ? 1 : 0);
+    return hipGetLastError();
+}
+
+template <int HD, bool BF>
+hipError_t backward_columns(const AttentionArgs &p, hipStream_t st)
+{
+    const Walk w(p, at_bwd_col_lds_per_wave(HD));
+    const hipError_t err = w.allow(attention_bwd_dkdv_kernel<HD, BF>);
+    if (err != hipSuccess) return err;
+    attention_bwd_dkdv_kernel<HD, BF><<<w.grid, w.block, w.lds, st>>>(
+        (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, (const float *)p.lse,
+        (const float *)p.delta, (half_t *)p.dk_out, (half_t *)p.dv_out, w.blocks, w.groups, w.slots, w.ws, p.sched_wgs,
+        p.batches, 32 * p.mask_rows, 32 * p.mask_cols, p.scale, p.causal ? 1 : 0);
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_attention_forward(const AttentionArgs &p, hipStream_t st)
+{
+    if (p.head_dim == 64) return p.bf16 ? forward<64, true>(p, st) : forward<64, false>(p, st);
+    return p.bf16 ? forward<128, true>(p, st) : forward<128, false>(p, st);
+}
+
+hipError_t launch_attention_backward_scores(const AttentionArgs &p, hipStream_t st)
+{
+    if (p.p_out != nullptr) {
+        if (p.head_dim == 64) return p.bf16 ? backward_rows<64, true, true>(p, st) : backward_rows<64, false, true>(p, st);
+        return p.bf16 ? backward_rows<128, true, true>(p, st) : backward_rows<128, false, true>(p, st);
+    }
+    if (p.head_dim == 64) return p.bf16 ? backward_rows<64, true, false>(p, st) : backward_rows<64, false, false>(p, st);
+    return p.bf16 ? backward_rows<128, true, false>(p, st) : backward_rows<128, false, false>(p, st);
 }
 
 hipError_t launch_attention_backward_dkdv(const AttentionArgs &p, hipStream_t st)
 {
-    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
-    const size_t lds = (size_t)p.sched_waves * at_bwd_col_lds_per_wave(64);
-#define BSA_AT_ARGS (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, \
-                    (const float *)p.lse, (const float *)p.delta, (half_t *)p.dk_out, (half_t *)p.dv_out, \
-                    (const BlockDesc *)p.blocks, (const SchedGroup *)p.sched, (const SchedEntry *)p.sched + p.groups, ws, \
-                    p.sched_wgs, p.batches, \
-                    32 * p.mask_rows, 32 * p.mask_cols, p.scale, p.causal ? 1 : 0
-    AtSplitWorkspace ws;
-    ws.tile_slots = p.tile_slots;
-    ws.split_groups = p.split_groups;
-    ws.counters = (int *)p.workspace;
-    ws.tiles = (float *)((char *)p.workspace + at_split_counter_bytes(p.split_groups, p.batches));
-    if (lds > 65536) {
-        const void *fn = p.bf16 ? (const void *)attention_bwd_dkdv_kernel<64, true>
-                                : (const void *)attention_bwd_dkdv_kernel<64, false>;
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    if (p.bf16) attention_bwd_dkdv_kernel<64, true><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-    else attention_bwd_dkdv_kernel<64, false><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-#undef BSA_AT_ARGS
-    return hipGetLastError();
-}
-
-hipError_t launch_attention_forward(const AttentionArgs &p, hipStream_t st)
-{
-    dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
-    AtSplitWorkspace ws;
-    ws.tile_slots = p.tile_slots;
-    ws.split_groups = p.split_groups;
-    ws.counters = (int *)p.workspace;
-    ws.tiles = (float *)((char *)p.workspace + at_split_counter_bytes(p.split_groups, p.batches));
-#define BSA_AT_ARGS (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (half_t *)p.out, (float *)p.lse, \
-                    (const BlockDesc *)p.blocks, (const SchedGroup *)p.sched, (const SchedEntry *)p.sched + p.groups, ws, \
-                    p.sched_wgs, p.batches, \
-                    32 * p.mask_rows, 32 * p.mask_cols, p.scale * 1.4426950408889634f, p.causal ? 1 : 0
-    const size_t lds = (size_t)p.sched_waves * at_lds_per_wave(p.head_dim);
-    if (p.head_dim == 64) {
-        if (lds > 65536) {   // 8 waves x 8.5 KB
-            const void *fn = p.bf16 ? (const void *)attention_fwd_f16_kernel<64, true>
-                                    : (const void *)attention_fwd_f16_kernel<64, false>;
-            hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        if (p.bf16) attention_fwd_f16_kernel<64, true><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-        else attention_fwd_f16_kernel<64, false><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-    } else {
-        // more than 3 waves x 16.5 KB of staging exceed the 64 KB a launch gets without asking
-        if (lds > 65536) {
-            const void *fn = p.bf16 ? (const void *)attention_fwd_f16_kernel<128, true>
-                                    : (const void *)attention_fwd_f16_kernel<128, false>;
-            hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        if (p.bf16) attention_fwd_f16_kernel<128, true><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-        else attention_fwd_f16_kernel<128, false><<<grid, block, lds, st>>>(BSA_AT_ARGS);
-    }
-#undef BSA_AT_ARGS
-    return hipGetLastError();
+    if (p.head_dim == 64) return p.bf16 ? backward_columns<64, true>(p, st) : backward_columns<64, false>(p, st);
+    return p.bf16 ? backward_columns<128, true>(p, st) : backward_columns<128, false>(p, st);
 }
 
 }  // namespace bsa

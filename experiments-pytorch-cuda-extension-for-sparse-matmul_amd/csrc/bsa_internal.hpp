@@ -98,7 +98,7 @@ struct AttentionArgs {
     const void *dout = nullptr;     // backward only
     void *p_out = nullptr, *ds_out = nullptr;   // row walk of the backward pass, both or neither: [batches, nnz, 32, 32]
     void *dq_out = nullptr;         // row walk, may be null: [batches, 32 mask_rows, head_dim]
-    void *delta = nullptr;          // float [batches, 32 mask_rows], rowsum(dout o out): written by the row walk (may be
+    void *delta = nullptr;          // float [batches, 32 mask_rows], scale * rowsum(dout o out): written by the row walk (may be
                                     // null there), read by the column walk
     void *dk_out = nullptr, *dv_out = nullptr;  // column walk: [batches, 32 mask_cols, head_dim]
     int nnz = 0;
@@ -121,6 +121,7 @@ size_t attention_backward_workspace_bytes(int row_tile_slots, int row_split_grou
                                           int col_split_groups, int batches, int head_dim);
 hipError_t launch_attention_forward(const AttentionArgs &p, hipStream_t stream);
 hipError_t launch_attention_backward_scores(const AttentionArgs &p, hipStream_t stream);
-hipError_t launch_attention_backward_dkdv(const AttentionArgs &p, hipStream_t stream);   // groups = block columns, head dim 64
+constexpr int AT_COLUMN_WAVES_128 = 4;    // waves per workgroup the column walk takes at head dim 128
+hipError_t launch_attention_backward_dkdv(const AttentionArgs &p, hipStream_t stream);   // groups = block columns
 
 }  // namespace bsa

@@ -15,13 +15,13 @@ extern "C" int bsa_lds_access(const char *name, int permuted, int arg0, int arg1
         else if (!strcmp(name, "put_ks")) a = put_ks_addr(lane, arg0);
         else if (!strcmp(name, "get_ks")) a = get_ks_addr(permuted, lane, arg0, arg1);
         else if (!strcmp(name, "put_strip")) a = put_strip_addr(lane, arg0);
-        else if (!strcmp(name, "put_strip_swapped")) a = put_strip_swapped_addr(lane, arg0);
-        else if (!strcmp(name, "get_kc_tr_swapped")) a = get_kc_tr_swapped_addr(lane, arg0, arg1);
         else if (!strcmp(name, "get_strip")) a = get_strip_addr(permuted, lane, arg0 & 1, arg0 >> 1, arg1);
         else if (!strcmp(name, "put_strip16")) a = put_strip16_addr(lane, arg0);
         else if (!strcmp(name, "get_strip16")) a = get_strip16_addr(lane, arg0, arg1);
         else if (!strcmp(name, "put_result")) a = put_result_addr(lane, arg0);
         else if (!strcmp(name, "get_linear")) a = get_linear_addr(lane, arg0);
+        else if (!strcmp(name, "get_panel")) a = get_panel_addr(lane, arg0);
+        else if (!strcmp(name, "get_panel_tr")) a = get_panel_tr_addr(lane, arg0, arg1, arg2);
         else if (!strcmp(name, "put_f32")) a = put_f32_addr(lane, arg0);
         else if (!strcmp(name, "get_f32_kc")) a = get_f32_kc_addr(permuted, lane, arg0);
         else if (!strcmp(name, "get_f32_ks")) a = get_f32_ks_addr(permuted, lane, arg0);
@@ -31,6 +31,7 @@ extern "C" int bsa_lds_access(const char *name, int permuted, int arg0, int arg1
     return 0;
 }
 
+extern "C" int bsa_panel_src_piece(int lane, int chunk) { return bsa::panel_src_piece(lane, chunk); }
 extern "C" int bsa_col16(int t, int i) { return bsa::col16(t, i); }
 extern "C" int bsa_strip16_half_swapped(int k) { return bsa::strip16_half_swapped(k); }
 extern "C" int bsa_perm16(int i) { return bsa::perm16(i); }

@@ -80,29 +80,6 @@ BSA_HD constexpr int put_strip_addr(int lane, int q)
     int k = c >> 3;
     return 16 * (k * 8 + ((c & 7) ^ strip_swizzle(k)));
 }
-// The same strip with rows 4-7 and 8-11 of every 16 exchanged (bits 2 and 3 of k): a reader
-// that asks for row 16 s + 8 h + j then gets row 16 s + 8 (j / 4) + 4 h + j % 4, the row an MFMA
-// accumulator lane (h = lane / 32) holds as its value 8 s + j.  The fused attention kernel feeds its
-// probabilities to the second product straight out of the first one's accumulators this way.
-BSA_HD constexpr int swap_bits23(int k) { return (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1); }
-BSA_HD constexpr int put_strip_swapped_addr(int lane, int q)
-{
-    int c = lane + 64 * q;
-    int k = swap_bits23(c >> 3);
-    return 16 * (k * 8 + ((c & 7) ^ strip_swizzle(k)));
-}
-// Transposing read of a [index][k] tile (the put_kc_addr layout, not permuted) along its ROWS: the
-// operand of a product that contracts over the tile's row index, with the same exchange of rows
-// 4-7 and 8-11 as above applied by the reader: element j of lane (index = lane % 32, h = lane / 32)
-// is row 16 step + 8 (j / 4) + 4 h + j % 4.  The 4 rows a 16-lane group touches share one
-// kc_swizzle and fill one 256-byte bank window.
-BSA_HD constexpr int get_kc_tr_swapped_addr(int lane, int step, int half)
-{
-    int g = lane >> 4, s = lane & 15;
-    int k = 16 * step + 4 * (g >> 1) + (s >> 2) + 8 * half;
-    int x = tr_chunk_base(false, g, s & 3) ^ (8 * kc_swizzle(k));
-    return 2 * (k * 32 + x);
-}
 BSA_HD constexpr int get_strip_addr(bool permuted, int lane, int step, int half, int x0)
 {
     int g = lane >> 4, s = lane & 15;
@@ -142,6 +119,34 @@ BSA_HD constexpr int get_linear_addr(int lane, int q)
     int c = lane + 64 * q;
     return 16 * kc_slot(c >> 2, c & 3);
 }
+
+// ---- [32 rows][64 halves] panel tile, 128-byte rows, filled by loads that go straight to LDS -------
+// Such a load writes 64 consecutive 16-byte slots, lane l slot l: the swizzle has to sit in the SOURCE address, so it
+// permutes the 8 pieces inside a row (the request still covers whole 128-byte lines).  The mask is bits 1-3 of the row,
+// reversed: a ds_read_b128 phase takes one piece of 16 consecutive rows, of which those of equal parity share a
+// 128-byte half of the bank window and must differ in all three bits; a transposing read takes four pieces (4 m .. 4 m
+// + 3) of 4 consecutive rows, and rows k, k + 2 must differ in bit 2.
+BSA_HD constexpr int panel_swizzle(int row) { return ((row >> 1) & 1) * 4 + ((row >> 2) & 1) * 2 + ((row >> 3) & 1); }
+// request `chunk` (0..3) of a tile fills rows 8 chunk .. + 7: which 16-byte piece of row 8 chunk + lane / 8 lane l fetches
+BSA_HD constexpr int panel_src_piece(int lane, int chunk) { return (lane & 7) ^ panel_swizzle(8 * chunk + (lane >> 3)); }
+// operand with the row as index and the column as contraction: row lane % 32, columns 16 step + 8 (lane / 32) .. + 7.
+// Rows r and r + 16 swizzle alike: a b128 read whose lanes 16-31 use other banks than lanes 0-15 runs at two thirds of
+// the rate (measured with lds_bank_probe).
+BSA_HD constexpr int get_panel_addr(int lane, int step)
+{
+    return 128 * (lane & 31) + 16 * ((2 * step + (lane >> 5)) ^ panel_swizzle(lane & 31));
+}
+// ds_read_b64_tr_b16 operand with column x0 + lane % 32 as index and the ROW as contraction: element j of lane half h
+// is row 16 step + 8 (j / 4) + 4 h + j % 4, the order in which an accumulator of the product before holds its rows
+BSA_HD constexpr int get_panel_tr_addr(int lane, int step, int half, int x0)
+{
+    int g = lane >> 4, s = lane & 15;
+    int k = 16 * step + 4 * (g >> 1) + (s >> 2) + 8 * half;
+    int x = x0 + 16 * (g & 1) + 4 * (s & 3);
+    return 128 * k + 16 * ((x >> 3) ^ panel_swizzle(k)) + 2 * (x & 7);
+}
+// result rows of 64 or 128 halves (8 or 16 pieces) on their way to whole-line stores: half h of piece p of row `row`
+BSA_HD constexpr int out_row_addr(int head, int row, int p, int h) { return 2 * head * row + 16 * (p ^ (row & 7)) + 8 * h; }
 
 // ---- fp32 tiles (32 x 32 floats = 4 KB, stored in their memory orientation) ---------------------
 // Row r of the tile starts 36 r floats into the LDS tile, rows 16-31 another 32 floats on.  A 16-lane

@@ -46,6 +46,12 @@ ATTENTION_SPLIT_ROWS = True       # groups longer than cap * waves are cut into 
 SCHEDULE_ATTENTION = (12, 4)           # forward: rows of more than 48 blocks are split across workgroups
 SCHEDULE_ATTENTION_BACKWARD = (12, 4)
 SCHEDULE_ATTENTION_BACKWARD_COLUMNS = (12, 2)
+# A launch of few blocks is one generation of waves and lasts as long as its longest chunk: shorter chunks.  Measured,
+# causal local-4 + stride-8 mask of 4096 tokens, head dim 64, chunks of 12 -> 6 (forward, rows, columns): 1 batch entry
+# (1530 blocks) 10.6 / 12.8 / 18.2 -> 8.1 / 10.0 / 16.2 us; 4 entries (6120) 11.6 / 13.8 / 18.3 -> 10.7 / 13.2 / 17.8; 8
+# entries of a random mask (13100) 15.2 / 18.0 / 19.5 -> 15.8 / 20.5 / 22.1.
+SCHEDULE_ATTENTION_SMALL = (6, 4)
+ATTENTION_SMALL_BLOCKS = 8192          # blocks of all batch entries together
 # block rows of at most this many blocks are handed whole to SOFTMAX_SLICES wavefronts (8 element rows
 # each), which keep them in registers and need no exchange; per dtype: forward, backward (the
 # backward walk keeps two inputs)
@@ -246,6 +252,13 @@ def _attention_schedule(layout, kind, split=False):
     if _longest_group(layout[1]) > cap * waves:
         waves = ATTENTION_WAVES_LONG_GROUPS
     return schedule_for(layout, (cap, waves, False))
+
+
+def _attention_schedule_for(layout, kind, batches):
+    """Schedule of a fused attention walk over ``batches`` entries: ``kind``, or shorter chunks for a small launch."""
+    if layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS:
+        kind = SCHEDULE_ATTENTION_SMALL
+    return _attention_schedule(layout, kind, split=ATTENTION_SPLIT_ROWS)
 
 
 def _softmax_schedule(layout, dtype, backward):
@@ -461,7 +474,7 @@ def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=F
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device) if return_lse else None
     if out.numel() > 0:
-        sched = _attention_schedule(row_layout, SCHEDULE_ATTENTION, split=ATTENTION_SPLIT_ROWS)
+        sched = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION, batches)
         with torch.cuda.device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = sched.attention_workspace(batches, head, stream)
@@ -511,13 +524,11 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
     """``(dq, dk, dv)`` of the fused attention in two launches (a walk over the rows, one over the
     columns), the probabilities and score gradients rebuilt in registers in both instead of stored:
     the seven launches of the unfused backward chain (sparse/matmul.py:27-52, sparse_softmax.cu:165-205)
-    without a block stack in memory.  fp16 / bf16, head dim 64."""
+    without a block stack in memory.  fp16 / bf16, head dim 64 or 128."""
     col_layout = (col_blocks, col_table)
     _check_layout(col_layout, "col_layout")
     row_layout, mask_rows, mask_cols, nnz, head, batches = _attention_common(q, k, v, row_blocks, row_table,
                                                                               col_layout)
-    if head != 64:
-        raise ValueError(f"the two-launch backward is built for head dim 64, got {head}")
     if dout.shape != q.shape or out.shape != q.shape or dout.dtype != q.dtype or out.dtype != q.dtype:
         raise ValueError("dout and out must match q in shape and dtype")
     if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
@@ -526,12 +537,12 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     if q.numel() > 0:
         delta = torch.empty_like(lse)
-        rs = _attention_schedule(row_layout, SCHEDULE_ATTENTION_BACKWARD, split=ATTENTION_SPLIT_ROWS)
-        cs = _attention_schedule(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, split=ATTENTION_SPLIT_ROWS)
+        rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
+        cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches)
         with torch.cuda.device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = rs.attention_backward_workspace(cs, batches, head, stream)
-            _launch(rs, _k.lib.bsa_attention_backward(
+            _launch(rs, _k.lib.bsa_attention_gradients(
                 _DTYPES[q.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), out.data_ptr(),
                 lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr(),
                 row_blocks.data_ptr(), row_table.data_ptr(), rs.table.data_ptr(), rs.workgroups, rs.waves,

@@ -51,6 +51,8 @@ SIGNATURES = {
                                            _i, _i, _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _f, _i, _vp]),
     "bsa_attention_backward": (_i, [_i] + [_vp] * 10 + [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i,
                                                         _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _f, _i, _vp]),
+    "bsa_attention_gradients": (_i, [_i] + [_vp] * 10 + [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i,
+                                                        _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _f, _i, _vp]),
 }
 
 

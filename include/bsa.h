@@ -325,7 +325,7 @@ int bsa_attention_backward_scores(int dtype, const void *q, const void *k, const
 /* The whole backward pass of that operator in two launches, with no block stack in memory: a walk over
  * the rows that rebuilds the probabilities and the score gradients in registers and accumulates
  *   dq_out = ds k                       [batches, 32 * mask_rows, head_dim]
- * (and leaves rowsum(dout o out) in `delta_ws`, float [batches, 32 * mask_rows], caller-provided), and
+ * (and leaves scale * rowsum(dout o out) in `delta_ws`, float [batches, 32 * mask_rows], caller-provided), and
  * a walk over the columns that rebuilds them a second time and accumulates
  *   dk_out = ds^T q,  dv_out = p^T dout [batches, 32 * mask_cols, head_dim].
  * Seven launches in the unfused chain (sparse/matmul.py:27-52 three times over, sparse_softmax.cu:165-205,233-258).
@@ -337,6 +337,20 @@ int bsa_attention_backward_scores(int dtype, const void *q, const void *k, const
  * bsa_matmul calls).
  */
 int bsa_attention_backward(int dtype, const void *q, const void *k, const void *v, const void *dout,
+                           const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
+                           float *delta_ws,
+                           const int32_t *row_blocks, const int32_t *row_offsets,
+                           const int32_t *row_sched, int row_sched_wgs, int row_sched_waves,
+                           int row_tile_slots, int row_split_groups,
+                           const int32_t *col_blocks, const int32_t *col_offsets,
+                           const int32_t *col_sched, int col_sched_wgs, int col_sched_waves,
+                           int col_tile_slots, int col_split_groups,
+                           void *workspace, size_t workspace_bytes,
+                           int mask_rows, int mask_cols, int nnz, int batches, int head_dim,
+                           float scale, int causal, void *stream);
+
+/* bsa_attention_backward for head_dim 64 and 128.  At 128 the column schedule has at most 4 waves per workgroup. */
+int bsa_attention_gradients(int dtype, const void *q, const void *k, const void *v, const void *dout,
                            const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
                            float *delta_ws,
                            const int32_t *row_blocks, const int32_t *row_offsets,

@@ -1,0 +1,44 @@
+"""GPU: the fused attention walks on both of their chunk lengths (small launches take shorter chunks), at both head dims,
+where they can go wrong: empty rows and columns, single blocks, rows and columns that are cut into parts, a zero and a
+negative scale."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention_oracle as ao
+from helpers import mask_zoo, rel_err, to_np
+
+pytestmark = pytest.mark.gpu
+ZOO = dict(mask_zoo())
+TOL = {torch.float16: 2e-3, torch.bfloat16: 1.6e-2}      # one rounding of probabilities and results; gradients round twice more
+
+
+@pytest.mark.parametrize("causal,scale", [(False, 0.11), (True, 0.11), (True, -0.2), (True, 0.0)])
+@pytest.mark.parametrize("dtype,head", [(torch.float16, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("small", [0, 8192], ids=["long_chunks", "short_chunks"])
+@pytest.mark.parametrize("name", ["one_cell", "empty_row_col_6x5", "rand16", "long_row_5x40", "long_col_70x3"])
+def test_forward_and_gradients(name, small, dtype, head, causal, scale, monkeypatch):
+    import sparse
+    from sparse import _ops
+    monkeypatch.setattr(_ops, "ATTENTION_SMALL_BLOCKS", small)
+    mask = np.asarray(ZOO[name])
+    rows, cols = mask.shape
+    L = sparse.SparseLayout(torch.as_tensor(mask))
+    g = torch.Generator().manual_seed(41)
+    mk = lambda n: torch.randn(2, 32 * n, head, generator=g).to(dtype).cuda()
+    q, k, v, dout = mk(rows).requires_grad_(), mk(cols).requires_grad_(), mk(cols).requires_grad_(), mk(rows)
+    out = sparse.attention(q, k, v, L, scale, causal)
+    grads = torch.autograd.grad(out, (q, k, v), dout)
+    qn, kn, vn, dn = (to_np(t.detach().float()) for t in (q, k, v, dout))
+    assert rel_err(to_np(out.detach().float()), ao.forward(qn, kn, vn, mask, scale, causal)) <= TOL[dtype]
+    want = ao.backward(qn, kn, vn, dn, mask, scale, causal)
+    for got, ref in zip(grads, want):
+        assert rel_err(to_np(got.float()), ref) <= 4 * TOL[dtype]
+
+
+def test_column_schedule_of_head_dim_128_is_checked():
+    from sparse import kernel as k
+    P = 0x1000
+    rc = k.lib.bsa_attention_gradients(1, P, P, P, P, P, P, P, P, P, P, P, P, P, 4, 4, 0, 0, P, P, P, 4, 8, 0, 0, None, 0,
+                                       4, 4, 5, 1, 128, 1.0, 0, None)
+    assert rc == -1 and "at most 4" in k.lib.bsa_last_error().decode()
