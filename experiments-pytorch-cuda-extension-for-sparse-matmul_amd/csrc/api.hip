@@ -288,6 +288,71 @@ int bsa_matmul_dsd_block64(int dtype, const void *a, const void *b, void *c,
     return check_launch(bsa::launch_dsd_block64(dtype, p, (hipStream_t)stream), who);
 }
 
+int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void *out, const int32_t *blocks,
+                          const int32_t *offsets, int mask_rows, int mask_cols, int nnz, int batches,
+                          int sparse_batches, int M, int tr_b, void *stream)
+{
+    const char *who = "bsa_matmul_dds_panels";
+    if (dtype != BSA_F16 && dtype != BSA_BF16)
+        return fail(BSA_ERR_UNSUPPORTED, "%s: fp16 (dtype 1) and bf16 (dtype 2) are built, got %d", who, dtype);
+    if (mask_rows < 1 || mask_rows > 32767 || mask_cols < 1 || mask_cols > 65535)
+        return fail(BSA_ERR_INVALID, "%s: mask shape %d x %d out of range", who, mask_rows, mask_cols);
+    if (nnz < 0 || (long long)nnz > (long long)mask_rows * mask_cols)
+        return fail(BSA_ERR_INVALID, "%s: nnz %d does not fit a %d x %d mask", who, nnz, mask_rows, mask_cols);
+    if (batches < 1 || batches > 65535 || (sparse_batches != batches && sparse_batches != 1))
+        return fail(BSA_ERR_INVALID, "%s: batches %d, sparse_batches %d", who, batches, sparse_batches);
+    if (M < 1 || M % BSA_BLOCK)
+        return fail(BSA_ERR_INVALID, "%s: %d dense rows are no positive multiple of %d", who, M, BSA_BLOCK);
+    const int kblocks = tr_b ? mask_cols : mask_rows, groups = tr_b ? mask_rows : mask_cols;
+    if (nnz > bsa::PANEL_MAX_NNZ || kblocks > bsa::PANEL_MAX_KBLOCKS)
+        return fail(BSA_ERR_UNSUPPORTED, "%s: %d blocks over %d block rows of the contraction, at most %d over %d are "
+                    "built (use bsa_matmul)", who, nnz, kblocks, bsa::PANEL_MAX_NNZ, bsa::PANEL_MAX_KBLOCKS);
+    if (!out || !dense || !offsets || ((!sparse || !blocks) && nnz > 0))
+        return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    if (((uintptr_t)out | (uintptr_t)dense | (uintptr_t)sparse) & 15)
+        return fail(BSA_ERR_UNSUPPORTED, "%s: operands must be aligned to 16 bytes (use bsa_matmul)", who);
+    // a shared weight sees the batch as one long matrix
+    const bool fold = sparse_batches == 1;
+    const long long rows = fold ? (long long)M * batches : M;
+    if (rows > (1LL << 30) || (rows / 64 + 1) * (groups / 8 + 1) > MAX_GRID / 8)
+        return fail(BSA_ERR_INVALID, "%s: %lld dense rows x %d groups are too large", who, rows, groups);
+    bsa::WeightPanelArgs p{dense, sparse, out, blocks, offsets, groups, nnz, (int)rows, BSA_BLOCK * kblocks,
+                           fold ? 1 : batches, tr_b != 0, fold};
+    return check_launch(bsa::launch_weight_panels(dtype, p, (hipStream_t)stream), who);
+}
+
+int bsa_weight_grad_shares(int mask_rows, int mask_cols, int tokens)
+{
+    if (mask_rows < 1 || mask_cols < 1 || tokens < BSA_BLOCK) return 0;
+    return bsa::weight_grad_shares(mask_rows, mask_cols, tokens);
+}
+
+int bsa_weight_grad(int dtype, const void *a, const void *b, void *out, const int32_t *row_blocks,
+                    const int32_t *row_offsets, int mask_rows, int mask_cols, int nnz, int tokens,
+                    int shares, float *parts, size_t parts_bytes, void *stream)
+{
+    const char *who = "bsa_weight_grad";
+    if (dtype != BSA_F16 && dtype != BSA_BF16)
+        return fail(BSA_ERR_UNSUPPORTED, "%s: fp16 (dtype 1) and bf16 (dtype 2) are built, got %d", who, dtype);
+    if (mask_rows < 1 || mask_rows > 32767 || mask_cols < 1 || mask_cols > 65535)
+        return fail(BSA_ERR_INVALID, "%s: mask shape %d x %d out of range", who, mask_rows, mask_cols);
+    if (nnz < 0 || (long long)nnz > (long long)mask_rows * mask_cols)
+        return fail(BSA_ERR_INVALID, "%s: nnz %d does not fit a %d x %d mask", who, nnz, mask_rows, mask_cols);
+    if (tokens < BSA_BLOCK || tokens % BSA_BLOCK)
+        return fail(BSA_ERR_INVALID, "%s: %d tokens are no positive multiple of %d", who, tokens, BSA_BLOCK);
+    if (nnz == 0) return BSA_OK;
+    if (!a || !b || !out || !row_blocks || !row_offsets || !parts)
+        return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    if (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b | (uintptr_t)parts) & 15)
+        return fail(BSA_ERR_UNSUPPORTED, "%s: operands must be aligned to 16 bytes", who);
+    if (shares < 1 || (long long)shares * ((mask_rows + 7) / 8) * ((mask_cols + 7) / 8) > MAX_GRID / 8)
+        return fail(BSA_ERR_INVALID, "%s: %d shares of %d x %d cells do not fit a launch", who, shares, mask_rows, mask_cols);
+    if (parts_bytes < (size_t)shares * nnz * BSA_BLOCK * BSA_BLOCK * sizeof(float))
+        return fail(BSA_ERR_INVALID, "%s: %zu bytes for %d shares of %d blocks", who, parts_bytes, shares, nnz);
+    bsa::WeightGradArgs p{a, b, out, parts, row_blocks, row_offsets, mask_rows, mask_cols, nnz, tokens, shares};
+    return check_launch(bsa::launch_weight_grad(dtype, p, (hipStream_t)stream), who);
+}
+
 int64_t bsa_run_schedule_bytes(int mask_rows, int nnz)
 {
     if (mask_rows < 1 || nnz < 0) return 0;

@@ -75,6 +75,28 @@ struct RunsArgs {
 };
 hipError_t launch_dsd_runs(int dtype, const RunsArgs &p, hipStream_t stream);
 
+// products of a block-sparse weight with many dense rows, and the weight's gradient (weight_panels.hip)
+constexpr int PANEL_MAX_KBLOCKS = 1024;            // the k-block table of eight groups: 32 KB of LDS
+constexpr int PANEL_MAX_NNZ = (1 << 20) - 1;       // 2 KB blocks within a 31-bit buffer range
+struct WeightPanelArgs {
+    const void *dense, *sparse;
+    void *out;
+    const int32_t *blocks, *offsets;
+    int groups, nnz, rows, KT, batches;            // rows: dense rows of one launch entry
+    bool row_groups, sparse_shared;
+};
+hipError_t launch_weight_panels(int dtype, const WeightPanelArgs &p, hipStream_t stream);
+struct WeightGradArgs {
+    const void *a, *b;
+    void *out;
+    float *parts;                                  // [shares][nnz][1024]
+    const int32_t *blocks, *offsets;               // row table
+    int mask_rows, mask_cols, nnz;
+    int tokens, shares;
+};
+int weight_grad_shares(int mask_rows, int mask_cols, int tokens);
+hipError_t launch_weight_grad(int dtype, const WeightGradArgs &p, hipStream_t stream);
+
 struct SoftmaxArgs {
     const void *x;    // forward: scores; backward: y
     const void *dy;   // backward only

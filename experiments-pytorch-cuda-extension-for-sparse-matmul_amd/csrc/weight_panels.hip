@@ -1,0 +1,419 @@
+// Products of a block-sparse weight with many dense rows (a sparse linear layer), for gfx950, fp16 / bf16.
+//
+// The group walk of matmul.hip gives a wave 64 dense rows and a chunk of one group's blocks: it fetches 4 KB of dense
+// operand for every 2 KB block, from rows that lie a whole matrix row apart, and nothing it fetched serves another
+// group.  With a few attention heads of 64 columns that is what there is to do; a linear layer has thousands of
+// dense rows and dozens of groups that read the same columns of them.  Here a workgroup of eight waves owns PANEL_ROWS dense
+// rows and eight neighbouring groups, walks ALL of the contraction in steps of 128 and keeps the dense panel of a step in LDS
+// for the eight waves; a wave multiplies it by the blocks its group has there.
+#include "bsa_device.hpp"
+#include "lds_tiles.hpp"
+#include "bsa_internal.hpp"
+#include "group_walk.hpp"
+#include "../../include/bsa.h"
+
+namespace bsa {
+
+// Consecutive work items on one XCD (its workgroups are every eighth): neighbours share operands in its L2.
+__device__ __forceinline__ int xcd_contiguous(int total)
+{
+    const int per_xcd = (total + 7) >> 3, w = (int)blockIdx.x;
+    const int item = (w & 7) * per_xcd + (w >> 3);
+    return (w >> 3) < per_xcd && item < total ? item : -1;
+}
+
+constexpr int PANEL_WAVES = 8;                  // groups of a workgroup, one wave each
+constexpr int PANEL_KB = 4;                     // k-blocks of 32 per step
+
+// ---------------------------------------------------------------------------
+// out[row][32 g + x] = sum over the blocks (k-block kb) of group g, sum over k of dense[row][32 kb + k] * block(x, k)
+//
+// dense [rows][KT] and out [rows][XT] of one batch entry, or of all of them as one matrix when the weight is shared.
+//   S_KC  the stored block is [x][k] (row groups): operands straight from memory
+//         otherwise [k][x] (column groups): through a wave-private LDS tile, read transposed
+// A wave first spreads its group's pairs over a table indexed by k-block (LDS, -1 where nothing is stored), so the
+// steady state needs no search and no branch around a load: the requests of absent blocks carry an offset beyond the
+// descriptor's range, which the memory pipeline answers with zeros without a fetch.
+// ---------------------------------------------------------------------------
+template <int ROWS, bool S_KC, bool BF>
+__global__ __launch_bounds__(64 * PANEL_WAVES, 4) void weight_panel_kernel(
+    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
+    int groups, int nnz, int rows, int KT, int XT, int sp_shared, int row_tiles, int group_sets)
+{
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int RT = ROWS / 32, Q = ROWS * 16 / (64 * PANEL_WAVES);      // 32-row tiles; 16-byte pieces per thread and step
+    constexpr int PANEL_BYTES = ROWS * 256;
+    const int item = xcd_contiguous(row_tiles * group_sets);
+    if (item < 0) return;                                                  // whole workgroup leaves together
+    const int tile = item / group_sets, set = item - tile * group_sets;
+    const int batch = (int)blockIdx.y, w = wave_id(), l = lane_id(), tid = (int)threadIdx.x;
+    const int y0 = tile * ROWS, g = set * PANEL_WAVES + w;
+    const int kblocks = KT / BS, steps = (kblocks + PANEL_KB - 1) / PANEL_KB;
+    // Workgroups start at different steps: rows a multiple of 4 KB apart have their 256 bytes of a step in ONE of the 16
+    // channels of an L2, and workgroups that walk the contraction in unison would all ask that channel.
+    const int start = item % steps;
+    auto wrapped = [&](int s) { s += start; return s < steps ? s : s - steps; };
+
+    half_t *priv = reinterpret_cast<half_t *>(lds_raw + 2 * PANEL_BYTES) + w * BS2;
+    int *table = reinterpret_cast<int *>(lds_raw + 2 * PANEL_BYTES + (S_KC ? 0 : PANEL_WAVES * BS2 * 2)) +
+                 (size_t)w * (steps + 1) * PANEL_KB;
+    const half_t *dnb = dn + (size_t)batch * rows * KT;
+
+    // 16-byte piece `tid & 15` of rows tid / 16, + 32, ..: whole 256-byte runs of a row.  Rows behind the last and
+    // k behind the last k-block repeat what is there (never multiplied into a stored result).
+    const int prow = tid >> 4, piece = tid & 15;
+    const half_t *src[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int y = y0 + prow + 32 * q;
+        src[q] = dnb + (size_t)(y < rows ? y : rows - 1) * KT;
+    }
+    uint4 dense[Q];
+    auto request_panel = [&](int step) {
+        int k = step * (BS * PANEL_KB) + 8 * piece;
+        k = k < KT ? k : KT - 8;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) dense[q] = ldg16(src[q] + k);
+    };
+    request_panel(wrapped(0));
+
+    for (int t = l; t < (steps + 1) * PANEL_KB; t += WAVE) table[t] = -1;
+    wave_lds_fence();
+    if (g < groups) {
+        const int end = offsets[g + 1];
+        for (int p = offsets[g] + l; p < end; p += WAVE) {
+            const BlockDesc d = blocks[p];
+            const int kb = S_KC ? d.col() : d.row();
+            if (kb < kblocks) table[kb] = d.idx;
+        }
+    }
+    wave_lds_fence();
+
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<half_t *>(sp + (sp_shared ? 0 : (size_t)batch * nnz * BS2)), 0, nnz * BS2 * 2, 0x00020000);
+    // S_KC: lane (i, h) takes row perm16(i) of the block, k = 16 s + 8 h; otherwise the linear pieces l and l + 64
+    const int off0 = S_KC ? 64 * perm16(l & 31) + 16 * (l >> 5) : 16 * l, off1 = off0 + (S_KC ? 32 : 1024);
+    uint4 blk[PANEL_KB][2];
+    int now[PANEL_KB], next[PANEL_KB];
+    auto lookup = [&](int step, int (&idx)[PANEL_KB]) {
+        const int4 e = *reinterpret_cast<const int4 *>(table + step * PANEL_KB);
+        idx[0] = __builtin_amdgcn_readfirstlane(e.x);
+        idx[1] = __builtin_amdgcn_readfirstlane(e.y);
+        idx[2] = __builtin_amdgcn_readfirstlane(e.z);
+        idx[3] = __builtin_amdgcn_readfirstlane(e.w);
+    };
+    auto request_block = [&](int idx, uint4 (&b)[2]) {
+        const unsigned base = idx >= 0 ? (unsigned)idx * (BS2 * 2) : 0x80000000u;
+        b[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, base + off0, 0, 0));
+        b[1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, base + off1, 0, 0));
+    };
+    lookup(wrapped(0), now);
+#pragma unroll
+    for (int j = 0; j < PANEL_KB; ++j) {
+        request_block(now[j], blk[j]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    f16v acc[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t] = f16v{0};
+    const int i = l & 31, h = l >> 5;
+
+    for (int step = 0; step < steps; ++step) {
+        // rows of 16 pieces, piece p of row r in slot p ^ (r & 15): 16 lanes that read one piece of 16 rows, or write the
+        // 16 pieces of one row, meet no bank twice
+        unsigned char *panel = lds_raw + (step & 1) * PANEL_BYTES;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int r = prow + 32 * q;
+            *reinterpret_cast<uint4 *>(panel + 256 * r + 16 * (piece ^ (r & 15))) = dense[q];
+        }
+        lds_barrier();          // the other panel's readers passed this barrier one step ago at the latest
+        const int ahead = step + 1 < steps ? wrapped(step + 1) : steps;    // behind the last step: the table holds no block
+        request_panel(ahead);
+        __builtin_amdgcn_sched_barrier(0);
+        lookup(ahead, next);
+#pragma unroll
+        for (int j = 0; j < PANEL_KB; ++j) {
+            if (now[j] >= 0) {
+                h8 sop[2];
+                if (S_KC) {
+                    sop[0] = as_h8(blk[j][0]);
+                    sop[1] = as_h8(blk[j][1]);
+                } else {
+                    wave_lds_fence();
+                    lds_put_ks(priv, blk[j]);
+                    wave_lds_fence();
+                    sop[0] = lds_get_ks<true>(priv, 0);
+                    sop[1] = lds_get_ks<true>(priv, 1);
+                }
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) {
+                        const int r = 32 * t + i;
+                        const h8 dop = *reinterpret_cast<const h8 *>(panel + 256 * r + 16 * ((4 * j + 2 * s + h) ^ (r & 15)));
+                        acc[t] = mfma_16<BF>(sop[s], dop, acc[t]);
+                    }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            request_block(next[j], blk[j]);
+            __builtin_amdgcn_sched_barrier(0);
+            now[j] = next[j];
+        }
+    }
+
+    if (g < groups) {
+        half_t *ob = out + (size_t)batch * rows * XT + BS * g + 16 * h;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int y = y0 + 32 * t + i;
+            uint4 lo, hi;
+            pack16<BF>(acc[t], lo, hi);
+            if (y < rows) {
+                stg16(ob + (size_t)y * XT, lo);
+                stg16(ob + (size_t)y * XT + 8, hi);
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Gradient of the weight: w[block (r, c)] = sum over tokens t of a[t][32 r + .] b[t][32 c + .]
+//
+// A workgroup owns 8 x 8 cells of the mask and a share of the tokens; per step of 32 tokens it fetches 256 columns
+// of a and of b (512-byte runs), and wave r multiplies its 32 columns of a by those of the up to eight stored blocks of its
+// row.  Partial sums of the shares leave as fp32 and are added up in share order by weight_sum_kernel.
+// ---------------------------------------------------------------------------
+constexpr int WG_EDGE = 8;                       // cells along a side
+constexpr int WG_TILE = 2048 + 64;               // a 32 x 32 tile; 64 bytes on, so that four tiles of a row write to different banks
+constexpr int WG_SIDE = WG_EDGE * WG_TILE;
+
+template <bool BF>
+__global__ __launch_bounds__(512, 2) void weight_grad_kernel(
+    const half_t *__restrict__ a, const half_t *__restrict__ b, float *__restrict__ parts,
+    const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
+    int R, int C, int nnz, int steps_total, int shares, int sets_r, int sets_c)
+{
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int item = xcd_contiguous(shares * sets_r * sets_c);
+    if (item < 0) return;
+    const int share = item / (sets_r * sets_c), cell = item - share * (sets_r * sets_c);
+    const int r0 = WG_EDGE * (cell / sets_c), c0 = WG_EDGE * (cell % sets_c);
+    const int w = wave_id(), l = lane_id(), tid = (int)threadIdx.x;
+    const int first = (int)((long long)steps_total * share / shares), last = (int)((long long)steps_total * (share + 1) / shares);
+    const int M = BS * R, N = BS * C;
+
+    // the stored cells, dealt evenly to the waves in row-major order: cells w, w + 8, ..
+    int *table = reinterpret_cast<int *>(lds_raw + 4 * WG_SIDE);
+    if (tid < WG_EDGE * WG_EDGE) table[tid] = -1;
+    lds_barrier();
+    if (r0 + w < R) {
+        const int end = offsets[r0 + w + 1];
+        for (int p = offsets[r0 + w] + l; p < end; p += WAVE) {
+            const BlockDesc d = blocks[p];
+            const int c = d.col() - c0;
+            if (c >= 0 && c < WG_EDGE) table[w * WG_EDGE + c] = d.idx;
+        }
+    }
+    lds_barrier();
+    const int mine_idx = table[l];
+    unsigned long long stored = __ballot(mine_idx >= 0);
+    const int count = (__popcll(stored) - w + WG_EDGE - 1) / WG_EDGE;      // of this wave
+    int idx[WG_EDGE], at_a[WG_EDGE], at_b[WG_EDGE];
+    for (int j = 0; j < w && stored; ++j) stored &= stored - 1;
+#pragma unroll
+    for (int j = 0; j < WG_EDGE; ++j) {
+        const int cell_of = stored ? __builtin_ctzll(stored) : 0;
+        idx[j] = __builtin_amdgcn_readlane(mine_idx, cell_of);
+        at_a[j] = (cell_of >> 3) * WG_TILE;
+        at_b[j] = WG_SIDE + (cell_of & 7) * WG_TILE;
+        for (int t = 0; t < WG_EDGE; ++t) stored &= stored ? stored - 1 : 0;
+    }
+
+    // piece `tid & 31` of tokens tid / 32 and + 16; columns behind the last repeat the first (never stored)
+    const int trow = tid >> 5, piece = tid & 31;
+    const int ca = 256 * (r0 / WG_EDGE) + 8 * piece, cb = 256 * (c0 / WG_EDGE) + 8 * piece;
+    const half_t *pa = a + (ca < M ? ca : 0), *pb = b + (cb < N ? cb : 0);
+    struct Raw { uint4 a[2], b[2]; };
+    auto request = [&](int step, Raw &f) {
+        step = step < last ? step : last - 1;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const size_t t = (size_t)32 * step + trow + 16 * q;
+            f.a[q] = ldg16(pa + t * M);
+            f.b[q] = ldg16(pb + t * N);
+        }
+    };
+    f16v acc[WG_EDGE];
+#pragma unroll
+    for (int c = 0; c < WG_EDGE; ++c) acc[c] = f16v{0};
+
+    auto step_of = [&](int parity, const Raw &f) {
+        unsigned char *ta = lds_raw + parity * 2 * WG_SIDE, *tb = ta + WG_SIDE;
+        const int to = (piece >> 2) * WG_TILE;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int at = to + 16 * ks_slot(trow + 16 * q, piece & 3);
+            *reinterpret_cast<uint4 *>(ta + at) = f.a[q];
+            *reinterpret_cast<uint4 *>(tb + at) = f.b[q];
+        }
+        lds_barrier();
+    };
+    auto multiply = [&](int parity) {
+        const unsigned char *panel = lds_raw + parity * 2 * WG_SIDE;
+        auto operands = [&](int j, h8 (&x)[4]) {
+            int oa = at_a[j], ob = at_b[j];
+            asm volatile("" : "+s"(oa), "+s"(ob));      // added where they are used: hoisted, the sums take 64 registers
+            const half_t *ta = reinterpret_cast<const half_t *>(panel + oa);
+            const half_t *tb = reinterpret_cast<const half_t *>(panel + ob);
+            x[0] = lds_get_ks<false>(ta, 0); x[1] = lds_get_ks<true>(tb, 0);
+            x[2] = lds_get_ks<false>(ta, 1); x[3] = lds_get_ks<true>(tb, 1);
+        };
+#pragma unroll
+        for (int j = 0; j < WG_EDGE; j += 2) {
+            if (j < count) {                       // a pair at a time; the second repeats a cell when there is none
+                h8 x[4], y[4];
+                operands(j, x);
+                operands(j + 1, y);
+                acc[j] = mfma_16<BF>(x[1], x[0], acc[j]);
+                acc[j + 1] = mfma_16<BF>(y[1], y[0], acc[j + 1]);
+                acc[j] = mfma_16<BF>(x[3], x[2], acc[j]);
+                acc[j + 1] = mfma_16<BF>(y[3], y[2], acc[j + 1]);
+            }
+        }
+    };
+    if (first < last) {
+        // three steps in flight (the operands of a long batch come from HBM); a panel is overwritten two steps later,
+        // when every wave has passed the barrier between
+        Raw f[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            request(first + d, f[d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        int s = first;
+        for (; s + 6 <= last; s += 6) {
+#pragma unroll
+            for (int d = 0; d < 6; ++d) {
+                step_of(d & 1, f[d % 3]);
+                request(s + 3 + d, f[d % 3]);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(d & 1);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < 5; ++d) {
+            if (s + d < last) {
+                step_of(d & 1, f[d % 3]);
+                if (s + d + 3 < last) request(s + 3 + d, f[d % 3]);
+                multiply(d & 1);
+            }
+        }
+    }
+    float *dst = parts + (size_t)share * nnz * BS2 + (l & 31) * BS + 16 * (l >> 5);
+#pragma unroll
+    for (int c = 0; c < WG_EDGE; ++c) {
+        if (c < count) {
+            float *o = dst + (size_t)idx[c] * BS2;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                *reinterpret_cast<float4 *>(o + 4 * t) =
+                    make_float4(acc[c][4 * t], acc[c][4 * t + 1], acc[c][4 * t + 2], acc[c][4 * t + 3]);
+        }
+    }
+}
+
+// out[e] = sum over the shares of parts[share][e]: 8 elements a thread
+template <bool BF>
+__global__ __launch_bounds__(256) void weight_sum_kernel(const float *__restrict__ parts, half_t *__restrict__ out,
+                                                         size_t elements, int shares)
+{
+    const size_t e = 8 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+    if (e >= elements) return;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < shares; ++p) {
+        const float4 *src = reinterpret_cast<const float4 *>(parts + (size_t)p * elements + e);
+        const float4 x = src[0], y = src[1];
+        s[0] += x.x; s[1] += x.y; s[2] += x.z; s[3] += x.w;
+        s[4] += y.x; s[5] += y.y; s[6] += y.z; s[7] += y.w;
+    }
+    h8 o;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) o[v] = narrow_16<BF>(s[v]);
+    stg16(out + e, __builtin_bit_cast(uint4, o));
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+// ---------------------------------------------------------------------------
+constexpr int PANEL_ROWS = 96;
+template <int ROWS, bool S_KC, bool BF>
+static hipError_t launch_panel(const WeightPanelArgs &p, hipStream_t st)
+{
+    const int tiles = (p.rows + ROWS - 1) / ROWS, sets = (p.groups + PANEL_WAVES - 1) / PANEL_WAVES;
+    const int steps = (p.KT / BS + PANEL_KB - 1) / PANEL_KB;
+    const size_t lds = 2 * ROWS * 256 + (S_KC ? 0 : PANEL_WAVES * BS2 * 2) +
+                       (size_t)PANEL_WAVES * (steps + 1) * PANEL_KB * sizeof(int);
+    auto kernel = weight_panel_kernel<ROWS, S_KC, BF>;
+    if (lds > 65536) {
+        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (err != hipSuccess) return err;
+    }
+    dim3 grid((unsigned)((tiles * sets + 7) / 8 * 8), (unsigned)p.batches);
+    kernel<<<grid, 64 * PANEL_WAVES, lds, st>>>((const half_t *)p.sparse, (const half_t *)p.dense, (half_t *)p.out,
+                                                (const BlockDesc *)p.blocks, p.offsets, p.groups, p.nnz, p.rows, p.KT,
+                                                BS * p.groups, p.sparse_shared ? 1 : 0, tiles, sets);
+    return hipGetLastError();
+}
+
+hipError_t launch_weight_panels(int dtype, const WeightPanelArgs &p, hipStream_t st)
+{
+    if (dtype == BSA_BF16)
+        return p.row_groups ? launch_panel<PANEL_ROWS, true, true>(p, st) : launch_panel<PANEL_ROWS, false, true>(p, st);
+    return p.row_groups ? launch_panel<PANEL_ROWS, true, false>(p, st) : launch_panel<PANEL_ROWS, false, false>(p, st);
+}
+
+// Shares of at least eight steps: the fewest (at most eight) that leave at most a sixth of the machine idle in the last
+// generation of workgroups (one per compute unit at a time: 66 KB of panels, 256 registers), else the best there is.
+int weight_grad_shares(int mask_rows, int mask_cols, int tokens)
+{
+    const long long cells = (long long)((mask_rows + WG_EDGE - 1) / WG_EDGE) * ((mask_cols + WG_EDGE - 1) / WG_EDGE);
+    const int steps = tokens / BS;
+    int best = 1;
+    double best_use = 0.;
+    for (int s = 1; s <= (cells < 32 ? 256 / cells : 8) && (s == 1 || steps / s >= 8); ++s) {
+        const long long wgs = cells * s;
+        const double use = (double)wgs / (double)((wgs + 255) / 256 * 256);
+        if (use > best_use + 0.01) {
+            best = s;
+            best_use = use;
+        }
+        if (use > 5. / 6.) break;
+    }
+    return best;
+}
+
+hipError_t launch_weight_grad(int dtype, const WeightGradArgs &p, hipStream_t st)
+{
+    const int sets_r = (p.mask_rows + WG_EDGE - 1) / WG_EDGE, sets_c = (p.mask_cols + WG_EDGE - 1) / WG_EDGE;
+    const size_t lds = 4 * WG_SIDE + WG_EDGE * WG_EDGE * sizeof(int);
+    auto kernel = dtype == BSA_BF16 ? weight_grad_kernel<true> : weight_grad_kernel<false>;
+    hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (err != hipSuccess) return err;
+    const unsigned grid = ((unsigned)p.shares * sets_r * sets_c + 7) / 8 * 8;
+    kernel<<<grid, 64 * WG_EDGE, lds, st>>>((const half_t *)p.a, (const half_t *)p.b, p.parts, (const BlockDesc *)p.blocks,
+                                            p.offsets, p.mask_rows, p.mask_cols, p.nnz, p.tokens / BS, p.shares, sets_r, sets_c);
+    err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    const size_t elements = (size_t)p.nnz * BS2;
+    const unsigned wgs = (unsigned)((elements / 8 + 255) / 256);
+    if (dtype == BSA_BF16) weight_sum_kernel<true><<<wgs, 256, 0, st>>>(p.parts, (half_t *)p.out, elements, p.shares);
+    else weight_sum_kernel<false><<<wgs, 256, 0, st>>>(p.parts, (half_t *)p.out, elements, p.shares);
+    return hipGetLastError();
+}
+
+}  // namespace bsa

@@ -41,6 +41,23 @@ RUN_WALK_PAIRS_MIN = 48
 RUN_WALK_STRIPS = 32             # 4 per wave; with 10 waves and up to 39 strips (rows of 33-39 blocks) the walk of
                                  # bsa_matmul is 3-6 % faster at 8192 tokens
 RUN_WALK_MIN_REUSE = 2.0
+# DDS over many dense rows (a block-sparse linear layer): panels of the dense operand shared by eight groups
+# (bsa_matmul_dds_panels), when the mask is dense enough that a panel serves several of them and the launch has
+# workgroups for most of the machine.  Measured against the group walk, fp16 / bf16, us: stored share of the cells times used
+# share of the panels' rows 0.08 (96 x 96 blocks, 8 x 1024 rows) 88 -> 97, 0.10 (64 x 64, 4 x 1056) 36 -> 30, 0.12 (96 x 96, 8 x
+# 1024) 111 -> 98, 0.18 155 -> 107, 0.30 238 -> 117; at a stored share of 0.2 by workgroups: 96 32 x 96 blocks 10 -> 24,
+# 128 (64 x 64, 16 x 96 rows) 16 -> 18, 176 (64 x 64, 2 x 1056) 28 -> 20.
+PANEL_WALK = True
+PANEL_ROWS, PANEL_GROUPS = 96, 8       # of a workgroup
+PANEL_MIN_WORKGROUPS = 160
+PANEL_MIN_DENSITY = 0.12
+PANEL_MAX_KBLOCKS = 1024
+PANEL_MAX_NNZ = 2 ** 20 - 1
+# Its weight gradient (bsa_weight_grad) against a stack per batch entry and a sum over them: 0.12 stored (96 x 96 blocks, 8192
+# tokens) 104 -> 114 us, 0.18 179 -> 126, 0.25 (64 x 64, 4224 tokens) 67 -> 40; 0.2, 1056 tokens 60 -> 24; 0.3 (16 x 16), 256
+# tokens 12 -> 16.
+WEIGHT_GRAD_MIN_TOKENS = 1024
+WEIGHT_GRAD_MIN_DENSITY = 0.15
 ATTENTION_WAVES_LONG_GROUPS = 8
 ATTENTION_SPLIT_ROWS = True       # groups longer than cap * waves are cut into parts across workgroups
 SCHEDULE_ATTENTION = (12, 4)           # forward: rows of more than 48 blocks are split across workgroups
@@ -368,6 +385,18 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
                     mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_n, _k.current_stream()))
             return c
 
+    if (PANEL_WALK and mode == "dds" and not trans_a and a.dtype != torch.float32
+            and size_m % BLOCK == 0 and size_k == BLOCK * (mask_cols if trans_b else mask_rows)
+            and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
+            and _takes_panels(num_blocks, size_m * batches if shared else size_m, 1 if shared else batches,
+                              size_k // BLOCK, size_n // BLOCK)):
+        with torch.cuda.device(a.device):
+            _k.check(_k.lib.bsa_matmul_dds_panels(
+                _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
+                mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_m, int(trans_b),
+                _k.current_stream()))
+        return c
+
     if mode == "sdd":
         sched = schedule_for(layout, SCHEDULE_SDD_F32 if a.dtype == torch.float32 else SCHEDULE_SDD)
     else:
@@ -383,6 +412,44 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
             mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_m, size_n, size_k,
             int(trans_a), int(trans_b), stream))
     return c
+
+
+def _takes_panels(nnz, rows, entries, kblocks, groups):
+    """Whether a DDS product of ``entries`` matrices of ``rows`` dense rows takes the panel walk
+    (bsa_matmul_dds_panels)."""
+    tiles, sets = -(-rows // PANEL_ROWS), -(-groups // PANEL_GROUPS)
+    return (kblocks <= PANEL_MAX_KBLOCKS and nnz <= PANEL_MAX_NNZ and entries <= 65535 and rows <= 2 ** 30
+            and tiles * sets * entries >= PANEL_MIN_WORKGROUPS
+            and nnz * rows >= PANEL_MIN_DENSITY * kblocks * groups * tiles * PANEL_ROWS)
+
+
+def sparse_weight_gradient(a, b, row_layout, col_layout, trans_a, trans_b):
+    """``sparse_matmul(a, b, 'sdd', ..)`` summed over the batch: the gradient of a sparse operand that the batch shared.
+    With both operands stored tokens-first (``trans_a``, not ``trans_b``) the batch and the tokens are one contraction,
+    summed in fp32 by bsa_weight_grad; the other forms write a stack per batch entry and add them up."""
+    nnz = row_layout[0].numel() // 2
+    rows, cols = row_layout[1].numel() - 1, col_layout[1].numel() - 1
+    tokens = a.numel() // max(a.size(-1), 1)
+    folds = (trans_a and not trans_b and a.dtype in (torch.float16, torch.bfloat16) and a.dtype == b.dtype
+             and a.shape[:-1] == b.shape[:-1] and a.size(-2) % BLOCK == 0 and WEIGHT_GRAD_MIN_TOKENS <= tokens < 2 ** 31
+             and a.size(-1) == BLOCK * rows and b.size(-1) == BLOCK * cols and a.is_cuda and a.device == b.device
+             and row_layout[0].device == a.device and nnz > 0 and nnz >= WEIGHT_GRAD_MIN_DENSITY * rows * cols)
+    if folds:
+        a, b = a.contiguous(), b.contiguous()
+        folds = a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
+    if folds:
+        _check_layout(row_layout, "row_layout")
+        out = torch.empty((nnz, BLOCK, BLOCK), dtype=a.dtype, device=a.device)
+        shares = _k.lib.bsa_weight_grad_shares(rows, cols, tokens)
+        parts = torch.empty(shares * nnz * BLOCK * BLOCK, dtype=torch.float32, device=a.device)
+        with torch.cuda.device(a.device):
+            _k.check(_k.lib.bsa_weight_grad(
+                _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), out.data_ptr(), row_layout[0].data_ptr(),
+                row_layout[1].data_ptr(), rows, cols, nnz, tokens, shares, parts.data_ptr(), 4 * parts.numel(),
+                _k.current_stream()))
+        return out
+    stack = sparse_matmul(a, b, "sdd", row_layout, col_layout, trans_a, trans_b)
+    return stack.sum(dim=tuple(range(stack.dim() - 3)))
 
 
 def _softmax_common(x, row_layout, col_layout, name):

@@ -36,6 +36,9 @@ SIGNATURES = {
     "bsa_matmul_noalloc": (_i, [_i, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i,
                                 _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "bsa_matmul_dsd_block64": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "bsa_matmul_dds_panels": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "bsa_weight_grad_shares": (_i, [_i, _i, _i]),
+    "bsa_weight_grad": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t, _vp]),
     "bsa_run_schedule_bytes": (ctypes.c_int64, [_i, _i]),
     "bsa_run_schedule_build": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, ctypes.c_int64, _vp, _vp]),
     "bsa_matmul_dsd_runs": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),

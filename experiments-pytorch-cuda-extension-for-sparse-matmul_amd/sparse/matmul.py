@@ -30,15 +30,19 @@ class SparseMatMul(torch.autograd.Function):
         trans_a, trans_b = ctx.trans_a, ctx.trans_b
         dc = dc.contiguous()
         da = db = None
-
+        # a sparse input given without batch dimensions was shared by the batch: its gradient is the sum
         if ctx.needs_input_grad[0]:
             # d op(a) = dc @ op(b)^T, stored back in a's orientation (matmul.py:30-39)
             if trans_a:
                 da_mode, lhs, rhs = mode[1] + mode[2] + mode[0], b, dc
             else:
                 da_mode, lhs, rhs = mode[1] + mode[0] + mode[2], dc, b
-            da = sparse_ops.sparse_matmul(lhs, rhs, da_mode, layout.row_layout, layout.col_layout,
-                                          trans_a and trans_b, trans_a or not trans_b)
+            if mode[1] == "s" and a.dim() == 3:
+                da = sparse_ops.sparse_weight_gradient(lhs, rhs, layout.row_layout, layout.col_layout,
+                                                       trans_a and trans_b, trans_a or not trans_b)
+            else:
+                da = sparse_ops.sparse_matmul(lhs, rhs, da_mode, layout.row_layout, layout.col_layout,
+                                              trans_a and trans_b, trans_a or not trans_b)
 
         if ctx.needs_input_grad[1]:
             # d op(b) = op(a)^T @ dc, stored back in b's orientation (matmul.py:41-50)
@@ -46,14 +50,12 @@ class SparseMatMul(torch.autograd.Function):
                 db_mode, lhs, rhs = mode[2] + mode[0] + mode[1], dc, a
             else:
                 db_mode, lhs, rhs = mode[2] + mode[1] + mode[0], a, dc
-            db = sparse_ops.sparse_matmul(lhs, rhs, db_mode, layout.row_layout, layout.col_layout,
-                                          not trans_a or trans_b, trans_a and trans_b)
-
-        # a sparse input given without batch dimensions was shared by the batch: its gradient is the sum
-        if da is not None and da.dim() > a.dim():
-            da = da.sum(dim=tuple(range(da.dim() - a.dim())))
-        if db is not None and db.dim() > b.dim():
-            db = db.sum(dim=tuple(range(db.dim() - b.dim())))
+            if mode[2] == "s" and b.dim() == 3:
+                db = sparse_ops.sparse_weight_gradient(lhs, rhs, layout.row_layout, layout.col_layout,
+                                                       not trans_a or trans_b, trans_a and trans_b)
+            else:
+                db = sparse_ops.sparse_matmul(lhs, rhs, db_mode, layout.row_layout, layout.col_layout,
+                                              not trans_a or trans_b, trans_a and trans_b)
         return da, db, None, None, None, None
 
 

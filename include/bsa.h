@@ -363,6 +363,27 @@ int bsa_attention_gradients(int dtype, const void *q, const void *k, const void 
                            int mask_rows, int mask_cols, int nnz, int batches, int head_dim,
                            float scale, int causal, void *stream);
 
+/* DDS with a weight that many dense rows meet: out = dense op(b), dense [batches, M, K] (K contiguous) and out
+ * [batches, M, N] as in bsa_matmul(mode 2, tr_a = 0, tr_b), by a walk that keeps panels of the dense operand on the chip
+ * for eight groups at a time (no schedule, no workspace).  Tables: the row table with tr_b, the column table without.
+ * With sparse_batches = 1 the batch is walked as one matrix of batches * M rows.  fp16 / bf16; at most 2^20 - 1
+ * blocks and a contraction of at most 1024 blocks (BSA_ERR_UNSUPPORTED otherwise: use bsa_matmul).
+ */
+int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void *out, const int32_t *blocks,
+                          const int32_t *offsets, int mask_rows, int mask_cols, int nnz, int batches,
+                          int sparse_batches, int M, int tr_b, void *stream);
+
+/* Gradient of a block-sparse weight that a whole batch shared: out[block (r, c)] = sum over all tokens t of
+ * a[t][32 r + .] b[t][32 c + .], a [tokens, 32 * mask_rows], b [tokens, 32 * mask_cols], the batch folded into the
+ * tokens (a multiple of 32); the sum stays in fp32 until the block is written.  `parts` is scratch of
+ * shares * nnz * 4096 bytes with any contents; bsa_weight_grad_shares says how many shares fill the machine.
+ * Row table.  fp16 / bf16.
+ */
+int bsa_weight_grad_shares(int mask_rows, int mask_cols, int tokens);
+int bsa_weight_grad(int dtype, const void *a, const void *b, void *out, const int32_t *row_blocks,
+                    const int32_t *row_offsets, int mask_rows, int mask_cols, int nnz, int tokens,
+                    int shares, float *parts, size_t parts_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

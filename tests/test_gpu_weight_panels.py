@@ -1,0 +1,92 @@
+"""GPU: the panel walk of a block-sparse weight (``bsa_matmul_dds_panels``) and its gradient (``bsa_weight_grad``) at the
+edges of their tiles, against float64.  Bound: one rounding of the result (2^-11 fp16, 2^-8 bf16 of the element) beside an
+fp32 sum of at most 40 x 32 products, taken over the 2-norm."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+REL = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _layout(rows, cols, density, seed):
+    import sparse
+    g = torch.Generator().manual_seed(seed)
+    mask = (torch.rand(rows, cols, generator=g) < density).long()
+    mask[0, -1] = 1
+    if rows > 1 and cols > 1:
+        mask[:, 0] = 0                    # an empty group in either direction
+        mask[1, :] = 0
+    return sparse.SparseLayout(mask.cuda())
+
+
+def _rel(got, want):
+    assert torch.isfinite(got).all()
+    return ((got.double() - want).norm() / want.norm().clamp_min(1e-30)).item()
+
+
+@pytest.fixture
+def any_size(monkeypatch):
+    from sparse import _ops
+    monkeypatch.setattr(_ops, "PANEL_MIN_WORKGROUPS", 1)
+    monkeypatch.setattr(_ops, "PANEL_MIN_DENSITY", 0.0)
+    monkeypatch.setattr(_ops, "WEIGHT_GRAD_MIN_TOKENS", 32)
+    monkeypatch.setattr(_ops, "WEIGHT_GRAD_MIN_DENSITY", 0.0)
+
+
+# one block; fewer groups than waves; contraction of 1, 4, 5 and 40 blocks (steps of 4, a wrapped start); rows of one tile,
+# one more than a tile, several; a full mask (four blocks a step)
+@pytest.mark.parametrize("rows,cols,density,batch,m", [
+    (1, 1, 1.0, 1, 32), (4, 3, 0.9, 2, 96), (5, 8, 0.6, 3, 128), (40, 9, 0.2, 1, 224), (9, 40, 0.3, 5, 32),
+    (16, 17, 1.0, 2, 192)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_panels(any_size, rows, cols, density, batch, m, trans_b, shared, dtype):
+    from sparse import _ops
+    L = _layout(rows, cols, density, rows + 100 * cols)
+    k = 32 * (cols if trans_b else rows)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(batch, m, k, generator=g, device="cuda").to(dtype)
+    w = torch.randn(*(() if shared else (batch,)), L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
+    W = L.to_dense(w).double().cpu()
+    want = (x.double().cpu() @ (W.transpose(-1, -2).contiguous() if trans_b else W)).cuda()
+    got = _ops.sparse_matmul(x, w, "dds", L.row_layout, L.col_layout, False, trans_b)
+    assert _rel(got, want) <= REL[dtype]
+
+
+@pytest.mark.parametrize("rows,cols,density", [(1, 1, 1.0), (8, 8, 1.0), (9, 7, 0.5), (20, 33, 0.3)])
+@pytest.mark.parametrize("batch,tokens", [(1, 32), (1, 160), (3, 224), (5, 64)])      # 1, 5, 21 and 10 steps: every tail
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_weight_gradient(any_size, rows, cols, density, batch, tokens, dtype):
+    from sparse import _ops
+    L = _layout(rows, cols, density, rows + cols)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    a = torch.randn(batch, tokens, 32 * rows, generator=g, device="cuda").to(dtype)
+    b = torch.randn(batch, tokens, 32 * cols, generator=g, device="cuda").to(dtype)
+    dense = a.double().cpu().flatten(0, 1).t().contiguous() @ b.double().cpu().flatten(0, 1)
+    pos = L.sparse_positions.cpu()
+    want = torch.stack([dense[32 * r:32 * r + 32, 32 * c:32 * c + 32] for r, c in pos.tolist()]).cuda()
+    got = _ops.sparse_weight_gradient(a, b, L.row_layout, L.col_layout, True, False)
+    assert got.shape == want.shape and _rel(got, want) <= REL[dtype]
+
+
+def test_linear_layer_takes_both_and_agrees_with_the_group_walk(monkeypatch):
+    import sparse
+    from sparse import _ops
+    L = _layout(24, 32, 0.4, 7)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(4, 1056, 32 * 24, generator=g, device="cuda").half().requires_grad_()
+    w = (0.05 * torch.randn(L.num_blocks, 32, 32, generator=g, device="cuda")).half().requires_grad_()
+    dy = torch.randn(4, 1056, 32 * 32, generator=g, device="cuda").half()
+
+    def step():
+        y = sparse.matmul(x, w, "dds", L)
+        return (y.detach(),) + torch.autograd.grad(y, (x, w), dy)
+
+    assert _ops._takes_panels(L.num_blocks, 4 * 1056, 1, 24, 32)
+    new = step()
+    monkeypatch.setattr(_ops, "PANEL_WALK", False)
+    monkeypatch.setattr(_ops, "WEIGHT_GRAD_MIN_TOKENS", 2 ** 31)
+    for n, o in zip(new, step()):
+        assert n.shape == o.shape and _rel(n, o.double()) <= 4 * REL[torch.float16]
+
