@@ -5,6 +5,8 @@ reference does not make.  ``sparse_matmul`` keeps the reference's positional
 signature (``native/sparse_ops.h:10-14``); the softmax entry points keep those of
 ``sparse_softmax.cu:208-210,233-236`` with ``scale`` / ``causal`` appended.
 """
+import functools
+
 import torch
 
 from . import kernel as _k
@@ -87,7 +89,7 @@ class Schedule:
         capacity = _k.lib.bsa_schedule_capacity(groups, nnz, cap, waves)
         self.table = torch.empty(4 * capacity, dtype=torch.int32, device=offsets.device)
         counts = torch.empty(4, dtype=torch.int32, device=offsets.device)
-        with torch.cuda.device(offsets.device):
+        with _k.on_device(offsets.device):
             _k.check(_k.lib.bsa_schedule_build(offsets.data_ptr(), groups, cap, waves,
                                                int(bool(allow_split)) | (2 if longest_first else 0), slice_max,
                                                slices, self.table.data_ptr(), capacity, counts.data_ptr(),
@@ -106,12 +108,18 @@ class Schedule:
     def workspace(self, mode: int, batches: int, size_m: int, size_n: int, stream: int):
         """Zeroed scratch for split groups, one per (shape, stream): launches on one stream run in
         order and each leaves the buffer zero again; launches on different streams may overlap."""
+        if self.tile_slots == 0:
+            self.last_key = None
+            return None, 0
         need = _k.lib.bsa_matmul_workspace_bytes(mode, self.tile_slots, self.split_groups, batches, size_m, size_n)
         self.last_key = (mode, batches, size_m, size_n, stream)
         return self._zeroed(self.last_key, need)
 
     def attention_workspace(self, batches: int, head_dim: int, stream: int):
         """The same for the split rows of the fused attention forward."""
+        if self.tile_slots == 0:
+            self.last_key = None
+            return None, 0
         need = _k.lib.bsa_attention_workspace_bytes(self.tile_slots, self.split_groups, batches, head_dim)
         self.last_key = ("attention", batches, head_dim, stream)
         return self._zeroed(self.last_key, need)
@@ -183,12 +191,17 @@ class RunSchedule:
         need = _k.lib.bsa_run_schedule_bytes(rows, nnz)
         self.table = torch.empty(need, dtype=torch.uint8, device=offsets.device)
         counts = torch.empty(4, dtype=torch.int32, device=offsets.device)
-        with torch.cuda.device(offsets.device):
+        with _k.on_device(offsets.device):
             _k.check(_k.lib.bsa_run_schedule_build(blocks.data_ptr(), offsets.data_ptr(), rows, nnz, target_pairs,
                                                    max_strips, self.table.data_ptr(), need, counts.data_ptr(),
                                                    _k.current_stream()))
         self.runs, self.strips, self.strips_total, self.pairs = (int(v) for v in counts.tolist())
         self.reuse = nnz / self.strips_total if self.strips_total else 0.0
+
+
+@functools.lru_cache(maxsize=None)
+def _compute_units(device_index: int) -> int:
+    return torch.cuda.get_device_properties(device_index).multi_processor_count
 
 
 def _run_schedule(layout, batches, strips_n):
@@ -198,7 +211,7 @@ def _run_schedule(layout, batches, strips_n):
     blocks, offsets = layout
     nnz = blocks.numel() // 2
     entries = batches * strips_n
-    cus = torch.cuda.get_device_properties(offsets.device).multi_processor_count
+    cus = _compute_units(offsets.device.index)
     if nnz * entries < cus * RUN_WALK_PAIRS_MIN:
         return None
     generations = max(1, round(nnz * entries / (cus * RUN_WALK_PAIRS)))
@@ -290,12 +303,16 @@ def _softmax_schedule(layout, dtype, backward):
     return schedule_for(layout, (cap, waves, False, slice_max, slices, SOFTMAX_LONGEST_FIRST))
 
 
+def _is_table(t):
+    return (isinstance(t, torch.Tensor) and t.dtype == torch.int32 and t.is_cuda and t.dim() == 1
+            and t.is_contiguous())
+
+
 def _check_layout(layout, name):
     blocks, offsets = layout
-    for t, what in ((blocks, "blocks"), (offsets, "offset_table")):
-        if not (isinstance(t, torch.Tensor) and t.dtype == torch.int32 and t.is_cuda and t.dim() == 1
-                and t.is_contiguous()):
-            raise ValueError(f"{name}.{what} must be a contiguous 1-D int32 tensor on the GPU")
+    if not (_is_table(blocks) and _is_table(offsets)):
+        what = "offset_table" if _is_table(blocks) else "blocks"
+        raise ValueError(f"{name}.{what} must be a contiguous 1-D int32 tensor on the GPU")
     if blocks.numel() % 2 or offsets.numel() < 2:
         raise ValueError(f"{name} is malformed")
 
@@ -367,7 +384,7 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
             and a.dtype != torch.float32 and size_n % 64 == 0 and num_blocks > 0):
         (cblocks, coffsets), crows, ccols = coarse
         sched = schedule_for((cblocks, coffsets), SCHEDULE_BLOCK64)
-        with torch.cuda.device(a.device):
+        with _k.on_device(a.device):
             _k.check(_k.lib.bsa_matmul_dsd_block64(
                 _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), cblocks.data_ptr(), coffsets.data_ptr(),
                 sched.table.data_ptr(), sched.workgroups, sched.waves, crows, ccols, cblocks.numel() // 2, batches,
@@ -378,7 +395,7 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
             and size_n % 64 == 0):
         runs = _run_schedule(layout, batches, size_n // 64)
         if runs is not None:
-            with torch.cuda.device(a.device):
+            with _k.on_device(a.device):
                 _k.check(_k.lib.bsa_matmul_dsd_runs(
                     _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(),
                     layout[1].data_ptr(), runs.table.data_ptr(), runs.runs, runs.strips, runs.pairs, runs.waves,
@@ -390,7 +407,7 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
             and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
             and _takes_panels(num_blocks, size_m * batches if shared else size_m, 1 if shared else batches,
                               size_k // BLOCK, size_n // BLOCK)):
-        with torch.cuda.device(a.device):
+        with _k.on_device(a.device):
             _k.check(_k.lib.bsa_matmul_dds_panels(
                 _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
                 mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_m, int(trans_b),
@@ -401,7 +418,7 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
         sched = schedule_for(layout, SCHEDULE_SDD_F32 if a.dtype == torch.float32 else SCHEDULE_SDD)
     else:
         sched = _group_walk_schedule(layout)
-    with torch.cuda.device(a.device):
+    with _k.on_device(a.device):
         stream = _k.current_stream()
         ws, ws_bytes = sched.workspace(_k.MODES[mode], batches, size_m, size_n, stream)
         _launch(sched, _k.lib.bsa_matmul(
@@ -442,7 +459,7 @@ def sparse_weight_gradient(a, b, row_layout, col_layout, trans_a, trans_b):
         out = torch.empty((nnz, BLOCK, BLOCK), dtype=a.dtype, device=a.device)
         shares = _k.lib.bsa_weight_grad_shares(rows, cols, tokens)
         parts = torch.empty(shares * nnz * BLOCK * BLOCK, dtype=torch.float32, device=a.device)
-        with torch.cuda.device(a.device):
+        with _k.on_device(a.device):
             _k.check(_k.lib.bsa_weight_grad(
                 _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), out.data_ptr(), row_layout[0].data_ptr(),
                 row_layout[1].data_ptr(), rows, cols, nnz, tokens, shares, parts.data_ptr(), 4 * parts.numel(),
@@ -477,7 +494,7 @@ def sparse_softmax_forward(x, row_blocks, row_table, scale=1.0, causal=False, co
     if nnz == 0 or x.numel() == 0:
         return y
     sched = _softmax_schedule(row_layout, x.dtype, False)
-    with torch.cuda.device(x.device):
+    with _k.on_device(x.device):
         _k.check(_k.lib.bsa_softmax_forward(
             _DTYPES[x.dtype], x.data_ptr(), y.data_ptr(), row_blocks.data_ptr(), row_table.data_ptr(),
             sched.table.data_ptr(), sched.workgroups, sched.waves, mask_rows, mask_cols, nnz, batches,
@@ -497,7 +514,7 @@ def sparse_softmax_backward(y, dy, row_blocks, row_table, scale=1.0, col_layout=
     if nnz == 0 or y.numel() == 0:
         return dx
     sched = _softmax_schedule(row_layout, y.dtype, True)
-    with torch.cuda.device(y.device):
+    with _k.on_device(y.device):
         _k.check(_k.lib.bsa_softmax_backward(
             _DTYPES[y.dtype], y.data_ptr(), dy.data_ptr(), dx.data_ptr(), row_blocks.data_ptr(),
             row_table.data_ptr(), sched.table.data_ptr(), sched.workgroups, sched.waves,
@@ -542,7 +559,7 @@ def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=F
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device) if return_lse else None
     if out.numel() > 0:
         sched = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION, batches)
-        with torch.cuda.device(q.device):
+        with _k.on_device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = sched.attention_workspace(batches, head, stream)
             _launch(sched, _k.lib.bsa_attention_forward(
@@ -573,7 +590,7 @@ def sparse_attention_backward_scores(q, k, v, dout, out, lse, row_blocks, row_ta
     dq = torch.empty_like(q) if with_dq else None
     if q.numel() > 0:
         sched = _attention_schedule(row_layout, SCHEDULE_ATTENTION_BACKWARD, split=ATTENTION_SPLIT_ROWS)
-        with torch.cuda.device(q.device):
+        with _k.on_device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = sched.attention_backward_workspace(None, batches, head, stream) if with_dq else (None, 0)
             _launch(sched, _k.lib.bsa_attention_backward_scores(
@@ -606,7 +623,7 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
         delta = torch.empty_like(lse)
         rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
         cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches)
-        with torch.cuda.device(q.device):
+        with _k.on_device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = rs.attention_backward_workspace(cs, batches, head, stream)
             _launch(rs, _k.lib.bsa_attention_gradients(

@@ -7,6 +7,7 @@ opened with ctypes; torch tensors cross the boundary as raw device pointers and
 the current HIP stream.  If the library is missing the import fails loudly:
 there is no fallback path.
 """
+import contextlib
 import ctypes
 import os
 
@@ -83,8 +84,25 @@ def check(status: int) -> None:
         raise BsaError(f"bsa status {status}: {lib.bsa_last_error().decode()}")
 
 
+# The stream and device queries every call makes, as torch's own generated code makes them: 0.1 us each against 3.1 us
+# for torch.cuda.current_stream() (which builds a Stream object) and 1.5 us for entering torch.cuda.device.
+_current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else torch.cuda.current_device
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def current_stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current stream of the current device."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing to enter when that is the current device already."""
+    return _SAME_DEVICE if device.index == _current_device() else torch.cuda.device(device)
 
 
 from . import _ops as sparse_ops  # noqa: E402  (module with the reference's sparse_matmul signature)

@@ -71,7 +71,7 @@ class SparseLayout:
         nnz_dev = torch.empty(1, dtype=torch.int32, device=self.device)
         workspace = torch.empty(_k.lib.bsa_layout_workspace_bytes(rows, cols), dtype=torch.uint8,
                                 device=self.device)
-        with torch.cuda.device(self.device):
+        with _k.on_device(self.device):
             _k.check(_k.lib.bsa_layout_build(
                 mask.data_ptr(), rows, cols, row_blocks.data_ptr(), row_offsets.data_ptr(),
                 col_blocks.data_ptr(), col_offsets.data_ptr(), nnz_dev.data_ptr(),
@@ -94,7 +94,7 @@ class SparseLayout:
             co = torch.empty(crows + 1, dtype=torch.int32, device=self.device)
             co2 = torch.empty(ccols + 1, dtype=torch.int32, device=self.device)
             cws = torch.empty(_k.lib.bsa_layout_workspace_bytes(crows, ccols), dtype=torch.uint8, device=self.device)
-            with torch.cuda.device(self.device):
+            with _k.on_device(self.device):
                 _k.check(_k.lib.bsa_layout_build(cmask.data_ptr(), crows, ccols, cb.data_ptr(), co.data_ptr(),
                                                  cb2.data_ptr(), co2.data_ptr(), nnz_dev.data_ptr(), cws.data_ptr(),
                                                  _k.current_stream()))
@@ -125,7 +125,7 @@ class SparseLayout:
             batches *= n
         if out.numel() == 0 or batches == 0:
             return out
-        with torch.cuda.device(self.device):
+        with _k.on_device(self.device):
             if gather:
                 _k.check(_k.lib.bsa_to_sparse(_COPY_DTYPES[x.dtype], x.data_ptr(), out.data_ptr(),
                                               self.row_layout[0].data_ptr(), rows, cols, self.num_blocks, batches,
