@@ -74,6 +74,21 @@ int bsa_layout_build(const uint8_t *mask, int mask_rows, int mask_cols,
                         "bsa_layout_build");
 }
 
+int bsa_layout_finish(const int32_t *row_in, const int32_t *col_in, int nnz, int mask_rows, int mask_cols,
+                      int32_t *row_blocks, int32_t *col_blocks, int64_t *positions, int64_t *cells, void *stream)
+{
+    const char *who = "bsa_layout_finish";
+    if (mask_rows < 1 || mask_rows > 32767 || mask_cols < 1 || mask_cols > 65535)
+        return fail(BSA_ERR_INVALID, "%s: mask shape %d x %d out of range", who, mask_rows, mask_cols);
+    if (nnz < 0 || (long long)nnz > (long long)mask_rows * mask_cols)
+        return fail(BSA_ERR_INVALID, "%s: nnz %d does not fit a %d x %d mask", who, nnz, mask_rows, mask_cols);
+    if (nnz == 0) return BSA_OK;
+    if (!row_in || !col_in || !row_blocks || !col_blocks || !positions || !cells)
+        return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    return check_launch(bsa::launch_layout_finish(row_in, col_in, nnz, mask_cols, row_blocks, col_blocks, positions, cells,
+                                                  (hipStream_t)stream), who);
+}
+
 static int check_block_copy(const char *who, int dtype, const void *a, const void *b, const void *t0, const void *t1,
                             int mask_rows, int mask_cols, int nnz, int batches)
 {

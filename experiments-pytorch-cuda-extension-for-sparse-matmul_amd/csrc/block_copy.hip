@@ -42,28 +42,37 @@ __global__ __launch_bounds__(64 * BC_WAVES) void to_sparse_kernel(
 }
 
 // ordinal_of[cell] = number of stored blocks in front of the cell in row-major order (what
-// layout_build_kernel leaves in its workspace): the block index of a stored cell
+// layout_build_kernel leaves in its workspace): the block index of a stored cell.
+// Bound by what it writes, mostly zeros: a wave takes as many neighbouring cells of a mask row as make 256 bytes of a
+// dense row (four of fp16, two of fp32), so that a request writes whole lines; a lane keeps to one column piece, i.e. to one
+// cell.  One fp16 cell a wave wrote 64-byte halves of lines: 8 matrices of 2048 x 2048, a tenth of the cells stored,
+// 20.9 -> 18.5 us.
 template <int ES>
 __global__ __launch_bounds__(64 * BC_WAVES) void to_dense_kernel(
     const unsigned char *__restrict__ sparse, unsigned char *__restrict__ dense,
     const uint8_t *__restrict__ mask, const int *__restrict__ ordinal_of, int nnz, int batches, int R, int C)
 {
-    const int cell = (int)blockIdx.x * BC_WAVES + wave_id();
-    if (cell >= R * C) return;
-    const int l = lane_id();
-    const int r = cell / C, c = cell - r * C;
-    const bool stored = mask[cell] != 0;
-    const int idx = stored ? ordinal_of[cell] : 0;
+    constexpr int CELLS = 8 / ES;                        // of a wave
+    const int chunks = (C + CELLS - 1) / CELLS;
+    const int chunk = (int)blockIdx.x * BC_WAVES + wave_id();
+    if (chunk >= R * chunks) return;
+    const int l = lane_id(), piece = l & 15;
+    const int r = chunk / chunks, c0 = (chunk - r * chunks) * CELLS, c = c0 + piece / (2 * ES);
+    if (c >= C) return;
+    const bool stored = mask[(size_t)r * C + c] != 0;
+    const int idx = stored ? ordinal_of[(size_t)r * C + c] : 0;
     const size_t row_bytes = (size_t)C * BS * ES;
     for (int b = (int)blockIdx.y; b < batches; b += (int)gridDim.y) {
-        unsigned char *dst = dense + ((size_t)b * R * BS + (size_t)BS * r) * row_bytes + (size_t)BS * ES * c;
-        const unsigned char *src = sparse + ((size_t)b * nnz + idx) * BS2 * ES;
+        unsigned char *dst = dense + ((size_t)b * R * BS + (size_t)BS * r + (l >> 4)) * row_bytes + (size_t)BS * ES * c0 + 16 * piece;
+        const unsigned char *src = sparse + ((size_t)b * nnz + idx) * BS2 * ES + (size_t)(l >> 4) * BS * ES + 16 * (piece % (2 * ES));
+        uint4 v[8];
 #pragma unroll
-        for (int q = 0; q < ES; ++q) {
-            const int p = l + WAVE * q;
-            const uint4 v = stored ? ldg16_stream(src + 16 * p) : make_uint4(0, 0, 0, 0);
-            stg16_stream(dst + dense_piece_offset<ES>(p, row_bytes), v);
+        for (int q = 0; q < 8; ++q) {
+            v[q] = make_uint4(0, 0, 0, 0);
+            if (stored) v[q] = ldg16_stream(src + (size_t)4 * q * BS * ES);
         }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) stg16_stream(dst + (size_t)4 * q * row_bytes, v[q]);
     }
 }
 
@@ -83,7 +92,8 @@ hipError_t launch_to_sparse(int elem_size, const void *dense, void *sparse, cons
 hipError_t launch_to_dense(int elem_size, const void *sparse, void *dense, const uint8_t *mask,
                            const int32_t *ordinal_of, int nnz, int batches, int R, int C, hipStream_t st)
 {
-    dim3 grid((unsigned)((R * C + BC_WAVES - 1) / BC_WAVES), (unsigned)(batches < 65535 ? batches : 65535)), block(64 * BC_WAVES);
+    const int cells = 8 / elem_size, chunks = R * ((C + cells - 1) / cells);
+    dim3 grid((unsigned)((chunks + BC_WAVES - 1) / BC_WAVES), (unsigned)(batches < 65535 ? batches : 65535)), block(64 * BC_WAVES);
     if (elem_size == 2)
         to_dense_kernel<2><<<grid, block, 0, st>>>((const unsigned char *)sparse, (unsigned char *)dense, mask,
                                                   ordinal_of, nnz, batches, R, C);

@@ -10,6 +10,9 @@ hipError_t launch_layout_build(const uint8_t *mask, int R, int C, int32_t *row_b
                                int32_t *row_off, int32_t *col_blocks, int32_t *col_off,
                                int32_t *nnz_out, void *workspace, hipStream_t stream);
 
+hipError_t launch_layout_finish(const int32_t *row_in, const int32_t *col_in, int nnz, int C, int32_t *row_blocks,
+                                int32_t *col_blocks, int64_t *positions, int64_t *cells, hipStream_t stream);
+
 hipError_t launch_schedule_build(const int32_t *offsets, int groups, int cap, int waves,
                                  int flags, int slice_max, int slices, int32_t *sched, int64_t capacity,
                                  int32_t *counts_out, hipStream_t stream);

@@ -88,6 +88,32 @@ __global__ __launch_bounds__(LB_THREADS) void layout_build_kernel(
     }
 }
 
+// What a layout keeps, once its number of blocks is known: both tables at their exact size and, from the row table, the
+// (row, column) and the cell number of every block.  One launch in place of two copies and seven elementwise ones.
+__global__ __launch_bounds__(256) void layout_finish_kernel(
+    const int2 *__restrict__ row_in, const int2 *__restrict__ col_in, int nnz, int C,
+    int2 *__restrict__ row_blocks, int2 *__restrict__ col_blocks, longlong2 *__restrict__ positions,
+    long long *__restrict__ cells)
+{
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (i >= nnz) return;
+    const int2 d = row_in[i];
+    row_blocks[i] = d;
+    col_blocks[i] = col_in[i];
+    const long long r = (long long)((unsigned)d.y >> 16), c = (long long)(d.y & 0xFFFF);
+    positions[i] = make_longlong2(r, c);
+    cells[i] = r * C + c;
+}
+
+hipError_t launch_layout_finish(const int32_t *row_in, const int32_t *col_in, int nnz, int C, int32_t *row_blocks,
+                                int32_t *col_blocks, int64_t *positions, int64_t *cells, hipStream_t st)
+{
+    layout_finish_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, st>>>((const int2 *)row_in, (const int2 *)col_in, nnz, C,
+                                                                        (int2 *)row_blocks, (int2 *)col_blocks,
+                                                                        (longlong2 *)positions, (long long *)cells);
+    return hipGetLastError();
+}
+
 // ---- schedule -------------------------------------------------------------
 // Buffer layout (int4 units): [0, groups) per-group meta, then the wavefront slots.
 //   meta[g] = (first slot of part 0, first partial-tile slot or -1, ordinal among split groups or -1, parts)

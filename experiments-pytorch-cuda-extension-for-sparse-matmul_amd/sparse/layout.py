@@ -59,30 +59,38 @@ class SparseLayout:
         self.tile_shape = (rows, cols)                  # the mask the tables describe, in 32x32 tiles
         self.device = torch.device(device)
 
-        mask = (pattern != 0).to(device=self.device, dtype=torch.uint8)
+        mask = (pattern != 0).to(device=self.device).view(torch.uint8)      # one byte a cell either way
         if per_side > 1:
             mask = mask.repeat_interleave(per_side, 0).repeat_interleave(per_side, 1)
         mask = mask.contiguous()
         cells = rows * cols
-        row_blocks = torch.empty(2 * cells, dtype=torch.int32, device=self.device)
-        col_blocks = torch.empty(2 * cells, dtype=torch.int32, device=self.device)
+        # tables of a full mask, the number of blocks behind them: what is stored is known when the kernel has run
+        scratch = torch.empty(4 * cells + 1, dtype=torch.int32, device=self.device)
+        row_cap, col_cap = scratch.data_ptr(), scratch.data_ptr() + 8 * cells
         row_offsets = torch.empty(rows + 1, dtype=torch.int32, device=self.device)
         col_offsets = torch.empty(cols + 1, dtype=torch.int32, device=self.device)
-        nnz_dev = torch.empty(1, dtype=torch.int32, device=self.device)
         workspace = torch.empty(_k.lib.bsa_layout_workspace_bytes(rows, cols), dtype=torch.uint8,
                                 device=self.device)
         with _k.on_device(self.device):
             _k.check(_k.lib.bsa_layout_build(
-                mask.data_ptr(), rows, cols, row_blocks.data_ptr(), row_offsets.data_ptr(),
-                col_blocks.data_ptr(), col_offsets.data_ptr(), nnz_dev.data_ptr(),
-                workspace.data_ptr(), _k.current_stream()))
-        nnz = int(nnz_dev.item())
+                mask.data_ptr(), rows, cols, row_cap, row_offsets.data_ptr(), col_cap, col_offsets.data_ptr(),
+                row_cap + 16 * cells, workspace.data_ptr(), _k.current_stream()))
+        nnz = int(scratch[4 * cells].item())
         self.num_blocks = nnz                           # stored 32x32 tiles: the length of a block stack
         self._mask = mask
         self._ordinals = workspace          # int32[rows * cols]: block index of every stored cell
         # exact-size tensors: the boundary derives nnz from blocks.size(0) / 2 (sparse_kernels.cc:13)
-        self.row_layout: Tuple[torch.Tensor, torch.Tensor] = (row_blocks[:2 * nnz].clone(), row_offsets)
-        self.col_layout: Tuple[torch.Tensor, torch.Tensor] = (col_blocks[:2 * nnz].clone(), col_offsets)
+        row_blocks = torch.empty(2 * nnz, dtype=torch.int32, device=self.device)
+        col_blocks = torch.empty(2 * nnz, dtype=torch.int32, device=self.device)
+        # [nnz, 2] (row, col) in row-major order == torch.nonzero(pattern) (layout.py:8)
+        self.sparse_positions = torch.empty((nnz, 2), dtype=torch.int64, device=self.device)
+        self._cell_index = torch.empty(nnz, dtype=torch.int64, device=self.device)
+        with _k.on_device(self.device):
+            _k.check(_k.lib.bsa_layout_finish(
+                row_cap, col_cap, nnz, rows, cols, row_blocks.data_ptr(), col_blocks.data_ptr(),
+                self.sparse_positions.data_ptr(), self._cell_index.data_ptr(), _k.current_stream()))
+        self.row_layout: Tuple[torch.Tensor, torch.Tensor] = (row_blocks, row_offsets)
+        self.col_layout: Tuple[torch.Tensor, torch.Tensor] = (col_blocks, col_offsets)
 
         self.coarse_row_layout = None
         if per_side > 1:
@@ -93,6 +101,7 @@ class SparseLayout:
             cb2 = torch.empty_like(cb)
             co = torch.empty(crows + 1, dtype=torch.int32, device=self.device)
             co2 = torch.empty(ccols + 1, dtype=torch.int32, device=self.device)
+            nnz_dev = torch.empty(1, dtype=torch.int32, device=self.device)
             cws = torch.empty(_k.lib.bsa_layout_workspace_bytes(crows, ccols), dtype=torch.uint8, device=self.device)
             with _k.on_device(self.device):
                 _k.check(_k.lib.bsa_layout_build(cmask.data_ptr(), crows, ccols, cb.data_ptr(), co.data_ptr(),
@@ -100,11 +109,6 @@ class SparseLayout:
                                                  _k.current_stream()))
             self.coarse_row_layout = (cb[:nnz // 2].clone(), co)
             self.row_layout[1]._bsa_coarse = (self.coarse_row_layout, crows, ccols)
-
-        packed = self.row_layout[0].view(-1, 2)[:, 1].long()
-        # [nnz, 2] (row, col) in row-major order == torch.nonzero(pattern) (layout.py:8)
-        self.sparse_positions = torch.stack((packed >> 16, packed & 0xFFFF), dim=1)
-        self._cell_index = (self.sparse_positions[:, 0] * cols + self.sparse_positions[:, 1])
 
     def _index_on(self, device) -> torch.Tensor:
         if self._cell_index.device != device:

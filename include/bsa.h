@@ -85,6 +85,12 @@ int bsa_layout_build(const uint8_t *mask, int mask_rows, int mask_cols,
                      int32_t *col_blocks, int32_t *col_offsets,
                      int32_t *nnz_out, void *workspace, void *stream);
 
+/* What a layout keeps of those tables: their first nnz pairs at their exact size, and the position (row, column)
+ * (int64 [nnz, 2]) and the cell number row * mask_cols + column (int64 [nnz]) of every block in row-major order.
+ */
+int bsa_layout_finish(const int32_t *row_in, const int32_t *col_in, int nnz, int mask_rows, int mask_cols,
+                      int32_t *row_blocks, int32_t *col_blocks, int64_t *positions, int64_t *cells, void *stream);
+
 /* ---- dense matrix <-> stack of its stored blocks ---------------------------
  * Replace SparseLayout.to_sparse / to_dense (sparse/layout.py:40-57).
  *   dense   [batches, 32 * mask_rows, 32 * mask_cols], contiguous
