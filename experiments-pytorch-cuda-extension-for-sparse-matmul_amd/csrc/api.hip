@@ -622,8 +622,10 @@ static int attention_backward(const char *who, int dtype, const void *q, const v
     if (head_dim == 128 && col_sched_waves > bsa::AT_COLUMN_WAVES_128)
         return fail(BSA_ERR_INVALID, "%s: the column schedule has %d waves per workgroup, at most %d at head_dim 128", who,
                     col_sched_waves, bsa::AT_COLUMN_WAVES_128);
-    if (!q || !k || !v || !dout || !out || !lse || !dq_out || !dk_out || !dv_out || !delta_ws)
+    if (!q || !k || !v || !dout || !out || !lse || !dq_out || !delta_ws)
         return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    if ((dk_out == nullptr) != (dv_out == nullptr))
+        return fail(BSA_ERR_INVALID, "%s: dk_out and dv_out go together", who);
     rc = check_split_workspace(who, row_tile_slots, row_split_groups);
     if (rc) return rc;
     rc = check_split_workspace(who, col_tile_slots, col_split_groups);
@@ -645,7 +647,7 @@ static int attention_backward(const char *who, int dtype, const void *q, const v
     p.split_groups = row_split_groups;
     p.workspace = workspace;
     rc = check_launch(bsa::launch_attention_backward_scores(p, (hipStream_t)stream), who);
-    if (rc) return rc;
+    if (rc || !dk_out) return rc;
     p.blocks = col_blocks;
     p.sched = col_sched;
     p.groups = mask_cols;
@@ -676,6 +678,7 @@ int bsa_attention_backward(int dtype, const void *q, const void *k, const void *
         return fail(BSA_ERR_UNSUPPORTED,
                     "bsa_attention_backward: head_dim 64 is built, got %d (bsa_attention_gradients takes both)",
                     head_dim);
+    if (!dk_out || !dv_out) return fail(BSA_ERR_INVALID, "bsa_attention_backward: null pointer argument");
     return attention_backward("bsa_attention_backward", dtype, q, k, v, dout, out, lse, dq_out, dk_out, dv_out,
                               delta_ws, row_blocks, row_offsets, row_sched, row_sched_wgs, row_sched_waves,
                               row_tile_slots, row_split_groups, col_blocks, col_offsets, col_sched, col_sched_wgs, col_sched_waves, col_tile_slots,

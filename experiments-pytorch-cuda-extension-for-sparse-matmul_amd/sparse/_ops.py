@@ -604,11 +604,12 @@ def sparse_attention_backward_scores(q, k, v, dout, out, lse, row_blocks, row_ta
 
 
 def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, col_blocks, col_table, scale=1.0,
-                              causal=False):
+                              causal=False, with_dkdv=True):
     """``(dq, dk, dv)`` of the fused attention in two launches (a walk over the rows, one over the
     columns), the probabilities and score gradients rebuilt in registers in both instead of stored:
     the seven launches of the unfused backward chain (sparse/matmul.py:27-52, sparse_softmax.cu:165-205)
-    without a block stack in memory.  fp16 / bf16, head dim 64 or 128."""
+    without a block stack in memory.  fp16 / bf16, head dim 64 or 128.  ``with_dkdv=False``: dq alone (None for the
+    others), one launch."""
     col_layout = (col_blocks, col_table)
     _check_layout(col_layout, "col_layout")
     row_layout, mask_rows, mask_cols, nnz, head, batches = _attention_common(q, k, v, row_blocks, row_table,
@@ -618,7 +619,8 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
     if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
         raise ValueError("lse must be the float32 row statistics of the forward pass")
     q, k, v, dout, out, lse = (t.contiguous() for t in (q, k, v, dout, out, lse))
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    dq = torch.empty_like(q)
+    dk, dv = (torch.empty_like(k), torch.empty_like(v)) if with_dkdv else (None, None)
     if q.numel() > 0:
         delta = torch.empty_like(lse)
         rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
@@ -628,7 +630,8 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
             ws, ws_bytes = rs.attention_backward_workspace(cs, batches, head, stream)
             _launch(rs, _k.lib.bsa_attention_gradients(
                 _DTYPES[q.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), out.data_ptr(),
-                lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr(),
+                lse.data_ptr(), dq.data_ptr(), dk.data_ptr() if with_dkdv else None, dv.data_ptr() if with_dkdv else None,
+                delta.data_ptr(),
                 row_blocks.data_ptr(), row_table.data_ptr(), rs.table.data_ptr(), rs.workgroups, rs.waves,
                 rs.tile_slots, rs.split_groups,
                 col_blocks.data_ptr(), col_table.data_ptr(), cs.table.data_ptr(), cs.workgroups, cs.waves,

@@ -33,7 +33,8 @@ class SparseAttention(torch.autograd.Function):
         rows, cols = layout.row_layout, layout.col_layout
         # two launches, nothing stored per block: a walk over the rows for dq, one over the columns for dk and dv
         dq, dk, dv = sparse_ops.sparse_attention_backward(q, k, v, dout.contiguous(), out, lse, rows[0], rows[1], cols[0],
-                                                          cols[1], ctx.scale, ctx.causal)
+                                                          cols[1], ctx.scale, ctx.causal,
+                                                          with_dkdv=ctx.needs_input_grad[1] or ctx.needs_input_grad[2])
         return dq, dk, dv, None, None, None
 
 

@@ -355,7 +355,8 @@ int bsa_attention_backward(int dtype, const void *q, const void *k, const void *
                            int mask_rows, int mask_cols, int nnz, int batches, int head_dim,
                            float scale, int causal, void *stream);
 
-/* bsa_attention_backward for head_dim 64 and 128.  At 128 the column schedule has at most 4 waves per workgroup. */
+/* bsa_attention_backward for head_dim 64 and 128.  At 128 the column schedule has at most 4 waves per workgroup.
+ * dk_out and dv_out both null: dq alone, without the walk over the columns. */
 int bsa_attention_gradients(int dtype, const void *q, const void *k, const void *v, const void *dout,
                            const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
                            float *delta_ws,

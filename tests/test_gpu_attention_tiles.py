@@ -42,3 +42,24 @@ def test_column_schedule_of_head_dim_128_is_checked():
     rc = k.lib.bsa_attention_gradients(1, P, P, P, P, P, P, P, P, P, P, P, P, P, 4, 4, 0, 0, P, P, P, 4, 8, 0, 0, None, 0,
                                        4, 4, 5, 1, 128, 1.0, 0, None)
     assert rc == -1 and "at most 4" in k.lib.bsa_last_error().decode()
+
+
+@pytest.mark.parametrize("head", [64, 128])
+def test_queries_alone_need_no_column_walk(head):
+    import sparse
+    from sparse import kernel as k
+    mask = np.asarray(ZOO["rand16"])
+    L = sparse.SparseLayout(torch.as_tensor(mask))
+    g = torch.Generator().manual_seed(43)
+    mk = lambda n: torch.randn(2, 32 * n, head, generator=g).half().cuda()
+    q, kk, v, dout = mk(mask.shape[0]), mk(mask.shape[1]), mk(mask.shape[1]), mk(mask.shape[0])
+    q.requires_grad_()
+    k_grad = kk.clone().requires_grad_()
+    want = torch.autograd.grad(sparse.attention(q, k_grad, v, L, 0.11), (q, k_grad), dout)[0]
+    out = sparse.attention(q, kk, v, L, 0.11)
+    got, = torch.autograd.grad(out, q, dout)
+    assert torch.equal(got, want)
+    P = 0x1000
+    rc = k.lib.bsa_attention_gradients(1, P, P, P, P, P, P, P, None, P, P, P, P, P, 4, 4, 0, 0, P, P, P, 4, 4, 0, 0, None, 0,
+                                       4, 4, 5, 1, head, 1.0, 0, None)
+    assert rc == -1 and "go together" in k.lib.bsa_last_error().decode()
