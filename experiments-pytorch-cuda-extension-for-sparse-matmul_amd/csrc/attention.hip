@@ -510,38 +510,47 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                 const int r = win.get(p).row();
                 const bool last = p + 1 == seg_end, masked = causal && c >= r;
                 h8 pop[2], ds[2];                // queries 8 (v / 4) + 4 h + v % 4 of this lane's key
-                tile_wait<0>();
+                // The probabilities need Q and lse only: dO, requested last, has the whole of them to arrive in (one wait for
+                // both before: training pass of 48 heads of 8192 tokens 274.9 -> 271.8 us, bf16).
+                tile_wait<TileRequests<HD>::N>();            // everything but dO
+                f16v prob = {0};
                 {
-                    f16v sacc = {0}, dpacc = {0};
-                    {
-                        h8 qop[KS];
+                    h8 qop[KS];
 #pragma unroll
-                        for (int s = 0; s < KS; ++s) qop[s] = rd.rows(Q_TILE, s);
+                    for (int s = 0; s < KS; ++s) qop[s] = rd.rows(Q_TILE, s);
 #pragma unroll
-                        for (int s = 0; s < KS; ++s) sacc = mfma_16<BF>(qop[s], kop[s], sacc);
-                    }
-                    {
-                        h8 dop[KS];
-#pragma unroll
-                        for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
-#pragma unroll
-                        for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], vop[s], dpacc);
-                    }
+                    for (int s = 0; s < KS; ++s) prob = mfma_16<BF>(qop[s], kop[s], prob);
                     if (masked) {                // a hidden score has no probability
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            if (c > r || key > 8 * (v >> 2) + 4 * h + (v & 3)) sacc[v] = scale2 < 0.f ? __builtin_inff() : -__builtin_inff();
+                            if (c > r || key > 8 * (v >> 2) + 4 * h + (v & 3)) prob[v] = scale2 < 0.f ? __builtin_inff() : -__builtin_inff();
                     }
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f4v ls = *reinterpret_cast<const f4v *>(stats + 8 * g + 4 * h);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int v = 4 * g + j;
+                            prob[v] = at_exp2(__builtin_fmaf(prob[v], scale2, -ls[j]));
+                            pop[v >> 3][v & 7] = narrow_16<BF>(prob[v]);
+                        }
+                    }
+                }
+                tile_wait<0>();
+                {
+                    f16v dpacc = {0};
+                    h8 dop[KS];
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], vop[s], dpacc);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
                         const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h);
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const int v = 4 * g + j;
-                            const float pr = at_exp2(__builtin_fmaf(sacc[v], scale2, -ls[j]));
-                            pop[v >> 3][v & 7] = narrow_16<BF>(pr);
-                            ds[v >> 3][v & 7] = narrow_16<BF>(pr * __builtin_fmaf(dpacc[v], scale, -dl[j]));
+                            ds[v >> 3][v & 7] = narrow_16<BF>(prob[v] * __builtin_fmaf(dpacc[v], scale, -dl[j]));
                         }
                     }
                 }
