@@ -65,7 +65,7 @@ def kernel_sources_sha256() -> str:
 
 # kernel name fragment -> row of the traffic table (rocprofv3 --pmc, one counter per run)
 TRAFFIC_KERNELS = [("sdd_f16_kernel", "sdd"), ("dsd_runs_f16_kernel", "dsd"), ("gw_f16_kernel", "dds"),
-                   ("softmax_fwd_kernel", "softmax"), ("attention_fwd", "attn"), ("attention_bwd_scores", "bwd_rows"),
+                   ("softmax_fwd_kernel", "softmax"), ("attention_fwd", "attn"), ("attention_bwd_rows", "bwd_rows"),
                    ("attention_bwd_dkdv", "bwd_cols")]
 CALIBRATION_KIB = 65536.0          # what the cold 64 MiB torch.neg in front of the timed loops reads, and writes
 
