@@ -314,23 +314,24 @@ int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void
         return fail(BSA_ERR_INVALID, "%s: mask shape %d x %d out of range", who, mask_rows, mask_cols);
     if (nnz < 0 || (long long)nnz > (long long)mask_rows * mask_cols)
         return fail(BSA_ERR_INVALID, "%s: nnz %d does not fit a %d x %d mask", who, nnz, mask_rows, mask_cols);
-    if (batches < 1 || batches > 65535 || (sparse_batches != batches && sparse_batches != 1))
+    if (batches < 1 || (sparse_batches != batches && sparse_batches != 1))
         return fail(BSA_ERR_INVALID, "%s: batches %d, sparse_batches %d", who, batches, sparse_batches);
+    // a shared weight sees the batch as one long matrix: the second grid dimension counts entries that have weights of their own
+    const bool fold = sparse_batches == 1;
+    if (!fold && batches > 65535) return fail(BSA_ERR_INVALID, "%s: %d batches with a weight each, at most 65535", who, batches);
     if (M < 1 || M % BSA_BLOCK)
         return fail(BSA_ERR_INVALID, "%s: %d dense rows are no positive multiple of %d", who, M, BSA_BLOCK);
     const int kblocks = tr_b ? mask_cols : mask_rows, groups = tr_b ? mask_rows : mask_cols;
     if (nnz > bsa::PANEL_MAX_NNZ || kblocks > bsa::PANEL_MAX_KBLOCKS)
         return fail(BSA_ERR_UNSUPPORTED, "%s: %d blocks over %d block rows of the contraction, at most %d over %d are "
                     "built (use bsa_matmul)", who, nnz, kblocks, bsa::PANEL_MAX_NNZ, bsa::PANEL_MAX_KBLOCKS);
+    const long long rows = fold ? (long long)M * batches : M;
+    if (rows > (1LL << 30) || (rows / 64 + 1) * (groups / 8 + 1) > MAX_GRID / 8)
+        return fail(BSA_ERR_INVALID, "%s: %lld dense rows x %d groups are too large", who, rows, groups);
     if (!out || !dense || !offsets || ((!sparse || !blocks) && nnz > 0))
         return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
     if (((uintptr_t)out | (uintptr_t)dense | (uintptr_t)sparse) & 15)
         return fail(BSA_ERR_UNSUPPORTED, "%s: operands must be aligned to 16 bytes (use bsa_matmul)", who);
-    // a shared weight sees the batch as one long matrix
-    const bool fold = sparse_batches == 1;
-    const long long rows = fold ? (long long)M * batches : M;
-    if (rows > (1LL << 30) || (rows / 64 + 1) * (groups / 8 + 1) > MAX_GRID / 8)
-        return fail(BSA_ERR_INVALID, "%s: %lld dense rows x %d groups are too large", who, rows, groups);
     bsa::WeightPanelArgs p{dense, sparse, out, blocks, offsets, groups, nnz, (int)rows, BSA_BLOCK * kblocks,
                            fold ? 1 : batches, tr_b != 0, fold};
     return check_launch(bsa::launch_weight_panels(dtype, p, (hipStream_t)stream), who);

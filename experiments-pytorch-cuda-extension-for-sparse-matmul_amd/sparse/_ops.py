@@ -436,6 +436,7 @@ def _takes_panels(nnz, rows, entries, kblocks, groups):
     (bsa_matmul_dds_panels)."""
     tiles, sets = -(-rows // PANEL_ROWS), -(-groups // PANEL_GROUPS)
     return (kblocks <= PANEL_MAX_KBLOCKS and nnz <= PANEL_MAX_NNZ and entries <= 65535 and rows <= 2 ** 30
+            and (rows // 64 + 1) * (groups // 8 + 1) < 2 ** 28
             and tiles * sets * entries >= PANEL_MIN_WORKGROUPS
             and nnz * rows >= PANEL_MIN_DENSITY * kblocks * groups * tiles * PANEL_ROWS)
 

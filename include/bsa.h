@@ -373,7 +373,8 @@ int bsa_attention_gradients(int dtype, const void *q, const void *k, const void 
 /* DDS with a weight that many dense rows meet: out = dense op(b), dense [batches, M, K] (K contiguous) and out
  * [batches, M, N] as in bsa_matmul(mode 2, tr_a = 0, tr_b), by a walk that keeps panels of the dense operand on the chip
  * for eight groups at a time (no schedule, no workspace).  Tables: the row table with tr_b, the column table without.
- * With sparse_batches = 1 the batch is walked as one matrix of batches * M rows.  fp16 / bf16; at most 2^20 - 1
+ * With sparse_batches = 1 the batch is walked as one matrix of batches * M rows (any number of entries); with a weight
+ * per entry at most 65535 of them.  fp16 / bf16; at most 2^20 - 1
  * blocks and a contraction of at most 1024 blocks (BSA_ERR_UNSUPPORTED otherwise: use bsa_matmul).
  */
 int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void *out, const int32_t *blocks,

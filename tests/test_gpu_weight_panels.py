@@ -54,6 +54,18 @@ def test_panels(any_size, rows, cols, density, batch, m, trans_b, shared, dtype)
     assert _rel(got, want) <= REL[dtype]
 
 
+def test_more_batch_entries_than_a_grid_dimension_holds():
+    import sparse
+    from sparse import _ops
+    L = _layout(1, 1, 1.0, 1)
+    x = torch.randn(65537, 32, 32, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").half()
+    w = torch.randn(1, 32, 32, generator=torch.Generator(device="cuda").manual_seed(4), device="cuda").half()
+    assert _ops._takes_panels(1, 65537 * 32, 1, 1, 1)
+    got = sparse.matmul(x, w, "dds", L)
+    want = x.double().flatten(0, 1) @ w[0].double()
+    assert _rel(got.flatten(0, 1), want) <= REL[torch.float16]
+
+
 @pytest.mark.parametrize("rows,cols,density", [(1, 1, 1.0), (8, 8, 1.0), (9, 7, 0.5), (20, 33, 0.3)])
 @pytest.mark.parametrize("batch,tokens", [(1, 32), (1, 160), (3, 224), (5, 64)])      # 1, 5, 21 and 10 steps: every tail
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

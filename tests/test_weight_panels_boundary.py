@@ -34,3 +34,30 @@ def test_shares_are_bounded(rows, cols, tokens):
     assert 1 <= s <= 256 and (s == 1 or tokens // 32 >= 8 * s)
     cells = -(-rows // 8) * -(-cols // 8)
     assert s == 1 or s <= 8 or s * cells <= 256
+
+
+# An operand that is not aligned is what the call refuses last: whatever else it takes gets as far as that.
+@pytest.mark.parametrize("batches,m", [(1, 2 ** 20), (65535, 64), (65536, 32), (70000, 32), (2 ** 25, 32)])
+def test_every_size_the_rule_accepts_is_accepted(batches, m, monkeypatch):
+    """A shared weight folds the batch into its rows, so the number of batch entries alone is no limit."""
+    import sparse.kernel as k
+    from sparse import _ops
+    monkeypatch.setattr(_ops, "PANEL_MIN_WORKGROUPS", 1)
+    monkeypatch.setattr(_ops, "PANEL_MIN_DENSITY", 0.0)
+    for rows, cols, nnz in ((1, 1, 1), (4, 5, 7), (32, 64, 2048), (1024, 1024, 2 ** 20 - 1)):
+        for tb in (0, 1):
+            kblocks, groups = (cols, rows) if tb else (rows, cols)
+            for shared in (True, False):
+                entries = 1 if shared else batches
+                if not _ops._takes_panels(nnz, m * batches if shared else m, entries, kblocks, groups):
+                    assert batches == 2 ** 25 or not shared and batches > 65535
+                    continue
+                rc = _panels(k, dense=P + 2, rows=rows, cols=cols, nnz=nnz, batches=batches,
+                             sparse_batches=1 if shared else batches, m=m, tb=tb)
+                assert rc != 0 and "aligned" in k.lib.bsa_last_error().decode(), (rows, cols, tb, shared)
+
+
+def test_weights_of_their_own_are_a_grid_dimension():
+    import sparse.kernel as k
+    assert _panels(k, dense=P + 2, batches=65536, sparse_batches=65536) != 0
+    assert "at most 65535" in k.lib.bsa_last_error().decode()
