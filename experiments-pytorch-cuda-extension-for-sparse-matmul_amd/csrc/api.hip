@@ -5,6 +5,7 @@
 // validated on the host before a launch.
 #include <cstdarg>
 #include <cstdio>
+#include <initializer_list>
 
 #include "../../include/bsa.h"
 #include "bsa_internal.hpp"
@@ -491,6 +492,15 @@ static int check_attention(const char *who, int dtype, int head_dim, const int32
     return check_schedule(sched, sched_wgs, sched_waves, batches, who);
 }
 
+// Operands that go from memory straight into LDS, 16 bytes a lane.  Those loads are not specified for less alignment.
+static int check_operand_alignment(const char *who, std::initializer_list<const void *> operands)
+{
+    for (const void *p : operands)
+        if ((uintptr_t)p & 15)
+            return fail(BSA_ERR_UNSUPPORTED, "%s: q, k, v and dout must be aligned to 16 bytes", who);
+    return BSA_OK;
+}
+
 static void fill_attention(bsa::AttentionArgs &p, int dtype, const void *q, const void *k, const void *v,
                            const int32_t *blocks, const int32_t *sched, int groups, int sched_wgs, int sched_waves,
                            int mask_rows, int mask_cols, int nnz, int batches, int head_dim, float scale, int causal)
@@ -531,6 +541,8 @@ int bsa_attention_forward(int dtype, const void *q, const void *k, const void *v
                              mask_rows, mask_cols, nnz, batches);
     if (rc) return rc;
     if (!q || !k || !v || !out) return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    rc = check_operand_alignment(who, {q, k, v});
+    if (rc) return rc;
     if (sched_tile_slots < 0 || sched_split_groups < 0 || (sched_tile_slots > 0) != (sched_split_groups > 0))
         return fail(BSA_ERR_INVALID, "%s: schedule split counts %d, %d are inconsistent", who, sched_tile_slots,
                     sched_split_groups);
@@ -577,6 +589,8 @@ int bsa_attention_backward_scores(int dtype, const void *q, const void *k, const
     if (rc) return rc;
     if (nnz == 0 && !dq_out) return BSA_OK;      // no blocks to write
     if (!q || !k || !v || !dout || !out || !lse) return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    rc = check_operand_alignment(who, {q, k, v, dout});
+    if (rc) return rc;
     if ((p_out == nullptr) != (ds_out == nullptr))
         return fail(BSA_ERR_INVALID, "%s: p_out and ds_out go together", who);
     if (!p_out && !dq_out) return fail(BSA_ERR_INVALID, "%s: no output asked for", who);
@@ -625,6 +639,8 @@ static int attention_backward(const char *who, int dtype, const void *q, const v
                     col_sched_waves, bsa::AT_COLUMN_WAVES_128);
     if (!q || !k || !v || !dout || !out || !lse || !dq_out || !delta_ws)
         return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+    rc = check_operand_alignment(who, {q, k, v, dout});
+    if (rc) return rc;
     if ((dk_out == nullptr) != (dv_out == nullptr))
         return fail(BSA_ERR_INVALID, "%s: dk_out and dv_out go together", who);
     rc = check_split_workspace(who, row_tile_slots, row_split_groups);

@@ -547,6 +547,13 @@ def _attention_common(q, k, v, row_blocks, row_table, col_layout):
     return row_layout, mask_rows, mask_cols, row_blocks.numel() // 2, head, batches
 
 
+def _tile_operand(t):
+    """``t`` contiguous and at a multiple of 16 bytes: the attention walks load it straight to LDS, 16 bytes a lane.  A
+    contiguous view may start anywhere in its storage."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=False, col_layout=None,
                              return_lse=False):
     """``softmax(scale * q k^T on the stored blocks) v`` in one launch: the chain of
@@ -555,7 +562,7 @@ def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=F
     With ``return_lse`` also the fp32 row statistics the backward pass needs."""
     row_layout, mask_rows, mask_cols, nnz, head, batches = _attention_common(q, k, v, row_blocks, row_table,
                                                                               col_layout)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v = _tile_operand(q), _tile_operand(k), _tile_operand(v)
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device) if return_lse else None
     if out.numel() > 0:
@@ -584,7 +591,8 @@ def sparse_attention_backward_scores(q, k, v, dout, out, lse, row_blocks, row_ta
         raise ValueError("dout and out must match q in shape and dtype")
     if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
         raise ValueError("lse must be the float32 row statistics of the forward pass")
-    q, k, v, dout, out, lse = (t.contiguous() for t in (q, k, v, dout, out, lse))
+    q, k, v, dout = (_tile_operand(t) for t in (q, k, v, dout))
+    out, lse = out.contiguous(), lse.contiguous()
     shape = q.shape[:-2] + (nnz, BLOCK, BLOCK)
     p = torch.empty(shape, dtype=q.dtype, device=q.device)
     ds = torch.empty(shape, dtype=q.dtype, device=q.device)
@@ -619,7 +627,8 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
         raise ValueError("dout and out must match q in shape and dtype")
     if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
         raise ValueError("lse must be the float32 row statistics of the forward pass")
-    q, k, v, dout, out, lse = (t.contiguous() for t in (q, k, v, dout, out, lse))
+    q, k, v, dout = (_tile_operand(t) for t in (q, k, v, dout))
+    out, lse = out.contiguous(), lse.contiguous()
     dq = torch.empty_like(q)
     dk, dv = (torch.empty_like(k), torch.empty_like(v)) if with_dkdv else (None, None)
     if q.numel() > 0:

@@ -285,6 +285,7 @@ int bsa_softmax_backward(int dtype, const void *y, const void *dy, void *dx,
  * stored.  Same meaning as bsa_matmul(SDD, q, k, tr_b = 1), bsa_softmax_forward, bsa_matmul(DSD)
  * in a row; the probabilities are rounded to fp16 before the second product, as there.
  *   q    [batches, 32 * mask_rows, head_dim], k, v  [batches, 32 * mask_cols, head_dim], contiguous
+ *   q, k, v (and dout of the backward entry points) start at a multiple of 16 bytes (BSA_ERR_UNSUPPORTED otherwise)
  *   out  [batches, 32 * mask_rows, head_dim]; rows without stored (or unmasked) blocks give zeros
  *   lse  optional (may be NULL) float[batches, 32 * mask_rows]: log2 of every row's sum of
  *        2^(scale * log2(e) * score); +inf for a row that sees nothing.  The backward pass needs it.

@@ -63,3 +63,29 @@ def test_queries_alone_need_no_column_walk(head):
     rc = k.lib.bsa_attention_gradients(1, P, P, P, P, P, P, P, None, P, P, P, P, P, 4, 4, 0, 0, P, P, P, 4, 4, 0, 0, None, 0,
                                        4, 4, 5, 1, head, 1.0, 0, None)
     assert rc == -1 and "go together" in k.lib.bsa_last_error().decode()
+
+
+@pytest.mark.parametrize("head", [64, 128])
+def test_operands_that_start_anywhere(head):
+    """Contiguous views at odd offsets of a flat buffer: the bits of the aligned operands."""
+    import sparse
+    mask = np.asarray(ZOO["rand16"])
+    rows, cols = mask.shape
+    L = sparse.SparseLayout(torch.as_tensor(mask))
+    g = torch.Generator().manual_seed(47)
+    t = [torch.randn(2, 32 * n, head, generator=g).half().cuda() for n in (rows, cols, cols, rows)]
+
+    def step(q, k, v, dout):
+        q, k, v = (x.detach().requires_grad_() for x in (q, k, v))
+        out = sparse.attention(q, k, v, L, 0.11, True)
+        return (out.detach(),) + torch.autograd.grad(out, (q, k, v), dout)
+
+    def moved(x, off):
+        flat = torch.empty(x.numel() + off, dtype=x.dtype, device=x.device)
+        flat[off:] = x.flatten()
+        return flat[off:].view(x.shape)
+
+    want = step(*t)
+    for off in (1, 4, 7):
+        assert moved(t[0], off).data_ptr() % 16 != 0
+        assert all(torch.equal(a, b) for a, b in zip(step(*(moved(x, off) for x in t)), want))
