@@ -69,6 +69,8 @@ SCHEDULE_ATTENTION_BACKWARD_COLUMNS = (12, 2)
 # causal local-4 + stride-8 mask of 4096 tokens, head dim 64, chunks of 12 -> 6 (forward, rows, columns): 1 batch entry
 # (1530 blocks) 10.6 / 12.8 / 18.2 -> 8.1 / 10.0 / 16.2 us; 4 entries (6120) 11.6 / 13.8 / 18.3 -> 10.7 / 13.2 / 17.8; 8
 # entries of a random mask (13100) 15.2 / 18.0 / 19.5 -> 15.8 / 20.5 / 22.1.
+# The workgroup's share (cap * waves) stays what it is for a large launch wherever a group is longer than 24 blocks
+# (_attention_kinds): no launch needs a workspace that another batch count of the same layout does not need.
 SCHEDULE_ATTENTION_SMALL = (6, 4)
 ATTENTION_SMALL_BLOCKS = 8192          # blocks of all batch entries together
 # block rows of at most this many blocks are handed whole to SOFTMAX_SLICES wavefronts (8 element rows
@@ -272,23 +274,35 @@ def _group_walk_schedule(layout):
     return schedule_for(layout, kind)
 
 
-def _attention_schedule(layout, kind, split=False):
-    """Schedule of a fused attention walk.  With ``split`` (what every caller passes while
+def _attention_kind(layout, kind, split):
+    """Arguments of the schedule of a fused attention walk.  With ``split`` (what every caller passes while
     ``ATTENTION_SPLIT_ROWS`` is set) a group longer than the workgroup's share is cut into parts that
     meet in a workspace; without it such a table gets the most waves a workgroup holds instead."""
     cap, waves = kind
-    if split:
-        return schedule_for(layout, (cap, waves, True))
-    if _longest_group(layout[1]) > cap * waves:
+    if not split and _longest_group(layout[1]) > cap * waves:
         waves = ATTENTION_WAVES_LONG_GROUPS
-    return schedule_for(layout, (cap, waves, False))
+    return cap, waves, bool(split)
+
+
+def _attention_schedule(layout, kind, split=False):
+    return schedule_for(layout, _attention_kind(layout, kind, split))
+
+
+def _attention_kinds(kind, few_blocks):
+    """Schedules to consider for a launch, in this order: the first that cuts no group into parts, else the last."""
+    if not few_blocks:
+        return (kind,)
+    chunk = SCHEDULE_ATTENTION_SMALL[0]
+    return SCHEDULE_ATTENTION_SMALL, (chunk, kind[0] * kind[1] // chunk)
 
 
 def _attention_schedule_for(layout, kind, batches):
     """Schedule of a fused attention walk over ``batches`` entries: ``kind``, or shorter chunks for a small launch."""
-    if layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS:
-        kind = SCHEDULE_ATTENTION_SMALL
-    return _attention_schedule(layout, kind, split=ATTENTION_SPLIT_ROWS)
+    for k in _attention_kinds(kind, layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS):
+        sched = _attention_schedule(layout, k, split=ATTENTION_SPLIT_ROWS)
+        if sched.split_groups == 0:
+            break
+    return sched
 
 
 def _softmax_schedule(layout, dtype, backward):

@@ -1,4 +1,4 @@
-"""CPU: what the attention entry points ask of their operands before anything is launched."""
+"""CPU: what the attention entry points ask of their operands before anything is launched, and which schedules they use."""
 import pytest
 import torch
 
@@ -38,3 +38,38 @@ def test_a_view_that_starts_off_a_multiple_of_16_bytes_is_copied():
         assert (got.data_ptr() == t.data_ptr()) == (t.data_ptr() % 16 == 0)
     wide = flat[1:1 + 8 * 128].view(1, 8, 128)[..., :64]
     assert _ops._tile_operand(wide).data_ptr() % 16 == 0
+
+
+class _FakeSchedule:
+    """Split counts of a schedule, as plan_group of csrc/layout_build.hip counts them."""
+
+    def __init__(self, offsets, nnz, cap, waves, allow_split=True, *rest):
+        parts = [-(-int(n) // (cap * waves)) if allow_split else 1 for n in (offsets[1:] - offsets[:-1])]
+        self.cap, self.waves = cap, waves
+        self.split_groups = sum(p > 1 for p in parts)
+        self.tile_slots = sum(p for p in parts if p > 1)
+
+
+@pytest.fixture
+def layout_of(monkeypatch):
+    from sparse import _ops
+    monkeypatch.setattr(_ops, "Schedule", _FakeSchedule)
+    state = {"capturing": False}
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+
+    def layout_of_lengths(*lengths):
+        offsets = torch.tensor([0] + list(lengths)).cumsum(0).int()
+        return torch.zeros(2 * sum(lengths), dtype=torch.int32), offsets
+    layout_of_lengths.capture = lambda on: state.update(capturing=on)
+    return layout_of_lengths
+
+
+@pytest.mark.parametrize("lengths", [(1,), (24, 3), (25, 3), (48, 2, 30), (49, 1), (7, 200, 96, 97)])
+def test_every_batch_count_needs_the_same_workspace(layout_of, lengths):
+    from sparse import _ops
+    for kind in (_ops.SCHEDULE_ATTENTION, _ops.SCHEDULE_ATTENTION_BACKWARD, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS):
+        L = layout_of(*lengths)
+        few, many = (_ops._attention_schedule_for(L, kind, b) for b in (1, 10 ** 5))
+        assert few.cap < many.cap and few.waves <= 8
+        assert (few.split_groups, few.tile_slots) == (many.split_groups, many.tile_slots)
+        assert (few.split_groups == 0) == (max(lengths) <= kind[0] * kind[1])
