@@ -260,6 +260,11 @@ def schedule_for(layout, kind):
     return cache[kind]
 
 
+def _has_schedule(layout, kind) -> bool:
+    """Whether ``schedule_for(layout, kind)`` has nothing to build."""
+    return kind in getattr(layout[1], "_bsa_schedules", ())
+
+
 def _longest_group(offsets) -> int:
     """Pairs in the longest group of a table; measured once and kept on the offsets tensor."""
     longest = getattr(offsets, "_bsa_longest", None)
@@ -297,12 +302,20 @@ def _attention_kinds(kind, few_blocks):
 
 
 def _attention_schedule_for(layout, kind, batches):
-    """Schedule of a fused attention walk over ``batches`` entries: ``kind``, or shorter chunks for a small launch."""
-    for k in _attention_kinds(kind, layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS):
-        sched = _attention_schedule(layout, k, split=ATTENTION_SPLIT_ROWS)
-        if sched.split_groups == 0:
-            break
-    return sched
+    """Schedule of a fused attention walk over ``batches`` entries: ``kind``, or shorter chunks for a small launch.  Nothing
+    can be built under graph capture: there the other length serves when only that one has been used eagerly."""
+    few = layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS
+    for few_blocks in (few, not few):
+        kinds = _attention_kinds(kind, few_blocks)
+        for k in kinds:
+            if not _has_schedule(layout, _attention_kind(layout, k, ATTENTION_SPLIT_ROWS)) \
+                    and torch.cuda.is_current_stream_capturing():
+                break
+            sched = _attention_schedule(layout, k, split=ATTENTION_SPLIT_ROWS)
+            if sched.split_groups == 0 or k == kinds[-1]:
+                return sched
+    raise RuntimeError("fused attention has never run on this layout outside graph capture: call it once eagerly before "
+                       "capturing (building its schedule synchronises)")
 
 
 def _softmax_schedule(layout, dtype, backward):

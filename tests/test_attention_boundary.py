@@ -64,6 +64,24 @@ def layout_of(monkeypatch):
     return layout_of_lengths
 
 
+@pytest.mark.parametrize("first,captured", [(400, 4), (4, 400)])
+def test_capture_uses_the_schedule_that_was_built_eagerly(layout_of, first, captured):
+    from sparse import _ops
+    for kind in (_ops.SCHEDULE_ATTENTION, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS):
+        L = layout_of(20, 3, 0, 24, 1)
+        eager = _ops._attention_schedule_for(L, kind, first)
+        layout_of.capture(True)
+        assert _ops._attention_schedule_for(L, kind, captured) is eager
+        layout_of.capture(False)
+        other = _ops._attention_schedule_for(L, kind, captured)
+        assert other is not eager and other.cap != eager.cap
+        layout_of.capture(True)
+        assert _ops._attention_schedule_for(L, kind, captured) is other
+        with pytest.raises(RuntimeError, match="eagerly"):
+            _ops._attention_schedule_for(layout_of(20, 3), kind, captured)
+        layout_of.capture(False)
+
+
 @pytest.mark.parametrize("lengths", [(1,), (24, 3), (25, 3), (48, 2, 30), (49, 1), (7, 200, 96, 97)])
 def test_every_batch_count_needs_the_same_workspace(layout_of, lengths):
     from sparse import _ops

@@ -89,3 +89,39 @@ def test_operands_that_start_anywhere(head):
     for off in (1, 4, 7):
         assert moved(t[0], off).data_ptr() % 16 != 0
         assert all(torch.equal(a, b) for a, b in zip(step(*(moved(x, off) for x in t)), want))
+
+
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("eager_small", [False, True])
+def test_captured_at_another_batch_count(head, eager_small, monkeypatch):
+    """One eager call at any batch count is enough to capture another one (a mask that cuts nothing into parts): the
+    replays give the bits of an eager call on the schedule that was there."""
+    import sparse
+    from sparse import _ops
+    mask = np.asarray(ZOO["rand16"])
+    monkeypatch.setattr(_ops, "ATTENTION_SMALL_BLOCKS", 3 * int(mask.sum()))
+    L = sparse.SparseLayout(torch.as_tensor(mask))
+    (rb, ro), (cb, co) = L.row_layout, L.col_layout
+    g = torch.Generator().manual_seed(53)
+
+    def operands(batches):
+        return [torch.randn(batches, 512, head, generator=g).half().cuda() for _ in range(4)]
+
+    def step(q, k, v, dout):
+        out, lse = _ops.sparse_attention_forward(q, k, v, rb, ro, 0.11, True, (cb, co), return_lse=True)
+        return (out, lse) + _ops.sparse_attention_backward(q, k, v, dout, out, lse, rb, ro, cb, co, 0.11, True)
+
+    first, then = (2, 8) if eager_small else (8, 2)
+    step(*operands(first))
+    t = operands(then)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(*t)
+    monkeypatch.setattr(_ops, "ATTENTION_SMALL_BLOCKS", 10 ** 9 if eager_small else 0)      # the schedule of the first call
+    for _ in range(4):
+        for x, fresh in zip(t, operands(then)):
+            x.copy_(fresh)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, step(*t)))
