@@ -43,7 +43,11 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: SparseL
     """``softmax(scale * q @ k^T, over the stored blocks of each row) @ v`` for ``q [..., 32 R, D]``,
     ``k``, ``v [..., 32 C, D]`` and an ``R x C`` block layout.  fp16 / bf16 with ``D`` 64 or 128 take the
     fused kernels; fp32, or another ``D`` (a multiple of 32), is computed as the chain of the three
-    differentiable operators it stands for."""
+    differentiable operators it stands for.
+
+    A row is summed in chunks that are shorter while the stored blocks of all batch entries together are at most
+    ``_ops.ATTENTION_SMALL_BLOCKS``: an entry gives the same bits in every launch on the same side of that line, across it
+    the last bits can differ."""
     fused = q.dtype in (torch.float16, torch.bfloat16) and q.size(-1) in (64, 128)
     if fused or not (q.dtype == k.dtype == v.dtype and q.dtype in (torch.float16, torch.bfloat16, torch.float32)):
         return SparseAttention.apply(q, k, v, layout, scale, causal)     # the fused path also owns the argument checks

@@ -1,6 +1,7 @@
 """GPU: workgroups of every batch count reach every (batch, workgroup) once (``map_workgroup``): batches that fill the
 eight XCDs evenly, every remainder of eight, fewer workgroups than XCDs.  Each batch entry of a launch must give the
-bits it gives when launched alone."""
+bits it gives when launched alone (the fused attention: on the same side of ``ATTENTION_SMALL_BLOCKS``, which every
+launch here is)."""
 import numpy as np
 import pytest
 import torch
