@@ -274,9 +274,21 @@ def _longest_group(offsets) -> int:
     return longest
 
 
+def _group_walk_kind(longest):
+    return SCHEDULE_GROUP_WALK_LONG if longest > GROUP_WALK_LONG else SCHEDULE_GROUP_WALK
+
+
 def _group_walk_schedule(layout):
-    kind = SCHEDULE_GROUP_WALK_LONG if _longest_group(layout[1]) > GROUP_WALK_LONG else SCHEDULE_GROUP_WALK
-    return schedule_for(layout, kind)
+    return schedule_for(layout, _group_walk_kind(_longest_group(layout[1])))
+
+
+def _captured_without(layout, kind) -> bool:
+    """Whether a graph is being captured and the schedule ``kind`` of the table (None: of its group walk) is not there:
+    building one synchronises.  Calls that used a walk without a schedule eagerly stay with it then."""
+    if kind is None:
+        longest = getattr(layout[1], "_bsa_longest", None)
+        kind = longest if longest is None else _group_walk_kind(longest)
+    return not _has_schedule(layout, kind) and torch.cuda.is_current_stream_capturing()
 
 
 def _attention_kind(layout, kind, split):
@@ -433,7 +445,7 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
             and size_m % BLOCK == 0 and size_k == BLOCK * (mask_cols if trans_b else mask_rows)
             and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
             and _takes_panels(num_blocks, size_m * batches if shared else size_m, 1 if shared else batches,
-                              size_k // BLOCK, size_n // BLOCK)):
+                              size_k // BLOCK, size_n // BLOCK, lambda: _captured_without(layout, None))):
         with _k.on_device(a.device):
             _k.check(_k.lib.bsa_matmul_dds_panels(
                 _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
@@ -458,14 +470,15 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
     return c
 
 
-def _takes_panels(nnz, rows, entries, kblocks, groups):
+def _takes_panels(nnz, rows, entries, kblocks, groups, without_choice=lambda: False):
     """Whether a DDS product of ``entries`` matrices of ``rows`` dense rows takes the panel walk
-    (bsa_matmul_dds_panels)."""
+    (bsa_matmul_dds_panels): where it is the faster one, or, ``without_choice()``, wherever it can."""
     tiles, sets = -(-rows // PANEL_ROWS), -(-groups // PANEL_GROUPS)
-    return (kblocks <= PANEL_MAX_KBLOCKS and nnz <= PANEL_MAX_NNZ and entries <= 65535 and rows <= 2 ** 30
-            and (rows // 64 + 1) * (groups // 8 + 1) < 2 ** 28
-            and tiles * sets * entries >= PANEL_MIN_WORKGROUPS
-            and nnz * rows >= PANEL_MIN_DENSITY * kblocks * groups * tiles * PANEL_ROWS)
+    if (kblocks > PANEL_MAX_KBLOCKS or nnz > PANEL_MAX_NNZ or entries > 65535 or rows > 2 ** 30
+            or (rows // 64 + 1) * (groups // 8 + 1) >= 2 ** 28):
+        return False
+    return ((tiles * sets * entries >= PANEL_MIN_WORKGROUPS
+             and nnz * rows >= PANEL_MIN_DENSITY * kblocks * groups * tiles * PANEL_ROWS) or without_choice())
 
 
 def sparse_weight_gradient(a, b, row_layout, col_layout, trans_a, trans_b):
@@ -476,9 +489,11 @@ def sparse_weight_gradient(a, b, row_layout, col_layout, trans_a, trans_b):
     rows, cols = row_layout[1].numel() - 1, col_layout[1].numel() - 1
     tokens = a.numel() // max(a.size(-1), 1)
     folds = (trans_a and not trans_b and a.dtype in (torch.float16, torch.bfloat16) and a.dtype == b.dtype
-             and a.shape[:-1] == b.shape[:-1] and a.size(-2) % BLOCK == 0 and WEIGHT_GRAD_MIN_TOKENS <= tokens < 2 ** 31
+             and a.shape[:-1] == b.shape[:-1] and a.size(-2) % BLOCK == 0 and BLOCK <= tokens < 2 ** 31
              and a.size(-1) == BLOCK * rows and b.size(-1) == BLOCK * cols and a.is_cuda and a.device == b.device
-             and row_layout[0].device == a.device and nnz > 0 and nnz >= WEIGHT_GRAD_MIN_DENSITY * rows * cols)
+             and row_layout[0].device == a.device and nnz > 0
+             and ((tokens >= WEIGHT_GRAD_MIN_TOKENS and nnz >= WEIGHT_GRAD_MIN_DENSITY * rows * cols)
+                  or _captured_without(row_layout, SCHEDULE_SDD)))
     if folds:
         a, b = a.contiguous(), b.contiguous()
         folds = a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0

@@ -102,3 +102,35 @@ def test_linear_layer_takes_both_and_agrees_with_the_group_walk(monkeypatch):
     for n, o in zip(new, step()):
         assert n.shape == o.shape and _rel(n, o.double()) <= 4 * REL[torch.float16]
 
+
+
+def test_layer_captured_at_a_size_that_never_ran():
+    """One eager training step at any size is enough to capture a step at another one."""
+    import sparse
+    from sparse import _ops
+    L = _layout(24, 32, 0.4, 7)
+    g = torch.Generator(device="cuda").manual_seed(2)
+
+    def operands(batch, m):
+        mk = lambda *shape: torch.randn(*shape, generator=g, device="cuda").half()
+        return mk(batch, m, 32 * 24), 0.05 * mk(L.num_blocks, 32, 32), mk(batch, m, 32 * 32)
+
+    def step(x, w, dy):
+        mm = lambda a, b, mode, ta, tb: _ops.sparse_matmul(a, b, mode, L.row_layout, L.col_layout, ta, tb)
+        return (mm(x, w, "dds", False, False), mm(dy, w, "dds", False, True),
+                _ops.sparse_weight_gradient(x, dy, L.row_layout, L.col_layout, True, False))
+
+    assert _ops._takes_panels(L.num_blocks, 4 * 1056, 1, 24, 32) and not _ops._takes_panels(L.num_blocks, 64, 1, 24, 32)
+    step(*operands(4, 1056))
+    t = operands(2, 32)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(*t)
+    for _ in range(4):
+        for x, fresh in zip(t, operands(2, 32)):
+            x.copy_(fresh)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, step(*t)):
+            assert _rel(a, b.double()) <= 4 * REL[torch.float16]

@@ -61,3 +61,24 @@ def test_weights_of_their_own_are_a_grid_dimension():
     import sparse.kernel as k
     assert _panels(k, dense=P + 2, batches=65536, sparse_batches=65536) != 0
     assert "at most 65535" in k.lib.bsa_last_error().decode()
+
+
+def test_what_nobody_built_a_schedule_for_is_captured_without_one(monkeypatch):
+    """An eager call that took the panel walk, or folded the batch into the weight gradient, built no schedule; a captured
+    call of another size cannot build one either and takes the same walk."""
+    import torch
+    from sparse import _ops
+    state = {"capturing": False}
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    layout = (torch.zeros(8, dtype=torch.int32), torch.tensor([0, 1, 4], dtype=torch.int32))
+    small = (4, 32, 1, 2, 2)
+    captured = lambda kind: _ops._captured_without(layout, kind)
+    takes = lambda *size: _ops._takes_panels(*size, lambda: captured(None))
+    assert not takes(*small) and not captured(_ops.SCHEDULE_SDD)
+    state["capturing"] = True
+    assert takes(*small) and captured(_ops.SCHEDULE_SDD)
+    assert not takes(4, 32, 1, 1025, 2) and not takes(2 ** 20, 2048, 1, 1024, 1024)      # what the walk is not built for
+    layout[1]._bsa_longest = 3
+    assert takes(*small)
+    layout[1]._bsa_schedules = {_ops.SCHEDULE_GROUP_WALK: object(), _ops.SCHEDULE_SDD: object()}
+    assert not takes(*small) and not captured(_ops.SCHEDULE_SDD)
