@@ -61,6 +61,7 @@ PANEL_MAX_NNZ = 2 ** 20 - 1
 WEIGHT_GRAD_MIN_TOKENS = 1024
 WEIGHT_GRAD_MIN_DENSITY = 0.15
 ATTENTION_WAVES_LONG_GROUPS = 8
+ATTENTION_COLUMN_WAVES_128 = 4    # waves of a workgroup the column walk takes at head dim 128
 ATTENTION_SPLIT_ROWS = True       # groups longer than cap * waves are cut into parts across workgroups
 SCHEDULE_ATTENTION = (12, 4)           # forward: rows of more than 48 blocks are split across workgroups
 SCHEDULE_ATTENTION_BACKWARD = (12, 4)
@@ -291,18 +292,18 @@ def _captured_without(layout, kind) -> bool:
     return not _has_schedule(layout, kind) and torch.cuda.is_current_stream_capturing()
 
 
-def _attention_kind(layout, kind, split):
+def _attention_kind(layout, kind, split, most_waves=ATTENTION_WAVES_LONG_GROUPS):
     """Arguments of the schedule of a fused attention walk.  With ``split`` (what every caller passes while
     ``ATTENTION_SPLIT_ROWS`` is set) a group longer than the workgroup's share is cut into parts that
     meet in a workspace; without it such a table gets the most waves a workgroup holds instead."""
     cap, waves = kind
     if not split and _longest_group(layout[1]) > cap * waves:
-        waves = ATTENTION_WAVES_LONG_GROUPS
+        waves = most_waves
     return cap, waves, bool(split)
 
 
-def _attention_schedule(layout, kind, split=False):
-    return schedule_for(layout, _attention_kind(layout, kind, split))
+def _attention_schedule(layout, kind, split=False, most_waves=ATTENTION_WAVES_LONG_GROUPS):
+    return schedule_for(layout, _attention_kind(layout, kind, split, most_waves))
 
 
 def _attention_kinds(kind, few_blocks):
@@ -313,17 +314,17 @@ def _attention_kinds(kind, few_blocks):
     return SCHEDULE_ATTENTION_SMALL, (chunk, kind[0] * kind[1] // chunk)
 
 
-def _attention_schedule_for(layout, kind, batches):
+def _attention_schedule_for(layout, kind, batches, most_waves=ATTENTION_WAVES_LONG_GROUPS):
     """Schedule of a fused attention walk over ``batches`` entries: ``kind``, or shorter chunks for a small launch.  Nothing
     can be built under graph capture: there the other length serves when only that one has been used eagerly."""
     few = layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS
     for few_blocks in (few, not few):
         kinds = _attention_kinds(kind, few_blocks)
         for k in kinds:
-            if not _has_schedule(layout, _attention_kind(layout, k, ATTENTION_SPLIT_ROWS)) \
+            if not _has_schedule(layout, _attention_kind(layout, k, ATTENTION_SPLIT_ROWS, most_waves)) \
                     and torch.cuda.is_current_stream_capturing():
                 break
-            sched = _attention_schedule(layout, k, split=ATTENTION_SPLIT_ROWS)
+            sched = _attention_schedule(layout, k, ATTENTION_SPLIT_ROWS, most_waves)
             if sched.split_groups == 0 or k == kinds[-1]:
                 return sched
     raise RuntimeError("fused attention has never run on this layout outside graph capture: call it once eagerly before "
@@ -676,7 +677,8 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
     if q.numel() > 0:
         delta = torch.empty_like(lse)
         rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
-        cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches)
+        cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches,
+                                     ATTENTION_WAVES_LONG_GROUPS if head == 64 else ATTENTION_COLUMN_WAVES_128)
         with _k.on_device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = rs.attention_backward_workspace(cs, batches, head, stream)

@@ -91,3 +91,19 @@ def test_every_batch_count_needs_the_same_workspace(layout_of, lengths):
         assert few.cap < many.cap and few.waves <= 8
         assert (few.split_groups, few.tile_slots) == (many.split_groups, many.tile_slots)
         assert (few.split_groups == 0) == (max(lengths) <= kind[0] * kind[1])
+
+
+@pytest.mark.parametrize("batches", [1, 10 ** 5])
+def test_unsplit_columns_keep_to_the_waves_the_walk_takes(layout_of, batches, monkeypatch):
+    """What the column walk of head dim 128 is asked for without splitting is what bsa_attention_gradients allows."""
+    import sparse.kernel as k
+    from sparse import _ops
+    monkeypatch.setattr(_ops, "ATTENTION_SPLIT_ROWS", False)
+    L = layout_of(300, 30, 2)
+    sched = _ops._attention_schedule_for(L, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches, _ops.ATTENTION_COLUMN_WAVES_128)
+    assert sched.waves == _ops.ATTENTION_COLUMN_WAVES_128
+    assert _ops._attention_schedule_for(L, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches).waves == 8
+    columns = lambda waves: k.lib.bsa_attention_gradients(1, P, P, P, P, P, P, P, P, P, P, P, P, P, 4, 4, 0, 0, P, P, P, 4, waves,
+                                                          5, 1, None, 0, 4, 4, 5, 1, 128, 1.0, 0, None)
+    assert columns(sched.waves + 1) == -1 and "at most 4" in k.lib.bsa_last_error().decode()
+    assert columns(sched.waves) == -1 and "workspace" in k.lib.bsa_last_error().decode()

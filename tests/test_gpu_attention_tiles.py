@@ -125,3 +125,18 @@ def test_captured_at_another_batch_count(head, eager_small, monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, step(*t)))
+
+
+def test_long_groups_unsplit_at_head_dim_128(monkeypatch):
+    import sparse
+    from sparse import _ops
+    monkeypatch.setattr(_ops, "ATTENTION_SPLIT_ROWS", False)
+    mask = np.asarray(ZOO["long_col_70x3"])
+    L = sparse.SparseLayout(torch.as_tensor(mask))
+    g = torch.Generator().manual_seed(59)
+    mk = lambda n: torch.randn(2, 32 * n, 128, generator=g).half().cuda()
+    q, k, v, dout = mk(70).requires_grad_(), mk(3).requires_grad_(), mk(3).requires_grad_(), mk(70)
+    grads = torch.autograd.grad(sparse.attention(q, k, v, L, 0.11), (q, k, v), dout)
+    qn, kn, vn, dn = (to_np(t.detach()) for t in (q, k, v, dout))
+    for got, ref in zip(grads, ao.backward(qn, kn, vn, dn, mask, 0.11, False)):
+        assert rel_err(to_np(got), ref) <= 4 * TOL[torch.float16]
