@@ -631,12 +631,17 @@ static int attention_backward(const char *who, int dtype, const void *q, const v
     int rc = check_attention(who, dtype, head_dim, row_blocks, row_offsets, row_sched, row_sched_wgs, row_sched_waves,
                              mask_rows, mask_cols, nnz, batches);
     if (rc) return rc;
-    if (!col_offsets || (!col_blocks && nnz > 0)) return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
-    rc = check_schedule(col_sched, col_sched_wgs, col_sched_waves, batches, who);
-    if (rc) return rc;
-    if (head_dim == 128 && col_sched_waves > bsa::AT_COLUMN_WAVES_128)
-        return fail(BSA_ERR_INVALID, "%s: the column schedule has %d waves per workgroup, at most %d at head_dim 128", who,
-                    col_sched_waves, bsa::AT_COLUMN_WAVES_128);
+    const bool columns = dk_out != nullptr;      // without them the column arguments are not looked at
+    if (columns) {
+        if (!col_offsets || (!col_blocks && nnz > 0)) return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
+        rc = check_schedule(col_sched, col_sched_wgs, col_sched_waves, batches, who);
+        if (rc) return rc;
+        if (head_dim == 128 && col_sched_waves > bsa::AT_COLUMN_WAVES_128)
+            return fail(BSA_ERR_INVALID, "%s: the column schedule has %d waves per workgroup, at most %d at head_dim 128", who,
+                        col_sched_waves, bsa::AT_COLUMN_WAVES_128);
+    } else {
+        col_tile_slots = col_split_groups = 0;
+    }
     if (!q || !k || !v || !dout || !out || !lse || !dq_out || !delta_ws)
         return fail(BSA_ERR_INVALID, "%s: null pointer argument", who);
     rc = check_operand_alignment(who, {q, k, v, dout});
@@ -664,7 +669,7 @@ static int attention_backward(const char *who, int dtype, const void *q, const v
     p.split_groups = row_split_groups;
     p.workspace = workspace;
     rc = check_launch(bsa::launch_attention_backward_scores(p, (hipStream_t)stream), who);
-    if (rc || !dk_out) return rc;
+    if (rc || !columns) return rc;
     p.blocks = col_blocks;
     p.sched = col_sched;
     p.groups = mask_cols;

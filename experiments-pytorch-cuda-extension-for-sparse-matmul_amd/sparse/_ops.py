@@ -678,7 +678,10 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
         delta = torch.empty_like(lse)
         rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
         cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches,
-                                     ATTENTION_WAVES_LONG_GROUPS if head == 64 else ATTENTION_COLUMN_WAVES_128)
+                                     ATTENTION_WAVES_LONG_GROUPS if head == 64 else ATTENTION_COLUMN_WAVES_128) \
+            if with_dkdv else None
+        columns = (cs.table.data_ptr(), cs.workgroups, cs.waves, cs.tile_slots, cs.split_groups) if with_dkdv \
+            else (None, 0, 0, 0, 0)
         with _k.on_device(q.device):
             stream = _k.current_stream()
             ws, ws_bytes = rs.attention_backward_workspace(cs, batches, head, stream)
@@ -688,7 +691,6 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
                 delta.data_ptr(),
                 row_blocks.data_ptr(), row_table.data_ptr(), rs.table.data_ptr(), rs.workgroups, rs.waves,
                 rs.tile_slots, rs.split_groups,
-                col_blocks.data_ptr(), col_table.data_ptr(), cs.table.data_ptr(), cs.workgroups, cs.waves,
-                cs.tile_slots, cs.split_groups, ws.data_ptr() if ws is not None else None, ws_bytes,
+                col_blocks.data_ptr(), col_table.data_ptr(), *columns, ws.data_ptr() if ws is not None else None, ws_bytes,
                 mask_rows, mask_cols, nnz, batches, head, float(scale), int(bool(causal)), stream))
     return dq, dk, dv

@@ -357,7 +357,7 @@ int bsa_attention_backward(int dtype, const void *q, const void *k, const void *
                            float scale, int causal, void *stream);
 
 /* bsa_attention_backward for head_dim 64 and 128.  At 128 the column schedule has at most 4 waves per workgroup.
- * dk_out and dv_out both null: dq alone, without the walk over the columns. */
+ * dk_out and dv_out both null: dq alone, without the walk over the columns, whose arguments are not looked at. */
 int bsa_attention_gradients(int dtype, const void *q, const void *k, const void *v, const void *dout,
                            const void *out, const float *lse, void *dq_out, void *dk_out, void *dv_out,
                            float *delta_ws,

@@ -107,3 +107,13 @@ def test_unsplit_columns_keep_to_the_waves_the_walk_takes(layout_of, batches, mo
                                                           5, 1, None, 0, 4, 4, 5, 1, 128, 1.0, 0, None)
     assert columns(sched.waves + 1) == -1 and "at most 4" in k.lib.bsa_last_error().decode()
     assert columns(sched.waves) == -1 and "workspace" in k.lib.bsa_last_error().decode()
+
+
+def test_queries_alone_prepare_nothing_for_the_columns():
+    import sparse.kernel as k
+    call = lambda ws_bytes, ct, cs: k.lib.bsa_attention_gradients(
+        1, P, P, P, P, P, P, P, None, None, P, P, P, P, 4, 4, 5, 1, None, None, None, 0, 0, ct, cs, P, ws_bytes, 4, 4, 5, 1, 64,
+        1.0, 0, None)
+    need = k.lib.bsa_attention_backward_workspace_bytes(5, 1, 0, 0, 1, 64)
+    for counts in ((0, 0), (7, 2), (3, 0)):
+        assert call(need - 1, *counts) == -1 and f"workspace of {need} bytes" in k.lib.bsa_last_error().decode()

@@ -59,6 +59,9 @@ def test_queries_alone_need_no_column_walk(head):
     out = sparse.attention(q, kk, v, L, 0.11)
     got, = torch.autograd.grad(out, q, dout)
     assert torch.equal(got, want)
+    fresh = sparse.SparseLayout(torch.as_tensor(mask))
+    again, = torch.autograd.grad(sparse.attention(q, kk, v, fresh, 0.11), q, dout)
+    assert torch.equal(again, want) and not hasattr(fresh.col_layout[1], "_bsa_schedules")
     P = 0x1000
     rc = k.lib.bsa_attention_gradients(1, P, P, P, P, P, P, P, None, P, P, P, P, P, 4, 4, 0, 0, P, P, P, 4, 4, 0, 0, None, 0,
                                        4, 4, 5, 1, head, 1.0, 0, None)
