@@ -255,7 +255,7 @@ __global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attention_fwd_f16_kerne
 // straight from those registers.  K_c is read from LDS twice, along d for S and along its rows for dq;
 // both reads come first, so that the next K is requested before anything is multiplied.  dq alone (us, before -> after):
 // 16 heads of 4096 tokens 26.8 -> 20.6, 48 of 8192 116 -> 94; at head dim 128, where two stacks were stored, 69 -> 40.
-// Without STACKS nothing is stored per block and scale * delta is left for the column walk.
+// Without STACKS nothing is stored per block and delta is left for the column walk.
 // ---------------------------------------------------------------------------
 // per wave: K and V tiles (= the dq^T part of the merge), and with STACKS the two result blocks of 2 KB
 constexpr int at_bwd_lds_per_wave(int hd, bool stacks) { return 128 * hd + (stacks ? 4096 : 0); }
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kern
 #pragma unroll
                     for (int j = 0; j < 8; ++j) delta += widen_16<BF>(dop[s][j]) * widen_16<BF>(oop[s][j]);
                 delta += at_lane_xor32(delta);   // the other half of the head dim sits in lane ^ 32
-                if (delta_out != nullptr && w == e.first_wave() && e.part() == 0 && h == 0) delta_out[row0 + qq] = scale * delta;
+                if (delta_out != nullptr && w == e.first_wave() && e.part() == 0 && h == 0) delta_out[row0 + qq] = delta;
             } else {
                 kreq.issue(win.get(seg).col());
                 vreq.issue(win.get(seg).col());
@@ -434,16 +434,18 @@ __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kern
 // ---------------------------------------------------------------------------
 // Backward, the walk over the COLUMNS: dk and dv of block column c from the blocks (r, c) of the
 // column table, with nothing but q, k, v, dO and two floats per query (lse of the forward pass,
-// scale * delta of the row walk above) read: the probabilities and the score gradients are rebuilt in
+// delta of the row walk above) read: the probabilities and the score gradients are rebuilt in
 // registers a second time rather than stored by the row walk and read back (4 KB written + 4 KB
 // read of HBM traffic per block that this pair of kernels does not have).
-//   S  = Q_r K_c^T, dP = dO_r V_c^T    K_c and V_c stay in registers; a lane holds ONE key column, 16 queries, whose lse
-//                                      and delta come into LDS with the tiles
+//   S  = Q_r K_c^T, delta - dO_r V_c^T   K_c and -V_c stay in registers; a lane holds ONE key column, 16 queries, whose lse
+//                                      and delta come into LDS with the tiles; delta is where the second product starts
 //   dv^T += dO_r^T P,  dk^T += Q_r^T dS   the 16-bit P and dS values are the column operands straight from the
 //                                      accumulators, the Q_r and dO_r tiles are read a second time along their rows
-// The waves of a column add their parts through LDS.  Two waves per SIMD at head dim 64 (200 registers), one at 128 (its
+// The waves of a column add their parts through LDS.  Two waves per SIMD at head dim 64 (184 registers), one at 128 (its
 // four accumulators are 256); three at 64 spill the K operands and are slower.  us, before -> after: 16 heads of 4096
 // tokens 34.9 -> 29.6, 48 of 8192 150 -> 135; at head dim 128, as two products over stored stacks before, 69 -> 66.
+// Delta kept scaled in memory, or subtracted behind the product, makes no difference to the whole backward pass (50.7-51.6
+// against 51.2-51.7 us, 198.7-199.5 against 198.9-200.2, at head dim 128 102.6-104.2 against 101.2-104.3).
 // ---------------------------------------------------------------------------
 constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256; }   // Q + dO tiles (= one parked accumulator set) + lse, delta
 
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
 #pragma unroll
                 for (int s = 0; s < KS; ++s) {
                     kop[s] = rd.rows(Q_TILE, s);
-                    vop[s] = rd.rows(DO_TILE, s);
+                    vop[s] = negated_16(rd.rows(DO_TILE, s));
                 }
                 lds_reads_done();
             }
@@ -538,21 +540,20 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                 }
                 tile_wait<0>();
                 {
-                    f16v dpacc = {0};
+                    f16v acc;                    // delta - dP
                     h8 dop[KS];
-#pragma unroll
-                    for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
-#pragma unroll
-                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], vop[s], dpacc);
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int v = 4 * g + j;
-                            ds[v >> 3][v & 7] = narrow_16<BF>(prob[v] * __builtin_fmaf(dpacc[v], scale, -dl[j]));
-                        }
+                        for (int j = 0; j < 4; ++j) acc[4 * g + j] = dl[j];
                     }
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) acc = mfma_16<BF>(dop[s], vop[s], acc);
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) ds[v >> 3][v & 7] = narrow_16<BF>(prob[v] * (acc[v] * -scale));
                 }
                 // The tiles are read a second time, Q first: the requests for the next block go out as soon as each is free.
                 h8 tr[KT][2];

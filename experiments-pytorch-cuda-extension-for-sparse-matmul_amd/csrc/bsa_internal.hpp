@@ -123,7 +123,7 @@ struct AttentionArgs {
     const void *dout = nullptr;     // backward only
     void *p_out = nullptr, *ds_out = nullptr;   // row walk of the backward pass, both or neither: [batches, nnz, 32, 32]
     void *dq_out = nullptr;         // row walk, may be null: [batches, 32 mask_rows, head_dim]
-    void *delta = nullptr;          // float [batches, 32 mask_rows], scale * rowsum(dout o out): written by the row walk (may be
+    void *delta = nullptr;          // float [batches, 32 mask_rows], rowsum(dout o out): written by the row walk (may be
                                     // null there), read by the column walk
     void *dk_out = nullptr, *dv_out = nullptr;  // column walk: [batches, 32 mask_cols, head_dim]
     int nnz = 0;

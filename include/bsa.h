@@ -332,7 +332,7 @@ int bsa_attention_backward_scores(int dtype, const void *q, const void *k, const
 /* The whole backward pass of that operator in two launches, with no block stack in memory: a walk over
  * the rows that rebuilds the probabilities and the score gradients in registers and accumulates
  *   dq_out = ds k                       [batches, 32 * mask_rows, head_dim]
- * (and leaves scale * rowsum(dout o out) in `delta_ws`, float [batches, 32 * mask_rows], caller-provided), and
+ * (and leaves rowsum(dout o out) in `delta_ws`, float [batches, 32 * mask_rows], caller-provided), and
  * a walk over the columns that rebuilds them a second time and accumulates
  *   dk_out = ds^T q,  dv_out = p^T dout [batches, 32 * mask_cols, head_dim].
  * Seven launches in the unfused chain (sparse/matmul.py:27-52 three times over, sparse_softmax.cu:165-205,233-258).

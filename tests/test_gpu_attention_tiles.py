@@ -143,3 +143,29 @@ def test_long_groups_unsplit_at_head_dim_128(monkeypatch):
     qn, kn, vn, dn = (to_np(t.detach()) for t in (q, k, v, dout))
     for got, ref in zip(grads, ao.backward(qn, kn, vn, dn, mask, 0.11, False)):
         assert rel_err(to_np(got), ref) <= 4 * TOL[torch.float16]
+
+
+@pytest.mark.parametrize("entry,head", [("bsa_attention_backward", 64), ("bsa_attention_gradients", 64), ("bsa_attention_gradients", 128)])
+def test_delta_workspace_holds_the_row_sums(entry, head):
+    """What the header says the row walk leaves there, whatever the scale: rowsum(dout o out), an fp32 sum of ``head``
+    products of 16-bit values (bound: head ulps of the sum of their magnitudes)."""
+    import sparse
+    from sparse import _ops, kernel
+    mask = np.asarray(ZOO["rand16"])
+    L = sparse.SparseLayout(torch.as_tensor(mask))
+    (rb, ro), (cb, co) = L.row_layout, L.col_layout
+    g = torch.Generator().manual_seed(61)
+    q, k, v, dout = (torch.randn(2, 512, head, generator=g).half().cuda() for _ in range(4))
+    out, lse = _ops.sparse_attention_forward(q, k, v, rb, ro, 0.11, True, L.col_layout, return_lse=True)
+    dq, dk, dv, delta = (torch.empty_like(t) for t in (q, k, v, lse))
+    scheds = [_ops._attention_schedule_for(t, kind, 2) for t, kind in (
+        (L.row_layout, _ops.SCHEDULE_ATTENTION_BACKWARD), (L.col_layout, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS))]
+    assert all(s.split_groups == 0 for s in scheds)
+    tables = [x for (b, o), s in zip((L.row_layout, L.col_layout), scheds)
+              for x in (b.data_ptr(), o.data_ptr(), s.table.data_ptr(), s.workgroups, s.waves, 0, 0)]
+    kernel.check(getattr(kernel.lib, entry)(1, *(t.data_ptr() for t in (q, k, v, dout, out, lse, dq, dk, dv, delta)), *tables,
+                                            None, 0, 16, 16, L.num_blocks, 2, head, 0.11, 1, kernel.current_stream()))
+    terms = dout.double() * out.double()
+    assert ((delta.double() - terms.sum(-1)).abs() <= head * 2.0 ** -24 * terms.abs().sum(-1)).all()
+    want = _ops.sparse_attention_backward(q, k, v, dout, out, lse, rb, ro, cb, co, 0.11, True)
+    assert all(torch.equal(a, b) for a, b in zip((dq, dk, dv), want))
