@@ -22,15 +22,19 @@ __device__ __forceinline__ float at_finite_or_zero(float m) { return m == -__bui
 // ---- loads that go straight to LDS ------------------------------------------------------------------
 // 16 bytes per lane from `base` + off to LDS bytes lds .. lds + 1023 (lane l: lds + 16 l).  Written as assembly so that
 // the compiler, which would wait for every such load in flight before any LDS read, leaves the counting to tile_wait.
+// m0 is named as clobbered: the compiler reserves it (and says so in a warning) but merges its own settings of it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(const void *base, unsigned off, unsigned lds)
 {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
 // 4 bytes per lane from an address of its own
 __device__ __forceinline__ void dma4_gather(const void *address, unsigned lds)
 {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(address), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(address), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // all but the youngest N requests of the wave have landed, and its LDS reads are done
 template <int N>
 __device__ __forceinline__ void tile_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory"); }
