@@ -338,6 +338,13 @@ int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void
     return check_launch(bsa::launch_weight_panels(dtype, p, (hipStream_t)stream), who);
 }
 
+void bsa_matmul_dds_panels_limits(int32_t limits[3])
+{
+    limits[0] = bsa::PANEL_ROWS;
+    limits[1] = bsa::PANEL_MAX_KBLOCKS;
+    limits[2] = bsa::PANEL_MAX_NNZ;
+}
+
 int bsa_weight_grad_shares(int mask_rows, int mask_cols, int tokens)
 {
     if (mask_rows < 1 || mask_cols < 1 || tokens < BSA_BLOCK) return 0;

@@ -79,6 +79,7 @@ struct RunsArgs {
 hipError_t launch_dsd_runs(int dtype, const RunsArgs &p, hipStream_t stream);
 
 // products of a block-sparse weight with many dense rows, and the weight's gradient (weight_panels.hip)
+constexpr int PANEL_ROWS = 96;                     // dense rows of a workgroup
 constexpr int PANEL_MAX_KBLOCKS = 1024;            // the k-block table of eight groups: 32 KB of LDS
 constexpr int PANEL_MAX_NNZ = (1 << 20) - 1;       // 2 KB blocks within a 31-bit buffer range
 struct WeightPanelArgs {

@@ -348,7 +348,6 @@ __global__ __launch_bounds__(256) void weight_sum_kernel(const float *__restrict
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-constexpr int PANEL_ROWS = 96;
 template <int ROWS, bool S_KC, bool BF>
 static hipError_t launch_panel(const WeightPanelArgs &p, hipStream_t st)
 {

@@ -50,11 +50,10 @@ RUN_WALK_MIN_REUSE = 2.0
 # 1024) 111 -> 98, 0.18 155 -> 107, 0.30 238 -> 117; at a stored share of 0.2 by workgroups: 96 32 x 96 blocks 10 -> 24,
 # 128 (64 x 64, 16 x 96 rows) 16 -> 18, 176 (64 x 64, 2 x 1056) 28 -> 20.
 PANEL_WALK = True
-PANEL_ROWS, PANEL_GROUPS = 96, 8       # of a workgroup
+PANEL_ROWS, PANEL_MAX_KBLOCKS, PANEL_MAX_NNZ = _k.dds_panel_limits()      # of a workgroup, of a launch
+PANEL_GROUPS = 8                       # of a workgroup
 PANEL_MIN_WORKGROUPS = 160
 PANEL_MIN_DENSITY = 0.12
-PANEL_MAX_KBLOCKS = 1024
-PANEL_MAX_NNZ = 2 ** 20 - 1
 # Its weight gradient (bsa_weight_grad) against a stack per batch entry and a sum over them: 0.12 stored (96 x 96 blocks, 8192
 # tokens) 104 -> 114 us, 0.18 179 -> 126, 0.25 (64 x 64, 4224 tokens) 67 -> 40; 0.2, 1056 tokens 60 -> 24; 0.3 (16 x 16), 256
 # tokens 12 -> 16.

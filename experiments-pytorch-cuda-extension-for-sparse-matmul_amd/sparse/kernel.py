@@ -39,6 +39,7 @@ SIGNATURES = {
                                 _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "bsa_matmul_dsd_block64": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "bsa_matmul_dds_panels": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "bsa_matmul_dds_panels_limits": (None, [_vp]),
     "bsa_weight_grad_shares": (_i, [_i, _i, _i]),
     "bsa_weight_grad": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t, _vp]),
     "bsa_run_schedule_bytes": (ctypes.c_int64, [_i, _i]),
@@ -78,6 +79,13 @@ def load_library(path: str = LIBRARY_PATH) -> ctypes.CDLL:
 
 
 lib = load_library()
+
+
+def dds_panel_limits():
+    """Dense rows of a workgroup of the panel walk, block rows of the contraction and blocks it is built for."""
+    limits = (ctypes.c_int32 * 3)()
+    lib.bsa_matmul_dds_panels_limits(limits)
+    return tuple(limits)
 
 
 def check(status: int) -> None:

@@ -382,6 +382,9 @@ int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void
                           const int32_t *offsets, int mask_rows, int mask_cols, int nnz, int batches,
                           int sparse_batches, int M, int tr_b, void *stream);
 
+/* Constants of that walk: dense rows of a workgroup, block rows of the contraction and blocks it is built for. */
+void bsa_matmul_dds_panels_limits(int32_t limits[3]);
+
 /* Gradient of a block-sparse weight that a whole batch shared: out[block (r, c)] = sum over all tokens t of
  * a[t][32 r + .] b[t][32 c + .], a [tokens, 32 * mask_rows], b [tokens, 32 * mask_cols], the batch folded into the
  * tokens (a multiple of 32); the sum stays in fp32 until the block is written.  `parts` is scratch of

@@ -60,18 +60,20 @@ def test_long_rows_and_multi_dim_batch():
     assert rel_err(out, ref) <= TOL
 
 
+@pytest.mark.parametrize("small", [0, 8192], ids=["long_chunks", "short_chunks"])
 @pytest.mark.parametrize("dtype,head", [(torch.float16, 64), (torch.bfloat16, 64), (torch.float16, 128)])
 @pytest.mark.parametrize("causal", [False, True])
-def test_rows_split_across_workgroups(dtype, head, causal):
+def test_rows_split_across_workgroups(dtype, head, causal, small, monkeypatch):
     """Rows longer than one workgroup's share (cap x waves blocks) are cut into parts that meet in a
     workspace: same result as the oracle and, within rounding, as the unsplit walk; a second launch on
     the same workspace gives the same bits (the counters are left at zero); with the causal mask whole
     parts of a row are hidden (their maximum is -inf) and the row statistics still come out right."""
     import sparse
     from sparse import _ops
+    monkeypatch.setattr(_ops, "ATTENTION_SMALL_BLOCKS", small)
     rng = np.random.RandomState(9)
     mask = (rng.rand(6, 200) < 0.03).astype(np.int64)
-    mask[1, :] = 1                      # 200 blocks: four parts
+    mask[1, :] = 1                      # 200 blocks: five parts
     mask[3, 10:140] = 1                 # 130 blocks: three parts
     mask[4, :65] = 1                    # 65 blocks: two parts
     mask[5, 150:] = 1                   # all right of the diagonal under the causal mask
@@ -80,8 +82,8 @@ def test_rows_split_across_workgroups(dtype, head, causal):
     q, k, v = mk(6), mk(200), mk(200)
     L = sparse.SparseLayout(torch.as_tensor(mask))
     rl, cl = L.row_layout, L.col_layout
-    sched = _ops._attention_schedule(rl, _ops.SCHEDULE_ATTENTION, split=True)
-    assert sched.split_groups >= 3 and sched.tile_slots >= 9
+    sched = _ops._attention_schedule_for(rl, _ops.SCHEDULE_ATTENTION, 3)
+    assert sched.split_groups >= 3 and sched.tile_slots >= 9 and sched.cap == (6 if small else 12)
     run = lambda: _ops.sparse_attention_forward(q.cuda(), k.cuda(), v.cuda(), rl[0], rl[1], 0.11, causal, cl, return_lse=True)
     out, lse = run()
     out2, lse2 = run()
@@ -102,14 +104,16 @@ def test_rows_split_across_workgroups(dtype, head, causal):
     assert torch.allclose(lse[seen], lse_whole[seen], rtol=0, atol=2e-3)
 
 
+@pytest.mark.parametrize("small", [0, 8192], ids=["long_chunks", "short_chunks"])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_backward_groups_split_across_workgroups(dtype, causal):
+def test_backward_groups_split_across_workgroups(dtype, causal, small, monkeypatch):
     """Rows and columns longer than one workgroup's share in the two backward walks: parts add up in a
     workspace.  Gradients against the oracle and against the unsplit walks; two launches in a row give
     the same bits (counters left at zero); the stored-stack row walk (dq with p and ds) splits as well."""
     import sparse
     from sparse import _ops
+    monkeypatch.setattr(_ops, "ATTENTION_SMALL_BLOCKS", small)
     rng = np.random.RandomState(21)
     mask = (rng.rand(104, 104) < 0.02).astype(np.int64)
     mask[3, :] = 1                      # a row of 104 blocks
@@ -121,9 +125,9 @@ def test_backward_groups_split_across_workgroups(dtype, causal):
     q, k, v, dout = mk(), mk(), mk(), mk()
     L = sparse.SparseLayout(torch.as_tensor(mask))
     rl, cl = L.row_layout, L.col_layout
-    rs = _ops._attention_schedule(rl, _ops.SCHEDULE_ATTENTION_BACKWARD, split=True)
-    cs = _ops._attention_schedule(cl, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS, split=True)
-    assert rs.split_groups >= 2 and cs.split_groups >= 2
+    rs = _ops._attention_schedule_for(rl, _ops.SCHEDULE_ATTENTION_BACKWARD, 2)
+    cs = _ops._attention_schedule_for(cl, _ops.SCHEDULE_ATTENTION_BACKWARD_COLUMNS, 2)
+    assert rs.split_groups >= 2 and cs.split_groups >= 2 and rs.cap == cs.cap == (6 if small else 12)
     qd, kd, vd, dd = q.cuda(), k.cuda(), v.cuda(), dout.cuda()
     out, lse = _ops.sparse_attention_forward(qd, kd, vd, rl[0], rl[1], 0.125, causal, cl, return_lse=True)
     run = lambda: _ops.sparse_attention_backward(qd, kd, vd, dd, out, lse, rl[0], rl[1], cl[0], cl[1], 0.125, causal)
@@ -145,10 +149,12 @@ def test_backward_groups_split_across_workgroups(dtype, causal):
         assert rel_err(to_np(a), to_np(b)) <= tol, name
 
 
-def test_split_rows_at_head_dim_128():
-    """The row walk of the backward pass at head dim 128 (four accumulator tiles parked per part)."""
+@pytest.mark.parametrize("small", [0, 8192], ids=["long_chunks", "short_chunks"])
+def test_split_rows_at_head_dim_128(small, monkeypatch):
+    """The row walks at head dim 128 (four accumulator tiles parked per part), with and without stored stacks."""
     import sparse
     from sparse import _ops
+    monkeypatch.setattr(_ops, "ATTENTION_SMALL_BLOCKS", small)
     mask = np.zeros((4, 120), dtype=np.int64)
     mask[0, :] = 1
     mask[1, ::7] = 1
@@ -159,13 +165,16 @@ def test_split_rows_at_head_dim_128():
     q, k, v, dout = mk(4), mk(120), mk(120), mk(4)
     L = sparse.SparseLayout(torch.as_tensor(mask))
     rl, cl = L.row_layout, L.col_layout
-    assert _ops._attention_schedule(rl, _ops.SCHEDULE_ATTENTION_BACKWARD, split=True).split_groups == 2
+    assert _ops._attention_schedule_for(rl, _ops.SCHEDULE_ATTENTION_BACKWARD, 2).split_groups == 2
     out, lse = _ops.sparse_attention_forward(q.cuda(), k.cuda(), v.cuda(), rl[0], rl[1], 0.09, False, cl, return_lse=True)
     assert rel_err(to_np(out), ao.forward(to_np(q), to_np(k), to_np(v), mask, 0.09, False)) <= TOL
     p, ds, dq = _ops.sparse_attention_backward_scores(q.cuda(), k.cuda(), v.cuda(), dout.cuda(), out, lse, rl[0], rl[1],
                                                       0.09, False, cl)
-    ref_dq = ao.backward(to_np(q), to_np(k), to_np(v), to_np(dout), mask, 0.09, False)[0]
-    assert rel_err(to_np(dq), ref_dq) <= 4 * TOL
+    ref = ao.backward(to_np(q), to_np(k), to_np(v), to_np(dout), mask, 0.09, False)
+    assert rel_err(to_np(dq), ref[0]) <= 4 * TOL
+    grads = _ops.sparse_attention_backward(q.cuda(), k.cuda(), v.cuda(), dout.cuda(), out, lse, rl[0], rl[1], cl[0], cl[1], 0.09)
+    for got, want in zip(grads, ref):
+        assert rel_err(to_np(got), want) <= 4 * TOL
 
 
 def test_large_logits_stay_finite():
@@ -193,7 +202,7 @@ def test_matches_the_unfused_chain_on_config5():
 @pytest.mark.parametrize("head,causal,name", [(64, True, "rand16"), (64, False, "empty_row_col_6x5"), (128, True, "rand16"),
                                               (128, False, "long_row_5x40"), (64, True, "long_col_70x3")])
 def test_gradients_match_the_unfused_chain(head, causal, name):
-    """Autograd through sparse.attention (two-launch backward at head dim 64, stored-stack backward at 128)
+    """Autograd through sparse.attention (a backward of two launches)
     against the chain of the three differentiable operators and against float64 autograd of the dense meaning."""
     import sparse
     mask = np.asarray(ZOO[name])

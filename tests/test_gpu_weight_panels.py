@@ -67,7 +67,8 @@ def test_more_batch_entries_than_a_grid_dimension_holds():
 
 
 @pytest.mark.parametrize("rows,cols,density", [(1, 1, 1.0), (8, 8, 1.0), (9, 7, 0.5), (20, 33, 0.3)])
-@pytest.mark.parametrize("batch,tokens", [(1, 32), (1, 160), (3, 224), (5, 64)])      # 1, 5, 21 and 10 steps: every tail
+# steps of a share: 1, 5, 6, 8, 10, 21 (or 10 and 11) and 15: every remainder of the six-step loop
+@pytest.mark.parametrize("batch,tokens", [(1, 32), (1, 160), (1, 192), (1, 256), (5, 64), (3, 224), (1, 480)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_weight_gradient(any_size, rows, cols, density, batch, tokens, dtype):
     from sparse import _ops
