@@ -255,7 +255,8 @@ __global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attention_fwd_f16_kerne
 // straight from those registers.  K_c is read from LDS twice, along d for S and along its rows for dq;
 // both reads come first, so that the next K is requested before anything is multiplied.  dq alone (us, before -> after):
 // 16 heads of 4096 tokens 26.8 -> 20.6, 48 of 8192 116 -> 94; at head dim 128, where two stacks were stored, 69 -> 40.
-// Without STACKS nothing is stored per block and delta is left for the column walk.
+// Without STACKS nothing is stored per block and delta is left for the column walk: what sparse.attention runs.  STACKS
+// serves bsa_attention_backward_scores alone, for callers that finish with products over the stored blocks.
 // ---------------------------------------------------------------------------
 // per wave: K and V tiles (= the dq^T part of the merge), and with STACKS the two result blocks of 2 KB
 constexpr int at_bwd_lds_per_wave(int hd, bool stacks) { return 128 * hd + (stacks ? 4096 : 0); }

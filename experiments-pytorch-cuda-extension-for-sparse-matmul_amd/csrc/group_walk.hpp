@@ -1,4 +1,4 @@
-// Pieces the walks over groups of a block table share (matmul.hip, bin_walk.hip): where a wave's
+// Pieces the walks over groups of a block table share (matmul.hip, dsd_runs.hip): where a wave's
 // 32 x 64 result tile goes, and how the parts of a group that was cut across workgroups meet.
 #pragma once
 

@@ -70,7 +70,9 @@ SCHEDULE_ATTENTION_BACKWARD_COLUMNS = (12, 2)
 # (1530 blocks) 10.6 / 12.8 / 18.2 -> 8.1 / 10.0 / 16.2 us; 4 entries (6120) 11.6 / 13.8 / 18.3 -> 10.7 / 13.2 / 17.8; 8
 # entries of a random mask (13100) 15.2 / 18.0 / 19.5 -> 15.8 / 20.5 / 22.1.
 # The workgroup's share (cap * waves) stays what it is for a large launch wherever a group is longer than 24 blocks
-# (_attention_kinds): no launch needs a workspace that another batch count of the same layout does not need.
+# (_attention_kinds): no launch needs a workspace that another batch count of the same layout does not need.  Chunks of 6
+# in 4 and in 8 waves, one entry, forward / backward: causal local-4 + stride-8 of 8192 tokens (rows of up to 36) 9.5 / 30.0 ->
+# 8.7 / 30.1 us, a quarter of 128 x 128 blocks (44) 10.8 / 21.9 -> 10.5 / 22.0, at head dim 128 14.5 / 35.3 -> 15.4 / 37.5.
 SCHEDULE_ATTENTION_SMALL = (6, 4)
 ATTENTION_SMALL_BLOCKS = 8192          # blocks of all batch entries together
 # block rows of at most this many blocks are handed whole to SOFTMAX_SLICES wavefronts (8 element rows
