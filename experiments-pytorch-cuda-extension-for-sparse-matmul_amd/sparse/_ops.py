@@ -307,26 +307,36 @@ def _attention_schedule(layout, kind, split=False, most_waves=ATTENTION_WAVES_LO
     return schedule_for(layout, _attention_kind(layout, kind, split, most_waves))
 
 
-def _attention_kinds(kind, few_blocks):
+def _attention_kinds(layout, kind, few_blocks):
     """Schedules to consider for a launch, in this order: the first that cuts no group into parts, else the last."""
     if not few_blocks:
         return (kind,)
-    chunk = SCHEDULE_ATTENTION_SMALL[0]
-    return SCHEDULE_ATTENTION_SMALL, (chunk, kind[0] * kind[1] // chunk)
+    cap, waves = SCHEDULE_ATTENTION_SMALL
+    same_share = cap, kind[0] * kind[1] // cap
+    some_group_is_longer = layout[0].numel() // 2 > cap * waves * (layout[1].numel() - 1)      # longer than the average
+    return (same_share,) if some_group_is_longer else (SCHEDULE_ATTENTION_SMALL, same_share)
 
 
 def _attention_schedule_for(layout, kind, batches, most_waves=ATTENTION_WAVES_LONG_GROUPS):
     """Schedule of a fused attention walk over ``batches`` entries: ``kind``, or shorter chunks for a small launch.  Nothing
     can be built under graph capture: there the other length serves when only that one has been used eagerly."""
     few = layout[0].numel() // 2 * batches <= ATTENTION_SMALL_BLOCKS
+    chosen = getattr(layout[1], "_bsa_attention", None)
+    if chosen is None:
+        chosen = layout[1]._bsa_attention = {}
+    key = (kind, few, ATTENTION_SPLIT_ROWS, most_waves)
+    if key in chosen:
+        return chosen[key]
     for few_blocks in (few, not few):
-        kinds = _attention_kinds(kind, few_blocks)
+        kinds = _attention_kinds(layout, kind, few_blocks)
         for k in kinds:
             if not _has_schedule(layout, _attention_kind(layout, k, ATTENTION_SPLIT_ROWS, most_waves)) \
                     and torch.cuda.is_current_stream_capturing():
                 break
             sched = _attention_schedule(layout, k, ATTENTION_SPLIT_ROWS, most_waves)
             if sched.split_groups == 0 or k == kinds[-1]:
+                if few_blocks == few:
+                    chosen[key] = sched
                 return sched
     raise RuntimeError("fused attention has never run on this layout outside graph capture: call it once eagerly before "
                        "capturing (building its schedule synchronises)")
@@ -591,11 +601,10 @@ def _attention_common(q, k, v, row_blocks, row_table, col_layout):
     return row_layout, mask_rows, mask_cols, row_blocks.numel() // 2, head, batches
 
 
-def _tile_operand(t):
-    """``t`` contiguous and at a multiple of 16 bytes: the attention walks load it straight to LDS, 16 bytes a lane.  A
+def _at_16_bytes(*operands):
+    """Contiguous operands at multiples of 16 bytes: the attention walks load them straight to LDS, 16 bytes a lane, and a
     contiguous view may start anywhere in its storage."""
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
+    return tuple(t if t.data_ptr() & 15 == 0 else t.clone() for t in operands)
 
 
 def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=False, col_layout=None,
@@ -606,7 +615,9 @@ def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=F
     With ``return_lse`` also the fp32 row statistics the backward pass needs."""
     row_layout, mask_rows, mask_cols, nnz, head, batches = _attention_common(q, k, v, row_blocks, row_table,
                                                                               col_layout)
-    q, k, v = _tile_operand(q), _tile_operand(k), _tile_operand(v)
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr()) & 15:
+        q, k, v = _at_16_bytes(q, k, v)
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device) if return_lse else None
     if out.numel() > 0:
@@ -635,8 +646,9 @@ def sparse_attention_backward_scores(q, k, v, dout, out, lse, row_blocks, row_ta
         raise ValueError("dout and out must match q in shape and dtype")
     if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
         raise ValueError("lse must be the float32 row statistics of the forward pass")
-    q, k, v, dout = (_tile_operand(t) for t in (q, k, v, dout))
-    out, lse = out.contiguous(), lse.contiguous()
+    q, k, v, dout, out, lse = (t.contiguous() for t in (q, k, v, dout, out, lse))
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr() | dout.data_ptr()) & 15:
+        q, k, v, dout = _at_16_bytes(q, k, v, dout)
     shape = q.shape[:-2] + (nnz, BLOCK, BLOCK)
     p = torch.empty(shape, dtype=q.dtype, device=q.device)
     ds = torch.empty(shape, dtype=q.dtype, device=q.device)
@@ -671,8 +683,9 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
         raise ValueError("dout and out must match q in shape and dtype")
     if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
         raise ValueError("lse must be the float32 row statistics of the forward pass")
-    q, k, v, dout = (_tile_operand(t) for t in (q, k, v, dout))
-    out, lse = out.contiguous(), lse.contiguous()
+    q, k, v, dout, out, lse = (t.contiguous() for t in (q, k, v, dout, out, lse))
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr() | dout.data_ptr()) & 15:
+        q, k, v, dout = _at_16_bytes(q, k, v, dout)
     dq = torch.empty_like(q)
     dk, dv = (torch.empty_like(k), torch.empty_like(v)) if with_dkdv else (None, None)
     if q.numel() > 0:
