@@ -438,15 +438,16 @@ __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kern
 // delta of the row walk above) read: the probabilities and the score gradients are rebuilt in
 // registers a second time rather than stored by the row walk and read back (4 KB written + 4 KB
 // read of HBM traffic per block that this pair of kernels does not have).
-//   S  = Q_r K_c^T, delta - dO_r V_c^T   K_c and -V_c stay in registers; a lane holds ONE key column, 16 queries, whose lse
-//                                      and delta come into LDS with the tiles; delta is where the second product starts
+//   S  = Q_r K_c^T, dP = dO_r V_c^T    K_c and V_c stay in registers; a lane holds ONE key column, 16 queries, whose lse
+//                                      and delta come into LDS with the tiles
 //   dv^T += dO_r^T P,  dk^T += Q_r^T dS   the 16-bit P and dS values are the column operands straight from the
 //                                      accumulators, the Q_r and dO_r tiles are read a second time along their rows
-// The waves of a column add their parts through LDS.  Two waves per SIMD at head dim 64 (184 registers), one at 128 (its
+// The waves of a column add their parts through LDS.  Two waves per SIMD at head dim 64 (200 registers), one at 128 (its
 // four accumulators are 256); three at 64 spill the K operands and are slower.  us, before -> after: 16 heads of 4096
 // tokens 34.9 -> 29.6, 48 of 8192 150 -> 135; at head dim 128, as two products over stored stacks before, 69 -> 66.
-// Delta kept scaled in memory, or subtracted behind the product, makes no difference to the whole backward pass (50.7-51.6
-// against 51.2-51.7 us, 198.7-199.5 against 198.9-200.2, at head dim 128 102.6-104.2 against 101.2-104.3).
+// Delta is scaled as it is read; with scale * delta in memory the whole backward pass takes 1 % less (48.4-49.0 against 49.3-50.1
+// us).  Starting the second product at delta, 184 registers, takes as long and is further from float64 (dk of fp16, causal:
+// 3.1957e-4 against 3.1949e-4, at head dim 128 3.4662e-4 against 3.4642e-4).
 // ---------------------------------------------------------------------------
 constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256; }   // Q + dO tiles (= one parked accumulator set) + lse, delta
 
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
 #pragma unroll
                 for (int s = 0; s < KS; ++s) {
                     kop[s] = rd.rows(Q_TILE, s);
-                    vop[s] = negated_16(rd.rows(DO_TILE, s));
+                    vop[s] = rd.rows(DO_TILE, s);
                 }
                 lds_reads_done();
             }
@@ -541,20 +542,21 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                 }
                 tile_wait<0>();
                 {
-                    f16v acc;                    // delta - dP
+                    f16v dpacc = {0};
                     h8 dop[KS];
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[4 * g + j] = dl[j];
-                    }
 #pragma unroll
                     for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
 #pragma unroll
-                    for (int s = 0; s < KS; ++s) acc = mfma_16<BF>(dop[s], vop[s], acc);
+                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], vop[s], dpacc);
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) ds[v >> 3][v & 7] = narrow_16<BF>(prob[v] * (acc[v] * -scale));
+                    for (int g = 0; g < 4; ++g) {
+                        const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h) * scale;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int v = 4 * g + j;
+                            ds[v >> 3][v & 7] = narrow_16<BF>(prob[v] * __builtin_fmaf(dpacc[v], scale, -dl[j]));
+                        }
+                    }
                 }
                 // The tiles are read a second time, Q first: the requests for the next block go out as soon as each is free.
                 h8 tr[KT][2];

@@ -12,11 +12,6 @@ __device__ __forceinline__ float at_lane_xor32(float x)
 {
     return __int_as_float(__builtin_amdgcn_ds_bpermute((lane_id() ^ 32) << 2, __float_as_int(x)));
 }
-__device__ __forceinline__ h8 negated_16(h8 x)      // either 16-bit type
-{
-    const uint4 b = __builtin_bit_cast(uint4, x);
-    return as_h8(make_uint4(b.x ^ 0x80008000u, b.y ^ 0x80008000u, b.z ^ 0x80008000u, b.w ^ 0x80008000u));
-}
 __device__ __forceinline__ float at_finite_or_zero(float m) { return m == -__builtin_inff() ? 0.f : m; }
 
 // ---- loads that go straight to LDS ------------------------------------------------------------------
