@@ -442,17 +442,23 @@ __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kern
 //                                      and delta come into LDS with the tiles
 //   dv^T += dO_r^T P,  dk^T += Q_r^T dS   the 16-bit P and dS values are the column operands straight from the
 //                                      accumulators, the Q_r and dO_r tiles are read a second time along their rows
-// The waves of a column add their parts through LDS.  Two waves per SIMD at head dim 64 (200 registers), one at 128 (its
-// four accumulators are 256); three at 64 spill the K operands and are slower.  us, before -> after: 16 heads of 4096
-// tokens 34.9 -> 29.6, 48 of 8192 150 -> 135; at head dim 128, as two products over stored stacks before, 69 -> 66.
+// The waves of a column add their parts through LDS.  Three waves per SIMD at head dim 64 (168 registers: V is read out of
+// LDS for every block, the exponentials stay in front of the second product), one at 128 (its four accumulators are 256).
+// us, both sides in turn on one box, two waves per SIMD (200 registers) -> three: 48 heads of 8192 tokens 114.1 -> 105.8, the
+// training pass 275.2 -> 266.3.  At 128 a second stage of tiles, requested a whole block ahead, took 63.1 -> 66.1 us at 16
+// heads of 4096 tokens.  At 64 one workgroup per residency slot that walks several columns and requests the next one's
+// tiles early took 111 -> 129 us (its neighbours drift apart and leave the L2's working set), forward and rows likewise.
 // Delta is scaled as it is read; with scale * delta in memory the whole backward pass takes 1 % less (48.4-49.0 against 49.3-50.1
 // us).  Starting the second product at delta, 184 registers, takes as long and is further from float64 (dk of fp16, causal:
 // 3.1957e-4 against 3.1949e-4, at head dim 128 3.4662e-4 against 3.4642e-4).
 // ---------------------------------------------------------------------------
-constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256; }   // Q + dO tiles (= one parked accumulator set) + lse, delta
+// Q + dO tiles (= one parked accumulator set) + lse, delta; at head dim 64 also V, whose operands are read again for every
+// block: kept in registers they are the 16 that stand between the walk and three waves per SIMD
+constexpr bool at_bwd_col_keeps_v(int hd) { return hd == 64; }
+constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256 + (at_bwd_col_keeps_v(hd) ? 64 * hd : 0); }
 
 template <int HD, bool BF>
-__global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64 ? 2 : 1) void attention_bwd_dkdv_kernel(
+__global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64 ? 3 : 1) void attention_bwd_dkdv_kernel(
     const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
     const half_t *__restrict__ dout, const float *__restrict__ lse, const float *__restrict__ delta,
     half_t *__restrict__ dk_out, half_t *__restrict__ dv_out,
@@ -475,7 +481,8 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
 
     unsigned char *tile_q = lds_raw + (size_t)w * LDS_PER_WAVE, *tile_do = tile_q + 64 * HD;
     const TileReader rd(tile_q);
-    constexpr unsigned Q_TILE = 0, DO_TILE = 64 * HD;
+    constexpr bool KEEPS_V = at_bwd_col_keeps_v(HD);
+    constexpr unsigned Q_TILE = 0, DO_TILE = 64 * HD, V_TILE = KEEPS_V ? 128 * HD + 256 : DO_TILE;
     const float *stats = reinterpret_cast<const float *>(tile_q + 128 * HD);      // 32 lse, 32 delta of the block's queries
     const TileRequests<HD> qreq(q + (size_t)batch * rows_q * HD, tile_q), doreq(dout + (size_t)batch * rows_q * HD, tile_do);
     const float *my_stat = (l < 32 ? lse : delta) + (size_t)batch * rows_q + (l & 31);
@@ -490,7 +497,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
         h8 kop[KS], vop[KS];
         // K_c and V_c go through the tiles, as Q_r does in the forward walk, while the block rows are fetched
         TileRequests<HD>(k + (size_t)batch * rows_k * HD, tile_q).issue(c);
-        TileRequests<HD>(v + (size_t)batch * rows_k * HD, tile_do).issue(c);
+        TileRequests<HD>(v + (size_t)batch * rows_k * HD, tile_q + V_TILE).issue(c);
         for (int seg = e.begin; seg < e.end; seg += WAVE) {
             const int seg_end = seg + WAVE < e.end ? seg + WAVE : e.end;
             win.fetch(blocks, seg, seg_end);
@@ -504,7 +511,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
 #pragma unroll
                 for (int s = 0; s < KS; ++s) {
                     kop[s] = rd.rows(Q_TILE, s);
-                    vop[s] = rd.rows(DO_TILE, s);
+                    if (!KEEPS_V) vop[s] = rd.rows(V_TILE, s);
                 }
                 lds_reads_done();
             }
@@ -525,9 +532,11 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
 #pragma unroll
                     for (int s = 0; s < KS; ++s) prob = mfma_16<BF>(qop[s], kop[s], prob);
                     if (masked) {                // a hidden score has no probability
+                        int first = key - 4 * h;
+                        asm volatile("" : "+v"(first));      // its comparisons stay here: 16 masks would be kept through the walk
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            if (c > r || key > 8 * (v >> 2) + 4 * h + (v & 3)) prob[v] = scale2 < 0.f ? __builtin_inff() : -__builtin_inff();
+                            if (c > r || first > 8 * (v >> 2) + (v & 3)) prob[v] = scale2 < 0.f ? __builtin_inff() : -__builtin_inff();
                     }
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
@@ -536,10 +545,13 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                         for (int j = 0; j < 4; ++j) {
                             const int v = 4 * g + j;
                             prob[v] = at_exp2(__builtin_fmaf(prob[v], scale2, -ls[j]));
-                            pop[v >> 3][v & 7] = narrow_16<BF>(prob[v]);
+                            if (!KEEPS_V) pop[v >> 3][v & 7] = narrow_16<BF>(prob[v]);
                         }
                     }
                 }
+                // The exponentials come here.  The compiler moved them behind the products below, which wait for dO, and kept
+                // the 32 statistics in registers beside the scores.
+                if (KEEPS_V) asm volatile("" : "+v"(prob));
                 tile_wait<0>();
                 {
                     f16v dpacc = {0};
@@ -547,7 +559,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
 #pragma unroll
                     for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
 #pragma unroll
-                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], vop[s], dpacc);
+                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], KEEPS_V ? rd.rows(V_TILE, s) : vop[s], dpacc);
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h) * scale;
@@ -555,6 +567,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                         for (int j = 0; j < 4; ++j) {
                             const int v = 4 * g + j;
                             ds[v >> 3][v & 7] = narrow_16<BF>(prob[v] * __builtin_fmaf(dpacc[v], scale, -dl[j]));
+                            if (KEEPS_V) pop[v >> 3][v & 7] = narrow_16<BF>(prob[v]);
                         }
                     }
                 }
