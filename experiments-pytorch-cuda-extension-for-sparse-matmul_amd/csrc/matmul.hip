@@ -319,10 +319,55 @@ __device__ __forceinline__ void lds_get_f32(const float *tile, float (&v)[16])
     }
 }
 
+// fp32 products on the bf16 matrix instructions.  An fp32 value is the sum of three bfloat16 values (24 = 3 x 8 bits of
+// significand; each is the rounding of what the ones before leave, and the last remainder is exact), and of the nine products of
+// two such sums the six down to 2^-16 of the first carry what an fp32 sum can hold:
+//   lo hi + mid mid + hi lo, then mid hi + hi mid, then hi hi, smallest first into the fp32 accumulator.
+// 16 steps of k cost 6 x 32 clocks of the matrix pipe instead of 8 x 64 of v_mfma_f32_32x32x2_f32, and unlike that instruction
+// they leave the vector datapath to the other waves (beside an fp32 chain another wave's FMA took 92 clocks instead of 7).
+// What bfloat16 cannot split is seen in the result, and the wave takes its products again on the fp32 instruction: an infinity or
+// NaN, or a value that rounds to infinity, leaves a remainder of NaN; below 2^-109 the last part falls under the smallest
+// bfloat16, which shows while the other operand is below 2^49 / k as results that are all below 2^-60 in a lane.
+// Error against float64 (2-norm, normal operands; fp32 instruction -> split): k = 32 1.03e-7 -> 0.69e-7, 64 1.44e-7 -> 1.09e-7,
+// 128 2.03e-7 -> 1.63e-7; the same from 1e-17 to 1e15.  us, fp32 instruction, one block a wave -> split, four blocks (16 heads of
+// 4096 tokens, 24480 blocks, head dim 64) 43.3 -> 36.0, 48 heads 122 -> 96, 16 heads of 2048 17.6 -> 15.0: the stores remain.
+struct SplitF32 {
+    h8 hi, mid, lo;                          // eight values of k
+};
+__device__ __forceinline__ SplitF32 split_f32(const float *v)
+{
+    SplitF32 o;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        o.hi[t] = narrow_16<true>(v[t]);
+        const float r = v[t] - widen_16<true>(o.hi[t]);
+        o.mid[t] = narrow_16<true>(r);
+        o.lo[t] = narrow_16<true>(r - widen_16<true>(o.mid[t]));
+    }
+    return o;
+}
+__device__ __forceinline__ f16v mfma_split(const SplitF32 &a, const SplitF32 &b, f16v acc)
+{
+    acc = mfma_16<true>(a.lo, b.hi, acc);
+    acc = mfma_16<true>(a.mid, b.mid, acc);
+    acc = mfma_16<true>(a.hi, b.lo, acc);
+    acc = mfma_16<true>(a.mid, b.hi, acc);
+    acc = mfma_16<true>(a.hi, b.mid, acc);
+    return mfma_16<true>(a.hi, b.hi, acc);
+}
+// whether some lane's results say that the split did not hold (uniform across the wave)
+__device__ __forceinline__ bool split_failed(const f16v &acc)
+{
+    float sum = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sum += __builtin_fabsf(acc[v]);
+    return __builtin_amdgcn_ballot_w64(!(sum < __builtin_inff()) || (sum != 0.f && sum < 0x1p-60f)) != 0ull;
+}
+
 // SDD fp32 with K = 32 KBT <= 128: the operands of the wave's block row stay in registers (16 KBT floats per
-// lane), the tiles of block p + 1 are requested as soon as those of block p have left their registers for LDS,
+// lane, or their three parts), the tiles of block p + 1 are requested as soon as those of block p have left their registers for LDS,
 // and the products of block p run while they arrive.
-template <bool A_KC, bool B_KC, int KBT>
+template <bool A_KC, bool B_KC, int KBT, bool SPLIT>
 __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
     const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c,
     const BlockDesc *__restrict__ blocks, const SchedEntry *__restrict__ sched,
@@ -342,7 +387,8 @@ __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
     const int r = e.group;
 
     uint4 raw[KBT][4];
-    float aop[KBT][16];
+    SplitF32 aop[KBT][2];
+    float aop32[KBT][16];                    // without SPLIT
     DescWindow win;
     const int first_end = e.begin + WAVE < e.end ? e.begin + WAVE : e.end;
     win.fetch(blocks, e.begin, first_end);
@@ -365,15 +411,35 @@ __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
         for (int kb = 0; kb < KBT; ++kb) lds_put_f32(tiles + kb * (F32_TILE_BYTES / 4), raw[kb]);
         wave_lds_fence();
     };
+    // the products on the fp32 instruction: the row's operands come from memory again
+    auto multiply_f32 = [&]() {
+        f16v acc = {0};
+#pragma unroll 1
+        for (int kb = 0; kb < KBT; ++kb) {
+            float av[16], bop[16];
+            if (A_KC) ldg_tile_f32<true, false>(ab + (size_t)(BS * r) * K + BS * kb, K, av);
+            else ldg_tile_f32<false, false>(ab + (size_t)(BS * kb) * M + BS * r, M, av);
+            lds_get_f32<B_KC, true>(tiles + kb * (F32_TILE_BYTES / 4), bop);
+#pragma unroll
+            for (int t = 0; t < 16; ++t) acc = mfma_f32(bop[t], av[t], acc);
+        }
+        return acc;
+    };
     auto multiply = [&](int p) {
         f16v acc = {0};
 #pragma unroll
         for (int kb = 0; kb < KBT; ++kb) {
             float bop[16];
             lds_get_f32<B_KC, true>(tiles + kb * (F32_TILE_BYTES / 4), bop);
+            if (SPLIT) {
 #pragma unroll
-            for (int t = 0; t < 16; ++t) acc = mfma_f32(bop[t], aop[kb][t], acc);
+                for (int s = 0; s < 2; ++s) acc = mfma_split(split_f32(bop + 8 * s), aop[kb][s], acc);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 16; ++t) acc = mfma_f32(bop[t], aop32[kb][t], acc);
+            }
         }
+        if (SPLIT && split_failed(acc)) acc = multiply_f32();
         // a lane holds 16 consecutive columns of one row; the block leaves through LDS as four whole
         // kilobytes (64-byte pieces at 128-byte stride straight from the registers write at a third of the rate)
         wave_lds_fence();
@@ -389,12 +455,19 @@ __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
                          *reinterpret_cast<const uint4 *>(tiles + put_f32_addr(l, j) / 4));
     };
     park();
+    request(e.begin);        // the first block's tiles arrive while the row's operands are split
 #pragma unroll
-    for (int kb = 0; kb < KBT; ++kb) lds_get_f32<A_KC, false>(tiles + kb * (F32_TILE_BYTES / 4), aop[kb]);
+    for (int kb = 0; kb < KBT; ++kb) {
+        lds_get_f32<A_KC, false>(tiles + kb * (F32_TILE_BYTES / 4), aop32[kb]);
+#pragma unroll
+        for (int s = 0; SPLIT && s < 2; ++s) aop[kb][s] = split_f32(aop32[kb] + 8 * s);
+    }
     for (int seg = e.begin; seg < e.end; seg += WAVE) {
         const int seg_end = seg + WAVE < e.end ? seg + WAVE : e.end;
-        if (seg != e.begin) win.fetch(blocks, seg, seg_end);
-        request(seg);
+        if (seg != e.begin) {
+            win.fetch(blocks, seg, seg_end);
+            request(seg);
+        }
         for (int p = seg; p + 1 < seg_end; ++p) {
             park();
             request(p + 1);
@@ -1063,11 +1136,21 @@ static hipError_t launch_sdd_f32(const MatmulArgs &p, hipStream_t st)
             kernel<<<grid, block, lds, st>>>(BSA_SDD_ARGS);
             return hipGetLastError();
         };
+        // With less than a block for each of the 1024 SIMDs nothing overlaps, and the fp32 instruction is the shorter chain:
+        // 80 blocks 4.4 us against 4.7 split, 744 4.2 against 4.5, 1012 6.2 against 5.7.
+        if ((long long)p.nnz * p.batches < 800) {
+            switch (kbs) {
+                case 1: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 1, false>);
+                case 2: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 2, false>);
+                case 3: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 3, false>);
+                default: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 4, false>);
+            }
+        }
         switch (kbs) {
-            case 1: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 1>);
-            case 2: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 2>);
-            case 3: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 3>);
-            default: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 4>);
+            case 1: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 1, true>);
+            case 2: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 2, true>);
+            case 3: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 3, true>);
+            default: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 4, true>);
         }
     }
     sdd_f32_kernel<A_KC, B_KC><<<grid, block, 0, st>>>(BSA_SDD_ARGS);

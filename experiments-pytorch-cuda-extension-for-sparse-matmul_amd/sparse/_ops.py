@@ -18,7 +18,15 @@ SCHEDULE_GROUP_WALK = (12, 4, True, -1, 2, True)        # groups of at most GROU
 SCHEDULE_GROUP_WALK_LONG = (10, 4, True, -1, 2, True)    # tables with longer groups (columns of causal / strided masks)
 GROUP_WALK_LONG = 24
 SCHEDULE_SDD = (4, 2)
-SCHEDULE_SDD_F32 = (1, 4)              # fp32 SDD reloads both operands per block anyway: one block per wave
+# fp32: a wave splits its row's operands once, so chunks pay where the launch fills the machine with them; below, one block a
+# wave is the shorter chain.  us, chunks of 1 in 4 waves -> of 4 in 2: 1012 blocks 5.7 -> 7.9, 8096 16.2 -> 15.2, 10144 (window
+# of 5) 22.3 -> 17.0, 24480 42.9 -> 36.0, 73440 123.6 -> 95.3.
+SCHEDULE_SDD_F32 = (1, 4)
+SCHEDULE_SDD_F32_LARGE = (4, 2)
+SDD_F32_LARGE_BLOCKS = 8000            # of all batch entries together
+# fp32 groups of at most GROUP_WALK_LONG pairs: chunks of 6 in 4 waves hold such a group in one workgroup too.  us, chunks of 12
+# -> 6 (DSD): 744 blocks 13.6 -> 11.2, 1012 19.7 -> 12.8, 8096 25.2 -> 20.3, 11912 29.4 -> 24.6, 73440 114 -> 114.
+SCHEDULE_GROUP_WALK_F32 = (6, 4, True, -1, 2, True)
 SCHEDULE_SOFTMAX = (4, 4)
 SOFTMAX_LONGEST_FIRST = True     # long rows are dispatched first: they would otherwise finish on a draining machine
 SOFTMAX_WAVES_LONG_ROWS = 8
@@ -280,8 +288,28 @@ def _group_walk_kind(longest):
     return SCHEDULE_GROUP_WALK_LONG if longest > GROUP_WALK_LONG else SCHEDULE_GROUP_WALK
 
 
-def _group_walk_schedule(layout):
-    return schedule_for(layout, _group_walk_kind(_longest_group(layout[1])))
+def _group_walk_schedule(layout, dtype=torch.float16):
+    kind = _group_walk_kind(_longest_group(layout[1]))
+    if dtype == torch.float32 and kind is SCHEDULE_GROUP_WALK:
+        return _schedule_or(layout, SCHEDULE_GROUP_WALK_F32, kind)
+    return schedule_for(layout, kind)
+
+
+def _sdd_schedule(layout, dtype, batches):
+    if dtype != torch.float32:
+        return schedule_for(layout, SCHEDULE_SDD)
+    if layout[0].numel() * batches >= 2 * SDD_F32_LARGE_BLOCKS:
+        return _schedule_or(layout, SCHEDULE_SDD_F32_LARGE, SCHEDULE_SDD_F32)
+    return _schedule_or(layout, SCHEDULE_SDD_F32, SCHEDULE_SDD_F32_LARGE)
+
+
+def _schedule_or(layout, kind, other):
+    """The schedule ``kind``, or, where a graph is being captured and only ``other`` is there, that one: building
+    synchronises."""
+    there = getattr(layout[1], "_bsa_schedules", ())
+    if kind in there:
+        return there[kind]
+    return schedule_for(layout, other if other in there and torch.cuda.is_current_stream_capturing() else kind)
 
 
 def _captured_without(layout, kind) -> bool:
@@ -466,9 +494,9 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
         return c
 
     if mode == "sdd":
-        sched = schedule_for(layout, SCHEDULE_SDD_F32 if a.dtype == torch.float32 else SCHEDULE_SDD)
+        sched = _sdd_schedule(layout, a.dtype, batches)
     else:
-        sched = _group_walk_schedule(layout)
+        sched = _group_walk_schedule(layout, a.dtype)
     with _k.on_device(a.device):
         stream = _k.current_stream()
         ws, ws_bytes = sched.workspace(_k.MODES[mode], batches, size_m, size_n, stream)
