@@ -12,6 +12,7 @@ SOURCES = ["api.hip", "layout_build.hip", "matmul.hip", "dsd_runs.hip", "softmax
            "weight_panels.hip"]
 HEADERS = ["bench_yardstick.hip", "bsa_device.hpp", "lds_tiles.hpp", "lds_index_math.hpp", "bsa_internal.hpp", "group_walk.hpp", "attention_tiles.hpp", os.path.join("..", "..", "include", "bsa.h")]
 LIB = os.path.join(HERE, "libbsa_hip.so")
+HOST_CALLS = os.path.join(HERE, "bsa_host_calls.so")
 
 # The same library built with the compile-time alternative of a hand-rolled sequence, for the test that pins the
 # default against it (tests/test_gpu_build_variants.py): full agent-scope fences around the counter of split
@@ -29,10 +30,10 @@ FLAGS = [
 
 
 def out_of_date() -> bool:
-    if not os.path.exists(LIB) or not all(os.path.exists(path) for path, _ in CHECK_VARIANTS.values()):
+    if not all(os.path.exists(path) for path in [LIB, HOST_CALLS] + [path for path, _ in CHECK_VARIANTS.values()]):
         return True
     t = os.path.getmtime(LIB)
-    return any(os.path.getmtime(os.path.join(HERE, f)) > t for f in SOURCES + HEADERS + ["build.py"])
+    return any(os.path.getmtime(os.path.join(HERE, f)) > t for f in SOURCES + HEADERS + ["host_calls.cpp", "build.py"])
 
 
 def build(force: bool = False, verbose: bool = False, extra_flags=(), lib: str = LIB) -> str:
@@ -70,6 +71,7 @@ def build(force: bool = False, verbose: bool = False, extra_flags=(), lib: str =
         raise RuntimeError("hipcc failed linking " + os.path.basename(lib))
     if lib == LIB:
         build_index_host(verbose)
+        build_host_calls(verbose)
         build_bench_yardstick(verbose)
         for _, (path, flags) in CHECK_VARIANTS.items():
             build(force=True, verbose=verbose, extra_flags=flags, lib=path)
@@ -98,6 +100,25 @@ def build_index_host(verbose: bool = False) -> str:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
     return out
+
+
+def build_host_calls(verbose: bool = False) -> str:
+    """g++ build of the package's native host side (a Python module against torch's headers; no GPU code)."""
+    import sysconfig
+
+    import torch
+    home = os.path.dirname(torch.__file__)
+    include = [os.path.join(home, "include"), os.path.join(home, "include", "torch", "csrc", "api", "include"),
+               sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    cmd += [flag for path in include for flag in ("-isystem", path)]
+    cmd += [os.path.join(HERE, "host_calls.cpp"), "-o", HOST_CALLS, "-L" + os.path.join(home, "lib")]
+    cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    return HOST_CALLS
 
 
 if __name__ == "__main__":

@@ -1,3 +1,4 @@
+from . import _native
 from .layout import SparseLayout
 from .matmul import matmul
 from .softmax import softmax

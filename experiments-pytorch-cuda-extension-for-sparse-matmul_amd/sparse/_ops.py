@@ -396,8 +396,9 @@ def _check_layout(layout, name):
         raise ValueError(f"{name} is malformed")
 
 
-def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=False):
-    """``c = op(a) @ op(b)`` with one of a, b, c block-sparse (sparse_kernels.cc:7-50)."""
+def _matmul_route(a, b, mode, row_layout, col_layout, trans_a, trans_b):
+    """Checks a product and says how it goes: (walk, its schedule, the table it walks, contiguous operands, shape of the
+    result, whether the batch shares the sparse operand, batch entries, M, N, K)."""
     if mode not in _k.MODES:
         raise ValueError(f"mode must be one of 'sdd', 'dsd', 'dds', got {mode!r}")
     if a.dtype != b.dtype or a.dtype not in _DTYPES:
@@ -456,57 +457,65 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
         shape = batch_a + (size_m, size_n)
     else:
         shape = batch_a + (num_blocks, BLOCK, BLOCK)
-    c = torch.empty(shape, dtype=a.dtype, device=a.device)
+    def route(walk, sched=None):
+        return walk, sched, layout, a, b, shape, shared, batches, size_m, size_n, size_k
 
     coarse = getattr(row_layout[1], "_bsa_coarse", None)
     if (USE_BLOCK64_KERNEL and coarse is not None and mode == "dsd" and not trans_a and not trans_b
             and a.dtype != torch.float32 and size_n % 64 == 0 and num_blocks > 0):
-        (cblocks, coffsets), crows, ccols = coarse
-        sched = schedule_for((cblocks, coffsets), SCHEDULE_BLOCK64)
-        with _k.on_device(a.device):
-            _k.check(_k.lib.bsa_matmul_dsd_block64(
-                _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), cblocks.data_ptr(), coffsets.data_ptr(),
-                sched.table.data_ptr(), sched.workgroups, sched.waves, crows, ccols, cblocks.numel() // 2, batches,
-                1 if shared else batches, size_n, _k.current_stream()))
-        return c
+        return route("block64", schedule_for(coarse[0], SCHEDULE_BLOCK64))
 
     if (RUN_WALK and mode == "dsd" and not trans_a and not trans_b and a.dtype != torch.float32
             and size_n % 64 == 0):
         runs = _run_schedule(layout, batches, size_n // 64)
         if runs is not None:
-            with _k.on_device(a.device):
-                _k.check(_k.lib.bsa_matmul_dsd_runs(
-                    _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(),
-                    layout[1].data_ptr(), runs.table.data_ptr(), runs.runs, runs.strips, runs.pairs, runs.waves,
-                    mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_n, _k.current_stream()))
-            return c
+            return route("runs", runs)
 
     if (PANEL_WALK and mode == "dds" and not trans_a and a.dtype != torch.float32
             and size_m % BLOCK == 0 and size_k == BLOCK * (mask_cols if trans_b else mask_rows)
             and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
             and _takes_panels(num_blocks, size_m * batches if shared else size_m, 1 if shared else batches,
                               size_k // BLOCK, size_n // BLOCK, lambda: _captured_without(layout, None))):
-        with _k.on_device(a.device):
-            _k.check(_k.lib.bsa_matmul_dds_panels(
-                _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
-                mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_m, int(trans_b),
-                _k.current_stream()))
-        return c
+        return route("panels")
 
     if mode == "sdd":
-        sched = _sdd_schedule(layout, a.dtype, batches)
-    else:
-        sched = _group_walk_schedule(layout, a.dtype)
+        return route("walk", _sdd_schedule(layout, a.dtype, batches))
+    return route("walk", _group_walk_schedule(layout, a.dtype))
+
+
+def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=False):
+    """``c = op(a) @ op(b)`` with one of a, b, c block-sparse (sparse_kernels.cc:7-50)."""
+    walk, sched, layout, a, b, shape, shared, batches, size_m, size_n, size_k = _matmul_route(
+        a, b, mode, row_layout, col_layout, trans_a, trans_b)
+    c = torch.empty(shape, dtype=a.dtype, device=a.device)
+    dtype, num_blocks, sparse_batches = _DTYPES[a.dtype], layout[0].numel() // 2, 1 if shared else batches
+    mask_rows, mask_cols = row_layout[1].numel() - 1, col_layout[1].numel() - 1
     with _k.on_device(a.device):
         stream = _k.current_stream()
-        ws, ws_bytes = sched.workspace(_k.MODES[mode], batches, size_m, size_n, stream)
-        _launch(sched, _k.lib.bsa_matmul(
-            _k.MODES[mode], _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), c.data_ptr(),
-            layout[0].data_ptr(), layout[1].data_ptr(), layout[1].numel() - 1,
-            sched.table.data_ptr(), sched.workgroups, sched.waves, sched.tile_slots, sched.split_groups,
-            ws.data_ptr() if ws is not None else None, ws_bytes,
-            mask_rows, mask_cols, num_blocks, batches, 1 if shared else batches, size_m, size_n, size_k,
-            int(trans_a), int(trans_b), stream))
+        if walk == "block64":
+            (cblocks, coffsets), crows, ccols = row_layout[1]._bsa_coarse
+            _k.check(_k.lib.bsa_matmul_dsd_block64(
+                dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(), cblocks.data_ptr(), coffsets.data_ptr(),
+                sched.table.data_ptr(), sched.workgroups, sched.waves, crows, ccols, cblocks.numel() // 2, batches,
+                sparse_batches, size_n, stream))
+        elif walk == "runs":
+            _k.check(_k.lib.bsa_matmul_dsd_runs(
+                dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
+                sched.table.data_ptr(), sched.runs, sched.strips, sched.pairs, sched.waves, mask_rows, mask_cols, num_blocks,
+                batches, sparse_batches, size_n, stream))
+        elif walk == "panels":
+            _k.check(_k.lib.bsa_matmul_dds_panels(
+                dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
+                mask_rows, mask_cols, num_blocks, batches, sparse_batches, size_m, int(bool(trans_b)), stream))
+        else:
+            ws, ws_bytes = sched.workspace(_k.MODES[mode], batches, size_m, size_n, stream)
+            _launch(sched, _k.lib.bsa_matmul(
+                _k.MODES[mode], dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(),
+                layout[0].data_ptr(), layout[1].data_ptr(), layout[1].numel() - 1,
+                sched.table.data_ptr(), sched.workgroups, sched.waves, sched.tile_slots, sched.split_groups,
+                ws.data_ptr() if ws is not None else None, ws_bytes,
+                mask_rows, mask_cols, num_blocks, batches, sparse_batches, size_m, size_n, size_k,
+                int(bool(trans_a)), int(bool(trans_b)), stream))
     return c
 
 
@@ -525,31 +534,39 @@ def sparse_weight_gradient(a, b, row_layout, col_layout, trans_a, trans_b):
     """``sparse_matmul(a, b, 'sdd', ..)`` summed over the batch: the gradient of a sparse operand that the batch shared.
     With both operands stored tokens-first (``trans_a``, not ``trans_b``) the batch and the tokens are one contraction,
     summed in fp32 by bsa_weight_grad; the other forms write a stack per batch entry and add them up."""
+    if _folds(a, b, row_layout, col_layout, trans_a, trans_b):
+        a, b = a.contiguous(), b.contiguous()
+        if a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0:
+            return _folded_weight_gradient(a, b, row_layout, col_layout)
+    stack = sparse_matmul(a, b, "sdd", row_layout, col_layout, trans_a, trans_b)
+    return stack.sum(dim=tuple(range(stack.dim() - 3)))
+
+
+def _folds(a, b, row_layout, col_layout, trans_a, trans_b):
     nnz = row_layout[0].numel() // 2
     rows, cols = row_layout[1].numel() - 1, col_layout[1].numel() - 1
     tokens = a.numel() // max(a.size(-1), 1)
-    folds = (trans_a and not trans_b and a.dtype in (torch.float16, torch.bfloat16) and a.dtype == b.dtype
+    return (trans_a and not trans_b and a.dtype in (torch.float16, torch.bfloat16) and a.dtype == b.dtype
              and a.shape[:-1] == b.shape[:-1] and a.size(-2) % BLOCK == 0 and BLOCK <= tokens < 2 ** 31
              and a.size(-1) == BLOCK * rows and b.size(-1) == BLOCK * cols and a.is_cuda and a.device == b.device
              and row_layout[0].device == a.device and nnz > 0
              and ((tokens >= WEIGHT_GRAD_MIN_TOKENS and nnz >= WEIGHT_GRAD_MIN_DENSITY * rows * cols)
                   or _captured_without(row_layout, SCHEDULE_SDD)))
-    if folds:
-        a, b = a.contiguous(), b.contiguous()
-        folds = a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
-    if folds:
-        _check_layout(row_layout, "row_layout")
-        out = torch.empty((nnz, BLOCK, BLOCK), dtype=a.dtype, device=a.device)
-        shares = _k.lib.bsa_weight_grad_shares(rows, cols, tokens)
-        parts = torch.empty(shares * nnz * BLOCK * BLOCK, dtype=torch.float32, device=a.device)
-        with _k.on_device(a.device):
-            _k.check(_k.lib.bsa_weight_grad(
-                _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), out.data_ptr(), row_layout[0].data_ptr(),
-                row_layout[1].data_ptr(), rows, cols, nnz, tokens, shares, parts.data_ptr(), 4 * parts.numel(),
-                _k.current_stream()))
-        return out
-    stack = sparse_matmul(a, b, "sdd", row_layout, col_layout, trans_a, trans_b)
-    return stack.sum(dim=tuple(range(stack.dim() - 3)))
+
+
+def _folded_weight_gradient(a, b, row_layout, col_layout):
+    _check_layout(row_layout, "row_layout")
+    nnz, tokens = row_layout[0].numel() // 2, a.numel() // a.size(-1)
+    rows, cols = row_layout[1].numel() - 1, col_layout[1].numel() - 1
+    out = torch.empty((nnz, BLOCK, BLOCK), dtype=a.dtype, device=a.device)
+    shares = _k.lib.bsa_weight_grad_shares(rows, cols, tokens)
+    parts = torch.empty(shares * nnz * BLOCK * BLOCK, dtype=torch.float32, device=a.device)
+    with _k.on_device(a.device):
+        _k.check(_k.lib.bsa_weight_grad(
+            _DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), out.data_ptr(), row_layout[0].data_ptr(),
+            row_layout[1].data_ptr(), rows, cols, nnz, tokens, shares, parts.data_ptr(), 4 * parts.numel(),
+            _k.current_stream()))
+    return out
 
 
 def _softmax_common(x, row_layout, col_layout, name):
@@ -696,6 +713,14 @@ def sparse_attention_backward_scores(q, k, v, dout, out, lse, row_blocks, row_ta
     return p, ds, dq
 
 
+def _attention_backward_schedules(row_layout, col_layout, batches, head, with_dkdv):
+    rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
+    cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches,
+                                 ATTENTION_WAVES_LONG_GROUPS if head == 64 else ATTENTION_COLUMN_WAVES_128) \
+        if with_dkdv else None
+    return rs, cs
+
+
 def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, col_blocks, col_table, scale=1.0,
                               causal=False, with_dkdv=True):
     """``(dq, dk, dv)`` of the fused attention in two launches (a walk over the rows, one over the
@@ -718,10 +743,7 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
     dk, dv = (torch.empty_like(k), torch.empty_like(v)) if with_dkdv else (None, None)
     if q.numel() > 0:
         delta = torch.empty_like(lse)
-        rs = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION_BACKWARD, batches)
-        cs = _attention_schedule_for(col_layout, SCHEDULE_ATTENTION_BACKWARD_COLUMNS, batches,
-                                     ATTENTION_WAVES_LONG_GROUPS if head == 64 else ATTENTION_COLUMN_WAVES_128) \
-            if with_dkdv else None
+        rs, cs = _attention_backward_schedules(row_layout, col_layout, batches, head, with_dkdv)
         columns = (cs.table.data_ptr(), cs.workgroups, cs.waves, cs.tile_slots, cs.split_groups) if with_dkdv \
             else (None, 0, 0, 0, 0)
         with _k.on_device(q.device):
@@ -736,3 +758,136 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
                 col_blocks.data_ptr(), col_table.data_ptr(), *columns, ws.data_ptr() if ws is not None else None, ws_bytes,
                 mask_rows, mask_cols, nnz, batches, head, float(scale), int(bool(causal)), stream))
     return dq, dk, dv
+
+
+# ---- plans: what csrc/host_calls.cpp needs to make a call of these shapes again without asking Python ----------------
+_LIB = _k.lib
+_MATMUL, _WEIGHT, _SOFTMAX, _SOFTMAX_BACKWARD, _ATTENTION, _ATTENTION_BACKWARD = range(6)
+_ROUTES = {"walk": 0, "runs": 1, "panels": 2}
+
+
+def _plans(layout, *operands):
+    """The layout's plans where a call on these operands may be planned: nothing under capture (what is missing there is not
+    built, and the walk that serves is not the one an eager call takes), nothing for operands off 16 bytes, which some walks do
+    not take, and nothing while the library is replaced."""
+    if _k.lib is not _LIB or torch.cuda.is_current_stream_capturing() or any(t.data_ptr() & 15 for t in operands):
+        return None
+    return getattr(layout, "_plans", None)
+
+
+def _planned(make):
+    """``make`` returns whether it left a plan; what it cannot do the general path does, or says why not."""
+    @functools.wraps(make)
+    def planned(*args):
+        try:
+            with _k.on_device(args[0].device):
+                return make(*args)
+        except Exception:
+            return False
+    return planned
+
+
+def _add(plans, op, flags, a, b, route, ints, tables, out=(), workspace=(None, 0), sched=None, aligned=False):
+    ws, ws_bytes = workspace
+    _k.host_calls.add_plan(plans, op, flags, a, b, route, _DTYPES[a.dtype], aligned, ints, tables, out, ws, ws_bytes,
+                           _k.current_stream(), sched, sched.last_key if ws is not None else None)
+    return True
+
+
+@_planned
+def plan_matmul(a, b, mode, layout, trans_a, trans_b):
+    plans = _plans(layout, a, b)
+    if plans is None:
+        return False
+    rows, cols = layout.row_layout, layout.col_layout
+    walk, sched, table, _, _, shape, shared, batches, m, n, k = _matmul_route(a, b, mode, rows, cols, trans_a, trans_b)
+    if walk not in _ROUTES:
+        return False
+    counts = (rows[1].numel() - 1, cols[1].numel() - 1, table[0].numel() // 2, batches, 1 if shared else batches)
+    flags = _k.MODES[mode] << 2 | bool(trans_a) << 1 | bool(trans_b)
+    add = functools.partial(_add, plans, _MATMUL, flags, a, b, _ROUTES[walk], out=tuple(shape))
+    if walk == "runs":
+        return add((sched.runs, sched.strips, sched.pairs, sched.waves) + counts + (n,), table + (sched.table,))
+    if walk == "panels":
+        return add(counts + (m, int(bool(trans_b))), table, aligned=True)
+    space = sched.workspace(_k.MODES[mode], batches, m, n, _k.current_stream())
+    return add((_k.MODES[mode], table[1].numel() - 1, sched.workgroups, sched.waves, sched.tile_slots, sched.split_groups) + counts +
+               (m, n, k, int(bool(trans_a)), int(bool(trans_b))), table + (sched.table,), workspace=space, sched=sched)
+
+
+@_planned
+def plan_weight(a, b, layout, trans_a, trans_b):
+    plans = _plans(layout, a, b)
+    rows, cols = layout.row_layout, layout.col_layout
+    if plans is None or not _folds(a, b, rows, cols, trans_a, trans_b):
+        return False
+    _check_layout(rows, "row_layout")
+    nnz, tokens = rows[0].numel() // 2, a.numel() // a.size(-1)
+    mask = rows[1].numel() - 1, cols[1].numel() - 1
+    shares = _k.lib.bsa_weight_grad_shares(*mask, tokens)
+    floats = shares * nnz * BLOCK * BLOCK
+    if floats >= 2 ** 31:
+        return False
+    return _add(plans, _WEIGHT, bool(trans_a) << 1 | bool(trans_b), a, b, 0, mask + (nnz, tokens, shares, floats), rows,
+                (nnz, BLOCK, BLOCK), aligned=True)
+
+
+def _plan_softmax(x, layout, backward):
+    plans = _plans(layout, x)
+    if plans is None:
+        return False
+    nnz, mask_rows, mask_cols, batches = _softmax_common(x, layout.row_layout, layout.col_layout, "x")
+    if nnz == 0 or x.numel() == 0:
+        return False
+    sched = _softmax_schedule(layout.row_layout, x.dtype, backward)
+    return _add(plans, _SOFTMAX_BACKWARD if backward else _SOFTMAX, 0, x, None, 0,
+                (sched.workgroups, sched.waves, mask_rows, mask_cols, nnz, batches), layout.row_layout + (sched.table,))
+
+
+@_planned
+def plan_softmax(x, layout):
+    return _plan_softmax(x, layout, False)
+
+
+@_planned
+def plan_softmax_backward(y, layout):
+    return _plan_softmax(y, layout, True)
+
+
+def _figures(sched):
+    return sched.workgroups, sched.waves, sched.tile_slots, sched.split_groups
+
+
+@_planned
+def plan_attention(q, k, v, layout):
+    plans = _plans(layout, q, k, v)
+    if plans is None or q.numel() == 0:
+        return False
+    rows, *counts = _attention_common(q, k, v, *layout.row_layout, layout.col_layout)
+    mask_rows, mask_cols, nnz, head, batches = counts
+    sched = _attention_schedule_for(rows, SCHEDULE_ATTENTION, batches)
+    space = sched.attention_workspace(batches, head, _k.current_stream())
+    return _add(plans, _ATTENTION, 0, q, k, 0, _figures(sched) + (mask_rows, mask_cols, nnz, batches, head), rows + (sched.table,),
+                workspace=space, sched=sched)
+
+
+@_planned
+def plan_attention_backward(q, k, v, layout, with_dkdv):
+    plans = _plans(layout, q, k, v)
+    if plans is None or q.numel() == 0:
+        return False
+    cols = layout.col_layout
+    _check_layout(cols, "col_layout")
+    rows, mask_rows, mask_cols, nnz, head, batches = _attention_common(q, k, v, *layout.row_layout, cols)
+    rs, cs = _attention_backward_schedules(rows, cols, batches, head, with_dkdv)
+    space = rs.attention_backward_workspace(cs, batches, head, _k.current_stream())
+    return _add(plans, _ATTENTION_BACKWARD, int(bool(with_dkdv)), q, k, 0,
+                _figures(rs) + (_figures(cs) if with_dkdv else (0, 0, 0, 0)) + (mask_rows, mask_cols, nnz, batches, head),
+                rows + (rs.table,) + cols + (cs.table if with_dkdv else None,), workspace=space, sched=rs)
+
+
+def failed(status, sched, key):
+    """Raises for a failed launch; its workspace is forgotten first (``_launch``)."""
+    if sched is not None:
+        sched.discard(key)
+    _k.check(status)

@@ -10,7 +10,7 @@ from typing import Any, Optional, Tuple
 
 import torch
 
-from .kernel import sparse_ops
+from .kernel import host_calls, sparse_ops
 from .layout import SparseLayout
 
 
@@ -50,7 +50,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: SparseL
     the last bits can differ."""
     fused = q.dtype in (torch.float16, torch.bfloat16) and q.size(-1) in (64, 128)
     if fused or not (q.dtype == k.dtype == v.dtype and q.dtype in (torch.float16, torch.bfloat16, torch.float32)):
-        return SparseAttention.apply(q, k, v, layout, scale, causal)     # the fused path also owns the argument checks
+        return host_calls.attention(q, k, v, layout, scale, causal)      # SparseAttention.apply, which also owns the argument checks
     from .matmul import matmul
     from .softmax import softmax
     scores = matmul(q, k, "sdd", layout, False, True)

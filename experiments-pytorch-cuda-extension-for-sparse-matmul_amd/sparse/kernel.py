@@ -9,6 +9,8 @@ there is no fallback path.
 """
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
@@ -79,6 +81,21 @@ def load_library(path: str = LIBRARY_PATH) -> ctypes.CDLL:
 
 
 lib = load_library()
+
+
+def load_host_calls():
+    """The native host side (``csrc/host_calls.cpp``), built beside the library; missing, the import fails as loudly."""
+    path = os.path.join(_CSRC, "bsa_host_calls.so")
+    if not os.path.exists(path):
+        raise ImportError(f"{path} is missing: build it with `python {os.path.join(_CSRC, 'build.py')}`")
+    spec = importlib.util.spec_from_file_location("bsa_host_calls", path,
+                                                  loader=importlib.machinery.ExtensionFileLoader("bsa_host_calls", path))
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+host_calls = load_host_calls()
 
 
 def dds_panel_limits():

@@ -92,6 +92,8 @@ class SparseLayout:
         self.row_layout: Tuple[torch.Tensor, torch.Tensor] = (row_blocks, row_offsets)
         self.col_layout: Tuple[torch.Tensor, torch.Tensor] = (col_blocks, col_offsets)
 
+        self._plans = _k.host_calls.new_plans(self.row_layout, self.col_layout)      # of calls on this layout
+
         self.coarse_row_layout = None
         if per_side > 1:
             # row table of the mask in 64x64 blocks, for the kernel that owns whole blocks
@@ -109,6 +111,13 @@ class SparseLayout:
                                                  _k.current_stream()))
             self.coarse_row_layout = (cb[:nnz // 2].clone(), co)
             self.row_layout[1]._bsa_coarse = (self.coarse_row_layout, crows, ccols)
+
+    def __getstate__(self):
+        return {name: value for name, value in self.__dict__.items() if name != "_plans"}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._plans = _k.host_calls.new_plans(self.row_layout, self.col_layout)
 
     def _index_on(self, device) -> torch.Tensor:
         if self._cell_index.device != device:

@@ -9,7 +9,7 @@ from typing import Any, Optional, Tuple
 
 import torch
 
-from .kernel import sparse_ops
+from .kernel import host_calls, sparse_ops
 from .layout import SparseLayout
 
 
@@ -59,5 +59,6 @@ class SparseMatMul(torch.autograd.Function):
         return da, db, None, None, None, None
 
 
-# Call this, not the class (matmul.py:55-57).
-matmul = SparseMatMul.apply
+# Call this, not the class (matmul.py:55-57).  It is SparseMatMul.apply, in native code where the layout has a plan for these
+# shapes (csrc/host_calls.cpp); the class is what serves every other call.
+matmul = host_calls.matmul

@@ -1,0 +1,234 @@
+"""GPU: calls that go by a plan (csrc/host_calls.cpp) against the Python autograd Functions the plans were made from: the same
+bits over modes, orders, types and sizes, and the same behaviour where a plan does not hold."""
+import copy
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import mask_zoo
+
+pytestmark = pytest.mark.gpu
+ZOO = dict(mask_zoo())
+TYPES = [torch.float32, torch.float16, torch.bfloat16]
+
+
+def _layout(name="long_col_70x3"):
+    import sparse
+    return sparse.SparseLayout(torch.as_tensor(np.asarray(ZOO[name])))
+
+
+def _randn(*shape, dtype, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def _product(L, mode, ta, tb, dim, dtype, lead=(2, 3), shared=False):
+    R, C = (32 * n for n in L.tile_shape)
+    stack = (() if shared else lead) + (L.num_blocks, 32, 32)
+    if mode == "sdd":
+        a, b = (dim, R) if ta else (R, dim), (C, dim) if tb else (dim, C)
+    elif mode == "dsd":
+        k = R if ta else C
+        a, b = None, (dim, k) if tb else (k, dim)
+    else:
+        k = C if tb else R
+        a, b = (k, dim) if ta else (dim, k), None
+    mk = lambda s, seed: _randn(*(stack if s is None else lead + s), dtype=dtype, seed=seed).requires_grad_()
+    return mk(a, 1), mk(b, 2)
+
+
+def _both(native, function, inputs):
+    """Results and gradients of the two, the native call twice (by a fresh plan and by the one that is there)."""
+    out = []
+    for f in (function, native, native):
+        y = f(*inputs)
+        g = _randn(*y.shape, dtype=y.dtype, seed=9)
+        out.append((y,) + torch.autograd.grad(y, [t for t in inputs if t.requires_grad], g))
+    for got in out[1:]:
+        assert all(torch.equal(x, w) for x, w in zip(got, out[0]))
+    return out[1][0]
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("mode,dim,shared", [("sdd", 64, False), ("dsd", 96, False), ("dds", 64, False), ("dsd", 64, True), ("dds", 128, True)])
+def test_products(mode, dim, shared, ta, tb, dtype):
+    import sparse
+    from sparse.matmul import SparseMatMul
+    L = _layout()
+    a, b = _product(L, mode, ta, tb, dim, dtype, shared=shared)
+    y = _both(lambda a, b: sparse.matmul(a, b, mode, L, ta, tb), lambda a, b: SparseMatMul.apply(a, b, mode, L, ta, tb), (a, b))
+    assert y.grad_fn.name() == "SparseMatMulBackward"
+
+
+@pytest.mark.parametrize("tokens", [32, 1056])
+def test_a_shared_weight(tokens, monkeypatch):
+    import sparse
+    from sparse import _ops
+    from sparse.matmul import SparseMatMul
+    for name in ("PANEL_MIN_WORKGROUPS", "PANEL_MIN_DENSITY", "WEIGHT_GRAD_MIN_TOKENS", "WEIGHT_GRAD_MIN_DENSITY"):
+        monkeypatch.setattr(_ops, name, 1 if "MIN_W" in name or "TOKENS" in name else 0.0)
+    L = _layout("rand16")
+    x, w = _product(L, "dds", False, False, tokens, torch.bfloat16, shared=True)
+    _both(lambda a, b: sparse.matmul(a, b, "dds", L), lambda a, b: SparseMatMul.apply(a, b, "dds", L), (x, w))
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("name", ["rand16", "long_row_5x40"])
+def test_softmax(name, dtype):
+    import sparse
+    from sparse.softmax import SparseSoftmax
+    L = _layout(name)
+    x = _randn(2, L.num_blocks, 32, 32, dtype=dtype).requires_grad_()
+    _both(lambda x: sparse.softmax(x, L, 0.3, True), lambda x: SparseSoftmax.apply(x, L, 0.3, True), (x,))
+
+
+@pytest.mark.parametrize("wants", [(True, True, True), (True, False, False), (False, True, True)])
+@pytest.mark.parametrize("dtype,head", [(torch.float16, 64), (torch.bfloat16, 128)])
+def test_attention(dtype, head, wants):
+    import sparse
+    from sparse.attention import SparseAttention
+    L = _layout("long_row_5x40")
+    R, C = (32 * n for n in L.tile_shape)
+    qkv = [_randn(3, n, head, dtype=dtype, seed=i).requires_grad_(w) for i, (n, w) in enumerate(zip((R, C, C), wants))]
+    _both(lambda *t: sparse.attention(*t, L, 0.2, True), lambda *t: SparseAttention.apply(*t, L, 0.2, True), qkv)
+    with torch.no_grad():
+        assert torch.equal(sparse.attention(*qkv, L, 0.2, True), SparseAttention.apply(*qkv, L, 0.2, True))
+
+
+def test_plans_are_taken(monkeypatch):
+    import sparse
+    from sparse import _ops
+    used = lambda *args, **kw: pytest.fail("a call without a plan")
+    for name in ("sparse_matmul", "sparse_weight_gradient", "sparse_softmax_forward", "sparse_softmax_backward", "sparse_attention_forward",
+                 "sparse_attention_backward"):
+        monkeypatch.setattr(_ops, name, used)
+    L = _layout()
+    R, C = (32 * n for n in L.tile_shape)
+    for _ in range(2):
+        for mode in ("sdd", "dsd", "dds"):
+            a, b = _product(L, mode, False, False, 64, torch.float16)
+            sparse.matmul(a, b, mode, L).sum().backward()
+        x = _randn(2, L.num_blocks, 32, 32, dtype=torch.float16).requires_grad_()
+        sparse.softmax(x, L, 0.3).sum().backward()
+        q, k, v = (_randn(2, n, 64, dtype=torch.float16).requires_grad_() for n in (R, C, C))
+        sparse.attention(q, k, v, L).sum().backward()
+
+
+def test_what_autograd_sees():
+    import sparse
+    L = _layout()
+    a, b = _product(L, "dds", False, False, 64, torch.float16)
+    sparse.matmul(a, b, "dds", L)                                       # the plan is there
+    y = sparse.matmul(a, b, "dds", L)
+    first = torch.autograd.grad(y.sum(), (a, b), retain_graph=True)
+    assert all(torch.equal(x, z) for x, z in zip(first, torch.autograd.grad(y.sum(), (a, b))))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(y.sum(), (a, b))
+    y = sparse.matmul(a, b, "dds", L)
+    with torch.no_grad():
+        a.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t, lambda t: t):
+        y = sparse.matmul(a, b, "dds", L)
+    assert packed == [a.shape, b.shape]
+    with torch.no_grad():
+        assert not sparse.matmul(a, b, "dds", L).requires_grad
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda t: sparse.matmul(t, b, "dds", L))(a[None])
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: sparse.matmul(t, b, "dds", L).float().sum())(a)
+    import torch.autograd.forward_ad as fw
+    with fw.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        sparse.matmul(fw.make_dual(a.detach(), torch.ones_like(a)), b.detach(), "dds", L)
+
+
+def test_operands_a_plan_does_not_hold():
+    import sparse
+    from sparse.matmul import SparseMatMul
+    L = _layout()
+    a, b = (t.detach() for t in _product(L, "dds", False, False, 64, torch.float16))
+    want = sparse.matmul(a, b, "dds", L)
+    at = a.transpose(-1, -2).contiguous().transpose(-1, -2)
+    assert not at.is_contiguous() and torch.equal(sparse.matmul(at, b, "dds", L), want)
+    flat = torch.empty(a.numel() + 1, dtype=a.dtype, device="cuda")
+    off = flat[1:].view(a.shape).copy_(a)
+    assert off.data_ptr() % 16 and torch.equal(sparse.matmul(off, b, "dds", L), want)
+    assert torch.equal(sparse.matmul(a, b, "".join(["d", "ds"]), L, 0, 0), want)
+    for bad in ((a.float(), b, "dds", L), (a, b, "ssd", L), (a.cpu(), b, "dds", L), (a[..., :32], b, "dds", L), (a[..., :32].contiguous(), b, "dds", L),
+                (a, b[:, :1], "dds", L)):
+        with pytest.raises(Exception) as native:
+            sparse.matmul(*bad)
+        with pytest.raises(Exception) as function:
+            SparseMatMul.apply(*bad)
+        assert type(native.value) is type(function.value) and str(native.value) == str(function.value)
+    with pytest.raises(TypeError):
+        sparse.matmul(a, b, "dds", L, trans_a=False)
+    assert torch.equal(sparse.matmul(torch.nn.Parameter(a), b, "dds", copy.deepcopy(L)), want)
+
+
+def test_a_setting_that_changes_drops_the_plans(monkeypatch):
+    import sparse
+    from sparse import _ops
+    L = _layout("rand16")
+    x = _randn(2, L.num_blocks, 32, 32, dtype=torch.float16)
+    v = _randn(2, 32 * L.tile_shape[1], 64, dtype=torch.float16)
+    for k in (_ops.SCHEDULE_GROUP_WALK, (3, 4, True, -1, 2, True), _ops.SCHEDULE_GROUP_WALK):
+        monkeypatch.setattr(_ops, "SCHEDULE_GROUP_WALK", k)
+        for _ in range(2):
+            sparse.matmul(x, v, "dsd", L)
+        assert k in L.row_layout[1]._bsa_schedules
+
+
+def test_streams_and_threads():
+    """Split groups: a workspace per stream, whichever thread calls."""
+    import sparse
+    L = _layout()
+    a, b = _product(L, "dds", False, False, 64, torch.float16)
+    want = sparse.matmul(a, b, "dds", L)
+    grads = torch.autograd.grad(want.float().sum(), (a, b))
+    torch.cuda.synchronize()
+    bad = []
+
+    def work():
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(20):
+                y = sparse.matmul(a, b, "dds", L)
+                got = torch.autograd.grad(y.float().sum(), (a, b))
+                if not (torch.equal(y, want) and all(torch.equal(x, z) for x, z in zip(got, grads))):
+                    bad.append(1)
+        s.synchronize()
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
+
+
+def test_captured_with_plans_there():
+    import sparse
+    L = _layout()
+    a, b = (t.detach() for t in _product(L, "dds", False, False, 64, torch.float16))
+    want = [sparse.matmul(a, b, "dds", L).clone() for _ in range(2)][1]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = sparse.matmul(a, b, "dds", L)
+    for _ in range(3):
+        graph.replay()
+        eager = sparse.matmul(a, b, "dds", L)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(eager, want)
+
+
+def test_plans_are_bounded():
+    import sparse
+    L = _layout("rand16")
+    for n in list(range(1, 80)) + [1]:
+        x = _randn(n, L.num_blocks, 32, 32, dtype=torch.float16)
+        y = sparse.softmax(x, L, 1.0, False)
+    assert y.shape == x.shape
