@@ -79,13 +79,10 @@ struct RunsArgs {
 hipError_t launch_dsd_runs(int dtype, const RunsArgs &p, hipStream_t stream);
 
 // products of a block-sparse weight with many dense rows, and the weight's gradient (weight_panels.hip)
-// Dense rows of a workgroup: 96 is what eight waves hold in 128 registers without spilling more than one (128 rows spill
-// 13-17).  bf16, us of the [k][x] / [x][k] walk at 64, 96 and 128 rows a workgroup: 64 x 64 blocks, a quarter stored, 4 x 1056
-// dense rows 41 / 42, 33 / 33, 87 / 57; 4 x 1024 rows 28 / 30, 32 / 32, 50 / 46; 2048 rows 18 / 17, 20 / 18, 42 / 40; 96 x
-// 96 blocks, a quarter stored, 8 x 1024 rows 105 / 114, 102 / 108, 205 / 160; 0.15 stored, 3 x 1312 rows 53 / 55, 42 / 43,
-// 115 / 77.  64 rows win where they make a whole number of workgroups a compute unit (512 and 256 on 256), 96 elsewhere.
+// Dense rows of a workgroup: 64 to 160, chosen by the launch; 96 is what callers that weigh this walk against bsa_matmul's
+// reckon with (their line was measured with it).
 constexpr int PANEL_ROWS = 96;
-constexpr int PANEL_MAX_KBLOCKS = 1024;            // the k-block table of eight groups: 32 KB of LDS
+constexpr int PANEL_MAX_KBLOCKS = 1024;            // the lists of eight groups: 32 KB of LDS
 constexpr int PANEL_MAX_NNZ = (1 << 20) - 1;       // 2 KB blocks within a 31-bit buffer range
 struct WeightPanelArgs {
     const void *dense, *sparse;

@@ -3,13 +3,14 @@
 // The group walk of matmul.hip gives a wave 64 dense rows and a chunk of one group's blocks: it fetches 4 KB of dense
 // operand for every 2 KB block, from rows that lie a whole matrix row apart, and nothing it fetched serves another
 // group.  With a few attention heads of 64 columns that is what there is to do; a linear layer has thousands of
-// dense rows and dozens of groups that read the same columns of them.  Here a workgroup of eight waves owns PANEL_ROWS dense
-// rows and eight neighbouring groups, walks ALL of the contraction in steps of 128 and keeps the dense panel of a step in LDS
-// for the eight waves; a wave multiplies it by the blocks its group has there.
+// dense rows and dozens of groups that read the same columns of them.  Here a workgroup owns 64 to 160 dense rows and eight
+// neighbouring groups, a wave each, walks ALL of the contraction in steps of 128 and keeps the dense panels of the present and
+// the next steps in LDS; a wave multiplies them by the blocks its group has there.
 #include "bsa_device.hpp"
 #include "lds_tiles.hpp"
 #include "bsa_internal.hpp"
 #include "group_walk.hpp"
+#include "attention_tiles.hpp"
 #include "../../include/bsa.h"
 
 namespace bsa {
@@ -24,6 +25,14 @@ __device__ __forceinline__ int xcd_contiguous(int total)
 
 constexpr int PANEL_WAVES = 8;                  // groups of a workgroup, one wave each
 constexpr int PANEL_KB = 4;                     // k-blocks of 32 per step
+constexpr int PANEL_RING = 4;                   // blocks of a wave in flight
+// panels in LDS at a time, and waves that do nothing but fetch them, one each: as many as a compute unit's 160 KB hold beside
+// the lists of the widest contraction
+constexpr int panel_stages(int rt) { return rt <= 3 ? 4 : 3; }
+constexpr int panel_threads(int rt) { return 64 * (PANEL_WAVES + panel_stages(rt)); }
+constexpr int PANEL_FLAGS = 64;                 // bytes in front of the lists: panels that are there, panels that are read
+constexpr int PANEL_NONE = -1;
+__host__ __device__ constexpr int panel_list_length(int kblocks) { return (kblocks + 2 * PANEL_RING + 3) / 4 * 4; }
 
 // ---------------------------------------------------------------------------
 // out[row][32 g + x] = sum over the blocks (k-block kb) of group g, sum over k of dense[row][32 kb + k] * block(x, k)
@@ -31,86 +40,136 @@ constexpr int PANEL_KB = 4;                     // k-blocks of 32 per step
 // dense [rows][KT] and out [rows][XT] of one batch entry, or of all of them as one matrix when the weight is shared.
 //   S_KC  the stored block is [x][k] (row groups): operands straight from memory
 //         otherwise [k][x] (column groups): through a wave-private LDS tile, read transposed
-// A wave first spreads its group's pairs over a table indexed by k-block (LDS, -1 where nothing is stored), so the
-// steady state needs no search and no branch around a load: the requests of absent blocks carry an offset beyond the
-// descriptor's range, which the memory pipeline answers with zeros without a fetch.
+// A wave per panel buffer requests panels straight into LDS, waits for them and says so in a flag; a multiplying wave waits
+// for the panel of its next block and says up to which panel it is done.  So the waits for panels are the fetching
+// waves' alone, the other waves' stay exact for the blocks, of which a wave has its next four on the way, and no wave waits
+// for the fullest of the eight in every step, only for the slowest where it is a whole set of buffers ahead.
+//
+// What bounds it: the wave with the most blocks, about 1000 clocks a block (its panel's flag, LDS reads, ten products), then
+// the panels (200 MB through the L2 -> LDS path: 18 us without the products).  us, panels through registers a step ahead and a
+// barrier per step, 96 rows a workgroup -> fetching waves and a barrier per step, 160 rows -> flags -> operands of a block read
+// together: 4224 rows x 2048 x 2048 at a quarter of its blocks, forward 31.3 -> 26.0 -> 24.6 -> 23.7, gradient of the dense operand
+// 32.3 -> 24.5 -> 24.3 -> 22.8; 8192 x 3072 x 3072 at 0.3 107 -> 91 and 111 -> 84; every block stored, 4224 rows 56 -> 46 and 56 -> 41.
+// A group that has a block in every k-block makes its wave the chain: 4800 rows, 48 x 80 blocks, such a column: 26.7 -> 31.8, its
+// gradient 37.2 -> 22.1.
 // ---------------------------------------------------------------------------
-template <int ROWS, bool S_KC, bool BF>
-__global__ __launch_bounds__(64 * PANEL_WAVES, 4) void weight_panel_kernel(
+template <int RT, bool S_KC, bool BF>
+__global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
     const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
     const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
     int groups, int nnz, int rows, int KT, int XT, int sp_shared, int row_tiles, int group_sets)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int RT = ROWS / 32, Q = ROWS * 16 / (64 * PANEL_WAVES);      // 32-row tiles; 16-byte pieces per thread and step
-    constexpr int PANEL_BYTES = ROWS * 256;
+    constexpr int ROWS = 32 * RT, STAGES = panel_stages(RT), PANEL_BYTES = ROWS * 256;
     const int item = xcd_contiguous(row_tiles * group_sets);
     if (item < 0) return;                                                  // whole workgroup leaves together
     const int tile = item / group_sets, set = item - tile * group_sets;
-    const int batch = (int)blockIdx.y, w = wave_id(), l = lane_id(), tid = (int)threadIdx.x;
+    const int batch = (int)blockIdx.y, w = wave_id(), l = lane_id();
     const int y0 = tile * ROWS, g = set * PANEL_WAVES + w;
     const int kblocks = KT / BS, steps = (kblocks + PANEL_KB - 1) / PANEL_KB;
     // Workgroups start at different steps: rows a multiple of 4 KB apart have their 256 bytes of a step in ONE of the 16
     // channels of an L2, and workgroups that walk the contraction in unison would all ask that channel.
     const int start = item % steps;
-    auto wrapped = [&](int s) { s += start; return s < steps ? s : s - steps; };
 
-    half_t *priv = reinterpret_cast<half_t *>(lds_raw + 2 * PANEL_BYTES) + w * BS2;
-    int *table = reinterpret_cast<int *>(lds_raw + 2 * PANEL_BYTES + (S_KC ? 0 : PANEL_WAVES * BS2 * 2)) +
-                 (size_t)w * (steps + 1) * PANEL_KB;
-    const half_t *dnb = dn + (size_t)batch * rows * KT;
-
-    // 16-byte piece `tid & 15` of rows tid / 16, + 32, ..: whole 256-byte runs of a row.  Rows behind the last and
-    // k behind the last k-block repeat what is there (never multiplied into a stored result).
-    const int prow = tid >> 4, piece = tid & 15;
-    const half_t *src[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int y = y0 + prow + 32 * q;
-        src[q] = dnb + (size_t)(y < rows ? y : rows - 1) * KT;
-    }
-    uint4 dense[Q];
-    auto request_panel = [&](int step) {
-        int k = step * (BS * PANEL_KB) + 8 * piece;
-        k = k < KT ? k : KT - 8;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) dense[q] = ldg16(src[q] + k);
+    half_t *privs = reinterpret_cast<half_t *>(lds_raw + STAGES * PANEL_BYTES);
+    int *flags = reinterpret_cast<int *>(lds_raw + STAGES * PANEL_BYTES + (S_KC ? 0 : PANEL_WAVES * BS2 * 2));
+    int *ready = flags, *done = flags + 4;       // of a buffer: panels up to and with the one in it; of a wave: panels it has done with
+    static_assert(STAGES <= 4 && 4 * (4 + PANEL_WAVES) <= PANEL_FLAGS, "flags");
+    auto load_flag = [](const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    auto store_flag = [](int *p, int v) {
+        wave_lds_fence();
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
-    request_panel(wrapped(0));
+    if (threadIdx.x < PANEL_FLAGS / 4) flags[threadIdx.x] = 0;
+    lds_barrier();
 
-    for (int t = l; t < (steps + 1) * PANEL_KB; t += WAVE) table[t] = -1;
-    wave_lds_fence();
+    if (w >= PANEL_WAVES) {
+        // Request r covers rows 4 r .. + 3, 16 pieces each; piece p of row y goes to slot p ^ (y & 15): 16 lanes that read one
+        // piece of 16 rows meet no bank twice.  Lane l fills slot l % 16 of row 4 r + l / 16.  Requests behind the last row
+        // repeat the last four (the rows of a launch are whole tiles of 32), pieces behind the last k-block the first: never
+        // multiplied into a stored result.
+        const int f = w - PANEL_WAVES;
+        const unsigned char *dnb = reinterpret_cast<const unsigned char *>(dn + (size_t)batch * rows * KT + (size_t)y0 * KT);
+        const int last = (rows - y0 < ROWS ? rows - y0 : ROWS) / 4 - 1;    // request of the last four rows
+        const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(lds_raw)) + (unsigned)f * PANEL_BYTES;
+        unsigned off[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) off[c] = 2u * (unsigned)((l >> 4) * KT) + 16u * (unsigned)((l & 15) ^ (4 * c + (l >> 4)));
+        const int whole = KT / (BS * PANEL_KB), pieces = 16 - (steps * 16 - KT / 8);      // the last step may have fewer pieces
+        for (int s = f; s < steps; s += STAGES) {
+            // the panel before in this buffer, s - STAGES, has been read by all
+            while (__ballot(l < PANEL_WAVES && load_flag(done + (l < PANEL_WAVES ? l : 0)) < s - STAGES + 1) != 0ull) __builtin_amdgcn_s_sleep(1);
+            int at = s + start;
+            at = at < steps ? at : at - steps;
+            unsigned o[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int piece = (l & 15) ^ (4 * c + (l >> 4));
+                o[c] = at >= whole && piece >= pieces ? off[c] - 16u * piece : off[c];
+            }
+            const unsigned char *from = dnb + 256 * at;
+#pragma unroll 1
+            for (int r = 0; r < 8 * RT; r += 4) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    dma16(from, o[c], to + 1024u * (r + c));
+                    from += r + c < last ? (size_t)8 * KT : 0;
+                }
+            }
+            tile_wait<0>();
+            if (l == 0) store_flag(ready + f, s + 1);
+        }
+        return;
+    }
+
+    // The group's pairs, in the order in which the steps come: block | k-block << 20, then PANEL_NONE
+    half_t *priv = privs + w * BS2;
+    int *list = flags + PANEL_FLAGS / 4 + w * panel_list_length(kblocks);
+    int n = 0;
     if (g < groups) {
-        const int end = offsets[g + 1];
-        for (int p = offsets[g] + l; p < end; p += WAVE) {
-            const BlockDesc d = blocks[p];
-            const int kb = S_KC ? d.col() : d.row();
-            if (kb < kblocks) table[kb] = d.idx;
+        const int begin = offsets[g];
+        n = offsets[g + 1] - begin;
+        n = n < 0 ? 0 : n < kblocks ? n : kblocks;
+        auto kblock = [&](const BlockDesc &d) { return S_KC ? d.col() : d.row(); };
+        const BlockDesc first = l < n ? blocks[begin + l] : BlockDesc{0, -1};
+        int before = __popcll(__ballot(l < n && kblock(first) < start * PANEL_KB));       // pairs of steps that come around again
+        for (int p = WAVE; p < n; p += WAVE) {
+            const int kb = p + l < n ? kblock(blocks[begin + p + l]) : kblocks;
+            before += __popcll(__ballot(kb < start * PANEL_KB));
+        }
+        for (int p = l; p < n; p += WAVE) {
+            const BlockDesc d = p < WAVE ? first : blocks[begin + p];
+            const bool inside = kblock(d) < kblocks;                       // else the walk below would wait for a step that never comes
+            list[p >= before ? p - before : p + n - before] = inside ? (d.idx & 0xFFFFF) | kblock(d) << 20 : PANEL_NONE;
         }
     }
+    n = __builtin_amdgcn_readfirstlane(n);
+    if (l < 2 * PANEL_RING) list[n + l] = PANEL_NONE;
     wave_lds_fence();
 
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<half_t *>(sp + (sp_shared ? 0 : (size_t)batch * nnz * BS2)), 0, nnz * BS2 * 2, 0x00020000);
     // S_KC: lane (i, h) takes row perm16(i) of the block, k = 16 s + 8 h; otherwise the linear pieces l and l + 64
     const int off0 = S_KC ? 64 * perm16(l & 31) + 16 * (l >> 5) : 16 * l, off1 = off0 + (S_KC ? 32 : 1024);
-    uint4 blk[PANEL_KB][2];
-    int now[PANEL_KB], next[PANEL_KB];
-    auto lookup = [&](int step, int (&idx)[PANEL_KB]) {
-        const int4 e = *reinterpret_cast<const int4 *>(table + step * PANEL_KB);
-        idx[0] = __builtin_amdgcn_readfirstlane(e.x);
-        idx[1] = __builtin_amdgcn_readfirstlane(e.y);
-        idx[2] = __builtin_amdgcn_readfirstlane(e.z);
-        idx[3] = __builtin_amdgcn_readfirstlane(e.w);
+    uint4 blk[PANEL_RING][2];
+    int now[PANEL_RING], next[PANEL_RING];
+    auto lookup = [&](int i, int (&e)[PANEL_RING]) {
+        const int4 x = *reinterpret_cast<const int4 *>(list + i);          // i is a multiple of 4
+        e[0] = __builtin_amdgcn_readfirstlane(x.x);
+        e[1] = __builtin_amdgcn_readfirstlane(x.y);
+        e[2] = __builtin_amdgcn_readfirstlane(x.z);
+        e[3] = __builtin_amdgcn_readfirstlane(x.w);
     };
-    auto request_block = [&](int idx, uint4 (&b)[2]) {
-        const unsigned base = idx >= 0 ? (unsigned)idx * (BS2 * 2) : 0x80000000u;
+    // the request of an absent block carries an offset beyond the descriptor's range, which the memory pipeline answers with
+    // zeros without a fetch: no load sits under a condition
+    auto request_block = [&](int e, uint4 (&b)[2]) {
+        const unsigned base = e >= 0 ? (unsigned)(e & 0xFFFFF) * (BS2 * 2) : 0x80000000u;
         b[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, base + off0, 0, 0));
         b[1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, base + off1, 0, 0));
     };
-    lookup(wrapped(0), now);
+    lookup(0, now);
 #pragma unroll
-    for (int j = 0; j < PANEL_KB; ++j) {
+    for (int j = 0; j < PANEL_RING; ++j) {
         request_block(now[j], blk[j]);
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -119,25 +178,26 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 4) void weight_panel_kernel(
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f16v{0};
     const int i = l & 31, h = l >> 5;
-
-    for (int step = 0; step < steps; ++step) {
-        // rows of 16 pieces, piece p of row r in slot p ^ (r & 15): 16 lanes that read one piece of 16 rows, or write the
-        // 16 pieces of one row, meet no bank twice
-        unsigned char *panel = lds_raw + (step & 1) * PANEL_BYTES;
+    int step = -1;                                                         // whose panel is there
+    const unsigned char *panel = lds_raw + 256 * i;                        // row i of it
+    auto walk_to = [&](int s) {
+        if (s == step) return;
+        if (l == 0) store_flag(done + w, s);                               // the reads before it are in front of it in LDS order
+        const int buffer = s % STAGES;
+        while (__builtin_amdgcn_readfirstlane(load_flag(ready + buffer)) < s + 1) __builtin_amdgcn_s_sleep(1);
+        wave_lds_fence();
+        panel = lds_raw + buffer * PANEL_BYTES + 256 * i;
+        step = s;
+    };
+    for (int p = 0; p < n; p += PANEL_RING) {
+        lookup(p + PANEL_RING, next);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const int r = prow + 32 * q;
-            *reinterpret_cast<uint4 *>(panel + 256 * r + 16 * (piece ^ (r & 15))) = dense[q];
-        }
-        lds_barrier();          // the other panel's readers passed this barrier one step ago at the latest
-        const int ahead = step + 1 < steps ? wrapped(step + 1) : steps;    // behind the last step: the table holds no block
-        request_panel(ahead);
-        __builtin_amdgcn_sched_barrier(0);
-        lookup(ahead, next);
-#pragma unroll
-        for (int j = 0; j < PANEL_KB; ++j) {
+        for (int j = 0; j < PANEL_RING; ++j) {
             if (now[j] >= 0) {
-                h8 sop[2];
+                const int kb = now[j] >> 20;
+                int s = kb / PANEL_KB - start;
+                // all operands first: two at a time, as the compiler has it, the LDS shows through five times a block
+                h8 sop[2], dop[2][RT];
                 if (S_KC) {
                     sop[0] = as_h8(blk[j][0]);
                     sop[1] = as_h8(blk[j][1]);
@@ -148,14 +208,18 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 4) void weight_panel_kernel(
                     sop[0] = lds_get_ks<true>(priv, 0);
                     sop[1] = lds_get_ks<true>(priv, 1);
                 }
+                walk_to(s < 0 ? s + steps : s);
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+                for (int u = 0; u < 2; ++u) {
+                    const unsigned char *at = panel + 16 * ((4 * (kb % PANEL_KB) + 2 * u + h) ^ (i & 15));
 #pragma unroll
-                    for (int t = 0; t < RT; ++t) {
-                        const int r = 32 * t + i;
-                        const h8 dop = *reinterpret_cast<const h8 *>(panel + 256 * r + 16 * ((4 * j + 2 * s + h) ^ (r & 15)));
-                        acc[t] = mfma_16<BF>(sop[s], dop, acc[t]);
-                    }
+                    for (int t = 0; t < RT; ++t) dop[u][t] = *reinterpret_cast<const h8 *>(at + 8192 * t);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) acc[t] = mfma_16<BF>(sop[u], dop[u][t], acc[t]);
             }
             __builtin_amdgcn_sched_barrier(0);
             request_block(next[j], blk[j]);
@@ -163,6 +227,7 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 4) void weight_panel_kernel(
             now[j] = next[j];
         }
     }
+    if (l == 0) store_flag(done + w, steps);
 
     if (g < groups) {
         half_t *ob = out + (size_t)batch * rows * XT + BS * g + 16 * h;
@@ -348,31 +413,58 @@ __global__ __launch_bounds__(256) void weight_sum_kernel(const float *__restrict
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-template <int ROWS, bool S_KC, bool BF>
+template <int RT, bool S_KC, bool BF>
 static hipError_t launch_panel(const WeightPanelArgs &p, hipStream_t st)
 {
+    constexpr int ROWS = 32 * RT;
     const int tiles = (p.rows + ROWS - 1) / ROWS, sets = (p.groups + PANEL_WAVES - 1) / PANEL_WAVES;
-    const int steps = (p.KT / BS + PANEL_KB - 1) / PANEL_KB;
-    const size_t lds = 2 * ROWS * 256 + (S_KC ? 0 : PANEL_WAVES * BS2 * 2) +
-                       (size_t)PANEL_WAVES * (steps + 1) * PANEL_KB * sizeof(int);
-    auto kernel = weight_panel_kernel<ROWS, S_KC, BF>;
+    const size_t lds = panel_stages(RT) * ROWS * 256 + (S_KC ? 0 : PANEL_WAVES * BS2 * 2) +
+                       PANEL_FLAGS + (size_t)PANEL_WAVES * panel_list_length(p.KT / BS) * sizeof(int);
+    auto kernel = weight_panel_kernel<RT, S_KC, BF>;
     if (lds > 65536) {
         hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (err != hipSuccess) return err;
     }
     dim3 grid((unsigned)((tiles * sets + 7) / 8 * 8), (unsigned)p.batches);
-    kernel<<<grid, 64 * PANEL_WAVES, lds, st>>>((const half_t *)p.sparse, (const half_t *)p.dense, (half_t *)p.out,
-                                                (const BlockDesc *)p.blocks, p.offsets, p.groups, p.nnz, p.rows, p.KT,
-                                                BS * p.groups, p.sparse_shared ? 1 : 0, tiles, sets);
+    kernel<<<grid, panel_threads(RT), lds, st>>>(
+        (const half_t *)p.sparse, (const half_t *)p.dense, (half_t *)p.out, (const BlockDesc *)p.blocks, p.offsets, p.groups, p.nnz,
+        p.rows, p.KT, BS * p.groups, p.sparse_shared ? 1 : 0, tiles, sets);
     return hipGetLastError();
+}
+
+// Tiles of 32 rows a workgroup takes: a compute unit holds one workgroup, so the fewest generations of them, counted with
+// a tile's worth of start and end.  Five leave no room for the lists of more than 700 k-blocks.
+static int panel_row_tiles(const WeightPanelArgs &p)
+{
+    const long long sets = (p.groups + PANEL_WAVES - 1) / PANEL_WAVES;
+    int best = 2;
+    long long best_cost = 0;
+    for (int rt = 2; rt <= (p.KT / BS <= 700 ? 5 : 4); ++rt) {
+        const long long wgs = (p.rows + 32 * rt - 1) / (32 * rt) * sets * p.batches, cost = (wgs + 255) / 256 * (rt + 1);
+        if (best_cost == 0 || cost < best_cost) {
+            best = rt;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <bool S_KC, bool BF>
+static hipError_t launch_panels(const WeightPanelArgs &p, hipStream_t st)
+{
+    switch (panel_row_tiles(p)) {
+        case 2: return launch_panel<2, S_KC, BF>(p, st);
+        case 3: return launch_panel<3, S_KC, BF>(p, st);
+        case 4: return launch_panel<4, S_KC, BF>(p, st);
+        default: return launch_panel<5, S_KC, BF>(p, st);
+    }
 }
 
 hipError_t launch_weight_panels(int dtype, const WeightPanelArgs &p, hipStream_t st)
 {
-    if (dtype == BSA_BF16)
-        return p.row_groups ? launch_panel<PANEL_ROWS, true, true>(p, st) : launch_panel<PANEL_ROWS, false, true>(p, st);
-    return p.row_groups ? launch_panel<PANEL_ROWS, true, false>(p, st) : launch_panel<PANEL_ROWS, false, false>(p, st);
+    if (dtype == BSA_BF16) return p.row_groups ? launch_panels<true, true>(p, st) : launch_panels<false, true>(p, st);
+    return p.row_groups ? launch_panels<true, false>(p, st) : launch_panels<false, false>(p, st);
 }
 
 // Shares of at least eight steps: the fewest (at most eight) that leave at most a sixth of the machine idle in the last

@@ -382,7 +382,8 @@ int bsa_matmul_dds_panels(int dtype, const void *dense, const void *sparse, void
                           const int32_t *offsets, int mask_rows, int mask_cols, int nnz, int batches,
                           int sparse_batches, int M, int tr_b, void *stream);
 
-/* Constants of that walk: dense rows of a workgroup, block rows of the contraction and blocks it is built for. */
+/* Constants of that walk: dense rows of a workgroup (64 to 160 are built; the figure a caller reckons with), block rows of
+ * the contraction and blocks it is built for. */
 void bsa_matmul_dds_panels_limits(int32_t limits[3]);
 
 /* Gradient of a block-sparse weight that a whole batch shared: out[block (r, c)] = sum over all tokens t of

@@ -135,3 +135,28 @@ def test_layer_captured_at_a_size_that_never_ran():
         torch.cuda.synchronize()
         for a, b in zip(got, step(*t)):
             assert _rel(a, b.double()) <= 4 * REL[torch.float16]
+
+
+# Launches of 64, 96, 128 and 160 rows a workgroup (the fewest generations of 256 workgroups), each with a tile that is cut; a
+# contraction that ends inside a step, a group with a block in every k-block beside empty ones, more k-blocks than a wave has lanes
+@pytest.mark.parametrize("rows,cols,density,batch,m", [
+    (5, 9, 0.7, 33, 32), (6, 70, 0.3, 31, 96), (70, 9, 0.3, 127, 160), (7, 16, 0.5, 255, 96), (66, 24, 0.2, 253, 96)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_panel_heights(any_size, rows, cols, density, batch, m, trans_b, dtype):
+    import sparse
+    from sparse import _ops
+    g = torch.Generator().manual_seed(rows)
+    mask = (torch.rand(rows, cols, generator=g) < density).long()
+    mask[:, 1] = 1
+    mask[:, 2] = 0
+    L = sparse.SparseLayout(mask.cuda())
+    k = 32 * (cols if trans_b else rows)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(batch, m, k, generator=g, device="cuda").to(dtype)
+    w = torch.randn(L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
+    W = L.to_dense(w).double()
+    got = _ops.sparse_matmul(x, w, "dds", L.row_layout, L.col_layout, False, trans_b).flatten(0, 1)
+    want = x.flatten(0, 1).double() @ (W.t().contiguous() if trans_b else W)
+    assert _rel(got, want) <= REL[dtype]
+    assert (got - want).abs().max() <= 8 * REL[dtype] * want.abs().max()       # no row of a cut tile is out of place
