@@ -248,12 +248,18 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
 // Gradient of the weight: w[block (r, c)] = sum over tokens t of a[t][32 r + .] b[t][32 c + .]
 //
 // A workgroup owns 8 x 8 cells of the mask and a share of the tokens; per step of 32 tokens it fetches 256 columns
-// of a and of b (512-byte runs), and wave r multiplies its 32 columns of a by those of the up to eight stored blocks of its
-// row.  Partial sums of the shares leave as fp32 and are added up in share order by weight_sum_kernel.
+// of a and of b, a 64-column panel a wave, and the stored cells are dealt evenly to the waves.  Partial sums of the shares
+// leave as fp32 and are added up in share order by weight_sum_kernel.
+// Bound by what the panels take from L2, 32 KB a step and workgroup (8.7 TB/s at 64 x 64 blocks).  They go straight to LDS:
+// through registers, three steps in flight took 48 of them (8 spilled), and an LDS write each.
+// A quarter of 64 x 64 blocks stored, 4224 tokens, with the sum: 38.5 -> 35.1 us; 96 x 96 at 0.3, 8192 tokens: 145 -> 128;
+// all of 64 x 64 stored: 74.6 -> 66.2.
 // ---------------------------------------------------------------------------
 constexpr int WG_EDGE = 8;                       // cells along a side
-constexpr int WG_TILE = 2048 + 64;               // a 32 x 32 tile; 64 bytes on, so that four tiles of a row write to different banks
-constexpr int WG_SIDE = WG_EDGE * WG_TILE;
+constexpr int WG_PANEL = 4096;                   // 32 tokens of 64 columns
+constexpr int WG_SIDE = WG_EDGE / 2 * WG_PANEL;
+constexpr int WG_STAGE = 2 * WG_SIDE;
+constexpr int WG_STAGES = 4;
 
 template <bool BF>
 __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
@@ -271,7 +277,7 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
     const int M = BS * R, N = BS * C;
 
     // the stored cells, dealt evenly to the waves in row-major order: cells w, w + 8, ..
-    int *table = reinterpret_cast<int *>(lds_raw + 4 * WG_SIDE);
+    int *table = reinterpret_cast<int *>(lds_raw + WG_STAGES * WG_STAGE);
     if (tid < WG_EDGE * WG_EDGE) table[tid] = -1;
     lds_barrier();
     if (r0 + w < R) {
@@ -286,105 +292,92 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
     const int mine_idx = table[l];
     unsigned long long stored = __ballot(mine_idx >= 0);
     const int count = (__popcll(stored) - w + WG_EDGE - 1) / WG_EDGE;      // of this wave
-    int idx[WG_EDGE], at_a[WG_EDGE], at_b[WG_EDGE];
+    int idx[WG_EDGE], at_a[WG_EDGE], at_b[WG_EDGE];      // at_: exclusive-ored into the address of an operand's first column
     for (int j = 0; j < w && stored; ++j) stored &= stored - 1;
 #pragma unroll
     for (int j = 0; j < WG_EDGE; ++j) {
         const int cell_of = stored ? __builtin_ctzll(stored) : 0;
         idx[j] = __builtin_amdgcn_readlane(mine_idx, cell_of);
-        at_a[j] = (cell_of >> 3) * WG_TILE;
-        at_b[j] = WG_SIDE + (cell_of & 7) * WG_TILE;
+        at_a[j] = (cell_of >> 4) * WG_PANEL + (cell_of >> 3 & 1) * 64;
+        at_b[j] = WG_SIDE + (cell_of >> 1 & 3) * WG_PANEL + (cell_of & 1) * 64;
         for (int t = 0; t < WG_EDGE; ++t) stored &= stored ? stored - 1 : 0;
     }
 
-    // piece `tid & 31` of tokens tid / 32 and + 16; columns behind the last repeat the first (never stored)
-    const int trow = tid >> 5, piece = tid & 31;
-    const int ca = 256 * (r0 / WG_EDGE) + 8 * piece, cb = 256 * (c0 / WG_EDGE) + 8 * piece;
-    const half_t *pa = a + (ca < M ? ca : 0), *pb = b + (cb < N ? cb : 0);
-    struct Raw { uint4 a[2], b[2]; };
-    auto request = [&](int step, Raw &f) {
-        step = step < last ? step : last - 1;
+    // Panel w % 4 of a (waves 0-3) or b; columns behind the last repeat the first (never stored).  A wave's offsets inside 32
+    // tokens fit 32 bits.
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds_raw));
+    const int width = w < WG_EDGE / 2 ? M : N, column0 = (w < WG_EDGE / 2 ? 32 * r0 : 32 * c0) + 64 * (w % (WG_EDGE / 2));
+    const unsigned char *operand = reinterpret_cast<const unsigned char *>(w < WG_EDGE / 2 ? a : b);
+    unsigned off[2];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const size_t t = (size_t)32 * step + trow + 16 * q;
-            f.a[q] = ldg16(pa + t * M);
-            f.b[q] = ldg16(pb + t * N);
-        }
+    for (int c = 0; c < 2; ++c) {
+        const int column = column0 + 8 * panel_src_piece(l, c);
+        off[c] = 2u * ((unsigned)(l >> 3) * (unsigned)width + (unsigned)(column < width ? column : 0));
+    }
+    auto request = [&](int step, int stage) {
+        step = step < last ? step : last - 1;
+        const unsigned char *rows = operand + (size_t)step * (64 * (size_t)width);
+        const unsigned to = lds0 + stage * WG_STAGE + w * WG_PANEL;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) dma16(rows + 16 * (size_t)width * c, off[c & 1], to + 1024 * c);
     };
     f16v acc[WG_EDGE];
 #pragma unroll
     for (int c = 0; c < WG_EDGE; ++c) acc[c] = f16v{0};
 
-    auto step_of = [&](int parity, const Raw &f) {
-        unsigned char *ta = lds_raw + parity * 2 * WG_SIDE, *tb = ta + WG_SIDE;
-        const int to = (piece >> 2) * WG_TILE;
+    const unsigned tr_lo = (unsigned)get_panel_tr_addr(l, 0, 0, 0), tr_hi = (unsigned)get_panel_tr_addr(l, 0, 1, 0);
+    auto multiply = [&](int stage) {
+        const unsigned base = lds0 + stage * WG_STAGE;
+        auto half_of = [&](int at, h8 (&x)[2]) {
+            asm volatile("" : "+s"(at));                // added where it is used: hoisted, the sums take 64 registers
+            typedef tr4 __attribute__((address_space(3))) *lds_tr4;
+            const unsigned lo = (tr_lo ^ (unsigned)at) + base, hi = (tr_hi ^ (unsigned)at) + base;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int at = to + 16 * ks_slot(trow + 16 * q, piece & 3);
-            *reinterpret_cast<uint4 *>(ta + at) = f.a[q];
-            *reinterpret_cast<uint4 *>(tb + at) = f.b[q];
-        }
-        lds_barrier();
-    };
-    auto multiply = [&](int parity) {
-        const unsigned char *panel = lds_raw + parity * 2 * WG_SIDE;
-        auto operands = [&](int j, h8 (&x)[4]) {
-            int oa = at_a[j], ob = at_b[j];
-            asm volatile("" : "+s"(oa), "+s"(ob));      // added where they are used: hoisted, the sums take 64 registers
-            const half_t *ta = reinterpret_cast<const half_t *>(panel + oa);
-            const half_t *tb = reinterpret_cast<const half_t *>(panel + ob);
-            x[0] = lds_get_ks<false>(ta, 0); x[1] = lds_get_ks<true>(tb, 0);
-            x[2] = lds_get_ks<false>(ta, 1); x[3] = lds_get_ks<true>(tb, 1);
+            for (int s = 0; s < 2; ++s) {
+                const tr4 p = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4)(uintptr_t)(lo + 2048u * s));
+                const tr4 q = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4)(uintptr_t)(hi + 2048u * s));
+                x[s] = __builtin_shufflevector(__builtin_bit_cast(h4, p), __builtin_bit_cast(h4, q), 0, 1, 2, 3, 4, 5, 6, 7);
+            }
         };
 #pragma unroll
         for (int j = 0; j < WG_EDGE; j += 2) {
             if (j < count) {                       // a pair at a time; the second repeats a cell when there is none
-                h8 x[4], y[4];
-                operands(j, x);
-                operands(j + 1, y);
-                acc[j] = mfma_16<BF>(x[1], x[0], acc[j]);
-                acc[j + 1] = mfma_16<BF>(y[1], y[0], acc[j + 1]);
-                acc[j] = mfma_16<BF>(x[3], x[2], acc[j]);
-                acc[j + 1] = mfma_16<BF>(y[3], y[2], acc[j + 1]);
+                h8 xa[2], xb[2], ya[2], yb[2];
+                half_of(at_a[j], xa);
+                half_of(at_b[j], xb);
+                half_of(at_a[j + 1], ya);
+                half_of(at_b[j + 1], yb);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    acc[j] = mfma_16<BF>(xb[s], xa[s], acc[j]);
+                    acc[j + 1] = mfma_16<BF>(yb[s], ya[s], acc[j + 1]);
+                }
             }
         }
     };
     if (first < last) {
-        // three steps in flight (the operands of a long batch come from HBM); a panel is overwritten two steps later,
-        // when every wave has passed the barrier between
-        Raw f[3];
+        // Three steps in flight (the operands of a long batch come from HBM).  A wave waits for its own panel of the step, the
+        // barrier for everybody's; behind it nobody reads the step before, whose buffer the next request takes.
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            request(first + d, f[d]);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int d = 0; d < WG_STAGES - 1; ++d) request(first + d, d);
+        int stage = 0;
+        for (int s = first; s < last; ++s) {
+            tile_wait<4 * (WG_STAGES - 2)>();
+            lds_barrier();
+            request(s + WG_STAGES - 1, (stage + WG_STAGES - 1) % WG_STAGES);
+            multiply(stage);
+            stage = (stage + 1) % WG_STAGES;
         }
-        int s = first;
-        for (; s + 6 <= last; s += 6) {
-#pragma unroll
-            for (int d = 0; d < 6; ++d) {
-                step_of(d & 1, f[d % 3]);
-                request(s + 3 + d, f[d % 3]);
-                __builtin_amdgcn_sched_barrier(0);
-                multiply(d & 1);
-            }
-        }
-#pragma unroll
-        for (int d = 0; d < 5; ++d) {
-            if (s + d < last) {
-                step_of(d & 1, f[d % 3]);
-                if (s + d + 3 < last) request(s + 3 + d, f[d % 3]);
-                multiply(d & 1);
-            }
-        }
+        tile_wait<0>();                            // requests past the last step write to LDS that is still this workgroup's
     }
-    float *dst = parts + (size_t)share * nnz * BS2 + (l & 31) * BS + 16 * (l >> 5);
+    float *dst = parts + (size_t)share * nnz * BS2 + (l & 31) * BS + 4 * (l >> 5);
 #pragma unroll
     for (int c = 0; c < WG_EDGE; ++c) {
         if (c < count) {
             float *o = dst + (size_t)idx[c] * BS2;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                *reinterpret_cast<float4 *>(o + 4 * t) =
+                *reinterpret_cast<float4 *>(o + 8 * t) =
                     make_float4(acc[c][4 * t], acc[c][4 * t + 1], acc[c][4 * t + 2], acc[c][4 * t + 3]);
         }
     }
@@ -468,7 +461,7 @@ hipError_t launch_weight_panels(int dtype, const WeightPanelArgs &p, hipStream_t
 }
 
 // Shares of at least eight steps: the fewest (at most eight) that leave at most a sixth of the machine idle in the last
-// generation of workgroups (one per compute unit at a time: 66 KB of panels, 256 registers), else the best there is.
+// generation of workgroups (one per compute unit at a time: 128 KB of panels, 256 registers), else the best there is.
 int weight_grad_shares(int mask_rows, int mask_cols, int tokens)
 {
     const long long cells = (long long)((mask_rows + WG_EDGE - 1) / WG_EDGE) * ((mask_cols + WG_EDGE - 1) / WG_EDGE);
@@ -490,7 +483,7 @@ int weight_grad_shares(int mask_rows, int mask_cols, int tokens)
 hipError_t launch_weight_grad(int dtype, const WeightGradArgs &p, hipStream_t st)
 {
     const int sets_r = (p.mask_rows + WG_EDGE - 1) / WG_EDGE, sets_c = (p.mask_cols + WG_EDGE - 1) / WG_EDGE;
-    const size_t lds = 4 * WG_SIDE + WG_EDGE * WG_EDGE * sizeof(int);
+    const size_t lds = WG_STAGES * WG_STAGE + WG_EDGE * WG_EDGE * sizeof(int);
     auto kernel = dtype == BSA_BF16 ? weight_grad_kernel<true> : weight_grad_kernel<false>;
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
