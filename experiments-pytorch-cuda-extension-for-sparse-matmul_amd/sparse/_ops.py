@@ -53,20 +53,19 @@ RUN_WALK_STRIPS = 32             # 4 per wave; with 10 waves and up to 39 strips
 RUN_WALK_MIN_REUSE = 2.0
 # DDS over many dense rows (a block-sparse linear layer): panels of the dense operand shared by eight groups
 # (bsa_matmul_dds_panels), when the mask is dense enough that a panel serves several of them and the launch has
-# workgroups for most of the machine.  Measured against the group walk, fp16 / bf16, us: stored share of the cells times used
-# share of the panels' rows 0.08 (96 x 96 blocks, 8 x 1024 rows) 88 -> 97, 0.10 (64 x 64, 4 x 1056) 36 -> 30, 0.12 (96 x 96, 8 x
-# 1024) 111 -> 98, 0.18 155 -> 107, 0.30 238 -> 117; at a stored share of 0.2 by workgroups: 96 32 x 96 blocks 10 -> 24,
-# 128 (64 x 64, 16 x 96 rows) 16 -> 18, 176 (64 x 64, 2 x 1056) 28 -> 20.
+# workgroups for most of the machine.  Measured against the group walk, bf16, us: stored share of the cells times used share of
+# the panels' rows 0.09 (96 x 96 blocks, 8 x 1024 rows) 95 -> 78, (64 x 64, 4 x 1056) 31 -> 25, 0.11 (64 x 64) 35 -> 26, 0.13
+# (96 x 96) 119 -> 81, 0.31 250 -> 91; one entry of 1056 rows, 64 x 64 at 0.2, 88 workgroups: 16.8 -> 17.5.
 PANEL_WALK = True
 PANEL_ROWS, PANEL_MAX_KBLOCKS, PANEL_MAX_NNZ = _k.dds_panel_limits()      # of a workgroup, of a launch
 PANEL_GROUPS = 8                       # of a workgroup
 PANEL_MIN_WORKGROUPS = 160
-PANEL_MIN_DENSITY = 0.12
-# Its weight gradient (bsa_weight_grad) against a stack per batch entry and a sum over them: 0.12 stored (96 x 96 blocks, 8192
-# tokens) 104 -> 114 us, 0.18 179 -> 126, 0.25 (64 x 64, 4224 tokens) 67 -> 40; 0.2, 1056 tokens 60 -> 24; 0.3 (16 x 16), 256
-# tokens 12 -> 16.
+PANEL_MIN_DENSITY = 0.08
+# Its weight gradient (bsa_weight_grad) against a stack per batch entry and a sum over them, us: 0.09 stored (96 x 96 blocks, 8192
+# tokens) 81 -> 87, 0.13 121 -> 94, 0.19 196 -> 107; 0.11 (64 x 64, 4224 tokens) 63 -> 27, 0.26 67 -> 36; 0.2, 1056 tokens
+# 60 -> 23; 0.3 (16 x 16), 256 tokens 12 -> 16.
 WEIGHT_GRAD_MIN_TOKENS = 1024
-WEIGHT_GRAD_MIN_DENSITY = 0.15
+WEIGHT_GRAD_MIN_DENSITY = 0.10
 ATTENTION_WAVES_LONG_GROUPS = 8
 ATTENTION_COLUMN_WAVES_128 = 4    # waves of a workgroup the column walk takes at head dim 128
 ATTENTION_SPLIT_ROWS = True       # groups longer than cap * waves are cut into parts across workgroups
