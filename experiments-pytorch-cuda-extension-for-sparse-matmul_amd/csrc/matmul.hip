@@ -325,12 +325,15 @@ __device__ __forceinline__ void lds_get_f32(const float *tile, float (&v)[16])
 //   lo hi + mid mid + hi lo, then mid hi + hi mid, then hi hi, smallest first into the fp32 accumulator.
 // 16 steps of k cost 6 x 32 clocks of the matrix pipe instead of 8 x 64 of v_mfma_f32_32x32x2_f32, and unlike that instruction
 // they leave the vector datapath to the other waves (beside an fp32 chain another wave's FMA took 92 clocks instead of 7).
-// What bfloat16 cannot split is seen in the result, and the wave takes its products again on the fp32 instruction: an infinity or
-// NaN, or a value that rounds to infinity, leaves a remainder of NaN; below 2^-109 the last part falls under the smallest
-// bfloat16, which shows while the other operand is below 2^49 / k as results that are all below 2^-60 in a lane.
+// The operands tell what three parts cannot hold, and the wave takes that block's products again on the fp32 instruction.  An
+// infinity or NaN, or a value that rounds to infinity, leaves a remainder of NaN, which reaches the result.  A value's last part is
+// a multiple of 2^-23 of the value's magnitude, which the smallest normal bfloat16, 2^-126, holds from 2^-103 on: a tile whose
+// smallest magnitude is below that is searched for an element that is not zero.  The results cannot show it: a lane has 16 columns
+// of a row, ordinary ones beside a small one, and small times large is ordinary.
 // Error against float64 (2-norm, normal operands; fp32 instruction -> split): k = 32 1.03e-7 -> 0.69e-7, 64 1.44e-7 -> 1.09e-7,
 // 128 2.03e-7 -> 1.63e-7; the same from 1e-17 to 1e15.  us, fp32 instruction, one block a wave -> split, four blocks (16 heads of
 // 4096 tokens, 24480 blocks, head dim 64) 43.3 -> 36.0, 48 heads 122 -> 96, 16 heads of 2048 17.6 -> 15.0: the stores remain.
+constexpr float SPLIT_HELD = 0x1p-103f;
 struct SplitF32 {
     h8 hi, mid, lo;                          // eight values of k
 };
@@ -355,13 +358,35 @@ __device__ __forceinline__ f16v mfma_split(const SplitF32 &a, const SplitF32 &b,
     acc = mfma_16<true>(a.hi, b.mid, acc);
     return mfma_16<true>(a.hi, b.hi, acc);
 }
-// whether some lane's results say that the split did not hold (uniform across the wave)
-__device__ __forceinline__ bool split_failed(const f16v &acc)
+// The smallest magnitude so far and of eight values: half an instruction a value, where the compiler's minimum of magnitudes takes
+// one and a half (and the kernel 3-6 % more time)
+__device__ __forceinline__ float smallest_f32(const float *v, float least)
+{
+#pragma unroll
+    for (int t = 0; t < 8; t += 2) asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(v[t]), "v"(v[t + 1]));
+    return least;
+}
+// whether some lane's 32 x 32 KBT operands in LDS have an element that three parts do not hold; zeros they do
+template <bool KC, bool PERMUTED, int KBT>
+__device__ __forceinline__ bool unsplittable(const float *tiles)
+{
+    bool small = false;
+#pragma unroll 1
+    for (int kb = 0; kb < KBT; ++kb) {
+        float v[16];
+        lds_get_f32<KC, PERMUTED>(tiles + kb * (F32_TILE_BYTES / 4), v);
+#pragma unroll
+        for (int t = 0; t < 16; ++t) small |= v[t] != 0.f && __builtin_fabsf(v[t]) < SPLIT_HELD;
+    }
+    return __builtin_amdgcn_ballot_w64(small) != 0ull;
+}
+// whether some lane's results are not all finite (uniform across the wave, as above)
+__device__ __forceinline__ bool not_finite(const f16v &acc)
 {
     float sum = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) sum += __builtin_fabsf(acc[v]);
-    return __builtin_amdgcn_ballot_w64(!(sum < __builtin_inff()) || (sum != 0.f && sum < 0x1p-60f)) != 0ull;
+    return __builtin_amdgcn_ballot_w64(!(sum < __builtin_inff())) != 0ull;
 }
 
 // SDD fp32 with K = 32 KBT <= 128: the operands of the wave's block row stay in registers (16 KBT floats per
@@ -425,21 +450,28 @@ __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
         }
         return acc;
     };
+    bool row_held = true;                    // by three parts: the operands of the block row
     auto multiply = [&](int p) {
         f16v acc = {0};
+        float least = 1.f;
 #pragma unroll
         for (int kb = 0; kb < KBT; ++kb) {
             float bop[16];
             lds_get_f32<B_KC, true>(tiles + kb * (F32_TILE_BYTES / 4), bop);
             if (SPLIT) {
 #pragma unroll
-                for (int s = 0; s < 2; ++s) acc = mfma_split(split_f32(bop + 8 * s), aop[kb][s], acc);
+                for (int s = 0; s < 2; ++s) {
+                    least = smallest_f32(bop + 8 * s, least);
+                    acc = mfma_split(split_f32(bop + 8 * s), aop[kb][s], acc);
+                }
             } else {
 #pragma unroll
                 for (int t = 0; t < 16; ++t) acc = mfma_f32(bop[t], aop32[kb][t], acc);
             }
         }
-        if (SPLIT && split_failed(acc)) acc = multiply_f32();
+        if (SPLIT && (!row_held || not_finite(acc) || (__builtin_amdgcn_ballot_w64(least < SPLIT_HELD) != 0ull &&
+                                                       unsplittable<B_KC, true, KBT>(tiles))))
+            acc = multiply_f32();
         // a lane holds 16 consecutive columns of one row; the block leaves through LDS as four whole
         // kilobytes (64-byte pieces at 128-byte stride straight from the registers write at a third of the rate)
         wave_lds_fence();
@@ -456,12 +488,17 @@ __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
     };
     park();
     request(e.begin);        // the first block's tiles arrive while the row's operands are split
+    float least = 1.f;
 #pragma unroll
     for (int kb = 0; kb < KBT; ++kb) {
         lds_get_f32<A_KC, false>(tiles + kb * (F32_TILE_BYTES / 4), aop32[kb]);
 #pragma unroll
-        for (int s = 0; SPLIT && s < 2; ++s) aop[kb][s] = split_f32(aop32[kb] + 8 * s);
+        for (int s = 0; SPLIT && s < 2; ++s) {
+            least = smallest_f32(aop32[kb] + 8 * s, least);
+            aop[kb][s] = split_f32(aop32[kb] + 8 * s);
+        }
     }
+    if (SPLIT) row_held = __builtin_amdgcn_ballot_w64(least < SPLIT_HELD) == 0ull || !unsplittable<A_KC, false, KBT>(tiles);
     for (int seg = e.begin; seg < e.end; seg += WAVE) {
         const int seg_end = seg + WAVE < e.end ? seg + WAVE : e.end;
         if (seg != e.begin) {

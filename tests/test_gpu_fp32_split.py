@@ -69,6 +69,33 @@ def test_operands_that_three_parts_cannot_hold(value):
     assert bool(((got.double()[fine] - want[fine]).abs() <= scale * 64 * 2 ** -24 + 64 * 2.0 ** -149).all())
 
 
+@pytest.mark.parametrize("k", [32, 64, 128])
+@pytest.mark.parametrize("small,large", [(1e-36, 1.0), (1e-38, 1.0), (1e-40, 1.0), (2.0 ** -115, 2.0 ** 60), (2.0 ** -124, 2.0 ** 80), (1e-37, 1e20),
+                                         (1e-41, 1e25), (0.0, 1.0), (2.0 ** -99, 2.0 ** 90), (2.0 ** -62, 2.0 ** -62), (2.0 ** -66, 2.0 ** -60)])
+@pytest.mark.parametrize("where", ["all", "a line", "a step of k"])
+@pytest.mark.parametrize("swapped", [False, True])
+def test_small_operands_beside_large_and_ordinary_ones(small, large, where, swapped, k):
+    """Every element against its own bound: the operands say whether three parts hold them, not the results."""
+    import sparse
+    L = sparse.SparseLayout(torch.as_tensor(MASK))
+    x, y = _operands(k, seed=5)
+    assert L.num_blocks * x.size(0) >= 800
+    x, y = (y.transpose(1, 2).contiguous(), x.transpose(1, 2).contiguous()) if swapped else (x, y)      # x [.., tokens, k] is the small one
+    if where == "all":
+        x, y = x * small, y * large
+    elif where == "a line":                      # one token of every batch entry, the others ordinary
+        x[:, 37] *= small
+        y *= max(large, 1.0) if large < 2.0 ** 70 else 1.0
+    else:
+        x[..., 5] *= small
+        y[:, 5] *= large
+    a, b = (y.transpose(1, 2).contiguous(), x.transpose(1, 2).contiguous()) if swapped else (x, y)
+    got, want = _product(a, b, False, True, L).cpu().double(), _want(a, b, L)
+    # k roundings of the running sum, and one of 2^-150 a step where they fall under the smallest normal number
+    bound = _want(a.abs(), b.abs(), L) * k * 2 ** -24 + k * 2.0 ** -149
+    assert bool(((got - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("mode", ["sdd", "dsd"])
 def test_captured_at_another_batch_count(mode, monkeypatch):
     import sparse
