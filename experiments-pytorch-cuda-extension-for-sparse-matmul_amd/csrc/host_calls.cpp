@@ -119,7 +119,8 @@ struct Plans {
         if (version != now) return nullptr;
         for (const PlanPtr &p : plans)
             if (p->op == op && p->flags == flags && p->dtype == a.scalar_type() && p->device == a.get_device() &&
-                a.sizes().equals(p->a) && (!b.defined() || b.sizes().equals(p->b)) &&
+                a.sizes().equals(p->a) &&
+                (!b.defined() || (b.sizes().equals(p->b) && b.scalar_type() == p->dtype && b.get_device() == p->device)) &&
                 (!p->workspace.defined() || p->stream == stream))
                 return p;
         return nullptr;

@@ -146,6 +146,31 @@ def test_what_autograd_sees():
         sparse.matmul(fw.make_dual(a.detach(), torch.ones_like(a)), b.detach(), "dds", L)
 
 
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("mode,dim,shared", [("sdd", 64, False), ("dsd", 64, False), ("dds", 64, False), ("dds", 1056, True)])
+def test_a_saved_operand_that_comes_back_as_another_type(mode, dim, shared, which, monkeypatch):
+    """An unpack hook decides what a backward pass is given: it is refused as it is without a plan."""
+    import sparse
+    from sparse import _ops
+    from sparse.matmul import SparseMatMul
+    monkeypatch.setattr(_ops, "WEIGHT_GRAD_MIN_DENSITY", 0.0)
+    L = _layout("rand16")
+    a, b = _product(L, mode, False, False, dim, torch.bfloat16, shared=shared)
+    native = lambda: sparse.matmul(a, b, mode, L)
+    native().float().sum().backward()                                   # the plans are there
+    for change in (lambda t: t.half(), lambda t: t.cpu()):
+        errors = []
+        for f in (native, lambda: SparseMatMul.apply(a, b, mode, L)):
+            saved = []
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t) or len(saved) - 1,
+                                                          lambda i: change(saved[i]) if i == which else saved[i]):
+                y = f()
+            with pytest.raises((TypeError, ValueError)) as error:
+                y.float().sum().backward()
+            errors.append((type(error.value), str(error.value)))
+        assert errors[0] == errors[1]
+
+
 def test_operands_a_plan_does_not_hold():
     import sparse
     from sparse.matmul import SparseMatMul
