@@ -76,6 +76,26 @@ struct PythonRef {
     }
 };
 
+// The zeroed workspace of a schedule's split groups, as the plans that launch with it share it.  The schedule owns it (_ops.Schedule)
+// and says when it is theirs no more: a launch that failed, the schedule's bound, a spare to be put back.
+struct Space {
+    std::mutex mutex;
+    Tensor buffer;
+    Tensor get()
+    {
+        std::lock_guard<std::mutex> lock(mutex);
+        return buffer;
+    }
+    void drop()
+    {
+        Tensor gone;                         // released behind the lock
+        std::lock_guard<std::mutex> lock(mutex);
+        std::swap(gone, buffer);
+    }
+};
+typedef std::shared_ptr<Space> SpacePtr;
+constexpr const char *SPACE = "bsa.space";
+
 struct Plan {
     int op, flags;
     at::ScalarType dtype;
@@ -86,16 +106,24 @@ struct Plan {
     std::vector<int> n;                      // sizes and schedule figures in the order of the launch below
     std::vector<Tensor> tables;
     std::vector<int64_t> out;
-    Tensor workspace;                        // of split groups: zero between launches, which one stream orders
+    SpacePtr space;                          // of split groups: zero between launches, which one stream orders
     size_t workspace_bytes = 0;
     hipStream_t stream = nullptr;            // of the workspace
     std::unique_ptr<PythonRef> schedule;     // the schedule and the key its workspace is kept under there
     std::unique_ptr<PythonRef> workspace_key;
     template <class T = int32_t>
     T *table(int i) const { return tables[i].defined() ? static_cast<T *>(tables[i].data_ptr()) : nullptr; }
-    void *ws() const { return workspace.defined() ? workspace.data_ptr() : nullptr; }
 };
 typedef std::shared_ptr<const Plan> PlanPtr;
+
+// A plan to launch by, with its workspace held until the launch is in the stream
+struct Found {
+    PlanPtr plan;
+    Tensor workspace;
+    const Plan *operator->() const { return plan.get(); }
+    explicit operator bool() const { return plan != nullptr; }
+    void *ws() const { return workspace.defined() ? workspace.data_ptr() : nullptr; }
+};
 
 uint64_t settings_version()
 {
@@ -112,18 +140,31 @@ struct Plans {
     std::vector<PlanPtr> plans;
     uint64_t version = 0;
     PyObject *row_layout, *col_layout;       // the tuples the plans were made from
-    PlanPtr find(int op, int flags, const Tensor &a, const Tensor &b, hipStream_t stream)
+    Found find(int op, int flags, const Tensor &a, const Tensor &b, hipStream_t stream)
     {
         const uint64_t now = settings_version();
+        Found found;
+        std::vector<PlanPtr> gone;           // released behind the lock
         std::lock_guard<std::mutex> lock(mutex);
-        if (version != now) return nullptr;
-        for (const PlanPtr &p : plans)
-            if (p->op == op && p->flags == flags && p->dtype == a.scalar_type() && p->device == a.get_device() &&
-                a.sizes().equals(p->a) &&
-                (!b.defined() || (b.sizes().equals(p->b) && b.scalar_type() == p->dtype && b.get_device() == p->device)) &&
-                (!p->workspace.defined() || p->stream == stream))
-                return p;
-        return nullptr;
+        if (version != now) return found;
+        for (size_t i = 0; i < plans.size(); ++i) {
+            const PlanPtr p = plans[i];
+            if (p->op != op || p->flags != flags || p->dtype != a.scalar_type() || p->device != a.get_device() ||
+                !a.sizes().equals(p->a) || (p->space && p->stream != stream))
+                continue;
+            if (b.defined() && !(b.sizes().equals(p->b) && b.scalar_type() == p->dtype && b.get_device() == p->device)) continue;
+            if (p->space) {
+                found.workspace = p->space->get();
+                if (!found.workspace.defined()) {
+                    gone.push_back(p);
+                    plans.erase(plans.begin() + i--);
+                    continue;
+                }
+            }
+            found.plan = p;
+            return found;
+        }
+        return found;
     }
     void add(PlanPtr plan)
     {
@@ -153,6 +194,42 @@ struct Plans {
 typedef std::shared_ptr<Plans> PlansPtr;
 constexpr const char *CAPSULE = "bsa.plans";
 
+PyObject *new_space(PyObject *, PyObject *workspace)
+{
+    HANDLE_TH_ERRORS
+    SpacePtr space = std::make_shared<Space>();
+    space->buffer = THPVariable_Unpack(workspace);
+    return PyCapsule_New(new SpacePtr(std::move(space)), SPACE,
+                         [](PyObject *c) { delete static_cast<SpacePtr *>(PyCapsule_GetPointer(c, SPACE)); });
+    END_HANDLE_TH_ERRORS
+}
+
+PyObject *drop_space(PyObject *, PyObject *capsule)
+{
+    HANDLE_TH_ERRORS
+    auto *space = static_cast<SpacePtr *>(PyCapsule_GetPointer(capsule, SPACE));
+    if (space == nullptr) return nullptr;
+    (*space)->drop();
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+// Address of each plan's workspace, 0 where it has none
+PyObject *plan_workspaces(PyObject *, PyObject *capsule)
+{
+    HANDLE_TH_ERRORS
+    auto *plans = static_cast<PlansPtr *>(PyCapsule_GetPointer(capsule, CAPSULE));
+    if (plans == nullptr) return nullptr;
+    py::list result;
+    std::lock_guard<std::mutex> lock((*plans)->mutex);
+    for (const PlanPtr &p : (*plans)->plans) {
+        const Tensor ws = p->space ? p->space->get() : Tensor();
+        result.append(ws.defined() ? reinterpret_cast<uintptr_t>(ws.data_ptr()) : 0);
+    }
+    return result.release().ptr();
+    END_HANDLE_TH_ERRORS
+}
+
 PyObject *new_plans(PyObject *, PyObject *args)
 {
     HANDLE_TH_ERRORS
@@ -173,15 +250,15 @@ PyObject *new_plans(PyObject *, PyObject *args)
     END_HANDLE_TH_ERRORS
 }
 
-// plans, op, flags, a, b, route, dtype, aligned, ints, tables, out, workspace, workspace bytes, stream, schedule, key
+// plans, op, flags, a, b, route, dtype, aligned, ints, tables, out, space, workspace bytes, stream, schedule, key
 PyObject *add_plan(PyObject *, PyObject *args)
 {
     HANDLE_TH_ERRORS
-    PyObject *capsule, *a, *b, *ints, *tables, *out, *workspace, *schedule, *key;
+    PyObject *capsule, *a, *b, *ints, *tables, *out, *space, *schedule, *key;
     int op, flags, route, dtype, aligned;
     unsigned long long bytes, stream;
     if (!PyArg_ParseTuple(args, "OiiOOiipO!O!O!OKKOO", &capsule, &op, &flags, &a, &b, &route, &dtype, &aligned, &PyTuple_Type, &ints,
-                          &PyTuple_Type, &tables, &PyTuple_Type, &out, &workspace, &bytes, &stream, &schedule, &key))
+                          &PyTuple_Type, &tables, &PyTuple_Type, &out, &space, &bytes, &stream, &schedule, &key))
         return nullptr;
     auto *plans = static_cast<PlansPtr *>(PyCapsule_GetPointer(capsule, CAPSULE));
     if (plans == nullptr) return nullptr;
@@ -203,8 +280,10 @@ PyObject *add_plan(PyObject *, PyObject *args)
     }
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(out); ++i) plan->out.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(out, i)));
     if (PyErr_Occurred()) return nullptr;
-    if (workspace != Py_None) {
-        plan->workspace = THPVariable_Unpack(workspace);
+    if (space != Py_None) {
+        auto *shared = static_cast<SpacePtr *>(PyCapsule_GetPointer(space, SPACE));
+        if (shared == nullptr) return nullptr;
+        plan->space = *shared;
         plan->workspace_bytes = bytes;
         plan->stream = reinterpret_cast<hipStream_t>(stream);
         plan->schedule = std::make_unique<PythonRef>(schedule);
@@ -245,18 +324,17 @@ bool plain_thread()
 hipStream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 // The plan of a call on these operands, if the call can go by one here and now
-PlanPtr find_plan(Plans &plans, int op, int flags, const Tensor &a, const Tensor &b)
+Found find_plan(Plans &plans, int op, int flags, const Tensor &a, const Tensor &b)
 {
-    const hipStream_t stream = current_stream();
-    PlanPtr p = plans.find(op, flags, a, b, stream);
-    if (p && p->workspace.defined() && c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
+    Found p = plans.find(op, flags, a, b, current_stream());
+    if (p && p->space && c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return Found();
     return p;
 }
-void check(int status, Plans &plans, const PlanPtr &p)
+void check(int status, Plans &plans, const Found &p)
 {
     if (status == 0) return;
-    // the launch may have left counters of the workspace non-zero: it is forgotten, here and in its schedule
-    plans.drop(p);
+    // the launch may have left counters of the workspace non-zero: its schedule forgets it and takes it from every plan
+    plans.drop(p.plan);
     py::gil_scoped_acquire gil;
     PyObject *none = PyObject_CallFunction(python.failed, "iOO", status, p->schedule ? p->schedule->object : Py_None,
                                            p->workspace_key ? p->workspace_key->object : Py_None);
@@ -267,7 +345,7 @@ void check(int status, Plans &plans, const PlanPtr &p)
     raise_pending();
 }
 
-Tensor run_matmul(Plans &plans, const PlanPtr &p, const Tensor &a, const Tensor &b)
+Tensor run_matmul(Plans &plans, const Found &p, const Tensor &a, const Tensor &b)
 {
     Tensor c = at::empty(p->out, a.options());
     const int *n = p->n.data();
@@ -281,7 +359,7 @@ Tensor run_matmul(Plans &plans, const PlanPtr &p, const Tensor &a, const Tensor 
                             n[5], n[6], st);
     else                                     // mode, groups, wgs, waves, tiles, splits, rows, cols, nnz, batches, sparse batches, M, N, K, ta, tb
         status = lib.matmul(n[0], p->bsa_dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(), p->table(0), p->table(1), n[1], p->table(2), n[2],
-                            n[3], n[4], n[5], p->ws(), p->workspace_bytes, n[6], n[7], n[8], n[9], n[10], n[11], n[12], n[13], n[14], n[15],
+                            n[3], n[4], n[5], p.ws(), p->workspace_bytes, n[6], n[7], n[8], n[9], n[10], n[11], n[12], n[13], n[14], n[15],
                             st);
     check(status, plans, p);
     return c;
@@ -307,7 +385,7 @@ Tensor unwrap_new(PyObject *result)          // steals
 Tensor product(Plans &plans, PyObject *layout, const Tensor &a, const Tensor &b, int mode, bool ta, bool tb)
 {
     const int flags = mode << 2 | ta << 1 | tb;
-    PlanPtr p = plain(a) && plain(b) && on_current_device(a) ? find_plan(plans, MATMUL, flags, a, b) : nullptr;
+    Found p = plain(a) && plain(b) && on_current_device(a) ? find_plan(plans, MATMUL, flags, a, b) : Found();
     if (!p || (p->aligned && !(at_16_bytes(a) && at_16_bytes(b)))) {
         py::gil_scoped_acquire gil;
         Borrow pa(a), pb(b);
@@ -316,7 +394,7 @@ Tensor product(Plans &plans, PyObject *layout, const Tensor &a, const Tensor &b,
         if (made == nullptr) raise_pending();
         const bool planned = made == Py_True;
         Py_DECREF(made);
-        p = planned && plain(a) && plain(b) && on_current_device(a) ? find_plan(plans, MATMUL, flags, a, b) : nullptr;
+        p = planned && plain(a) && plain(b) && on_current_device(a) ? find_plan(plans, MATMUL, flags, a, b) : Found();
         if (!p || (p->aligned && !(at_16_bytes(a) && at_16_bytes(b))))
             return unwrap_new(PyObject_CallFunctionObjArgs(python.run_matmul, pa.get(), pb.get(), python.modes[mode], layout, py_bool(ta),
                                                            py_bool(tb), nullptr));
@@ -326,11 +404,11 @@ Tensor product(Plans &plans, PyObject *layout, const Tensor &a, const Tensor &b,
 
 Tensor weight_gradient(Plans &plans, PyObject *layout, const Tensor &a, const Tensor &b, bool ta, bool tb)
 {
-    auto by_plan = [&]() -> PlanPtr {
-        if (!(plain(a) && plain(b) && on_current_device(a) && at_16_bytes(a) && at_16_bytes(b))) return nullptr;
+    auto by_plan = [&]() -> Found {
+        if (!(plain(a) && plain(b) && on_current_device(a) && at_16_bytes(a) && at_16_bytes(b))) return Found();
         return find_plan(plans, WEIGHT_GRAD, ta << 1 | tb, a, b);
     };
-    PlanPtr p = by_plan();
+    Found p = by_plan();
     if (!p) {
         py::gil_scoped_acquire gil;
         Borrow pa(a), pb(b);
@@ -338,7 +416,7 @@ Tensor weight_gradient(Plans &plans, PyObject *layout, const Tensor &a, const Te
         if (made == nullptr) raise_pending();
         const bool planned = made == Py_True;
         Py_DECREF(made);
-        p = planned ? by_plan() : nullptr;
+        p = planned ? by_plan() : Found();
         if (!p)
             return unwrap_new(PyObject_CallFunctionObjArgs(python.run_weight, pa.get(), pb.get(), layout, py_bool(ta), py_bool(tb), nullptr));
     }
@@ -412,12 +490,12 @@ struct SoftmaxNode : public Node {
         std::lock_guard<std::mutex> lock(mutex_);
         const Tensor y = y_.unpack(getptr()), dy = first_gradient(grads, *this);
         if (!task_should_compute_output(0)) return {Tensor()};
-        auto by_plan = [&]() -> PlanPtr {
+        auto by_plan = [&]() -> Found {
             if (!(plain(y) && plain(dy) && on_current_device(y) && y.sizes() == dy.sizes() && y.scalar_type() == dy.scalar_type()))
-                return nullptr;
+                return Found();
             return find_plan(*plans, SOFTMAX_BACKWARD, 0, y, Tensor());
         };
-        PlanPtr p = by_plan();
+        Found p = by_plan();
         if (!p) {
             py::gil_scoped_acquire gil;
             Borrow py_y(y), py_dy(dy);
@@ -425,7 +503,7 @@ struct SoftmaxNode : public Node {
             if (made == nullptr) raise_pending();
             const bool planned = made == Py_True;
             Py_DECREF(made);
-            p = planned ? by_plan() : nullptr;
+            p = planned ? by_plan() : Found();
             if (!p) {
                 py::object s = py::float_(scale);
                 return {unwrap_new(PyObject_CallFunctionObjArgs(python.run_softmax_backward, py_y.get(), py_dy.get(), layout->object, s.ptr(), nullptr))};
@@ -458,18 +536,18 @@ struct AttentionNode : public Node {
         const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(getptr()), lse = lse_.unpack();
         const Tensor dout = first_gradient(grads, *this);
         const bool dkdv = task_should_compute_output(1) || task_should_compute_output(2);
-        auto by_plan = [&]() -> PlanPtr {
+        auto by_plan = [&]() -> Found {
             for (const Tensor *t : {&q, &k, &v, &dout, &out, &lse})
-                if (!plain(*t) || t->get_device() != q.get_device()) return nullptr;
-            if (!(on_current_device(q) && at_16_bytes(q) && at_16_bytes(k) && at_16_bytes(v) && at_16_bytes(dout))) return nullptr;
+                if (!plain(*t) || t->get_device() != q.get_device()) return Found();
+            if (!(on_current_device(q) && at_16_bytes(q) && at_16_bytes(k) && at_16_bytes(v) && at_16_bytes(dout))) return Found();
             if (dout.sizes() != q.sizes() || out.sizes() != q.sizes() || v.sizes() != k.sizes() || lse.scalar_type() != at::kFloat ||
                 lse.sizes() != q.sizes().slice(0, q.dim() - 1))
-                return nullptr;
+                return Found();
             for (const Tensor *t : {&k, &v, &dout, &out})
-                if (t->scalar_type() != q.scalar_type()) return nullptr;
+                if (t->scalar_type() != q.scalar_type()) return Found();
             return find_plan(*plans, ATTENTION_BACKWARD, dkdv, q, k);
         };
-        PlanPtr p = by_plan();
+        Found p = by_plan();
         if (!p) {
             py::gil_scoped_acquire gil;
             Borrow pq(q), pk(k), pv(v), pd(dout), po(out), pl(lse);
@@ -477,7 +555,7 @@ struct AttentionNode : public Node {
             if (made == nullptr) raise_pending();
             const bool planned = made == Py_True;
             Py_DECREF(made);
-            p = planned ? by_plan() : nullptr;
+            p = planned ? by_plan() : Found();
             if (!p) {
                 py::object s = py::float_(scale);
                 PyObject *got = PyObject_CallFunctionObjArgs(python.run_attention_backward, pq.get(), pk.get(), pv.get(), pd.get(), po.get(), pl.get(),
@@ -498,7 +576,7 @@ struct AttentionNode : public Node {
         check(lib.attention_gradients(p->bsa_dtype, q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
                                       dq.data_ptr(), dkdv ? dk.data_ptr() : nullptr, dkdv ? dv.data_ptr() : nullptr, delta.data_ptr<float>(),
                                       p->table(0), p->table(1), p->table(2), n[0], n[1], n[2], n[3], p->table(3), p->table(4), p->table(5), n[4],
-                                      n[5], n[6], n[7], p->ws(), p->workspace_bytes, n[8], n[9], n[10], n[11], n[12], (float)scale, causal,
+                                      n[5], n[6], n[7], p.ws(), p->workspace_bytes, n[8], n[9], n[10], n[11], n[12], (float)scale, causal,
                                       current_stream()), *plans, p);
         return {dq, dk, dv};
     }
@@ -557,13 +635,13 @@ PyObject *matmul(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     const PlansPtr plans = plans_of(args[3]);
     if (plans == nullptr) return general(python.matmul, args, nargs);
     const int flags = mode << 2 | ta << 1 | tb;
-    PlanPtr p = find_plan(*plans, MATMUL, flags, a, b);
+    Found p = find_plan(*plans, MATMUL, flags, a, b);
     if (!p) {
         PyObject *made = PyObject_CallFunctionObjArgs(python.plan_matmul, args[0], args[1], args[2], args[3], py_bool(ta), py_bool(tb), nullptr);
         if (made == nullptr) return nullptr;
         const bool planned = made == Py_True;
         Py_DECREF(made);
-        p = planned ? find_plan(*plans, MATMUL, flags, a, b) : nullptr;
+        p = planned ? find_plan(*plans, MATMUL, flags, a, b) : Found();
     }
     if (!p || (p->aligned && !(at_16_bytes(a) && at_16_bytes(b)))) return general(python.matmul, args, nargs);
     std::shared_ptr<MatMulNode> node;
@@ -600,13 +678,13 @@ PyObject *softmax(PyObject *, PyObject *const *args, Py_ssize_t nargs)      // x
     if (plans == nullptr) return general(python.softmax, args, nargs);
     const double scale = PyFloat_AsDouble(args[2]);
     if (scale == -1.0 && PyErr_Occurred()) return nullptr;
-    PlanPtr p = find_plan(*plans, SOFTMAX_FORWARD, 0, x, Tensor());
+    Found p = find_plan(*plans, SOFTMAX_FORWARD, 0, x, Tensor());
     if (!p) {
         PyObject *made = PyObject_CallFunctionObjArgs(python.plan_softmax, args[0], args[1], nullptr);
         if (made == nullptr) return nullptr;
         const bool planned = made == Py_True;
         Py_DECREF(made);
-        p = planned ? find_plan(*plans, SOFTMAX_FORWARD, 0, x, Tensor()) : nullptr;
+        p = planned ? find_plan(*plans, SOFTMAX_FORWARD, 0, x, Tensor()) : Found();
     }
     if (!p) return general(python.softmax, args, nargs);
     std::shared_ptr<SoftmaxNode> node;
@@ -649,13 +727,13 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs)    // q
     if (plans == nullptr) return general(python.attention, args, nargs);
     const double scale = PyFloat_AsDouble(args[4]);
     if (scale == -1.0 && PyErr_Occurred()) return nullptr;
-    PlanPtr p = find_plan(*plans, ATTENTION_FORWARD, 0, q, k);
+    Found p = find_plan(*plans, ATTENTION_FORWARD, 0, q, k);
     if (!p) {
         PyObject *made = PyObject_CallFunctionObjArgs(python.plan_attention, args[0], args[1], args[2], args[3], nullptr);
         if (made == nullptr) return nullptr;
         const bool planned = made == Py_True;
         Py_DECREF(made);
-        p = planned ? find_plan(*plans, ATTENTION_FORWARD, 0, q, k) : nullptr;
+        p = planned ? find_plan(*plans, ATTENTION_FORWARD, 0, q, k) : Found();
     }
     if (!p) return general(python.attention, args, nargs);
     std::shared_ptr<AttentionNode> node;
@@ -677,7 +755,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs)    // q
         out = at::empty(q.sizes(), q.options());
         if (node) lse = at::empty(q.sizes().slice(0, q.dim() - 1), q.options().dtype(at::kFloat));
         check(lib.attention_forward(p->bsa_dtype, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), node ? lse.data_ptr<float>() : nullptr,
-                                    p->table(0), p->table(1), p->table(2), n[0], n[1], n[2], n[3], p->ws(), p->workspace_bytes, n[4], n[5], n[6],
+                                    p->table(0), p->table(1), p->table(2), n[0], n[1], n[2], n[3], p.ws(), p->workspace_bytes, n[4], n[5], n[6],
                                     n[7], n[8], (float)scale, causal, current_stream()), *plans, p);
     }
     if (node) {
@@ -745,6 +823,9 @@ PyMethodDef methods[] = {
     {"setup", setup, METH_VARARGS, nullptr},
     {"new_plans", new_plans, METH_VARARGS, nullptr},
     {"add_plan", add_plan, METH_VARARGS, nullptr},
+    {"new_space", new_space, METH_O, nullptr},
+    {"drop_space", drop_space, METH_O, nullptr},
+    {"plan_workspaces", plan_workspaces, METH_O, nullptr},
     {"matmul", (PyCFunction)(void (*)(void))matmul, METH_FASTCALL, "matmul(a, b, mode, layout, trans_a=False, trans_b=False)"},
     {"softmax", (PyCFunction)(void (*)(void))softmax, METH_FASTCALL, "softmax(x, layout, scale, causal)"},
     {"attention", (PyCFunction)(void (*)(void))attention, METH_FASTCALL, "attention(q, k, v, layout, scale, causal)"},

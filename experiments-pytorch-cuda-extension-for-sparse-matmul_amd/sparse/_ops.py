@@ -114,6 +114,7 @@ class Schedule:
         self._workspaces = {}
         self._captured = {}
         self._spares = {}
+        self._spaces = {}
         self.last_key = None
 
     def workspace(self, mode: int, batches: int, size_m: int, size_n: int, stream: int):
@@ -143,6 +144,7 @@ class Schedule:
         self.last_key = ("attention_backward", id(columns), batches, head_dim, stream)
         return self._zeroed(self.last_key, need)
 
+    _spaces = {}             # of a schedule that no plan launches by
     MAX_WORKSPACES = 16      # eager ones per schedule; the least recently used one goes first
 
     def _zeroed(self, key, need):
@@ -153,7 +155,10 @@ class Schedule:
 
         A buffer handed out under capture is never dropped: the captured graph holds its raw address and
         may be replayed at any time.  An eager one is dropped only after the stream it was used on has
-        drained (a launch still in flight parks partial tiles there)."""
+        drained (a launch still in flight parks partial tiles there).
+
+        Plans launch with an eager workspace without coming here (``plan_space``); they lose it, and the next call
+        comes here again, where it is dropped."""
         if need == 0:
             return None, 0
         capturing = torch.cuda.is_current_stream_capturing()
@@ -188,8 +193,20 @@ class Schedule:
         """Waits for the stream a workspace was used on before the workspace is given back to the allocator."""
         torch.cuda.ExternalStream(stream_handle, device=self.table.device).synchronize()
 
+    def plan_space(self, key, ws):
+        """What the plans that launch with the workspace ``ws`` of ``key`` share, and lose together."""
+        if key not in self._spaces:
+            self._spaces[key] = _k.host_calls.new_space(ws)
+        return self._spaces[key]
+
+    def _forget_plans(self, key):
+        space = self._spaces.pop(key, None)
+        if space is not None:
+            _k.host_calls.drop_space(space)
+
     def discard(self, key):
         """Forget the workspace of ``key``: a launch that failed may have left its counters non-zero."""
+        self._forget_plans(key)
         self._workspaces.pop(key, None)
         self._captured.pop(key, None)
 
@@ -788,8 +805,9 @@ def _planned(make):
 
 def _add(plans, op, flags, a, b, route, ints, tables, out=(), workspace=(None, 0), sched=None, aligned=False):
     ws, ws_bytes = workspace
-    _k.host_calls.add_plan(plans, op, flags, a, b, route, _DTYPES[a.dtype], aligned, ints, tables, out, ws, ws_bytes,
-                           _k.current_stream(), sched, sched.last_key if ws is not None else None)
+    key = sched.last_key if ws is not None else None
+    _k.host_calls.add_plan(plans, op, flags, a, b, route, _DTYPES[a.dtype], aligned, ints, tables, out,
+                           sched.plan_space(key, ws) if ws is not None else None, ws_bytes, _k.current_stream(), sched, key)
     return True
 
 

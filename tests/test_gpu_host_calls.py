@@ -250,6 +250,29 @@ def test_captured_with_plans_there():
         assert torch.equal(got, want) and torch.equal(eager, want)
 
 
+def test_a_failed_launch_takes_the_workspace_from_every_plan(monkeypatch):
+    """fp16 and bf16 calls, and other groupings of as many entries, launch with one workspace."""
+    import sparse
+    from sparse import kernel
+    from sparse.matmul import SparseMatMul
+    L = _layout()
+    calls = [_product(L, "dds", False, False, 64, dtype, lead=lead) for dtype, lead in ((torch.float16, (2, 3)), (torch.bfloat16, (2, 3)), (torch.float16, (6,)))]
+    calls = [(a.detach(), b.detach()) for a, b in calls]
+    want = [SparseMatMul.apply(a, b, "dds", L) for a, b in calls]
+    for a, b in calls[:2]:
+        sparse.matmul(a, b, "dds", L)
+    shared = kernel.host_calls.plan_workspaces(L._plans)
+    assert len(shared) == 2 and shared[0] == shared[1] != 0
+    real = kernel.host_calls.add_plan                                   # a plan that the library refuses: too small a workspace
+    monkeypatch.setattr(kernel.host_calls, "add_plan", lambda *args: real(*args[:12], 1, *args[13:]))
+    with pytest.raises(kernel.BsaError):
+        sparse.matmul(*calls[2], "dds", L)
+    monkeypatch.undo()
+    assert not any(kernel.host_calls.plan_workspaces(L._plans))
+    for (a, b), w in zip(calls, want):
+        assert torch.equal(sparse.matmul(a, b, "dds", L), w)
+
+
 def test_plans_are_bounded():
     import sparse
     L = _layout("rand16")
