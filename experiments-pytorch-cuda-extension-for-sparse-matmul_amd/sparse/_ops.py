@@ -185,6 +185,7 @@ class Schedule:
         self._workspaces[key] = ws                      # most recently used last
         while len(self._workspaces) > self.MAX_WORKSPACES:
             old_key = next(iter(self._workspaces))
+            self._forget_plans(old_key)
             self._drain(old_key[-1])
             self._workspaces.pop(old_key)
         return ws, need

@@ -273,10 +273,28 @@ def test_a_failed_launch_takes_the_workspace_from_every_plan(monkeypatch):
         assert torch.equal(sparse.matmul(a, b, "dds", L), w)
 
 
+def test_workspaces_that_plans_use_are_bounded():
+    import sparse
+    from sparse import _ops, kernel
+    from sparse.matmul import SparseMatMul
+    L = _layout()
+    a, b = (t.detach() for t in _product(L, "dds", False, False, 64, torch.float16, lead=(70,)))
+    want = SparseMatMul.apply(a, b, "dds", L)
+    for n in list(range(1, 71)) + [1, 60, 2, 70]:
+        for _ in range(2):
+            assert torch.equal(sparse.matmul(a[:n], b[:n], "dds", L), want[:n])
+        there = kernel.host_calls.plan_workspaces(L._plans)
+        assert len(there) <= 64 and sum(ws != 0 for ws in there) <= _ops.Schedule.MAX_WORKSPACES
+    assert any(there)
+
+
 def test_plans_are_bounded():
     import sparse
+    from sparse import kernel
+    from sparse.softmax import SparseSoftmax
     L = _layout("rand16")
-    for n in list(range(1, 80)) + [1]:
-        x = _randn(n, L.num_blocks, 32, 32, dtype=torch.float16)
-        y = sparse.softmax(x, L, 1.0, False)
-    assert y.shape == x.shape
+    x = _randn(80, L.num_blocks, 32, 32, dtype=torch.float16)
+    want = SparseSoftmax.apply(x, L, 1.0, False)
+    for i, n in enumerate(list(range(1, 81)) + [1, 80, 2]):
+        assert torch.equal(sparse.softmax(x[:n], L, 1.0, False), want[:n])
+        assert len(kernel.host_calls.plan_workspaces(L._plans)) == min(i + 1, 64)
