@@ -158,7 +158,7 @@ class Schedule:
         drained (a launch still in flight parks partial tiles there).
 
         Plans launch with an eager workspace without coming here (``plan_space``); they lose it, and the next call
-        comes here again, where it is dropped."""
+        comes here again, where it is dropped and where a capture took the shape's spare."""
         if need == 0:
             return None, 0
         capturing = torch.cuda.is_current_stream_capturing()
@@ -175,6 +175,8 @@ class Schedule:
                     raise RuntimeError("this operator and shape has never run outside graph capture: call it once "
                                        "eagerly before capturing (its workspace must be zeroed first)")
                 ws = spares.pop()
+                for other in [k for k in self._spaces if k[:-1] == key[:-1]]:
+                    self._forget_plans(other)           # one of their calls puts a spare back
             else:
                 ws = torch.zeros(need, dtype=torch.uint8, device=self.table.device)
         if not capturing and not spares:

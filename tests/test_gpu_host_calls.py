@@ -250,6 +250,27 @@ def test_captured_with_plans_there():
         assert torch.equal(got, want) and torch.equal(eager, want)
 
 
+def test_captured_on_several_streams():
+    """An eager call between two captures is what lets the second have a workspace of its own, by a plan too."""
+    import sparse
+    L = _layout()
+    a, b = (t.detach() for t in _product(L, "dds", False, False, 64, torch.float16))
+    want = sparse.matmul(a, b, "dds", L)
+    graphs = []
+    for _ in range(3):
+        assert torch.equal(sparse.matmul(a, b, "dds", L), want)
+        torch.cuda.synchronize()
+        graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=stream):
+            graphs.append((graph, sparse.matmul(a, b, "dds", L)))
+    for _ in range(3):
+        for graph, got in graphs:
+            graph.replay()
+            eager = sparse.matmul(a, b, "dds", L)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want) and torch.equal(eager, want)
+
+
 def test_a_failed_launch_takes_the_workspace_from_every_plan(monkeypatch):
     """fp16 and bf16 calls, and other groupings of as many entries, launch with one workspace."""
     import sparse
