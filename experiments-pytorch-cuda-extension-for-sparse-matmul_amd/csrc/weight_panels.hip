@@ -132,15 +132,33 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
         n = n < 0 ? 0 : n < kblocks ? n : kblocks;
         auto kblock = [&](const BlockDesc &d) { return S_KC ? d.col() : d.row(); };
         const BlockDesc first = l < n ? blocks[begin + l] : BlockDesc{0, -1};
-        int before = __popcll(__ballot(l < n && kblock(first) < start * PANEL_KB));       // pairs of steps that come around again
-        for (int p = WAVE; p < n; p += WAVE) {
-            const int kb = p + l < n ? kblock(blocks[begin + p + l]) : kblocks;
+        int before = 0, previous = -1;                                     // pairs of steps that come around again; the lane before this one's
+        bool ascending = true;
+        for (int p = 0; p < n; p += WAVE) {
+            const int kb = p + l >= n ? kblocks : kblock(p == 0 ? first : blocks[begin + p + l]), left = __shfl_up(kb, 1);
+            ascending &= kb >= (l == 0 ? previous : left);
             before += __popcll(__ballot(kb < start * PANEL_KB));
+            previous = __builtin_amdgcn_readlane(kb, WAVE - 1);
         }
-        for (int p = l; p < n; p += WAVE) {
-            const BlockDesc d = p < WAVE ? first : blocks[begin + p];
-            const bool inside = kblock(d) < kblocks;                       // else the walk below would wait for a step that never comes
-            list[p >= before ? p - before : p + n - before] = inside ? (d.idx & 0xFFFFF) | kblock(d) << 20 : PANEL_NONE;
+        if (__ballot(!ascending) == 0ull) {
+            for (int p = l; p < n; p += WAVE) {
+                const BlockDesc d = p < WAVE ? first : blocks[begin + p];
+                const bool inside = kblock(d) < kblocks;                   // else the walk below would wait for a step that never comes
+                list[p >= before ? p - before : p + n - before] = inside ? (d.idx & 0xFFFFF) | kblock(d) << 20 : PANEL_NONE;
+            }
+        } else {                                                           // a table in another order: collected step by step
+            int there = 0;
+            for (int s = 0; s < steps; ++s) {
+                const int at = s + start < steps ? s + start : s + start - steps;
+                for (int p = 0; p < n; p += WAVE) {
+                    const BlockDesc d = p + l < n ? blocks[begin + p + l] : BlockDesc{0, -1};
+                    const bool here = p + l < n && kblock(d) < kblocks && kblock(d) / PANEL_KB == at;
+                    const unsigned long long all = __ballot(here);
+                    if (here) list[there + __popcll(all & ((1ull << l) - 1ull))] = (d.idx & 0xFFFFF) | kblock(d) << 20;
+                    there += __popcll(all);
+                }
+            }
+            n = there;
         }
     }
     n = __builtin_amdgcn_readfirstlane(n);

@@ -373,7 +373,8 @@ int bsa_attention_gradients(int dtype, const void *q, const void *k, const void 
 
 /* DDS with a weight that many dense rows meet: out = dense op(b), dense [batches, M, K] (K contiguous) and out
  * [batches, M, N] as in bsa_matmul(mode 2, tr_a = 0, tr_b), by a walk that keeps panels of the dense operand on the chip
- * for eight groups at a time (no schedule, no workspace).  Tables: the row table with tr_b, the column table without.
+ * for eight groups at a time (no schedule, no workspace).  Tables: the row table with tr_b, the column table without; the
+ * pairs of a group may stand in any order (they are walked in ascending order of the contraction).
  * With sparse_batches = 1 the batch is walked as one matrix of batches * M rows (any number of entries); with a weight
  * per entry at most 65535 of them.  fp16 / bf16; at most 2^20 - 1
  * blocks and a contraction of at most 1024 blocks (BSA_ERR_UNSUPPORTED otherwise: use bsa_matmul).

@@ -54,6 +54,28 @@ def test_panels(any_size, rows, cols, density, batch, m, trans_b, shared, dtype)
     assert _rel(got, want) <= REL[dtype]
 
 
+@pytest.mark.parametrize("rows,cols,density", [(5, 9, 0.7), (70, 9, 0.6), (9, 150, 0.9)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_pairs_of_a_group_in_any_order(any_size, rows, cols, density, trans_b):
+    """Tables are the caller's: a group's pairs reversed, and in random order."""
+    from sparse import _ops
+    L = _layout(rows, cols, density, rows)
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(2, 96, 32 * (cols if trans_b else rows), generator=g).half().cuda()
+    w = torch.randn(L.num_blocks, 32, 32, generator=g).half().cuda()
+    W = L.to_dense(w).double()
+    want = x.double().flatten(0, 1) @ (W.t().contiguous() if trans_b else W)
+    for order in (lambda n: torch.arange(n - 1, -1, -1), lambda n: torch.randperm(n, generator=g)):
+        tables = []
+        for blocks, offsets in (L.row_layout, L.col_layout):
+            pairs, ends = blocks.cpu().view(-1, 2), offsets.cpu().tolist()
+            pairs = torch.cat([pairs[i:j][order(j - i)] for i, j in zip(ends, ends[1:])])
+            tables.append((pairs.flatten().cuda(), offsets))
+        assert not torch.equal(tables[0][0], L.row_layout[0])
+        got = _ops.sparse_matmul(x, w, "dds", *tables, False, trans_b).flatten(0, 1)
+        assert _rel(got, want) <= REL[torch.float16]
+
+
 def test_more_batch_entries_than_a_grid_dimension_holds():
     import sparse
     from sparse import _ops
