@@ -26,12 +26,21 @@ __device__ __forceinline__ int xcd_contiguous(int total)
 constexpr int PANEL_WAVES = 8;                  // groups of a workgroup, one wave each
 constexpr int PANEL_KB = 4;                     // k-blocks of 32 per step
 constexpr int PANEL_RING = 4;                   // blocks of a wave in flight
-// panels in LDS at a time, and waves that do nothing but fetch them, one each: as many as a compute unit's 160 KB hold beside
-// the lists of the widest contraction
+// panels in LDS at a time: as many as a compute unit's 160 KB hold beside the lists of the widest contraction
 constexpr int panel_stages(int rt) { return rt <= 3 ? 4 : 3; }
-constexpr int panel_threads(int rt) { return 64 * (PANEL_WAVES + panel_stages(rt)); }
+constexpr int PANEL_FETCHERS = 3;               // waves that do nothing but fetch them
+constexpr int PANEL_HELPER = PANEL_WAVES + PANEL_FETCHERS;                 // the last wave, if there is one: half of the longest group
+constexpr int PANEL_THREADS = 64 * (PANEL_HELPER + 1);
 constexpr int PANEL_FLAGS = 64;                 // bytes in front of the lists: panels that are there, panels that are read
+constexpr int PANEL_LDS = 160 * 1024;
 constexpr int PANEL_NONE = -1;
+// Blocks that the set's longest chain must get shorter by, to pay for two barriers and the helper's sums through LDS.  us, a
+// column of the weight full, without the helper -> with it: a quarter and a tenth of 64 x 64 blocks, 4224 rows 28.0 -> 25.1 and
+// 25.8 -> 21.5, 5632 rows 39.7 -> 34.1 and 38.0 -> 30.2; 96 x 96, 8192 rows 80.7 -> 68.6; masks without one as they were (23.4 ->
+// 23.5, 19.2 -> 19.2, 64.6 -> 64.5).  Two or five helpers that go to the longest chains one by one: 1 us slower at one such
+// column, faster at two of a set (38.7 -> 36.7); half of the longest group to the wave of the shortest, with a second set of sums:
+// its registers spill.
+constexpr int PANEL_CUT_FROM = 8;
 __host__ __device__ constexpr int panel_list_length(int kblocks) { return (kblocks + 2 * PANEL_RING + 3) / 4 * 4; }
 
 // ---------------------------------------------------------------------------
@@ -40,8 +49,8 @@ __host__ __device__ constexpr int panel_list_length(int kblocks) { return (kbloc
 // dense [rows][KT] and out [rows][XT] of one batch entry, or of all of them as one matrix when the weight is shared.
 //   S_KC  the stored block is [x][k] (row groups): operands straight from memory
 //         otherwise [k][x] (column groups): through a wave-private LDS tile, read transposed
-// A wave per panel buffer requests panels straight into LDS, waits for them and says so in a flag; a multiplying wave waits
-// for the panel of its next block and says up to which panel it is done.  So the waits for panels are the fetching
+// Three waves request panels straight into LDS, wait for them and say so in a flag; a multiplying wave waits for the panel of
+// its next block and says up to which panel it is done.  So the waits for panels are the fetching
 // waves' alone, the other waves' stay exact for the blocks, of which a wave has its next four on the way, and no wave waits
 // for the fullest of the eight in every step, only for the slowest where it is a whole set of buffers ahead.
 //
@@ -50,11 +59,13 @@ __host__ __device__ constexpr int panel_list_length(int kblocks) { return (kbloc
 // barrier per step, 96 rows a workgroup -> fetching waves and a barrier per step, 160 rows -> flags -> operands of a block read
 // together: 4224 rows x 2048 x 2048 at a quarter of its blocks, forward 31.3 -> 26.0 -> 24.6 -> 23.7, gradient of the dense operand
 // 32.3 -> 24.5 -> 24.3 -> 22.8; 8192 x 3072 x 3072 at 0.3 107 -> 91 and 111 -> 84; every block stored, 4224 rows 56 -> 46 and 56 -> 41.
-// A group that has a block in every k-block makes its wave the chain: 4800 rows, 48 x 80 blocks, such a column: 26.7 -> 31.8, its
-// gradient 37.2 -> 22.1.
+// A group that has a block in every k-block makes its wave the chain; half of it goes to another wave (PANEL_CUT_FROM).  Launches of
+// two generations of workgroups in which that does not help are slower than two workgroups of eight waves a compute unit were: two such
+// columns among eight, 5632 rows 31.7 -> 38.6 (input gradient 32.5 -> 34.3); half and all of 48 x 80 blocks stored, 4800 rows 35.7 ->
+// 37.6 and 59.3 -> 60.4 (44 -> 30 and 69 -> 46).
 // ---------------------------------------------------------------------------
 template <int RT, bool S_KC, bool BF>
-__global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
+__global__ __launch_bounds__(PANEL_THREADS, 3) void weight_panel_kernel(
     const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
     const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
     int groups, int nnz, int rows, int KT, int XT, int sp_shared, int row_tiles, int group_sets)
@@ -65,16 +76,16 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
     if (item < 0) return;                                                  // whole workgroup leaves together
     const int tile = item / group_sets, set = item - tile * group_sets;
     const int batch = (int)blockIdx.y, w = wave_id(), l = lane_id();
-    const int y0 = tile * ROWS, g = set * PANEL_WAVES + w;
+    const int y0 = tile * ROWS, walkers = ((int)blockDim.x >> 6) - PANEL_FETCHERS;
     const int kblocks = KT / BS, steps = (kblocks + PANEL_KB - 1) / PANEL_KB;
     // Workgroups start at different steps: rows a multiple of 4 KB apart have their 256 bytes of a step in ONE of the 16
     // channels of an L2, and workgroups that walk the contraction in unison would all ask that channel.
     const int start = item % steps;
 
     half_t *privs = reinterpret_cast<half_t *>(lds_raw + STAGES * PANEL_BYTES);
-    int *flags = reinterpret_cast<int *>(lds_raw + STAGES * PANEL_BYTES + (S_KC ? 0 : PANEL_WAVES * BS2 * 2));
+    int *flags = reinterpret_cast<int *>(lds_raw + STAGES * PANEL_BYTES + (S_KC ? 0 : walkers * BS2 * 2));
     int *ready = flags, *done = flags + 4;       // of a buffer: panels up to and with the one in it; of a wave: panels it has done with
-    static_assert(STAGES <= 4 && 4 * (4 + PANEL_WAVES) <= PANEL_FLAGS, "flags");
+    static_assert(STAGES <= 4 && 4 * (4 + PANEL_WAVES + 1) <= PANEL_FLAGS, "flags");
     auto load_flag = [](const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
     auto store_flag = [](int *p, int v) {
         wave_lds_fence();
@@ -83,7 +94,33 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
     if (threadIdx.x < PANEL_FLAGS / 4) flags[threadIdx.x] = 0;
     lds_barrier();
 
-    if (w >= PANEL_WAVES) {
+    // Pairs of the set's groups, a lane each
+    int begins = 0, lengths = 0;
+    auto look_at_the_set = [&]() {
+        const int q = set * PANEL_WAVES + l % PANEL_WAVES;
+        begins = offsets[q < groups ? q : groups];
+        lengths = offsets[q + 1 < groups ? q + 1 : groups];
+    };
+    // Where the longest group is so by PANEL_CUT_FROM blocks and more, the helper takes half of its pairs, every second one: a
+    // group with a block in every k-block (a dense column of the weight) would keep a workgroup waiting for its one wave.
+    int longest = 0, half = 0;
+    auto pairs = [&](int from, int to) { return to <= from ? 0 : to - from < kblocks ? to - from : kblocks; };
+    auto find_the_longest = [&]() {
+        lengths = pairs(begins, lengths);
+        if (walkers == PANEL_WAVES || __ballot(lengths >= 2 * PANEL_CUT_FROM) == 0ull) return;
+        int most = 0, second = 0;
+#pragma unroll
+        for (int j = 0; j < PANEL_WAVES; ++j) {
+            const int n = __builtin_amdgcn_readlane(lengths, j);
+            second = n > most ? most : n > second ? n : second;
+            longest = n > most ? j : longest;
+            most = n > most ? n : most;
+        }
+        half = most / 2;
+        if (most - (second > most - half ? second : most - half) < PANEL_CUT_FROM) half = 0;
+    };
+
+    if (w >= PANEL_WAVES && w < PANEL_HELPER) {
         // Request r covers rows 4 r .. + 3, 16 pieces each; piece p of row y goes to slot p ^ (y & 15): 16 lanes that read one
         // piece of 16 rows meet no bank twice.  Lane l fills slot l % 16 of row 4 r + l / 16.  Requests behind the last row
         // repeat the last four (the rows of a launch are whole tiles of 32), pieces behind the last k-block the first: never
@@ -91,14 +128,15 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
         const int f = w - PANEL_WAVES;
         const unsigned char *dnb = reinterpret_cast<const unsigned char *>(dn + (size_t)batch * rows * KT + (size_t)y0 * KT);
         const int last = (rows - y0 < ROWS ? rows - y0 : ROWS) / 4 - 1;    // request of the last four rows
-        const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(lds_raw)) + (unsigned)f * PANEL_BYTES;
+        const unsigned lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds_raw));
         unsigned off[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) off[c] = 2u * (unsigned)((l >> 4) * KT) + 16u * (unsigned)((l & 15) ^ (4 * c + (l >> 4)));
         const int whole = KT / (BS * PANEL_KB), pieces = 16 - (steps * 16 - KT / 8);      // the last step may have fewer pieces
-        for (int s = f; s < steps; s += STAGES) {
+        for (int s = f; s < steps; s += PANEL_FETCHERS) {
             // the panel before in this buffer, s - STAGES, has been read by all
-            while (__ballot(l < PANEL_WAVES && load_flag(done + (l < PANEL_WAVES ? l : 0)) < s - STAGES + 1) != 0ull) __builtin_amdgcn_s_sleep(1);
+            while (__ballot(load_flag(done + (l < walkers ? l : 0)) < s - STAGES + 1) != 0ull) __builtin_amdgcn_s_sleep(1);
+            const unsigned to = lds0 + (unsigned)(s % STAGES) * PANEL_BYTES;
             int at = s + start;
             at = at < steps ? at : at - steps;
             unsigned o[4];
@@ -117,48 +155,70 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
                 }
             }
             tile_wait<0>();
-            if (l == 0) store_flag(ready + f, s + 1);
+            if (l == 0) store_flag(ready + s % STAGES, s + 1);
+        }
+        look_at_the_set();
+        find_the_longest();
+        if (half > 0) {                          // the barriers at the end of the others
+            lds_barrier();
+            lds_barrier();
         }
         return;
     }
 
     // The group's pairs, in the order in which the steps come: block | k-block << 20, then PANEL_NONE
-    half_t *priv = privs + w * BS2;
-    int *list = flags + PANEL_FLAGS / 4 + w * panel_list_length(kblocks);
-    int n = 0;
-    if (g < groups) {
-        const int begin = offsets[g];
-        n = offsets[g + 1] - begin;
-        n = n < 0 ? 0 : n < kblocks ? n : kblocks;
-        auto kblock = [&](const BlockDesc &d) { return S_KC ? d.col() : d.row(); };
-        const BlockDesc first = l < n ? blocks[begin + l] : BlockDesc{0, -1};
+    const bool helper = w == PANEL_HELPER;
+    const int slot = helper ? PANEL_WAVES : w;
+    half_t *priv = privs + slot * BS2;
+    int *list = flags + PANEL_FLAGS / 4 + slot * panel_list_length(kblocks);
+    auto kblock = [&](const BlockDesc &d) { return S_KC ? d.col() : d.row(); };
+    look_at_the_set();
+    int g = set * PANEL_WAVES + w, begin = 0, length = 0;
+    BlockDesc first = {0, -1};                                             // pair l of the group
+    if (!helper) {
+        begin = offsets[g < groups ? g : groups];
+        length = pairs(begin, offsets[g + 1 < groups ? g + 1 : groups]);
+        if (l < length) first = blocks[begin + l];
+    }
+    find_the_longest();
+    if (helper && half > 0) {
+        g = set * PANEL_WAVES + longest;
+        begin = __builtin_amdgcn_readlane(begins, longest);
+        length = __builtin_amdgcn_readlane(lengths, longest);
+        if (l < length) first = blocks[begin + l];
+    }
+    const int apart = half > 0 && g == set * PANEL_WAVES + longest ? 1 : 0;                   // the wave's pairs: all, or the even or the odd ones
+    const int n_own = !apart ? length : helper ? half : length - half;
+    int n = n_own;
+    {
+        auto mine = [&](int p) { return p < length && ((p & apart) != 0) == (helper && apart); };
         int before = 0, previous = -1;                                     // pairs of steps that come around again; the lane before this one's
         bool ascending = true;
-        for (int p = 0; p < n; p += WAVE) {
-            const int kb = p + l >= n ? kblocks : kblock(p == 0 ? first : blocks[begin + p + l]), left = __shfl_up(kb, 1);
+        for (int p = 0; p < length; p += WAVE) {
+            const int kb = p + l >= length ? kblocks : kblock(p == 0 ? first : blocks[begin + p + l]), left = __shfl_up(kb, 1);
             ascending &= kb >= (l == 0 ? previous : left);
-            before += __popcll(__ballot(kb < start * PANEL_KB));
+            before += __popcll(__ballot(mine(p + l) && kb < start * PANEL_KB));
             previous = __builtin_amdgcn_readlane(kb, WAVE - 1);
         }
         if (__ballot(!ascending) == 0ull) {
-            for (int p = l; p < n; p += WAVE) {
+            for (int p = l; p < length; p += WAVE) {
                 const BlockDesc d = p < WAVE ? first : blocks[begin + p];
                 const bool inside = kblock(d) < kblocks;                   // else the walk below would wait for a step that never comes
-                list[p >= before ? p - before : p + n - before] = inside ? (d.idx & 0xFFFFF) | kblock(d) << 20 : PANEL_NONE;
+                const int q = p >> apart;
+                if (mine(p)) list[q >= before ? q - before : q + n_own - before] = inside ? (d.idx & 0xFFFFF) | kblock(d) << 20 : PANEL_NONE;
             }
         } else {                                                           // a table in another order: collected step by step
-            int there = 0;
+            n = 0;
             for (int s = 0; s < steps; ++s) {
                 const int at = s + start < steps ? s + start : s + start - steps;
-                for (int p = 0; p < n; p += WAVE) {
-                    const BlockDesc d = p + l < n ? blocks[begin + p + l] : BlockDesc{0, -1};
-                    const bool here = p + l < n && kblock(d) < kblocks && kblock(d) / PANEL_KB == at;
+                for (int p = 0; p < length; p += WAVE) {
+                    const BlockDesc d = p + l < length ? blocks[begin + p + l] : BlockDesc{0, -1};
+                    const bool here = mine(p + l) && kblock(d) < kblocks && kblock(d) / PANEL_KB == at;
                     const unsigned long long all = __ballot(here);
-                    if (here) list[there + __popcll(all & ((1ull << l) - 1ull))] = (d.idx & 0xFFFFF) | kblock(d) << 20;
-                    there += __popcll(all);
+                    if (here) list[n + __popcll(all & ((1ull << l) - 1ull))] = (d.idx & 0xFFFFF) | kblock(d) << 20;
+                    n += __popcll(all);
                 }
             }
-            n = there;
         }
     }
     n = __builtin_amdgcn_readfirstlane(n);
@@ -200,7 +260,7 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
     const unsigned char *panel = lds_raw + 256 * i;                        // row i of it
     auto walk_to = [&](int s) {
         if (s == step) return;
-        if (l == 0) store_flag(done + w, s);                               // the reads before it are in front of it in LDS order
+        if (l == 0) store_flag(done + slot, s);                             // the reads before it are in front of it in LDS order
         const int buffer = s % STAGES;
         while (__builtin_amdgcn_readfirstlane(load_flag(ready + buffer)) < s + 1) __builtin_amdgcn_s_sleep(1);
         wave_lds_fence();
@@ -245,9 +305,26 @@ __global__ __launch_bounds__(panel_threads(RT), 3) void weight_panel_kernel(
             now[j] = next[j];
         }
     }
-    if (l == 0) store_flag(done + w, steps);
+    if (l == 0) store_flag(done + slot, steps);
+    if (half > 0) {                              // the helper's sums go back through LDS, where all panels have been read
+        f4v *parts = reinterpret_cast<f4v *>(lds_raw) + l;
+        lds_barrier();
+        if (helper) {
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) parts[WAVE * (4 * t + v)] = f4v{acc[t][4 * v], acc[t][4 * v + 1], acc[t][4 * v + 2], acc[t][4 * v + 3]};
+        }
+        lds_barrier();
+        if (apart) {
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[t][v] += parts[WAVE * (4 * t + v / 4)][v % 4];
+        }
+    }
 
-    if (g < groups) {
+    if (!helper && g < groups) {
         half_t *ob = out + (size_t)batch * rows * XT + BS * g + 16 * h;
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
@@ -429,8 +506,11 @@ static hipError_t launch_panel(const WeightPanelArgs &p, hipStream_t st)
 {
     constexpr int ROWS = 32 * RT;
     const int tiles = (p.rows + ROWS - 1) / ROWS, sets = (p.groups + PANEL_WAVES - 1) / PANEL_WAVES;
-    const size_t lds = panel_stages(RT) * ROWS * 256 + (S_KC ? 0 : PANEL_WAVES * BS2 * 2) +
-                       PANEL_FLAGS + (size_t)PANEL_WAVES * panel_list_length(p.KT / BS) * sizeof(int);
+    auto lds_of = [&](int walkers) {
+        return panel_stages(RT) * ROWS * 256 + PANEL_FLAGS + walkers * ((S_KC ? 0 : BS2 * 2) + (size_t)panel_list_length(p.KT / BS) * sizeof(int));
+    };
+    const int walkers = PANEL_WAVES + (lds_of(PANEL_WAVES + 1) <= PANEL_LDS ? 1 : 0);
+    const size_t lds = lds_of(walkers);
     auto kernel = weight_panel_kernel<RT, S_KC, BF>;
     if (lds > 65536) {
         hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -438,7 +518,7 @@ static hipError_t launch_panel(const WeightPanelArgs &p, hipStream_t st)
         if (err != hipSuccess) return err;
     }
     dim3 grid((unsigned)((tiles * sets + 7) / 8 * 8), (unsigned)p.batches);
-    kernel<<<grid, panel_threads(RT), lds, st>>>(
+    kernel<<<grid, 64 * (walkers + PANEL_FETCHERS), lds, st>>>(
         (const half_t *)p.sparse, (const half_t *)p.dense, (half_t *)p.out, (const BlockDesc *)p.blocks, p.offsets, p.groups, p.nnz,
         p.rows, p.KT, BS * p.groups, p.sparse_shared ? 1 : 0, tiles, sets);
     return hipGetLastError();

@@ -76,6 +76,38 @@ def test_pairs_of_a_group_in_any_order(any_size, rows, cols, density, trans_b):
         assert _rel(got, want) <= REL[torch.float16]
 
 
+# A second wave takes half of a set's longest group where the longest chain gets shorter by 8 blocks: by 7, 8 and 2 of them, beside
+# empty groups, more pairs than a wave has lanes, several long groups in a set, the last set incomplete, rows that end inside a
+# tile; each with the pairs of the table ascending and descending
+@pytest.mark.parametrize("k,groups,long,short,m", [
+    (16, 8, (15,), 0, 224), (16, 8, (16,), 0, 224), (21, 9, (17, 19), 4, 224), (70, 9, (70, 1, 33), 7, 224), (150, 21, (150, 150, 64), 66, 96), (41, 8, (41, 41, 40, 39), 9, 96),
+    (41, 13, (41, 30), 9, 9312), (150, 16, (150, 149, 3), 11, 9312)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_long_group_is_cut(any_size, k, groups, long, short, m, trans_b, dtype):
+    import sparse
+    from sparse import _ops
+    g = torch.Generator().manual_seed(k)
+    mask = torch.zeros(groups, k, dtype=torch.long)
+    for r in range(groups):
+        length = long[r // 2] if r % 2 == 1 and r // 2 < len(long) else short
+        mask[r, torch.randperm(k, generator=g)[:length]] = 1
+    L = sparse.SparseLayout((mask if trans_b else mask.t().contiguous()).cuda())
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(1, m, 32 * k, generator=g, device="cuda").to(dtype)
+    w = torch.randn(L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
+    W = L.to_dense(w).double()
+    want = x[0].double() @ (W.t().contiguous() if trans_b else W)
+    walked = L.row_layout if trans_b else L.col_layout
+    pairs, ends = walked[0].cpu().view(-1, 2), walked[1].cpu().tolist()
+    turned = torch.cat([pairs[i:j].flip(0) for i, j in zip(ends, ends[1:])]).flatten().cuda()
+    for table in (walked, (turned, walked[1])):
+        tables = (table, L.col_layout) if trans_b else (L.row_layout, table)
+        got = _ops.sparse_matmul(x, w, "dds", *tables, False, trans_b)[0]
+        assert _rel(got, want) <= REL[dtype]
+        assert (got - want).abs().max() <= 8 * REL[dtype] * want.abs().max()
+
+
 def test_more_batch_entries_than_a_grid_dimension_holds():
     import sparse
     from sparse import _ops
