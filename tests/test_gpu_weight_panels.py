@@ -191,23 +191,32 @@ def test_layer_captured_at_a_size_that_never_ran():
             assert _rel(a, b.double()) <= 4 * REL[torch.float16]
 
 
-# Launches of 64, 96, 128 and 160 rows a workgroup (the fewest generations of 256 workgroups), each with a tile that is cut; a
-# contraction that ends inside a step, a group with a block in every k-block beside empty ones, more k-blocks than a wave has lanes
-@pytest.mark.parametrize("rows,cols,density,batch,m", [
-    (5, 9, 0.7, 33, 32), (6, 70, 0.3, 31, 96), (70, 9, 0.3, 127, 160), (7, 16, 0.5, 255, 96), (66, 24, 0.2, 253, 96)])
+def _row_tiles(groups, kblocks, rows):
+    """Tiles of 32 rows a workgroup takes: the fewest generations of 256 workgroups, a tile's worth of start and end each."""
+    sets = -(-groups // 8)
+    cost = lambda t: -(-(-(-rows // (32 * t)) * sets) // 256) * (t + 1)
+    return min(range(2, 6 if kblocks <= 700 else 5), key=cost)
+
+
+# Launches of 64, 96, 128 and 160 rows a workgroup, the last tile a row of 32 short; a contraction that ends inside a step, a
+# group with a block in every k-block beside empty ones, more k-blocks than a wave has lanes, as many as leave no room for the helper
+# beside 160 rows
+@pytest.mark.parametrize("tiles", [2, 3, 4, 5])
+@pytest.mark.parametrize("k,groups,density", [(9, 70, 0.3), (70, 9, 0.3), (33, 16, 0.5), (690, 3, 0.1)])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_panel_heights(any_size, rows, cols, density, batch, m, trans_b, dtype):
+def test_panel_heights(any_size, tiles, k, groups, density, trans_b, dtype):
     import sparse
     from sparse import _ops
-    g = torch.Generator().manual_seed(rows)
-    mask = (torch.rand(rows, cols, generator=g) < density).long()
-    mask[:, 1] = 1
-    mask[:, 2] = 0
-    L = sparse.SparseLayout(mask.cuda())
-    k = 32 * (cols if trans_b else rows)
-    g = torch.Generator(device="cuda").manual_seed(m)
-    x = torch.randn(batch, m, k, generator=g, device="cuda").to(dtype)
+    g = torch.Generator().manual_seed(k)
+    mask = (torch.rand(groups, k, generator=g) < density).long()
+    mask[1] = 1
+    mask[2] = 0
+    L = sparse.SparseLayout((mask if trans_b else mask.t().contiguous()).cuda())
+    batch = tiles * (256 // -(-groups // 8)) - 1
+    assert _row_tiles(groups, k, 32 * batch) == tiles and batch % tiles
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    x = torch.randn(batch, 32, 32 * k, generator=g, device="cuda").to(dtype)
     w = torch.randn(L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
     W = L.to_dense(w).double()
     got = _ops.sparse_matmul(x, w, "dds", L.row_layout, L.col_layout, False, trans_b).flatten(0, 1)
