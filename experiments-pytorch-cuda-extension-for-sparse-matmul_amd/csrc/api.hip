@@ -47,7 +47,7 @@ int check_schedule(const int32_t *sched, int sched_wgs, int sched_waves, int bat
 
 extern "C" {
 
-int bsa_version(void) { return 100; }
+int bsa_version(void) { return BSA_VERSION; }
 
 const char *bsa_last_error(void) { return g_error; }
 

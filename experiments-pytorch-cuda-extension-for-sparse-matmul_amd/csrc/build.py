@@ -29,17 +29,22 @@ FLAGS = [
 ]
 
 
+def _older(path, sources) -> bool:
+    return not os.path.exists(path) or any(os.path.getmtime(os.path.join(HERE, f)) > os.path.getmtime(path) for f in sources)
+
+
 def out_of_date() -> bool:
-    if not all(os.path.exists(path) for path in [LIB, HOST_CALLS] + [path for path, _ in CHECK_VARIANTS.values()]):
-        return True
-    t = os.path.getmtime(LIB)
-    return any(os.path.getmtime(os.path.join(HERE, f)) > t for f in SOURCES + HEADERS + ["host_calls.cpp", "build.py"])
+    libraries = [LIB] + [path for path, _ in CHECK_VARIANTS.values()]
+    return any(_older(path, SOURCES + HEADERS + ["build.py"]) for path in libraries) or \
+        _older(HOST_CALLS, ["host_calls.cpp", "build.py", os.path.join("..", "..", "include", "bsa.h")])
 
 
 def build(force: bool = False, verbose: bool = False, extra_flags=(), lib: str = LIB) -> str:
     """Compiles every source to an object file (in parallel, one hipcc each) and links them."""
     if not force and lib == LIB and not out_of_date():
         return LIB
+    if lib == LIB and os.path.exists(HOST_CALLS):
+        os.remove(HOST_CALLS)                   # it calls the library by address: none is better than one of another build
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     objdir = os.path.join(HERE, "build", os.path.basename(lib))
     os.makedirs(objdir, exist_ok=True)
@@ -111,7 +116,7 @@ def build_host_calls(verbose: bool = False) -> str:
     include = [os.path.join(home, "include"), os.path.join(home, "include", "torch", "csrc", "api", "include"),
                sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DBSA_TORCH_VERSION="{torch.__version__}"']
     cmd += [flag for path in include for flag in ("-isystem", path)]
     cmd += [os.path.join(HERE, "host_calls.cpp"), "-o", HOST_CALLS, "-L" + os.path.join(home, "lib")]
     cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]

@@ -778,6 +778,11 @@ PyObject *setup(PyObject *, PyObject *args)
         fn = reinterpret_cast<std::decay_t<decltype(fn)>>(x ? PyLong_AsUnsignedLongLong(x) : 0);
         if (fn == nullptr && !PyErr_Occurred()) PyErr_Format(PyExc_KeyError, "%s", name);
     };
+    decltype(&bsa_version) version = nullptr;
+    address("bsa_version", version);
+    if (version != nullptr && version() != BSA_VERSION)
+        PyErr_Format(PyExc_ImportError, "bsa_host_calls.so was built for version %d of the library, which is %d: build both", BSA_VERSION, version());
+    if (PyErr_Occurred()) return nullptr;
     address("bsa_matmul", lib.matmul);
     address("bsa_matmul_dsd_runs", lib.runs);
     address("bsa_matmul_dds_panels", lib.panels);
@@ -834,4 +839,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "bsa_host_calls", nullptr, -1, meth
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_bsa_host_calls() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_bsa_host_calls()
+{
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", BSA_TORCH_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

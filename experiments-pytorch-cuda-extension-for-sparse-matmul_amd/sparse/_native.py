@@ -6,7 +6,7 @@ from .attention import SparseAttention
 from .matmul import SparseMatMul
 from .softmax import SparseSoftmax
 
-_ENTRIES = ("bsa_matmul", "bsa_matmul_dsd_runs", "bsa_matmul_dds_panels", "bsa_weight_grad", "bsa_softmax_forward",
+_ENTRIES = ("bsa_version", "bsa_matmul", "bsa_matmul_dsd_runs", "bsa_matmul_dds_panels", "bsa_weight_grad", "bsa_softmax_forward",
             "bsa_softmax_backward", "bsa_attention_forward", "bsa_attention_gradients")
 
 

@@ -92,6 +92,8 @@ def load_host_calls():
                                                   loader=importlib.machinery.ExtensionFileLoader("bsa_host_calls", path))
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
+    if module.torch_version != torch.__version__:        # it uses torch's C++ interface, which no two versions share
+        raise ImportError(f"{path} was built for torch {module.torch_version}, this is {torch.__version__}: build it again")
     return module
 
 

@@ -57,7 +57,8 @@ enum bsa_status {
     BSA_ERR_UNSUPPORTED = -3
 };
 
-/* Library version, major * 10000 + minor * 100 + patch. */
+/* Library version, major * 10000 + minor * 100 + patch; the one these declarations are of. */
+#define BSA_VERSION 100
 int bsa_version(void);
 
 /* Message of the last failure on this thread ("" if none). Never NULL. */
