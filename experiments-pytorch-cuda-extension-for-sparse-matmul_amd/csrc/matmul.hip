@@ -1156,6 +1156,7 @@ static hipError_t launch_sdd_f16(const MatmulArgs &p, hipStream_t st)
     return hipGetLastError();
 }
 
+constexpr long long SDD_F32_SPLIT_BLOCKS = 3000;                           // of all batch entries together
 template <bool A_KC, bool B_KC>
 static hipError_t launch_sdd_f32(const MatmulArgs &p, hipStream_t st)
 {
@@ -1173,9 +1174,15 @@ static hipError_t launch_sdd_f32(const MatmulArgs &p, hipStream_t st)
             kernel<<<grid, block, lds, st>>>(BSA_SDD_ARGS);
             return hipGetLastError();
         };
-        // With less than a block for each of the 1024 SIMDs nothing overlaps, and the fp32 instruction is the shorter chain:
-        // 80 blocks 4.4 us against 4.7 split, 744 4.2 against 4.5, 1012 6.2 against 5.7.
-        if ((long long)p.nnz * p.batches < 800) {
+        // Three blocks for each of the 1024 SIMDs: below, little overlaps, the fp32 instruction is the shorter chain, and the split
+        // waits for its operands' parts.  us, k = 64 / 96 / 128, both operands with k contiguous, fp32 instruction in chunks of one
+        // block -> split in chunks of one, of four: 814 blocks 5.5 -> 5.4, - / 6.5 -> 6.8, - / 7.9 -> 8.5, -; 2368 8.2 -> 8.3, 8.8 / 10.5 ->
+        // 10.8, 11.4 / 12.8 -> 13.2, 13.8; 3552 10.3 -> 10.2, 9.3 / 14.3 -> 14.8, 12.5 / 16.5 -> 17.7, 14.7; 7104 16.0 -> 16.1, 12.8 / 24.4 ->
+        // 24.6, 20.2 / 29.1 -> 30.2, 26.9.  At k = 32 a block is half the work: twice as many; both operands contiguous are split with
+        // few instructions and pay from 1500 blocks (1776 5.2 -> 4.9, 2368 6.0 -> 5.5, 4736 7.9 -> 7.5), neither so does not at 3552, 6.2 ->
+        // 7.5, 6.9, nor 5920, 8.5 -> 10.2, 8.6.
+        const long long all = (long long)p.nnz * p.batches;
+        if (kbs > 1 ? all < SDD_F32_SPLIT_BLOCKS : all < (A_KC && B_KC ? SDD_F32_SPLIT_BLOCKS / 2 : 2 * SDD_F32_SPLIT_BLOCKS)) {
             switch (kbs) {
                 case 1: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 1, false>);
                 case 2: return launch(sdd_f32_tiled_kernel<A_KC, B_KC, 2, false>);

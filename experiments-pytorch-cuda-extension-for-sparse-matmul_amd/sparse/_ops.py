@@ -18,12 +18,13 @@ SCHEDULE_GROUP_WALK = (12, 4, True, -1, 2, True)        # groups of at most GROU
 SCHEDULE_GROUP_WALK_LONG = (10, 4, True, -1, 2, True)    # tables with longer groups (columns of causal / strided masks)
 GROUP_WALK_LONG = 24
 SCHEDULE_SDD = (4, 2)
-# fp32: a wave splits its row's operands once, so chunks pay where the launch fills the machine with them; below, one block a
-# wave is the shorter chain.  us, chunks of 1 in 4 waves -> of 4 in 2: 1012 blocks 5.7 -> 7.9, 8096 16.2 -> 15.2, 10144 (window
-# of 5) 22.3 -> 17.0, 24480 42.9 -> 36.0, 73440 123.6 -> 95.3.
+# fp32: a wave splits its row's operands into bf16 parts once, so chunks pay where the products are split: from as many blocks on as
+# bsa_matmul splits them (SDD_F32_SPLIT_BLOCKS in csrc/matmul.hip, with both sides' times).  us, the fp32 instruction in chunks of 1
+# in 4 waves -> split in chunks of 4 in 2, k = 64: 1012 blocks 6.2 -> 7.9, 2368 8.2 -> 8.8, 3552 10.3 -> 9.3, 8096 18.6 -> 15.0,
+# 24480 46.5 -> 38, 73440 120 -> 98.
 SCHEDULE_SDD_F32 = (1, 4)
 SCHEDULE_SDD_F32_LARGE = (4, 2)
-SDD_F32_LARGE_BLOCKS = 8000            # of all batch entries together
+SDD_F32_LARGE_BLOCKS = 3000            # of all batch entries together, at k = 64 and more
 # fp32 groups of at most GROUP_WALK_LONG pairs: chunks of 6 in 4 waves hold such a group in one workgroup too.  us, chunks of 12
 # -> 6 (DSD): 744 blocks 13.6 -> 11.2, 1012 19.7 -> 12.8, 8096 25.2 -> 20.3, 11912 29.4 -> 24.6, 73440 114 -> 114.
 SCHEDULE_GROUP_WALK_F32 = (6, 4, True, -1, 2, True)
@@ -314,10 +315,10 @@ def _group_walk_schedule(layout, dtype=torch.float16):
     return schedule_for(layout, kind)
 
 
-def _sdd_schedule(layout, dtype, batches):
+def _sdd_schedule(layout, dtype, batches, k):
     if dtype != torch.float32:
         return schedule_for(layout, SCHEDULE_SDD)
-    if layout[0].numel() * batches >= 2 * SDD_F32_LARGE_BLOCKS:
+    if layout[0].numel() // 2 * batches * min(k, 64) >= 64 * SDD_F32_LARGE_BLOCKS:
         return _schedule_or(layout, SCHEDULE_SDD_F32_LARGE, SCHEDULE_SDD_F32)
     return _schedule_or(layout, SCHEDULE_SDD_F32, SCHEDULE_SDD_F32_LARGE)
 
@@ -498,7 +499,7 @@ def _matmul_route(a, b, mode, row_layout, col_layout, trans_a, trans_b):
         return route("panels")
 
     if mode == "sdd":
-        return route("walk", _sdd_schedule(layout, a.dtype, batches))
+        return route("walk", _sdd_schedule(layout, a.dtype, batches, size_k))
     return route("walk", _group_walk_schedule(layout, a.dtype))
 
 

@@ -25,7 +25,7 @@ def _want(a, b, layout):
     return tiles[:, pos[:, 0], pos[:, 1]]
 
 
-def _operands(k, seed=0, batch=16):              # enough blocks for the split products
+def _operands(k, seed=0, batch=80):              # enough blocks for the split products
     g = torch.Generator().manual_seed(seed)
     return (torch.randn(batch, 32 * MASK.shape[0], k, generator=g).cuda(), torch.randn(batch, k, 32 * MASK.shape[1], generator=g).cuda())
 
@@ -39,7 +39,7 @@ def test_error_against_float64(k, trans_a, trans_b, chunks, monkeypatch):
     monkeypatch.setattr(_ops, "SDD_F32_LARGE_BLOCKS", chunks)
     L = sparse.SparseLayout(torch.as_tensor(MASK))
     a, b = _operands(k)
-    assert L.num_blocks * a.size(0) >= 800
+    assert L.num_blocks * a.size(0) * min(k, 64) >= 64 * 3000
     got = _product(a, b, trans_a, trans_b, L).cpu().double()
     # Of a product |a b| the dropped terms are at most 4 2^-26; an instruction sums 16 products to 2^-23 of the largest and
     # rounds once into the accumulator, 6 times for 16 steps of k.
@@ -54,7 +54,7 @@ def test_operands_that_three_parts_cannot_hold(value):
     import sparse
     L = sparse.SparseLayout(torch.as_tensor(MASK))
     a, b = _operands(64, seed=3)
-    assert L.num_blocks * a.size(0) >= 800
+    assert L.num_blocks * a.size(0) >= 3000
     if abs(value) < 1e-30:                       # a whole operand of them: all results are small
         a = a.sign() * value
     else:
@@ -79,7 +79,7 @@ def test_small_operands_beside_large_and_ordinary_ones(small, large, where, swap
     import sparse
     L = sparse.SparseLayout(torch.as_tensor(MASK))
     x, y = _operands(k, seed=5)
-    assert L.num_blocks * x.size(0) >= 800
+    assert L.num_blocks * x.size(0) * min(k, 64) >= 64 * 3000
     x, y = (y.transpose(1, 2).contiguous(), x.transpose(1, 2).contiguous()) if swapped else (x, y)      # x [.., tokens, k] is the small one
     if where == "all":
         x, y = x * small, y * large
