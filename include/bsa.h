@@ -167,6 +167,8 @@ int bsa_schedule_build(const int32_t *offsets, int groups, int cap, int waves,
  *   every launch leaves it zero again, so it can be reused by later launches
  *   on the same stream (launches that overlap in time need separate ones).
  *   SDD takes no workspace (null, 0).
+ *   fp32 SDD with K <= 128 changes its matrix instruction at 3000 blocks of all entries (K = 32: 1500 or 6000, by the operands'
+ *   orders): an entry has the same bits in every launch on one side of that line.
  *   sparse_batches is `batches`, or 1 (DSD / DDS only) when ONE sparse operand [nnz, 32, 32] serves
  *   every batch entry (a block-sparse weight); the reference has no such case.
  * fp16 and bf16 accumulate in fp32.  Empty groups give zero rows / columns.
