@@ -323,11 +323,20 @@ bool plain_thread()
 }
 hipStream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// Whether Python would make a plan of a call on these operands (_ops._plans): to ask takes 2 us
+bool plannable(std::initializer_list<const Tensor *> operands)
+{
+    for (const Tensor *t : operands)
+        if (!at_16_bytes(*t)) return false;
+    return !capturing();
+}
+
 // The plan of a call on these operands, if the call can go by one here and now
 Found find_plan(Plans &plans, int op, int flags, const Tensor &a, const Tensor &b)
 {
     Found p = plans.find(op, flags, a, b, current_stream());
-    if (p && p->space && c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return Found();
+    if (p && p->space && capturing()) return Found();
     return p;
 }
 void check(int status, Plans &plans, const Found &p)
@@ -385,16 +394,19 @@ Tensor unwrap_new(PyObject *result)          // steals
 Tensor product(Plans &plans, PyObject *layout, const Tensor &a, const Tensor &b, int mode, bool ta, bool tb)
 {
     const int flags = mode << 2 | ta << 1 | tb;
-    Found p = plain(a) && plain(b) && on_current_device(a) ? find_plan(plans, MATMUL, flags, a, b) : Found();
+    const bool direct = plain(a) && plain(b) && on_current_device(a);
+    Found p = direct ? find_plan(plans, MATMUL, flags, a, b) : Found();
     if (!p || (p->aligned && !(at_16_bytes(a) && at_16_bytes(b)))) {
         py::gil_scoped_acquire gil;
         Borrow pa(a), pb(b);
-        PyObject *made = PyObject_CallFunctionObjArgs(python.plan_matmul, pa.get(), pb.get(), python.modes[mode], layout, py_bool(ta), py_bool(tb),
-                                                      nullptr);
-        if (made == nullptr) raise_pending();
-        const bool planned = made == Py_True;
-        Py_DECREF(made);
-        p = planned && plain(a) && plain(b) && on_current_device(a) ? find_plan(plans, MATMUL, flags, a, b) : Found();
+        if (direct && plannable({&a, &b})) {
+            PyObject *made = PyObject_CallFunctionObjArgs(python.plan_matmul, pa.get(), pb.get(), python.modes[mode], layout, py_bool(ta),
+                                                          py_bool(tb), nullptr);
+            if (made == nullptr) raise_pending();
+            const bool planned = made == Py_True;
+            Py_DECREF(made);
+            p = planned ? find_plan(plans, MATMUL, flags, a, b) : Found();
+        }
         if (!p || (p->aligned && !(at_16_bytes(a) && at_16_bytes(b))))
             return unwrap_new(PyObject_CallFunctionObjArgs(python.run_matmul, pa.get(), pb.get(), python.modes[mode], layout, py_bool(ta),
                                                            py_bool(tb), nullptr));
@@ -412,11 +424,13 @@ Tensor weight_gradient(Plans &plans, PyObject *layout, const Tensor &a, const Te
     if (!p) {
         py::gil_scoped_acquire gil;
         Borrow pa(a), pb(b);
-        PyObject *made = PyObject_CallFunctionObjArgs(python.plan_weight, pa.get(), pb.get(), layout, py_bool(ta), py_bool(tb), nullptr);
-        if (made == nullptr) raise_pending();
-        const bool planned = made == Py_True;
-        Py_DECREF(made);
-        p = planned ? by_plan() : Found();
+        if (plain(a) && plain(b) && plannable({&a, &b})) {
+            PyObject *made = PyObject_CallFunctionObjArgs(python.plan_weight, pa.get(), pb.get(), layout, py_bool(ta), py_bool(tb), nullptr);
+            if (made == nullptr) raise_pending();
+            const bool planned = made == Py_True;
+            Py_DECREF(made);
+            p = planned ? by_plan() : Found();
+        }
         if (!p)
             return unwrap_new(PyObject_CallFunctionObjArgs(python.run_weight, pa.get(), pb.get(), layout, py_bool(ta), py_bool(tb), nullptr));
     }
@@ -499,11 +513,13 @@ struct SoftmaxNode : public Node {
         if (!p) {
             py::gil_scoped_acquire gil;
             Borrow py_y(y), py_dy(dy);
-            PyObject *made = PyObject_CallFunctionObjArgs(python.plan_softmax_backward, py_y.get(), layout->object, nullptr);
-            if (made == nullptr) raise_pending();
-            const bool planned = made == Py_True;
-            Py_DECREF(made);
-            p = planned ? by_plan() : Found();
+            if (plain(y) && plannable({&y})) {
+                PyObject *made = PyObject_CallFunctionObjArgs(python.plan_softmax_backward, py_y.get(), layout->object, nullptr);
+                if (made == nullptr) raise_pending();
+                const bool planned = made == Py_True;
+                Py_DECREF(made);
+                p = planned ? by_plan() : Found();
+            }
             if (!p) {
                 py::object s = py::float_(scale);
                 return {unwrap_new(PyObject_CallFunctionObjArgs(python.run_softmax_backward, py_y.get(), py_dy.get(), layout->object, s.ptr(), nullptr))};
@@ -551,11 +567,13 @@ struct AttentionNode : public Node {
         if (!p) {
             py::gil_scoped_acquire gil;
             Borrow pq(q), pk(k), pv(v), pd(dout), po(out), pl(lse);
-            PyObject *made = PyObject_CallFunctionObjArgs(python.plan_attention_backward, pq.get(), pk.get(), pv.get(), layout->object, py_bool(dkdv), nullptr);
-            if (made == nullptr) raise_pending();
-            const bool planned = made == Py_True;
-            Py_DECREF(made);
-            p = planned ? by_plan() : Found();
+            if (plain(q) && plain(k) && plain(v) && plannable({&q, &k, &v})) {
+                PyObject *made = PyObject_CallFunctionObjArgs(python.plan_attention_backward, pq.get(), pk.get(), pv.get(), layout->object, py_bool(dkdv), nullptr);
+                if (made == nullptr) raise_pending();
+                const bool planned = made == Py_True;
+                Py_DECREF(made);
+                p = planned ? by_plan() : Found();
+            }
             if (!p) {
                 py::object s = py::float_(scale);
                 PyObject *got = PyObject_CallFunctionObjArgs(python.run_attention_backward, pq.get(), pk.get(), pv.get(), pd.get(), po.get(), pl.get(),
@@ -636,7 +654,7 @@ PyObject *matmul(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     if (plans == nullptr) return general(python.matmul, args, nargs);
     const int flags = mode << 2 | ta << 1 | tb;
     Found p = find_plan(*plans, MATMUL, flags, a, b);
-    if (!p) {
+    if (!p && plannable({&a, &b})) {
         PyObject *made = PyObject_CallFunctionObjArgs(python.plan_matmul, args[0], args[1], args[2], args[3], py_bool(ta), py_bool(tb), nullptr);
         if (made == nullptr) return nullptr;
         const bool planned = made == Py_True;
@@ -679,7 +697,7 @@ PyObject *softmax(PyObject *, PyObject *const *args, Py_ssize_t nargs)      // x
     const double scale = PyFloat_AsDouble(args[2]);
     if (scale == -1.0 && PyErr_Occurred()) return nullptr;
     Found p = find_plan(*plans, SOFTMAX_FORWARD, 0, x, Tensor());
-    if (!p) {
+    if (!p && plannable({&x})) {
         PyObject *made = PyObject_CallFunctionObjArgs(python.plan_softmax, args[0], args[1], nullptr);
         if (made == nullptr) return nullptr;
         const bool planned = made == Py_True;
@@ -728,7 +746,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs)    // q
     const double scale = PyFloat_AsDouble(args[4]);
     if (scale == -1.0 && PyErr_Occurred()) return nullptr;
     Found p = find_plan(*plans, ATTENTION_FORWARD, 0, q, k);
-    if (!p) {
+    if (!p && plannable({&q, &k, &v})) {
         PyObject *made = PyObject_CallFunctionObjArgs(python.plan_attention, args[0], args[1], args[2], args[3], nullptr);
         if (made == nullptr) return nullptr;
         const bool planned = made == Py_True;
