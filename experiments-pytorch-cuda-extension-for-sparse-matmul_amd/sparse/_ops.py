@@ -54,9 +54,10 @@ RUN_WALK_STRIPS = 32             # 4 per wave; with 10 waves and up to 39 strips
 RUN_WALK_MIN_REUSE = 2.0
 # DDS over many dense rows (a block-sparse linear layer): panels of the dense operand shared by eight groups
 # (bsa_matmul_dds_panels), when the mask is dense enough that a panel serves several of them and the launch has
-# workgroups for most of the machine.  Measured against the group walk, bf16, us: stored share of the cells times used share of
-# the panels' rows 0.09 (96 x 96 blocks, 8 x 1024 rows) 95 -> 78, (64 x 64, 4 x 1056) 31 -> 25, 0.11 (64 x 64) 35 -> 26, 0.13
-# (96 x 96) 119 -> 81, 0.31 250 -> 91; one entry of 1056 rows, 64 x 64 at 0.2, 88 workgroups: 16.8 -> 17.5.
+# workgroups for most of the machine, both reckoned in tiles of PANEL_ROWS rows.  bf16, us, group walk -> panels: 0.1 of 64 x 64
+# blocks, 4 x 1056 rows 31.8 -> 19.2, with a full column 34.6 -> 21.5; 0.12 of 96 x 96, 8 x 1024 rows 112 -> 64.5 and 127 -> 68.6;
+# 0.25 of 64 x 64, 1920 rows (160 tiles) 28.9 -> 12.9 and 32.2 -> 16.2.  At the lines the panels are well ahead, and they stay ahead
+# for some way below them (1056 rows, 88 tiles 18.3 -> 11.7 and 19.6 -> 14.8; 0.1 at 1344 rows, 112 tiles 12.8 -> 9.5 and 13.7 -> 13.7).
 PANEL_WALK = True
 PANEL_ROWS, PANEL_MAX_KBLOCKS, PANEL_MAX_NNZ = _k.dds_panel_limits()      # of a workgroup, of a launch
 PANEL_GROUPS = 8                       # of a workgroup
