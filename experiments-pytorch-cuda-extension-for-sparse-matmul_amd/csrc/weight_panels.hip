@@ -37,9 +37,9 @@ constexpr int PANEL_NONE = -1;
 // Blocks that the set's longest chain must get shorter by, to pay for two barriers and the helper's sums through LDS.  us, a
 // column of the weight full, without the helper -> with it: a quarter and a tenth of 64 x 64 blocks, 4224 rows 28.0 -> 25.1 and
 // 25.8 -> 21.5, 5632 rows 39.7 -> 34.1 and 38.0 -> 30.2; 96 x 96, 8192 rows 80.7 -> 68.6; masks without one as they were (23.4 ->
-// 23.5, 19.2 -> 19.2, 64.6 -> 64.5).  Two or five helpers that go to the longest chains one by one: 1 us slower at one such
-// column, faster at two of a set (38.7 -> 36.7); half of the longest group to the wave of the shortest, with a second set of sums:
-// its registers spill.
+// 23.5, 19.2 -> 19.2, 64.6 -> 64.5).  Two helpers, half of each of the two longest: two full columns of a set 38.7 -> 36.1 and 71.3 ->
+// 62.6, everything else 1 % slower; two or five that go to the longest chains one by one: 1 us slower at one such column; half of the
+// longest group to the wave of the shortest, with a second set of sums: its registers spill.
 constexpr int PANEL_CUT_FROM = 8;
 __host__ __device__ constexpr int panel_list_length(int kblocks) { return (kblocks + 2 * PANEL_RING + 3) / 4 * 4; }
 
