@@ -441,10 +441,12 @@ __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kern
 //   dv^T += dO_r^T P,  dk^T += Q_r^T dS   the 16-bit P and dS values are the column operands straight from the
 //                                      accumulators, the Q_r and dO_r tiles are read a second time along their rows
 // The waves of a column add their parts through LDS.  Three waves per SIMD at head dim 64 (168 registers: V is read out of
-// LDS for every block, the exponentials stay in front of the second product), one at 128 (its four accumulators are 256).
-// us, both sides in turn on one box, two waves per SIMD (200 registers) -> three: 48 heads of 8192 tokens 114.1 -> 105.8, the
-// training pass 275.2 -> 266.3.  At 128 a second stage of tiles, requested a whole block ahead, took 63.1 -> 66.1 us at 16
-// heads of 4096 tokens.  At 64 one workgroup per residency slot that walks several columns and requests the next one's
+// LDS for every block, the exponentials stay in front of the second product), two at 128 (256 registers: accumulators 128, K
+// and V 64, so a tile's operands are read four at a time instead of all at once).
+// us, both sides in turn on one box, two waves per SIMD (200 registers) -> three at 64: 48 heads of 8192 tokens 114.1 -> 105.8,
+// the training pass 275.2 -> 266.3; one (368 registers) -> two at 128, where a wave alone had nothing to wait beside: 16 heads of
+// 4096 tokens 63 -> 51, the training pass 133.1 -> 120.9 (left to the compiler two waves spill 53 registers: 183).  There a second
+// stage of tiles, requested a whole block ahead, took one wave 63.1 -> 66.1 us.  At 64 one workgroup per residency slot that walks several columns and requests the next one's
 // tiles early took 111 -> 129 us (its neighbours drift apart and leave the L2's working set), forward and rows likewise.
 // Delta is scaled as it is read; with scale * delta in memory the whole backward pass takes 1 % less (48.4-49.0 against 49.3-50.1
 // us).  Starting the second product at delta, 184 registers, takes as long and is further from float64 (dk of fp16, causal:
@@ -456,7 +458,7 @@ constexpr bool at_bwd_col_keeps_v(int hd) { return hd == 64; }
 constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256 + (at_bwd_col_keeps_v(hd) ? 64 * hd : 0); }
 
 template <int HD, bool BF>
-__global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64 ? 3 : 1) void attention_bwd_dkdv_kernel(
+__global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64 ? 3 : 2) void attention_bwd_dkdv_kernel(
     const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
     const half_t *__restrict__ k, const half_t *__restrict__ v, const half_t *__restrict__ q, const half_t *__restrict__ dout,
     int rows_q, int rows_k, const float *__restrict__ lse, const float *__restrict__ delta, float scale, int causal,
@@ -502,6 +504,18 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                 dma4_gather(my_stat + BS * r, stat_lds);
                 qreq.issue(r);
             };
+            // acc += rows of a tile, four operands of it in registers at a time
+            auto products_of_rows = [&](unsigned tile, auto other, f16v &acc) {
+#pragma unroll
+                for (int s0 = 0; s0 < KS; s0 += 4) {
+                    h8 op[4];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) op[s] = rd.rows(tile, s0 + s);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) acc = mfma_16<BF>(op[s], other(s0 + s), acc);
+                    if (KS > 4) __builtin_amdgcn_sched_barrier(0);
+                }
+            };
             if (seg == e.begin) {
                 tile_wait<0>();
 #pragma unroll
@@ -522,11 +536,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                 tile_wait<TileRequests<HD>::N>();            // everything but dO
                 f16v prob = {0};
                 {
-                    h8 qop[KS];
-#pragma unroll
-                    for (int s = 0; s < KS; ++s) qop[s] = rd.rows(Q_TILE, s);
-#pragma unroll
-                    for (int s = 0; s < KS; ++s) prob = mfma_16<BF>(qop[s], kop[s], prob);
+                    products_of_rows(Q_TILE, [&](int s) { return kop[s]; }, prob);
                     if (masked) {                // a hidden score has no probability
                         int first = key - 4 * h;
                         asm volatile("" : "+v"(first));      // its comparisons stay here: 16 masks would be kept through the walk
@@ -551,11 +561,7 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                 tile_wait<0>();
                 {
                     f16v dpacc = {0};
-                    h8 dop[KS];
-#pragma unroll
-                    for (int s = 0; s < KS; ++s) dop[s] = rd.rows(DO_TILE, s);
-#pragma unroll
-                    for (int s = 0; s < KS; ++s) dpacc = mfma_16<BF>(dop[s], KEEPS_V ? rd.rows(V_TILE, s) : vop[s], dpacc);
+                    products_of_rows(DO_TILE, [&](int s) { return KEEPS_V ? rd.rows(V_TILE, s) : vop[s]; }, dpacc);
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f4v dl = *reinterpret_cast<const f4v *>(stats + 32 + 8 * g + 4 * h) * scale;
@@ -568,26 +574,25 @@ __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64
                     }
                 }
                 // The tiles are read a second time, Q first: the requests for the next block go out as soon as each is free.
-                h8 tr[KT][2];
-                auto read_columns = [&](unsigned tile) {
+                auto products_of_columns = [&](unsigned tile, const h8 (&op)[2], RowTile<HD> &acc, auto when_read) {
 #pragma unroll
-                    for (int t = 0; t < KT; ++t)
+                    for (int t0 = 0; t0 < KT; t0 += 2) {
+                        h8 tr[2][2];
 #pragma unroll
-                        for (int s = 0; s < 2; ++s) tr[t][s] = rd.columns(tile, t, s);
-                    lds_reads_done();
+                        for (int t = 0; t < 2; ++t)
+#pragma unroll
+                            for (int s = 0; s < 2; ++s) tr[t][s] = rd.columns(tile, t0 + t, s);
+                        lds_reads_done();
+                        if (t0 + 2 == KT) when_read();
+#pragma unroll
+                        for (int s = 0; s < 2; ++s)
+#pragma unroll
+                            for (int t = 0; t < 2; ++t) acc[t0 + t] = mfma_16<BF>(tr[t][s], op[s], acc[t0 + t]);
+                        if (KT > 2) __builtin_amdgcn_sched_barrier(0);
+                    }
                 };
-                read_columns(Q_TILE);
-                if (!last) request_q(p + 1);
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int t = 0; t < KT; ++t) dk[t] = mfma_16<BF>(tr[t][s], ds[s], dk[t]);
-                read_columns(DO_TILE);
-                if (!last) doreq.issue(win.get(p + 1).row());
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int t = 0; t < KT; ++t) dv[t] = mfma_16<BF>(tr[t][s], pop[s], dv[t]);
+                products_of_columns(Q_TILE, ds, dk, [&]() { if (!last) request_q(p + 1); });
+                products_of_columns(DO_TILE, pop, dv, [&]() { if (!last) doreq.issue(win.get(p + 1).row()); });
             }
         }
     }
