@@ -14,9 +14,18 @@ from . import kernel as _k
 BLOCK = 32
 # tuning of the wavefront schedules: (target pairs per wavefront, wavefronts per workgroup)
 # (cap, waves, split long groups, no row slicing, -, longest chunks first)
-SCHEDULE_GROUP_WALK = (12, 4, True, -1, 2, True)        # groups of at most GROUP_WALK_LONG pairs (rows of attention masks)
+# Group walks (DSD, DDS).  A launch of few pairs is one generation of waves and lasts as long as its fullest SIMD: shorter chunks,
+# spread over more of them.  Counted are the pairs of all batch entries and 64-column strips.  A table whose longest group fits
+# the workgroup of a large launch is not cut by shorter chunks either (_group_walk_kinds): no launch needs a workspace that another
+# batch count of the same layout does not need.  us, median of a graph, chunks of 12 -> now (fp16 DSD): 592 pairs, rows of up to 6
+# 5.2 -> 4.6, 2024 (12) 7.1 -> 4.8, 4048 7.4 -> 5.7, 6072 7.5 -> 6.7, 12144 13.3 -> 10.3, 12240 (20) 9.9 -> 8.8; 18112 (9) would be 13.3 ->
+# 14.9.  Tables with longer groups gain nothing in fp16 (506 to 14664 pairs, chunks of 4 to 10 within 3 % below 5000, slower above).
+SCHEDULE_GROUP_WALK = (4, 4, True, -1, 2, True)          # groups of at most GROUP_WALK_LONG pairs (rows of attention masks)
+SCHEDULE_GROUP_WALK_MIDDLE = (6, 4, True, -1, 2, True)
+SCHEDULE_GROUP_WALK_LARGE = (12, 4, True, -1, 2, True)
 SCHEDULE_GROUP_WALK_LONG = (10, 4, True, -1, 2, True)    # tables with longer groups (columns of causal / strided masks)
 GROUP_WALK_LONG = 24
+GROUP_WALK_SMALL_PAIRS, GROUP_WALK_MIDDLE_PAIRS = 4096, 14000
 SCHEDULE_SDD = (4, 2)
 # fp32: a wave splits its row's operands into bf16 parts once, so chunks pay where the products are split: from as many blocks on as
 # bsa_matmul splits them (SDD_F32_SPLIT_BLOCKS in csrc/matmul.hip, with both sides' times).  us, the fp32 instruction in chunks of 1
@@ -25,9 +34,16 @@ SCHEDULE_SDD = (4, 2)
 SCHEDULE_SDD_F32 = (1, 4)
 SCHEDULE_SDD_F32_LARGE = (4, 2)
 SDD_F32_LARGE_BLOCKS = 3000            # of all batch entries together, at k = 64 and more
-# fp32 groups of at most GROUP_WALK_LONG pairs: chunks of 6 in 4 waves hold such a group in one workgroup too.  us, chunks of 12
-# -> 6 (DSD): 744 blocks 13.6 -> 11.2, 1012 19.7 -> 12.8, 8096 25.2 -> 20.3, 11912 29.4 -> 24.6, 73440 114 -> 114.
-SCHEDULE_GROUP_WALK_F32 = (6, 4, True, -1, 2, True)
+# fp32: a pair keeps its SIMD's matrix pipe for 2048 clocks, so the chunks of the fullest SIMD are the launch.  us, chunks of 6 (10
+# in tables with longer groups) -> now: 592 pairs, rows of up to 6 11.5 -> 7.6, 2024 (12) 12.0 -> 8.2, (columns of 64) 17.9 -> 11.3;
+# 4048 (columns of 64) 19.5 -> 13.7, 6120 (rows of 20, columns of 128) 20.0 -> 15.5 and 21.8 -> 18.5, 8096 (12, 64) 20.3 -> 18.6 and 24.3 ->
+# 20.5, 10464
+# (rows of 7) 22.1 -> 21.5, 9776 (columns of 64) 24.5 -> 22.8; from 12000 pairs on chunks of 4 are ahead in some launches and behind in as
+# many (12144 29.2 -> 27.3, 13392 26.6 -> 27.1, 14664 26.9 -> 30.6).
+SCHEDULE_GROUP_WALK_F32 = (3, 4, True, -1, 2, True)
+SCHEDULE_GROUP_WALK_F32_MIDDLE = (4, 4, True, -1, 2, True)
+SCHEDULE_GROUP_WALK_F32_LARGE = (6, 4, True, -1, 2, True)      # 73440 pairs, chunks of 12 -> 6: 114 -> 114
+GROUP_WALK_F32_MIDDLE_PAIRS = 11000
 SCHEDULE_SOFTMAX = (4, 4)
 SOFTMAX_LONGEST_FIRST = True     # long rows are dispatched first: they would otherwise finish on a draining machine
 SOFTMAX_WAVES_LONG_ROWS = 8
@@ -145,6 +161,10 @@ class Schedule:
                                                              head_dim)
         self.last_key = ("attention_backward", id(columns), batches, head_dim, stream)
         return self._zeroed(self.last_key, need)
+
+    def has_workspace(self, key):
+        """Whether a graph can be given a workspace of ``key`` (a key without its stream)."""
+        return bool(self._spares.get(key)) or any(k[:-1] == key for k in self._captured)
 
     _spaces = {}             # of a schedule that no plan launches by
     MAX_WORKSPACES = 16      # eager ones per schedule; the least recently used one goes first
@@ -305,15 +325,39 @@ def _longest_group(offsets) -> int:
     return longest
 
 
-def _group_walk_kind(longest):
-    return SCHEDULE_GROUP_WALK_LONG if longest > GROUP_WALK_LONG else SCHEDULE_GROUP_WALK
+def _group_walk_kinds(longest, dtype, pairs):
+    """Schedules of a group walk over ``pairs`` pairs of all batch entries and strips: the one it takes, then what else serves
+    where that one cannot be built (the others of this type and of the 16-bit types)."""
+    short = longest <= GROUP_WALK_LONG
+    large = SCHEDULE_GROUP_WALK_LARGE if short else SCHEDULE_GROUP_WALK_LONG
+    half = [SCHEDULE_GROUP_WALK, SCHEDULE_GROUP_WALK_MIDDLE, large] if short else [large]
+    if dtype == torch.float32:
+        kinds = [SCHEDULE_GROUP_WALK_F32, SCHEDULE_GROUP_WALK_F32_MIDDLE, SCHEDULE_GROUP_WALK_F32_LARGE if short else large]
+        lines = GROUP_WALK_SMALL_PAIRS, GROUP_WALK_F32_MIDDLE_PAIRS
+    else:
+        kinds, lines = half, (GROUP_WALK_SMALL_PAIRS, GROUP_WALK_MIDDLE_PAIRS) if short else ()
+    first = kinds[sum(pairs > line for line in lines)]
+
+    def whole(kind):                # chunks that cut no group which the largest launches leave whole
+        cap, waves = kind[:2]
+        return (max(cap, -(-longest // waves)),) + kind[1:] if longest <= large[0] * large[1] else kind
+
+    return tuple(dict.fromkeys(whole(kind) for kind in [first] + kinds + half))
 
 
-def _group_walk_schedule(layout, dtype=torch.float16):
-    kind = _group_walk_kind(_longest_group(layout[1]))
-    if dtype == torch.float32 and kind is SCHEDULE_GROUP_WALK:
-        return _schedule_or(layout, SCHEDULE_GROUP_WALK_F32, kind)
-    return schedule_for(layout, kind)
+def _group_walk_schedule(layout, dtype=torch.float16, entries=None, key=None):
+    """Schedule of a group walk over ``entries`` batch entries times strips (None: as many as fill the machine).  Under graph
+    capture the first that is there and has the launch's workspace, ``key``."""
+    pairs = layout[0].numel() // 2 * entries if entries is not None else 2 ** 62
+    kinds = _group_walk_kinds(_longest_group(layout[1]), dtype, pairs)
+    if torch.cuda.is_current_stream_capturing():
+        there = [layout[1]._bsa_schedules[kind] for kind in kinds if _has_schedule(layout, kind)]
+        for sched in there:
+            if sched.tile_slots == 0 or key is None or sched.has_workspace(key):
+                return sched
+        if there:
+            return there[0]
+    return schedule_for(layout, kinds[0])
 
 
 def _sdd_schedule(layout, dtype, batches, k):
@@ -338,8 +382,10 @@ def _captured_without(layout, kind) -> bool:
     building one synchronises.  Calls that used a walk without a schedule eagerly stay with it then."""
     if kind is None:
         longest = getattr(layout[1], "_bsa_longest", None)
-        kind = longest if longest is None else _group_walk_kind(longest)
-    return not _has_schedule(layout, kind) and torch.cuda.is_current_stream_capturing()
+        kinds = () if longest is None else _group_walk_kinds(longest, torch.float16, 0)
+    else:
+        kinds = (kind,)
+    return not any(_has_schedule(layout, k) for k in kinds) and torch.cuda.is_current_stream_capturing()
 
 
 def _attention_kind(layout, kind, split, most_waves=ATTENTION_WAVES_LONG_GROUPS):
@@ -501,7 +547,8 @@ def _matmul_route(a, b, mode, row_layout, col_layout, trans_a, trans_b):
 
     if mode == "sdd":
         return route("walk", _sdd_schedule(layout, a.dtype, batches, size_k))
-    return route("walk", _group_walk_schedule(layout, a.dtype))
+    strips = -(-(size_n if mode == "dsd" else size_m) // 64)
+    return route("walk", _group_walk_schedule(layout, a.dtype, batches * strips, (_k.MODES[mode], batches, size_m, size_n)))
 
 
 def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=False):

@@ -47,7 +47,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: SparseL
 
     A row is summed in chunks that are shorter while the stored blocks of all batch entries together are at most
     ``_ops.ATTENTION_SMALL_BLOCKS``: an entry gives the same bits in every launch on the same side of that line, across it
-    the last bits can differ.  In fp32 the line is that of the scores (``sparse.matmul``, mode ``'sdd'``)."""
+    the last bits can differ.  In fp32 the lines are those of ``sparse.matmul``, modes ``'sdd'`` and ``'dsd'``."""
     fused = q.dtype in (torch.float16, torch.bfloat16) and q.size(-1) in (64, 128)
     if fused or not (q.dtype == k.dtype == v.dtype and q.dtype in (torch.float16, torch.bfloat16, torch.float32)):
         return host_calls.attention(q, k, v, layout, scale, causal)      # SparseAttention.apply, which also owns the argument checks

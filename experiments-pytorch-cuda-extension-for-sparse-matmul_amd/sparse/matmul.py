@@ -61,7 +61,8 @@ class SparseMatMul(torch.autograd.Function):
 
 # fp32 'sdd' with an inner dimension of at most 128: from 3000 stored blocks of all batch entries together on (at an inner dimension
 # of 32 from 1500 or 6000, by the operands' orders) the products are made on another matrix instruction, no less exact.  An entry
-# gives the same bits in every launch on one side of that line, across it the last bits can differ.
+# gives the same bits in every launch on one side of that line, across it the last bits can differ.  Likewise 'dsd' and 'dds',
+# whose sums are cut into shorter chunks in smaller launches (_ops.GROUP_WALK_SMALL_PAIRS and the lines beside it).
 # Call this, not the class (matmul.py:55-57).  It is SparseMatMul.apply, in native code where the layout has a plan for these
 # shapes (csrc/host_calls.cpp); the class is what serves every other call.
 matmul = host_calls.matmul

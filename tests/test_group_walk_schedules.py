@@ -1,0 +1,88 @@
+"""Chunks of the group walks (DSD, DDS) by the size of a launch: what a table is cut into does not depend on it where a large
+launch leaves its groups whole, every choice serves where another cannot be built, and each gives the product."""
+import pytest
+import torch
+
+LINES = (1, 4096, 4097, 11000, 11001, 14000, 14001, 10 ** 7)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("longest", [0, 1, 12, 13, 16, 17, 24, 25, 40, 41, 48, 130])
+def test_no_launch_cuts_a_group_that_another_leaves_whole(dtype, longest):
+    from sparse import _ops
+    large = _ops.SCHEDULE_GROUP_WALK_LONG if longest > _ops.GROUP_WALK_LONG else _ops.SCHEDULE_GROUP_WALK_LARGE
+    choices = [_ops._group_walk_kinds(longest, dtype, pairs) for pairs in LINES]
+    for kinds in choices:
+        assert set(kinds) == set(choices[0])
+        if longest <= large[0] * large[1]:
+            assert all(cap * waves >= longest for cap, waves, *_ in kinds)
+    caps = [kinds[0][0] for kinds in choices]
+    assert caps == sorted(caps)
+
+
+def _mask(longest, by_rows):
+    mask = torch.zeros(longest + 3, longest + 3, dtype=torch.long)
+    mask.fill_diagonal_(1)
+    mask[2, :longest] = 1
+    mask[5 % (longest + 3), 1:longest // 2 + 1] = 1
+    return mask if by_rows else mask.t().contiguous()
+
+
+def _products(L, s, v, dtype):
+    import sparse
+    for args in ((s, v, "dsd", L), (s, v, "dsd", L, True), (v.transpose(-1, -2).contiguous(), s, "dds", L),
+                 (v.transpose(-1, -2).contiguous(), s, "dds", L, False, True)):
+        yield sparse.matmul(*args)
+
+
+# lengths at, one above and below what four waves take in chunks of 3, 4 and 6, and such as every launch cuts
+@pytest.mark.gpu
+@pytest.mark.parametrize("longest", [12, 13, 16, 17, 24, 25, 41, 49])
+@pytest.mark.parametrize("by_rows", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("width", [64, 96])
+def test_products_on_every_side_of_the_lines(longest, by_rows, dtype, width, monkeypatch):
+    """Bound: the rounding of the result and of an fp32 sum of at most 49 x 32 products, over the 2-norm."""
+    import sparse
+    from sparse import _ops
+    L = sparse.SparseLayout(_mask(longest, by_rows).cuda())
+    g = torch.Generator(device="cuda").manual_seed(longest)
+    n = 32 * (longest + 3)
+    s = torch.randn(3, L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
+    v = torch.randn(3, n, width, generator=g, device="cuda").to(dtype)
+    S, V = L.to_dense(s).double().cpu(), v.double().cpu()
+    wants = [S @ V, S.transpose(1, 2).contiguous() @ V]
+    wants += [V.transpose(1, 2).contiguous() @ S, V.transpose(1, 2).contiguous() @ S.transpose(1, 2).contiguous()]
+    rel = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -21
+    for small, middle in ((10 ** 9, 10 ** 9), (1, 10 ** 9), (1, 1)):
+        monkeypatch.setattr(_ops, "GROUP_WALK_SMALL_PAIRS", small)
+        monkeypatch.setattr(_ops, "GROUP_WALK_MIDDLE_PAIRS", middle)
+        monkeypatch.setattr(_ops, "GROUP_WALK_F32_MIDDLE_PAIRS", middle)
+        fresh = sparse.SparseLayout(_mask(longest, by_rows).cuda())
+        for got, want in zip(_products(fresh, s, v, dtype), wants):
+            assert torch.isfinite(got).all()
+            assert (got.double().cpu() - want).norm() <= rel * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("longest", [12, 20, 30])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_captured_on_the_other_side_of_a_line(longest, dtype, monkeypatch):
+    """Groups that no launch cuts: the schedule of an eager launch of another size serves a captured one."""
+    import sparse
+    from sparse import _ops
+    L = sparse.SparseLayout(_mask(longest, True).cuda())
+    monkeypatch.setattr(_ops, "GROUP_WALK_SMALL_PAIRS", 2 * L.num_blocks)
+    g = torch.Generator(device="cuda").manual_seed(longest)
+    s = torch.randn(4, L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
+    v = torch.randn(4, 32 * (longest + 3), 64, generator=g, device="cuda").to(dtype)
+    want = [x[:2].clone() for x in _products(L, s, v, dtype)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = list(_products(L, s[:2], v[:2], dtype))
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(got, want):
+            assert (x.double() - y.double()).norm() <= (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -20) * y.double().norm()
