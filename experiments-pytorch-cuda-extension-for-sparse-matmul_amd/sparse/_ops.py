@@ -27,6 +27,10 @@ SCHEDULE_GROUP_WALK_LONG = (10, 4, True, -1, 2, True)    # tables with longer gr
 GROUP_WALK_LONG = 24
 GROUP_WALK_SMALL_PAIRS, GROUP_WALK_MIDDLE_PAIRS = 4096, 14000
 SCHEDULE_SDD = (4, 2)
+# SDD of few blocks (of all batch entries, times 64-value pieces of the inner dimension): more waves of two blocks each.  fp16, us,
+# chunks of 4 -> 2: 592 blocks 3.9 -> 3.4, 2024 4.6 -> 4.1, 4048 4.8 -> 4.6, 7156 5.8 -> 5.6; 12240 would be 7.4 -> 7.6.  The same bits.
+SCHEDULE_SDD_SMALL = (2, 2)
+SDD_SMALL_BLOCKS = 8000
 # fp32: a wave splits its row's operands into bf16 parts once, so chunks pay where the products are split: from as many blocks on as
 # bsa_matmul splits them (SDD_F32_SPLIT_BLOCKS in csrc/matmul.hip, with both sides' times).  us, the fp32 instruction in chunks of 1
 # in 4 waves -> split in chunks of 4 in 2, k = 64: 1012 blocks 6.2 -> 7.9, 2368 8.2 -> 8.8, 3552 10.3 -> 9.3, 8096 18.6 -> 15.0,
@@ -362,7 +366,8 @@ def _group_walk_schedule(layout, dtype=torch.float16, entries=None, key=None):
 
 def _sdd_schedule(layout, dtype, batches, k):
     if dtype != torch.float32:
-        return schedule_for(layout, SCHEDULE_SDD)
+        small = layout[0].numel() // 2 * batches * -(-k // 64) <= SDD_SMALL_BLOCKS
+        return _schedule_or(layout, *((SCHEDULE_SDD_SMALL, SCHEDULE_SDD) if small else (SCHEDULE_SDD, SCHEDULE_SDD_SMALL)))
     if layout[0].numel() // 2 * batches * min(k, 64) >= 64 * SDD_F32_LARGE_BLOCKS:
         return _schedule_or(layout, SCHEDULE_SDD_F32_LARGE, SCHEDULE_SDD_F32)
     return _schedule_or(layout, SCHEDULE_SDD_F32, SCHEDULE_SDD_F32_LARGE)
@@ -384,7 +389,7 @@ def _captured_without(layout, kind) -> bool:
         longest = getattr(layout[1], "_bsa_longest", None)
         kinds = () if longest is None else _group_walk_kinds(longest, torch.float16, 0)
     else:
-        kinds = (kind,)
+        kinds = (SCHEDULE_SDD, SCHEDULE_SDD_SMALL) if kind == SCHEDULE_SDD else (kind,)
     return not any(_has_schedule(layout, k) for k in kinds) and torch.cuda.is_current_stream_capturing()
 
 

@@ -86,3 +86,40 @@ def test_captured_on_the_other_side_of_a_line(longest, dtype, monkeypatch):
         torch.cuda.synchronize()
         for x, y in zip(got, want):
             assert (x.double() - y.double()).norm() <= (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -20) * y.double().norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k", [32, 64, 160])
+def test_scores_have_the_same_bits_on_both_sides_of_the_line(dtype, k, monkeypatch):
+    import sparse
+    from sparse import _ops
+    g = torch.Generator(device="cuda").manual_seed(k)
+    mask = _mask(21, True).cuda()
+    q, v = (torch.randn(3, 32 * 24, k, generator=g, device="cuda").to(dtype) for _ in range(2))
+    got = []
+    for line in (10 ** 9, 0):
+        monkeypatch.setattr(_ops, "SDD_SMALL_BLOCKS", line)
+        got.append(sparse.matmul(q, v, "sdd", sparse.SparseLayout(mask), False, True))
+    assert torch.equal(*got)
+    S = sparse.SparseLayout(mask).to_sparse((q.double() @ v.double().transpose(1, 2).contiguous()).float())
+    assert (got[0].double() - S.double()).norm() <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) * S.double().norm()
+
+
+@pytest.mark.gpu
+def test_scores_captured_on_the_other_side_of_the_line(monkeypatch):
+    import sparse
+    from sparse import _ops
+    L = sparse.SparseLayout(_mask(21, True).cuda())
+    monkeypatch.setattr(_ops, "SDD_SMALL_BLOCKS", 2 * L.num_blocks)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, v = (torch.randn(4, 32 * 24, 64, generator=g, device="cuda").half() for _ in range(2))
+    want = sparse.matmul(q, v, "sdd", L, False, True)[:2].clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = sparse.matmul(q[:2], v[:2], "sdd", L, False, True)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
