@@ -6,8 +6,6 @@
 // dense rows and dozens of groups that read the same columns of them.  Here a workgroup owns 64 to 160 dense rows and eight
 // neighbouring groups, a wave each, walks ALL of the contraction in steps of 128 and keeps the dense panels of the present and
 // the next steps in LDS; a wave multiplies them by the blocks its group has there.
-#include <type_traits>
-
 #include "bsa_device.hpp"
 #include "lds_tiles.hpp"
 #include "bsa_internal.hpp"
@@ -344,15 +342,12 @@ __global__ __launch_bounds__(PANEL_THREADS, 3) void weight_panel_kernel(
 // Gradient of the weight: w[block (r, c)] = sum over tokens t of a[t][32 r + .] b[t][32 c + .]
 //
 // A workgroup owns 8 x 8 cells of the mask and a share of the tokens; per step of 32 tokens it fetches 256 columns
-// of a and of b, a 64-column panel a wave, and a wave multiplies the stored cells of one row (or column) of the mask, whose
-// operand of a (of b) it reads once.  Partial sums of the shares leave as fp32 and are added up in share order by weight_sum_kernel.
-// A quarter of 64 x 64 blocks stored, 4224 tokens, without the sum: about 12 us for start, end and the barriers of 33 steps (the
-// stores 4 of it), panels alone 8 more (32 KB a step and workgroup out of L2), operands and products alone 13 more; the two
-// overlap by half.  us with the sum, cells dealt evenly, both operands of each read and a lone cell paired with itself -> now:
-// 35.2 -> 29.3, half stored 46.3 -> 39.2, all 65.9 -> 56.7; 96 x 96 at a quarter, 8192 tokens 114 -> 105; a tenth of 64 x 64 27.0 ->
-// 25.6, with two rows full 30.4 -> 27.1 (32.5 by rows alone), two columns 33.2 -> 28.4.  Sixteen waves of half a row each 2 us
-// slower; an eighth of the cells in row-major order to a wave, the row's operand read again where it changes, 15 (sums are copied
-// behind the branch).  Panels through registers, three steps in flight, took 48 of them (8 spilled).
+// of a and of b, a 64-column panel a wave, and the stored cells are dealt evenly to the waves.  Partial sums of the shares
+// leave as fp32 and are added up in share order by weight_sum_kernel.
+// Bound by what the panels take from L2, 32 KB a step and workgroup (8.7 TB/s at 64 x 64 blocks).  They go straight to LDS:
+// through registers, three steps in flight took 48 of them (8 spilled), and an LDS write each.
+// A quarter of 64 x 64 blocks stored, 4224 tokens, with the sum: 38.5 -> 35.1 us; 96 x 96 at 0.3, 8192 tokens: 145 -> 128;
+// all of 64 x 64 stored: 74.6 -> 66.2.
 // ---------------------------------------------------------------------------
 constexpr int WG_EDGE = 8;                       // cells along a side
 constexpr int WG_PANEL = 4096;                   // 32 tokens of 64 columns
@@ -375,7 +370,7 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
     const int first = (int)((long long)steps_total * share / shares), last = (int)((long long)steps_total * (share + 1) / shares);
     const int M = BS * R, N = BS * C;
 
-    // A row of cells to a wave, or a column where the fullest row has more than the fullest column: the slowest wave is the pace.
+    // the stored cells, dealt evenly to the waves in row-major order: cells w, w + 8, ..
     int *table = reinterpret_cast<int *>(lds_raw + WG_STAGES * WG_STAGE);
     if (tid < WG_EDGE * WG_EDGE) table[tid] = -1;
     lds_barrier();
@@ -389,24 +384,17 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
     }
     lds_barrier();
     const int mine_idx = table[l];
-    const unsigned long long stored = __ballot(mine_idx >= 0), a_row = 0xFFull, a_column = 0x0101010101010101ull;
-    int row_most = 0, column_most = 0;
+    unsigned long long stored = __ballot(mine_idx >= 0);
+    const int count = (__popcll(stored) - w + WG_EDGE - 1) / WG_EDGE;      // of this wave
+    int idx[WG_EDGE], at_a[WG_EDGE], at_b[WG_EDGE];      // at_: exclusive-ored into the address of an operand's first column
+    for (int j = 0; j < w && stored; ++j) stored &= stored - 1;
 #pragma unroll
     for (int j = 0; j < WG_EDGE; ++j) {
-        const int in_row = __popcll(stored & a_row << (WG_EDGE * j)), in_column = __popcll(stored & a_column << j);
-        row_most = in_row > row_most ? in_row : row_most;
-        column_most = in_column > column_most ? in_column : column_most;
-    }
-    const bool by_rows = row_most <= column_most;
-    unsigned long long mine = stored & (by_rows ? a_row << (WG_EDGE * w) : a_column << w);
-    const int count = __popcll(mine);
-    int idx[WG_EDGE], other[WG_EDGE];            // a cell's block, and its column in the row, or row in the column
-#pragma unroll
-    for (int j = 0; j < WG_EDGE; ++j) {
-        const int cell_of = mine ? __builtin_ctzll(mine) : 0;
+        const int cell_of = stored ? __builtin_ctzll(stored) : 0;
         idx[j] = __builtin_amdgcn_readlane(mine_idx, cell_of);
-        other[j] = by_rows ? cell_of % WG_EDGE : cell_of / WG_EDGE;
-        mine &= mine - 1;
+        at_a[j] = (cell_of >> 4) * WG_PANEL + (cell_of >> 3 & 1) * 64;
+        at_b[j] = WG_SIDE + (cell_of >> 1 & 3) * WG_PANEL + (cell_of & 1) * 64;
+        for (int t = 0; t < WG_EDGE; ++t) stored &= stored ? stored - 1 : 0;
     }
 
     // Panel w % 4 of a (waves 0-3) or b; columns behind the last repeat the first (never stored).  A wave's offsets inside 32
@@ -431,22 +419,13 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
 #pragma unroll
     for (int c = 0; c < WG_EDGE; ++c) acc[c] = f16v{0};
 
-    // LDS addresses of a cell's operands in the first stage, 8 rows apart (lo, hi); 16 tokens on are 2048 bytes on
     const unsigned tr_lo = (unsigned)get_panel_tr_addr(l, 0, 0, 0), tr_hi = (unsigned)get_panel_tr_addr(l, 0, 1, 0);
-    struct Operand { unsigned lo, hi; };
-    auto operand_of = [&](int k, unsigned side) {
-        const unsigned x = 64u * (k & 1), to = lds0 + side + (unsigned)(k >> 1) * WG_PANEL;
-        return Operand{(tr_lo ^ x) + to, (tr_hi ^ x) + to};
-    };
-    const Operand own = operand_of(w, by_rows ? 0 : WG_SIDE);
-    Operand others[WG_EDGE];
-#pragma unroll
-    for (int j = 0; j < WG_EDGE; ++j) others[j] = operand_of(other[j], by_rows ? WG_SIDE : 0);
-    auto multiply = [&](int stage, auto rows) {
-        const unsigned base = stage * WG_STAGE;
-        auto read = [&](const Operand &o, h8 (&x)[2]) {
+    auto multiply = [&](int stage) {
+        const unsigned base = lds0 + stage * WG_STAGE;
+        auto half_of = [&](int at, h8 (&x)[2]) {
+            asm volatile("" : "+s"(at));                // added where it is used: hoisted, the sums take 64 registers
             typedef tr4 __attribute__((address_space(3))) *lds_tr4;
-            const unsigned lo = o.lo + base, hi = o.hi + base;
+            const unsigned lo = (tr_lo ^ (unsigned)at) + base, hi = (tr_hi ^ (unsigned)at) + base;
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 const tr4 p = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4)(uintptr_t)(lo + 2048u * s));
@@ -454,19 +433,19 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
                 x[s] = __builtin_shufflevector(__builtin_bit_cast(h4, p), __builtin_bit_cast(h4, q), 0, 1, 2, 3, 4, 5, 6, 7);
             }
         };
-        h8 own_op[2];
-        read(own, own_op);
 #pragma unroll
         for (int j = 0; j < WG_EDGE; j += 2) {
             if (j < count) {                       // a pair at a time; the second repeats a cell when there is none
-                h8 op[2][2];
-                read(others[j], op[0]);
-                read(others[j + 1], op[1]);
+                h8 xa[2], xb[2], ya[2], yb[2];
+                half_of(at_a[j], xa);
+                half_of(at_b[j], xb);
+                half_of(at_a[j + 1], ya);
+                half_of(at_b[j + 1], yb);
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int c = 0; c < 2; ++c)
-                        acc[j + c] = rows.value ? mfma_16<BF>(op[c][s], own_op[s], acc[j + c]) : mfma_16<BF>(own_op[s], op[c][s], acc[j + c]);
+                for (int s = 0; s < 2; ++s) {
+                    acc[j] = mfma_16<BF>(xb[s], xa[s], acc[j]);
+                    acc[j + 1] = mfma_16<BF>(yb[s], ya[s], acc[j + 1]);
+                }
             }
         }
     };
@@ -475,47 +454,40 @@ __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
         // barrier for everybody's; behind it nobody reads the step before, whose buffer the next request takes.
 #pragma unroll
         for (int d = 0; d < WG_STAGES - 1; ++d) request(first + d, d);
-        auto walk = [&](auto rows) {
-            int stage = 0;
-            for (int s = first; s < last; ++s) {
-                tile_wait<4 * (WG_STAGES - 2)>();
-                lds_barrier();
-                request(s + WG_STAGES - 1, (stage + WG_STAGES - 1) % WG_STAGES);
-                multiply(stage, rows);
-                stage = (stage + 1) % WG_STAGES;
-            }
-        };
-        if (by_rows) walk(std::true_type{});
-        else walk(std::false_type{});
+        int stage = 0;
+        for (int s = first; s < last; ++s) {
+            tile_wait<4 * (WG_STAGES - 2)>();
+            lds_barrier();
+            request(s + WG_STAGES - 1, (stage + WG_STAGES - 1) % WG_STAGES);
+            multiply(stage);
+            stage = (stage + 1) % WG_STAGES;
+        }
         tile_wait<0>();                            // requests past the last step write to LDS that is still this workgroup's
     }
-    // a part is kept as the accumulators hold it: whole kilobytes a store (weight_sum_kernel puts the elements in order)
-    float *dst = parts + (size_t)share * nnz * BS2 + 4 * l;
+    float *dst = parts + (size_t)share * nnz * BS2 + (l & 31) * BS + 4 * (l >> 5);
 #pragma unroll
     for (int c = 0; c < WG_EDGE; ++c) {
         if (c < count) {
             float *o = dst + (size_t)idx[c] * BS2;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                *reinterpret_cast<float4 *>(o + 4 * WAVE * t) =
+                *reinterpret_cast<float4 *>(o + 8 * t) =
                     make_float4(acc[c][4 * t], acc[c][4 * t + 1], acc[c][4 * t + 2], acc[c][4 * t + 3]);
         }
     }
 }
 
-// out = sum over the shares of parts[share]: 8 elements a thread, row r, columns 8 t .. + 7 of a block, which lie in the parts as
-// four of lane r and four of lane r + 32 of store t
+// out[e] = sum over the shares of parts[share][e]: 8 elements a thread
 template <bool BF>
 __global__ __launch_bounds__(256) void weight_sum_kernel(const float *__restrict__ parts, half_t *__restrict__ out,
                                                          size_t elements, int shares)
 {
     const size_t e = 8 * ((size_t)blockIdx.x * 256 + threadIdx.x);
     if (e >= elements) return;
-    const size_t at = e / BS2 * BS2 + e % BS / 8 * (4 * WAVE) + e % BS2 / BS * 4;
     float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int p = 0; p < shares; ++p) {
-        const float4 *src = reinterpret_cast<const float4 *>(parts + (size_t)p * elements + at);
-        const float4 x = src[0], y = src[BS];
+        const float4 *src = reinterpret_cast<const float4 *>(parts + (size_t)p * elements + e);
+        const float4 x = src[0], y = src[1];
         s[0] += x.x; s[1] += x.y; s[2] += x.z; s[3] += x.w;
         s[4] += y.x; s[5] += y.y; s[6] += y.z; s[7] += y.w;
     }

@@ -137,27 +137,6 @@ def test_weight_gradient(any_size, rows, cols, density, batch, tokens, dtype):
     assert got.shape == want.shape and _rel(got, want) <= REL[dtype]
 
 
-# A wave takes a row of eight by eight cells, or a column where some row has more of them than every column: a row full, a
-# column full, both in different corners of the mask, one cell alone
-@pytest.mark.parametrize("rows,cols,cells", [
-    (8, 8, [(3, None)]), (8, 8, [(None, 6)]), (17, 12, [(2, None), (None, 9), (16, 3)]), (9, 8, [(8, 7)])])
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_weight_gradient_by_rows_and_by_columns(any_size, rows, cols, cells, dtype):
-    import sparse
-    from sparse import _ops
-    mask = torch.zeros(rows, cols, dtype=torch.long)
-    for r, c in cells:
-        mask[slice(None) if r is None else r, slice(None) if c is None else c] = 1
-    L = sparse.SparseLayout(mask.cuda())
-    g = torch.Generator(device="cuda").manual_seed(rows)
-    a = torch.randn(3, 160, 32 * rows, generator=g, device="cuda").to(dtype)
-    b = torch.randn(3, 160, 32 * cols, generator=g, device="cuda").to(dtype)
-    dense = a.double().cpu().flatten(0, 1).t().contiguous() @ b.double().cpu().flatten(0, 1)
-    want = torch.stack([dense[32 * r:32 * r + 32, 32 * c:32 * c + 32] for r, c in L.sparse_positions.cpu().tolist()]).cuda()
-    got = _ops.sparse_weight_gradient(a, b, L.row_layout, L.col_layout, True, False)
-    assert got.shape == want.shape and _rel(got, want) <= REL[dtype]
-
-
 def test_linear_layer_takes_both_and_agrees_with_the_group_walk(monkeypatch):
     import sparse
     from sparse import _ops
