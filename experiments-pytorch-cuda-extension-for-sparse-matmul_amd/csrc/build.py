@@ -24,10 +24,6 @@ CHECK_VARIANTS = {
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-fno-gpu-rdc", "-Wall", "-Wno-unused-function",
-    # The first 56 bytes of a kernel's arguments are in scalar registers when a wave starts, instead of a load away: every kernel
-    # takes the arguments it needs first (schedule, batch mapping, table, operands) in front.  us, without -> with: DSD of 2048
-    # tokens 7.20 -> 6.98, fused attention of 3 x 5 heads of 2976 13.2 -> 12.9, the longer kernels 0.1-0.2 each.
-    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     # keep the compiler from forming packed-fp32 instructions out of scalar float code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
