@@ -1,9 +1,10 @@
 // Host build (g++) of the LDS index arithmetic for the bank-model tests: exports the very
 // functions the kernels use, one C entry point that fills the 64 per-lane byte addresses
-// of a named access.
+// of a named access; and of the rule by which the panel walk refills its buffers.
 #include <cstring>
 
 #include "lds_index_math.hpp"
+#include "panel_ring.hpp"
 
 extern "C" int bsa_lds_access(const char *name, int permuted, int arg0, int arg1, int arg2, int *addr64)
 {
@@ -36,3 +37,10 @@ extern "C" int bsa_col16(int t, int i) { return bsa::col16(t, i); }
 extern "C" int bsa_strip16_half_swapped(int k) { return bsa::strip16_half_swapped(k); }
 extern "C" int bsa_perm16(int i) { return bsa::perm16(i); }
 extern "C" int bsa_invperm16(int i) { return bsa::invperm16(i); }
+
+extern "C" int bsa_panel_stages(int row_tiles) { return bsa::panel_stages(row_tiles); }
+extern "C" int bsa_panel_fetchers() { return bsa::PANEL_FETCHERS; }
+extern "C" int bsa_panel_ready() { return bsa::PANEL_READY; }
+extern "C" int bsa_panel_done() { return bsa::PANEL_DONE; }
+extern "C" int bsa_panel_refill_flag(int lane, int walkers, int s, int stages) { return bsa::panel_refill_flag(lane, walkers, s, stages); }
+extern "C" int bsa_panel_refill_from(int s, int stages) { return bsa::panel_refill_from(s, stages); }

@@ -11,6 +11,7 @@
 #include "bsa_internal.hpp"
 #include "group_walk.hpp"
 #include "attention_tiles.hpp"
+#include "panel_ring.hpp"
 #include "../../include/bsa.h"
 
 namespace bsa {
@@ -26,9 +27,6 @@ __device__ __forceinline__ int xcd_contiguous(int total)
 constexpr int PANEL_WAVES = 8;                  // groups of a workgroup, one wave each
 constexpr int PANEL_KB = 4;                     // k-blocks of 32 per step
 constexpr int PANEL_RING = 4;                   // blocks of a wave in flight
-// panels in LDS at a time: as many as a compute unit's 160 KB hold beside the lists of the widest contraction
-constexpr int panel_stages(int rt) { return rt <= 3 ? 4 : 3; }
-constexpr int PANEL_FETCHERS = 3;               // waves that do nothing but fetch them
 constexpr int PANEL_HELPER = PANEL_WAVES + PANEL_FETCHERS;                 // the last wave, if there is one: half of the longest group
 constexpr int PANEL_THREADS = 64 * (PANEL_HELPER + 1);
 constexpr int PANEL_FLAGS = 64;                 // bytes in front of the lists: panels that are there, panels that are read
@@ -50,9 +48,9 @@ __host__ __device__ constexpr int panel_list_length(int kblocks) { return (kbloc
 //   S_KC  the stored block is [x][k] (row groups): operands straight from memory
 //         otherwise [k][x] (column groups): through a wave-private LDS tile, read transposed
 // Three waves request panels straight into LDS, wait for them and say so in a flag; a multiplying wave waits for the panel of
-// its next block and says up to which panel it is done.  So the waits for panels are the fetching
-// waves' alone, the other waves' stay exact for the blocks, of which a wave has its next four on the way, and no wave waits
-// for the fullest of the eight in every step, only for the slowest where it is a whole set of buffers ahead.
+// its next block and says up to which panel it is done (panel_ring.hpp: when a buffer may be filled again).  So the waits for
+// panels are the fetching waves' alone, the other waves' stay exact for the blocks, of which a wave has its next four on the way,
+// and no wave waits for the fullest of the eight in every step, only for the slowest where it is a whole set of buffers ahead.
 //
 // What bounds it: the wave with the most blocks, about 1000 clocks a block (its panel's flag, LDS reads, ten products), then
 // the panels (200 MB through the L2 -> LDS path: 18 us without the products).  us, panels through registers a step ahead and a
@@ -83,8 +81,8 @@ __global__ __launch_bounds__(PANEL_THREADS, 3) void weight_panel_kernel(
 
     half_t *privs = reinterpret_cast<half_t *>(lds_raw + STAGES * PANEL_BYTES);
     int *flags = reinterpret_cast<int *>(lds_raw + STAGES * PANEL_BYTES + (S_KC ? 0 : walkers * BS2 * 2));
-    int *ready = flags, *done = flags + 4;       // of a buffer: panels up to and with the one in it; of a wave: panels it has done with
-    static_assert(STAGES <= 4 && 4 * (4 + PANEL_WAVES + 1) <= PANEL_FLAGS, "flags");
+    int *ready = flags + PANEL_READY, *done = flags + PANEL_DONE;
+    static_assert(STAGES <= PANEL_DONE - PANEL_READY && 4 * (PANEL_DONE + PANEL_WAVES + 1) <= PANEL_FLAGS, "flags");
     auto load_flag = [](const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
     auto store_flag = [](int *p, int v) {
         wave_lds_fence();
@@ -133,8 +131,9 @@ __global__ __launch_bounds__(PANEL_THREADS, 3) void weight_panel_kernel(
         for (int c = 0; c < 4; ++c) off[c] = 2u * (unsigned)((l >> 4) * KT) + 16u * (unsigned)((l & 15) ^ (4 * c + (l >> 4)));
         const int whole = KT / (BS * PANEL_KB), pieces = 16 - (steps * 16 - KT / 8);      // the last step may have fewer pieces
         for (int s = f; s < steps; s += PANEL_FETCHERS) {
-            // the panel before in this buffer, s - STAGES, has been read by all
-            while (__ballot(load_flag(done + (l < walkers ? l : 0)) < s - STAGES + 1) != 0ull) __builtin_amdgcn_s_sleep(1);
+            // the panel before in this buffer, s - STAGES, is there and has been read by all
+            const int *watched = flags + panel_refill_flag(l, walkers, s, STAGES);
+            while (__ballot(load_flag(watched) < panel_refill_from(s, STAGES)) != 0ull) __builtin_amdgcn_s_sleep(1);
             const unsigned to = lds0 + (unsigned)(s % STAGES) * PANEL_BYTES;
             int at = s + start;
             at = at < steps ? at : at - steps;

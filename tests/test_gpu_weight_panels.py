@@ -223,3 +223,32 @@ def test_panel_heights(any_size, tiles, k, groups, density, trans_b, dtype):
     want = x.flatten(0, 1).double() @ (W.t().contiguous() if trans_b else W)
     assert _rel(got, want) <= REL[dtype]
     assert (got - want).abs().max() <= 8 * REL[dtype] * want.abs().max()       # no row of a cut tile is out of place
+
+
+# Panels that no wave of a set has a block in, of which a wave says that it is done with them while they are on their way: a last set
+# of one group, with gaps of one to six steps and its blocks bunched or apart; a set without a block; as many k-blocks as leave
+# no room for the helper.  Four buffers (64 and 96 rows a workgroup) and three.
+@pytest.mark.parametrize("tiles", [2, 3, 4])
+@pytest.mark.parametrize("k,groups", [(48, 9), (330, 17), (690, 9)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_steps_that_no_group_of_a_set_uses(any_size, tiles, k, groups, trans_b):
+    import sparse
+    from sparse import _ops
+    g = torch.Generator().manual_seed(k)
+    mask = (torch.rand(groups, k, generator=g) < 0.01).long()
+    mask[8] = 0
+    mask[8, [4 * s + j for s in (1, 4, 5, 8, 9) for j in range(1 + s % 2)]] = 1
+    mask[8, 48:] = (torch.rand(k - 48, generator=g) < 0.05).long()
+    mask[9:] = 0
+    L = sparse.SparseLayout((mask if trans_b else mask.t().contiguous()).cuda())
+    batch = tiles * (256 // -(-groups // 8)) - 1
+    assert _row_tiles(groups, k, 32 * batch) == tiles
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    x = torch.randn(batch, 32, 32 * k, generator=g, device="cuda").half()
+    w = torch.randn(L.num_blocks, 32, 32, generator=g, device="cuda").half()
+    W = L.to_dense(w).double()
+    want = x.flatten(0, 1).double() @ (W.t().contiguous() if trans_b else W)
+    for _ in range(3):
+        got = _ops.sparse_matmul(x, w, "dds", L.row_layout, L.col_layout, False, trans_b).flatten(0, 1)
+        assert _rel(got, want) <= REL[torch.float16]
+        assert (got - want).abs().max() <= 8 * REL[torch.float16] * want.abs().max()
