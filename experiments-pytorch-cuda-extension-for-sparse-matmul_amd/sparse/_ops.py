@@ -329,24 +329,24 @@ def _longest_group(offsets) -> int:
     return longest
 
 
-def _group_walk_kinds(longest, dtype, pairs):
+def _group_walk_kinds(longest, dtype, pairs, of_others=True):
     """Schedules of a group walk over ``pairs`` pairs of all batch entries and strips: the one it takes, then what else serves
-    where that one cannot be built (the others of this type and of the 16-bit types)."""
+    where that one cannot be built (the others of this type; with ``of_others`` also what calls of another type have built)."""
     short = longest <= GROUP_WALK_LONG
     large = SCHEDULE_GROUP_WALK_LARGE if short else SCHEDULE_GROUP_WALK_LONG
     half = [SCHEDULE_GROUP_WALK, SCHEDULE_GROUP_WALK_MIDDLE, large] if short else [large]
+    single = [SCHEDULE_GROUP_WALK_F32, SCHEDULE_GROUP_WALK_F32_MIDDLE, SCHEDULE_GROUP_WALK_F32_LARGE if short else large]
     if dtype == torch.float32:
-        kinds = [SCHEDULE_GROUP_WALK_F32, SCHEDULE_GROUP_WALK_F32_MIDDLE, SCHEDULE_GROUP_WALK_F32_LARGE if short else large]
-        lines = GROUP_WALK_SMALL_PAIRS, GROUP_WALK_F32_MIDDLE_PAIRS
+        kinds, others, lines = single, half, (GROUP_WALK_SMALL_PAIRS, GROUP_WALK_F32_MIDDLE_PAIRS)
     else:
-        kinds, lines = half, (GROUP_WALK_SMALL_PAIRS, GROUP_WALK_MIDDLE_PAIRS) if short else ()
+        kinds, others, lines = half, single, (GROUP_WALK_SMALL_PAIRS, GROUP_WALK_MIDDLE_PAIRS) if short else ()
     first = kinds[sum(pairs > line for line in lines)]
 
     def whole(kind):                # chunks that cut no group which the largest launches leave whole
         cap, waves = kind[:2]
         return (max(cap, -(-longest // waves)),) + kind[1:] if longest <= large[0] * large[1] else kind
 
-    return tuple(dict.fromkeys(whole(kind) for kind in [first] + kinds + half))
+    return tuple(dict.fromkeys(whole(kind) for kind in [first] + kinds + (others if of_others else [])))
 
 
 def _group_walk_schedule(layout, dtype=torch.float16, entries=None, key=None):
@@ -367,27 +367,30 @@ def _group_walk_schedule(layout, dtype=torch.float16, entries=None, key=None):
 def _sdd_schedule(layout, dtype, batches, k):
     if dtype != torch.float32:
         small = layout[0].numel() // 2 * batches * -(-k // 64) <= SDD_SMALL_BLOCKS
-        return _schedule_or(layout, *((SCHEDULE_SDD_SMALL, SCHEDULE_SDD) if small else (SCHEDULE_SDD, SCHEDULE_SDD_SMALL)))
+        kinds = (SCHEDULE_SDD_SMALL, SCHEDULE_SDD) if small else (SCHEDULE_SDD, SCHEDULE_SDD_SMALL)
+        return _schedule_or(layout, *kinds, SCHEDULE_SDD_F32)
     if layout[0].numel() // 2 * batches * min(k, 64) >= 64 * SDD_F32_LARGE_BLOCKS:
-        return _schedule_or(layout, SCHEDULE_SDD_F32_LARGE, SCHEDULE_SDD_F32)
-    return _schedule_or(layout, SCHEDULE_SDD_F32, SCHEDULE_SDD_F32_LARGE)
+        return _schedule_or(layout, SCHEDULE_SDD_F32_LARGE, SCHEDULE_SDD_F32, SCHEDULE_SDD_SMALL)
+    return _schedule_or(layout, SCHEDULE_SDD_F32, SCHEDULE_SDD_F32_LARGE, SCHEDULE_SDD_SMALL)
 
 
-def _schedule_or(layout, kind, other):
-    """The schedule ``kind``, or, where a graph is being captured and only ``other`` is there, that one: building
-    synchronises."""
+def _schedule_or(layout, kind, *others):
+    """The schedule ``kind``, or, where a graph is being captured and it is not there, the first of ``others`` that is (they may
+    be what calls of another type have built): building synchronises."""
     there = getattr(layout[1], "_bsa_schedules", ())
     if kind in there:
         return there[kind]
-    return schedule_for(layout, other if other in there and torch.cuda.is_current_stream_capturing() else kind)
+    if torch.cuda.is_current_stream_capturing():
+        kind = next((other for other in others if other in there), kind)
+    return schedule_for(layout, kind)
 
 
 def _captured_without(layout, kind) -> bool:
-    """Whether a graph is being captured and the schedule ``kind`` of the table (None: of its group walk) is not there:
+    """Whether a graph is being captured and the schedule ``kind`` of the table (None: of its 16-bit group walk) is not there:
     building one synchronises.  Calls that used a walk without a schedule eagerly stay with it then."""
     if kind is None:
         longest = getattr(layout[1], "_bsa_longest", None)
-        kinds = () if longest is None else _group_walk_kinds(longest, torch.float16, 0)
+        kinds = () if longest is None else _group_walk_kinds(longest, torch.float16, 0, of_others=False)
     else:
         kinds = (SCHEDULE_SDD, SCHEDULE_SDD_SMALL) if kind == SCHEDULE_SDD else (kind,)
     return not any(_has_schedule(layout, k) for k in kinds) and torch.cuda.is_current_stream_capturing()

@@ -123,3 +123,59 @@ def test_scores_captured_on_the_other_side_of_the_line(monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+TYPES = [torch.float16, torch.bfloat16, torch.float32]
+
+
+@pytest.mark.parametrize("longest", [0, 1, 12, 13, 24, 25, 30, 40, 41, 64, 130])
+def test_whatever_a_call_built_serves_a_captured_one(longest, monkeypatch):
+    """A table that a call of any type and size has used, captured in any type and size: nothing is left to build."""
+    from sparse import _ops
+    for pairs in LINES:
+        for dtype in TYPES:
+            built = _ops._group_walk_kinds(longest, dtype, pairs)[0]
+            assert all(built in _ops._group_walk_kinds(longest, t, n) for t in TYPES for n in LINES)
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    layout = (torch.zeros(2 * 100, dtype=torch.int32), torch.tensor([0, 100], dtype=torch.int32))
+    for built in (_ops.SCHEDULE_SDD, _ops.SCHEDULE_SDD_SMALL, _ops.SCHEDULE_SDD_F32, _ops.SCHEDULE_SDD_F32_LARGE):
+        layout[1]._bsa_schedules = {built: object()}
+        for t in TYPES:
+            for batches in (1, 29, 30, 80, 81, 10 ** 5):
+                assert _ops._sdd_schedule(layout, t, batches, 64) is layout[1]._bsa_schedules[built]
+
+
+def _operands(L, n, mode, batches, dtype):
+    g = torch.Generator(device="cuda").manual_seed(n + batches)
+    dense = lambda: torch.randn(batches, n, 64, generator=g, device="cuda").to(dtype)
+    if mode == "sdd":
+        return dense(), dense(), "sdd", L, False, True
+    stack = torch.randn(batches, L.num_blocks, 32, 32, generator=g, device="cuda").to(dtype)
+    return (stack, dense(), "dsd", L) if mode == "dsd" else (dense().transpose(-1, -2).contiguous(), stack, "dds", L)
+
+
+# groups that a workgroup takes whole, and such as the launch of every type cuts: 30 and 64 pairs
+@pytest.mark.gpu
+@pytest.mark.parametrize("longest", [30, 64])
+@pytest.mark.parametrize("mode", ["sdd", "dsd", "dds"])
+@pytest.mark.parametrize("eager,captured", [(torch.float32, torch.float16), (torch.float32, torch.bfloat16), (torch.float16, torch.float32)])
+def test_captured_in_another_type(longest, mode, eager, captured):
+    """Bound: two results of an fp32 sum of at most 64 x 32 products, rounded once each, over the 2-norm."""
+    import sparse
+    L = sparse.SparseLayout(_mask(longest, mode != "dds").cuda())
+    n = 32 * (longest + 3)
+    sparse.matmul(*_operands(L, n, mode, 2, eager))
+    args = _operands(L, n, mode, 2, captured)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = sparse.matmul(*args)
+    rel = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7, torch.float32: 2.0 ** -20}[captured]
+    for _ in range(3):
+        for x, fresh in zip(args[:2], _operands(L, n, mode, 2, captured)):
+            x.copy_(-fresh)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = sparse.matmul(*args)
+        assert (got.double() - want.double()).norm() <= rel * want.double().norm()
