@@ -167,8 +167,9 @@ class Schedule:
         return self._zeroed(self.last_key, need)
 
     def has_workspace(self, key):
-        """Whether a graph can be given a workspace of ``key`` (a key without its stream)."""
-        return bool(self._spares.get(key)) or any(k[:-1] == key for k in self._captured)
+        """Whether a launch that is being captured can be given the workspace of ``key`` (its last item is the stream): one
+        that the stream has, or a spare.  What a graph of another stream has is that graph's."""
+        return key in self._captured or key in self._workspaces or bool(self._spares.get(key[:-1]))
 
     _spaces = {}             # of a schedule that no plan launches by
     MAX_WORKSPACES = 16      # eager ones per schedule; the least recently used one goes first
@@ -351,13 +352,15 @@ def _group_walk_kinds(longest, dtype, pairs, of_others=True):
 
 def _group_walk_schedule(layout, dtype=torch.float16, entries=None, key=None):
     """Schedule of a group walk over ``entries`` batch entries times strips (None: as many as fill the machine).  Under graph
-    capture the first that is there and has the launch's workspace, ``key``."""
+    capture the first that is there and has the launch's workspace, ``key`` (without its stream)."""
     pairs = layout[0].numel() // 2 * entries if entries is not None else 2 ** 62
     kinds = _group_walk_kinds(_longest_group(layout[1]), dtype, pairs)
     if torch.cuda.is_current_stream_capturing():
         there = [layout[1]._bsa_schedules[kind] for kind in kinds if _has_schedule(layout, kind)]
+        with _k.on_device(layout[1].device):
+            stream = _k.current_stream()
         for sched in there:
-            if sched.tile_slots == 0 or key is None or sched.has_workspace(key):
+            if sched.tile_slots == 0 or key is None or sched.has_workspace(key + (stream,)):
                 return sched
         if there:
             return there[0]

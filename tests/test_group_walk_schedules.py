@@ -179,3 +179,35 @@ def test_captured_in_another_type(longest, mode, eager, captured):
         torch.cuda.synchronize()
         want = sparse.matmul(*args)
         assert (got.double() - want.double()).norm() <= rel * want.double().norm()
+
+
+@pytest.mark.gpu
+def test_captured_where_another_schedule_has_the_workspace():
+    """A column of 64 pairs, cut by every launch: the schedule that an fp32 launch takes has no workspace left for a second graph,
+    or none of this shape; that of the 16-bit calls has."""
+    import sparse
+    L = sparse.SparseLayout(_mask(64, True).cuda())
+    n = 32 * 67
+    args = {b: _operands(L, n, "dsd", b, torch.float32) for b in (2, 3)}
+    half = {b: _operands(L, n, "dsd", b, torch.float16) for b in (2, 3)}
+    graphs = []
+
+    def capture(b):
+        torch.cuda.synchronize()
+        graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=stream):
+            got = sparse.matmul(*args[b])
+        graphs.append((graph, got, b, stream))
+
+    sparse.matmul(*args[2])
+    capture(2)                                                        # takes the fp32 schedule's spare
+    sparse.matmul(*half[2])
+    capture(2)                                                        # another stream's graph: the 16-bit schedule's spare
+    sparse.matmul(*half[3])
+    capture(3)                                                        # a shape that only 16-bit calls have had
+    for _ in range(3):
+        for graph, got, b, _ in graphs:
+            graph.replay()
+            torch.cuda.synchronize()
+            want = sparse.matmul(*args[b])
+            assert (got.double() - want.double()).norm() <= 2.0 ** -20 * want.double().norm()

@@ -66,3 +66,61 @@ def test_an_eager_buffer_moves_to_the_graph_that_captures_it(sched):
     assert later.data_ptr() == eager.data_ptr()
     sched.discard(key)                                          # a failed launch: forget it wherever it is
     assert key not in sched._captured and key not in sched._workspaces
+
+
+def test_has_workspace_says_what_a_capture_is_given(sched):
+    key, here, there = ("dsd", 2, 64, 64), 1, 2
+
+    def agrees(stream):
+        says = sched.has_workspace(key + (stream,))
+        kept = {name: {k: list(v) if isinstance(v, list) else v for k, v in getattr(sched, name).items()}
+                for name in ("_workspaces", "_captured", "_spares")}
+        sched.state["capturing"] = True
+        try:
+            sched._zeroed(key + (stream,), 64)
+            given = True
+        except RuntimeError:
+            given = False
+        sched.state["capturing"] = False
+        for name, value in kept.items():
+            setattr(sched, name, value)
+        assert says == given
+        return says
+
+    assert not agrees(here) and not agrees(there)                     # never used
+    sched._zeroed(key + (here,), 64)
+    assert agrees(here) and agrees(there)                             # its own, the spare
+    sched.state["capturing"] = True
+    sched._zeroed(key + (there,), 64)                                 # a graph takes the spare
+    sched.state["capturing"] = False
+    assert agrees(here) and agrees(there) and not agrees(3)           # what the graph of another stream has serves no third one
+    sched.discard(key + (here,))
+    assert not agrees(here) and agrees(there)
+
+
+def test_a_capture_takes_a_schedule_whose_workspace_it_can_have(sched, monkeypatch):
+    from sparse import _ops
+    state = {"stream": 1}
+    monkeypatch.setattr(_ops._k, "current_stream", lambda: state["stream"])
+    monkeypatch.setattr(_ops._k, "on_device", lambda device: _ops._k._SAME_DEVICE)
+    other = _ops.Schedule.__new__(_ops.Schedule)
+    other.table, other.tile_slots, sched.tile_slots = sched.table, 4, 4
+    other._workspaces, other._captured, other._spares = {}, {}, {}
+    key = ("dsd", 2, 64, 64)
+    layout = (torch.zeros(2 * 64, dtype=torch.int32), torch.tensor([0, 64], dtype=torch.int32))
+    first, *_, last = _ops._group_walk_kinds(64, torch.float32, 64)
+    layout[1]._bsa_schedules = {first: sched, last: other}
+    sched._zeroed(key + (1,), 64)
+    sched.state["capturing"] = True
+    chosen = lambda: _ops._group_walk_schedule(layout, torch.float32, 1, key)
+    state["stream"] = 2
+    assert chosen() is sched
+    sched._zeroed(key + (2,), 64)                                     # a graph takes its spare
+    assert chosen() is sched
+    state["stream"] = 3
+    sched.state["capturing"] = False
+    other._zeroed(key + (1,), 64)
+    sched.state["capturing"] = True
+    assert chosen() is other                                          # the first would refuse: its graph is that of stream 2
+    state["stream"] = 1
+    assert chosen() is sched
