@@ -70,10 +70,10 @@ size_t attention_backward_workspace_bytes(int row_tile_slots, int row_split_grou
 
 template <int HD, bool BF>
 __global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attention_fwd_f16_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v, int rows_q, int rows_k,
-    float scale2 /* scale * log2(e) */, int causal, half_t *__restrict__ out, float *__restrict__ lse,
-    const SchedGroup *__restrict__ sched_groups, AtSplitWorkspace ws)
+    const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
+    half_t *__restrict__ out, float *__restrict__ lse, const BlockDesc *__restrict__ blocks,
+    const SchedGroup *__restrict__ sched_groups, const SchedEntry *__restrict__ sched, AtSplitWorkspace ws,
+    int n_swg, int batches, int rows_q, int rows_k, float scale2 /* scale * log2(e) */, int causal)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int KS = HD / 16, KT = HD / 32, LDS_PER_WAVE = at_lds_per_wave(HD), STAT_OFF = 128 * HD;
@@ -267,11 +267,13 @@ __device__ __forceinline__ float exponent_scale(float scale) { return scale == 0
 
 template <int HD, bool BF, bool STACKS>
 __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ q, const half_t *__restrict__ dout, const half_t *__restrict__ k, const half_t *__restrict__ v,
-    int rows_q, int rows_k, const half_t *__restrict__ out, const float *__restrict__ lse, float scale,
-    float log2_scale /* of |scale| */, int causal, int nnz, half_t *__restrict__ p_out, half_t *__restrict__ ds_out,
-    half_t *__restrict__ dq_out, float *__restrict__ delta_out, const SchedGroup *__restrict__ sched_groups, AtSplitWorkspace ws)
+    const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
+    const half_t *__restrict__ dout, const half_t *__restrict__ out, const float *__restrict__ lse,
+    half_t *__restrict__ p_out, half_t *__restrict__ ds_out, half_t *__restrict__ dq_out,
+    float *__restrict__ delta_out,
+    const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
+    const SchedEntry *__restrict__ sched, AtSplitWorkspace ws,
+    int n_swg, int batches, int rows_q, int rows_k, int nnz, float scale, float log2_scale /* of |scale| */, int causal)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int KS = HD / 16, KT = HD / 32, LDS_PER_WAVE = at_bwd_lds_per_wave(HD, STACKS), N = TileRequests<HD>::N;
@@ -459,10 +461,12 @@ constexpr int at_bwd_col_lds_per_wave(int hd) { return 128 * hd + 256 + (at_bwd_
 
 template <int HD, bool BF>
 __global__ __launch_bounds__(HD == 64 ? 512 : 64 * AT_COLUMN_WAVES_128, HD == 64 ? 3 : 2) void attention_bwd_dkdv_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ k, const half_t *__restrict__ v, const half_t *__restrict__ q, const half_t *__restrict__ dout,
-    int rows_q, int rows_k, const float *__restrict__ lse, const float *__restrict__ delta, float scale, int causal,
-    half_t *__restrict__ dk_out, half_t *__restrict__ dv_out, const SchedGroup *__restrict__ sched_groups, AtSplitWorkspace ws)
+    const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
+    const half_t *__restrict__ dout, const float *__restrict__ lse, const float *__restrict__ delta,
+    half_t *__restrict__ dk_out, half_t *__restrict__ dv_out,
+    const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
+    const SchedEntry *__restrict__ sched, AtSplitWorkspace ws,
+    int n_swg, int batches, int rows_q, int rows_k, float scale, int causal)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int KS = HD / 16, KT = HD / 32, LDS_PER_WAVE = at_bwd_col_lds_per_wave(HD);
@@ -671,8 +675,8 @@ hipError_t forward(const AttentionArgs &p, hipStream_t st)
     const hipError_t err = w.allow(attention_fwd_f16_kernel<HD, BF>);
     if (err != hipSuccess) return err;
     attention_fwd_f16_kernel<HD, BF><<<w.grid, w.block, w.lds, st>>>(
-        w.slots, p.sched_wgs, p.batches, w.blocks, (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, 32 * p.mask_rows,
-        32 * p.mask_cols, p.scale * 1.4426950408889634f, p.causal ? 1 : 0, (half_t *)p.out, (float *)p.lse, w.groups, w.ws);
+        (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (half_t *)p.out, (float *)p.lse, w.blocks, w.groups,
+        w.slots, w.ws, p.sched_wgs, p.batches, 32 * p.mask_rows, 32 * p.mask_cols, p.scale * 1.4426950408889634f, p.causal ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -683,10 +687,10 @@ hipError_t backward_rows(const AttentionArgs &p, hipStream_t st)
     const hipError_t err = w.allow(attention_bwd_rows_kernel<HD, BF, STACKS>);
     if (err != hipSuccess) return err;
     attention_bwd_rows_kernel<HD, BF, STACKS><<<w.grid, w.block, w.lds, st>>>(
-        w.slots, p.sched_wgs, p.batches, w.blocks, (const half_t *)p.q, (const half_t *)p.dout, (const half_t *)p.k,
-        (const half_t *)p.v, 32 * p.mask_rows, 32 * p.mask_cols, (const half_t *)p.out, (const float *)p.lse, p.scale,
-        log2f(fabsf(p.scale)), p.causal ? 1 : 0, p.nnz, (half_t *)p.p_out, (half_t *)p.ds_out, (half_t *)p.dq_out,
-        (float *)p.delta, w.groups, w.ws);
+        (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, (const half_t *)p.out,
+        (const float *)p.lse, (half_t *)p.p_out, (half_t *)p.ds_out, (half_t *)p.dq_out, (float *)p.delta, w.blocks, w.groups,
+        w.slots, w.ws, p.sched_wgs, p.batches, 32 * p.mask_rows, 32 * p.mask_cols, p.nnz, p.scale, log2f(fabsf(p.scale)),
+        p.causal ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -697,9 +701,9 @@ hipError_t backward_columns(const AttentionArgs &p, hipStream_t st)
     const hipError_t err = w.allow(attention_bwd_dkdv_kernel<HD, BF>);
     if (err != hipSuccess) return err;
     attention_bwd_dkdv_kernel<HD, BF><<<w.grid, w.block, w.lds, st>>>(
-        w.slots, p.sched_wgs, p.batches, w.blocks, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.q,
-        (const half_t *)p.dout, 32 * p.mask_rows, 32 * p.mask_cols, (const float *)p.lse, (const float *)p.delta, p.scale,
-        p.causal ? 1 : 0, (half_t *)p.dk_out, (half_t *)p.dv_out, w.groups, w.ws);
+        (const half_t *)p.q, (const half_t *)p.k, (const half_t *)p.v, (const half_t *)p.dout, (const float *)p.lse,
+        (const float *)p.delta, (half_t *)p.dk_out, (half_t *)p.dv_out, w.blocks, w.groups, w.slots, w.ws, p.sched_wgs,
+        p.batches, 32 * p.mask_rows, 32 * p.mask_cols, p.scale, p.causal ? 1 : 0);
     return hipGetLastError();
 }
 }  // namespace

@@ -159,9 +159,10 @@ __device__ __forceinline__ void mailbox_add(f4v (&acc)[8], const float *box)
 // part of the design and the compiler may not move them across the barriers.
 template <bool BF, int MAXW>
 __global__ __launch_bounds__(64 * MAXW) void dsd_runs_f16_kernel(
-    const RunRecord *__restrict__ runs, int n_runs, int batches, const BlockDesc *__restrict__ blocks,
-    const unsigned char *__restrict__ pair_byte, const half_t *sp, const half_t *dn, int nnz, int DN, int KT, int XT,
-    int sp_shared, int info_off, int box_off, int strips, const int *__restrict__ offsets, half_t *__restrict__ out)
+    const half_t *sp, const half_t *dn, half_t *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
+    const RunRecord *__restrict__ runs, const unsigned char *__restrict__ pair_byte,
+    int n_runs, int batches, int nnz, int DN, int KT, int XT, int sp_shared, int info_off, int box_off, int strips)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, ri;
@@ -374,9 +375,9 @@ static hipError_t launch_runs(Kernel kernel, const RunsArgs &p, hipStream_t st)
     dim3 grid(grid_workgroups(p.n_runs, p.batches), (unsigned)(p.N / 64)), block(64 * p.waves);
     const RunRecord *runs = reinterpret_cast<const RunRecord *>(p.sched);
     const unsigned char *pair_byte = reinterpret_cast<const unsigned char *>(p.sched) + (size_t)p.mask_rows * sizeof(RunRecord);
-    kernel<<<grid, block, lds, st>>>(runs, p.n_runs, p.batches, (const BlockDesc *)p.blocks, pair_byte, (const half_t *)p.a,
-                                     (const half_t *)p.b, p.nnz, p.N, 32 * p.mask_cols, 32 * p.mask_rows, p.sparse_shared ? 1 : 0,
-                                     info_off, box_off, p.strips, p.offsets, (half_t *)p.c);
+    kernel<<<grid, block, lds, st>>>((const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, (const BlockDesc *)p.blocks,
+                                     p.offsets, runs, pair_byte, p.n_runs, p.batches, p.nnz, p.N, 32 * p.mask_cols,
+                                     32 * p.mask_rows, p.sparse_shared ? 1 : 0, info_off, box_off, p.strips);
     return hipGetLastError();
 }
 

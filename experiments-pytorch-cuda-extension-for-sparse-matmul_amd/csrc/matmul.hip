@@ -52,8 +52,9 @@ constexpr int SDD_LDS_PER_WAVE = 2048 * (1 + SDD_KB_MAX);   // a / result tile +
 // ---------------------------------------------------------------------------
 template <bool A_KC, bool B_KC, int KBT, bool BF>
 __global__ __launch_bounds__(512) void sdd_f16_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ a, const half_t *__restrict__ b, half_t *__restrict__ c, int nnz, int M, int N, int K)
+    const half_t *__restrict__ a, const half_t *__restrict__ b, half_t *__restrict__ c,
+    const BlockDesc *__restrict__ blocks, const SchedEntry *__restrict__ sched,
+    int n_swg, int batches, int nnz, int M, int N, int K)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, swg;
@@ -229,8 +230,9 @@ __device__ __forceinline__ void store16_f32(float *o, const f16v &acc)
 
 template <bool A_KC, bool B_KC>
 __global__ __launch_bounds__(512) void sdd_f32_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c, int nnz, int M, int N, int K)
+    const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c,
+    const BlockDesc *__restrict__ blocks, const SchedEntry *__restrict__ sched,
+    int n_swg, int batches, int nnz, int M, int N, int K)
 {
     int batch, swg;
     if (!map_workgroup(n_swg, batches, batch, swg)) return;
@@ -392,8 +394,9 @@ __device__ __forceinline__ bool not_finite(const f16v &acc)
 // and the products of block p run while they arrive.
 template <bool A_KC, bool B_KC, int KBT, bool SPLIT>
 __global__ __launch_bounds__(512) void sdd_f32_tiled_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c, int nnz, int M, int N, int K)
+    const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c,
+    const BlockDesc *__restrict__ blocks, const SchedEntry *__restrict__ sched,
+    int n_swg, int batches, int nnz, int M, int N, int K)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, swg;
@@ -565,9 +568,10 @@ __device__ __forceinline__ bool team_reduce(V (&acc)[NT], const SchedEntry &e, i
 // four times.
 template <bool S_KC, bool D_KC, bool DSD, int DEPTH, bool BF, bool FULL>
 __global__ __launch_bounds__(512) void gw_f16_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out, int nnz, int DN, int KT, int XT,
-    const SchedGroup *__restrict__ sched_groups, SplitWorkspace ws, int sp_shared, int idx_is_pos)
+    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
+    const SchedEntry *__restrict__ sched, SplitWorkspace ws,
+    int n_swg, int batches, int nnz, int DN, int KT, int XT, int sp_shared, int idx_is_pos)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, swg;
@@ -719,9 +723,10 @@ __global__ __launch_bounds__(512) void gw_f16_kernel(
 // ---------------------------------------------------------------------------
 template <bool BF>
 __global__ __launch_bounds__(512) void dsd_rows_f16_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out, int nnz, int DN, int KT, int XT,
-    const SchedGroup *__restrict__ sched_groups, SplitWorkspace ws, int sp_shared)
+    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
+    const SchedEntry *__restrict__ sched, SplitWorkspace ws,
+    int n_swg, int batches, int nnz, int DN, int KT, int XT, int sp_shared)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, swg;
@@ -856,9 +861,9 @@ constexpr int GW64_LDS_PER_WAVE = 16384;    // the strip (4 KB) while walking, t
 
 template <bool BF>
 __global__ __launch_bounds__(256) void dsd_rows64_f16_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out, const int *__restrict__ offsets,
-    int tiles, int DN, int KT, int XT, int sp_shared)
+    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets, const SchedEntry *__restrict__ sched,
+    int n_swg, int batches, int tiles, int DN, int KT, int XT, int sp_shared)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, swg;
@@ -989,9 +994,10 @@ __global__ __launch_bounds__(256) void dsd_rows64_f16_kernel(
 
 template <bool S_KC, bool D_KC, bool DSD>
 __global__ __launch_bounds__(512) void gw_f32_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const float *__restrict__ sp, const float *__restrict__ dn, float *__restrict__ out, int nnz, int DN, int KT, int XT,
-    const SchedGroup *__restrict__ sched_groups, SplitWorkspace ws, int sp_shared)
+    const float *__restrict__ sp, const float *__restrict__ dn, float *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
+    const SchedEntry *__restrict__ sched, SplitWorkspace ws,
+    int n_swg, int batches, int nnz, int DN, int KT, int XT, int sp_shared)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     int batch, swg;
@@ -1047,9 +1053,10 @@ __global__ __launch_bounds__(512) void gw_f32_kernel(
 // of pair p are issued.
 template <bool S_KC, bool D_KC, bool DSD>
 __global__ __launch_bounds__(512) void gw_f32_tiled_kernel(
-    const SchedEntry *__restrict__ sched, int n_swg, int batches, const BlockDesc *__restrict__ blocks,
-    const float *__restrict__ sp, const float *__restrict__ dn, float *__restrict__ out, int nnz, int DN, int KT, int XT,
-    const SchedGroup *__restrict__ sched_groups, SplitWorkspace ws, int sp_shared)
+    const float *__restrict__ sp, const float *__restrict__ dn, float *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const SchedGroup *__restrict__ sched_groups,
+    const SchedEntry *__restrict__ sched, SplitWorkspace ws,
+    int n_swg, int batches, int nnz, int DN, int KT, int XT, int sp_shared)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     static_assert(F32_TILE_BYTES <= GW_LDS_PER_WAVE, "the operand tile shares the wave's reduce area");
@@ -1136,8 +1143,8 @@ static hipError_t launch_sdd_f16(const MatmulArgs &p, hipStream_t st)
 {
     dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
     size_t lds = (size_t)p.sched_waves * SDD_LDS_PER_WAVE;
-#define BSA_SDD_ARGS sched_slots(p), p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, \
-                     (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, p.nnz, p.M, p.N, p.K
+#define BSA_SDD_ARGS (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, (const BlockDesc *)p.blocks, \
+                     sched_slots(p), p.sched_wgs, p.batches, p.nnz, p.M, p.N, p.K
     switch (p.K / BS) {
         case 1: sdd_f16_kernel<A_KC, B_KC, 1, BF><<<grid, block, lds, st>>>(BSA_SDD_ARGS); break;
         case 2: sdd_f16_kernel<A_KC, B_KC, 2, BF><<<grid, block, lds, st>>>(BSA_SDD_ARGS); break;
@@ -1154,8 +1161,8 @@ template <bool A_KC, bool B_KC>
 static hipError_t launch_sdd_f32(const MatmulArgs &p, hipStream_t st)
 {
     dim3 grid(grid_workgroups(p.sched_wgs, p.batches)), block(64 * p.sched_waves);
-#define BSA_SDD_ARGS sched_slots(p), p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, \
-                     (const float *)p.a, (const float *)p.b, (float *)p.c, p.nnz, p.M, p.N, p.K
+#define BSA_SDD_ARGS (const float *)p.a, (const float *)p.b, (float *)p.c, (const BlockDesc *)p.blocks, \
+                     sched_slots(p), p.sched_wgs, p.batches, p.nnz, p.M, p.N, p.K
     const int kbs = p.K / BS;
     const size_t lds = (size_t)p.sched_waves * kbs * F32_TILE_BYTES;
     if (kbs <= 4 && lds <= 163840) {      // at most 8 waves x 4 tiles of 4864 bytes: a compute unit's 160 KB hold it
@@ -1224,13 +1231,13 @@ static hipError_t launch_gw_t(int dtype, const void *sp, const void *dn, const M
     ws.split_groups = p.split_groups;
     ws.counters = (int *)p.workspace;
     ws.tiles = (float *)((char *)p.workspace + gw_counter_bytes(p.split_groups, p.batches, DN));
-#define BSA_GW_ARGS sched_slots(p), p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, (const half_t *)sp, \
-                    (const half_t *)dn, (half_t *)p.c, p.nnz, DN, KT, XT, sched_groups(p), ws, p.sparse_shared ? 1 : 0, \
+#define BSA_GW_ARGS (const half_t *)sp, (const half_t *)dn, (half_t *)p.c, (const BlockDesc *)p.blocks, \
+                    sched_groups(p), sched_slots(p), ws, p.sched_wgs, p.batches, p.nnz, DN, KT, XT, p.sparse_shared ? 1 : 0, \
                     p.row_table ? 1 : 0
     const bool full = DN % 64 == 0;
     if (S_KC && !D_KC && DSD && full && p.row_table && dtype != BSA_F32) {
-#define BSA_DR_ARGS sched_slots(p), p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, (const half_t *)sp, \
-                    (const half_t *)dn, (half_t *)p.c, p.nnz, DN, KT, XT, sched_groups(p), ws, p.sparse_shared ? 1 : 0
+#define BSA_DR_ARGS (const half_t *)sp, (const half_t *)dn, (half_t *)p.c, (const BlockDesc *)p.blocks, \
+                    sched_groups(p), sched_slots(p), ws, p.sched_wgs, p.batches, p.nnz, DN, KT, XT, p.sparse_shared ? 1 : 0
         if (dtype == BSA_F16) dsd_rows_f16_kernel<false><<<grid, block, lds, st>>>(BSA_DR_ARGS);
         else dsd_rows_f16_kernel<true><<<grid, block, lds, st>>>(BSA_DR_ARGS);
 #undef BSA_DR_ARGS
@@ -1245,8 +1252,8 @@ static hipError_t launch_gw_t(int dtype, const void *sp, const void *dn, const M
     } else
 #undef BSA_GW_ARGS
     {
-#define BSA_GW32_ARGS sched_slots(p), p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, (const float *)sp, \
-                      (const float *)dn, (float *)p.c, p.nnz, DN, KT, XT, sched_groups(p), ws, p.sparse_shared ? 1 : 0
+#define BSA_GW32_ARGS (const float *)sp, (const float *)dn, (float *)p.c, (const BlockDesc *)p.blocks, \
+                      sched_groups(p), sched_slots(p), ws, p.sched_wgs, p.batches, p.nnz, DN, KT, XT, p.sparse_shared ? 1 : 0
         if (full) gw_f32_tiled_kernel<S_KC, D_KC, DSD><<<grid, block, lds, st>>>(BSA_GW32_ARGS);
         else gw_f32_kernel<S_KC, D_KC, DSD><<<grid, block, lds, st>>>(BSA_GW32_ARGS);
 #undef BSA_GW32_ARGS
@@ -1265,15 +1272,15 @@ hipError_t launch_dsd_block64(int dtype, const Block64Args &p, hipStream_t st)
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (err != hipSuccess) return err;
         dsd_rows64_f16_kernel<false><<<grid, block, lds, st>>>(
-            slots, p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c,
-            p.offsets, 4 * p.coarse_nnz, p.N, 64 * p.coarse_cols, 64 * p.coarse_rows, p.sparse_shared ? 1 : 0);
+            (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, (const BlockDesc *)p.blocks, p.offsets, slots,
+            p.sched_wgs, p.batches, 4 * p.coarse_nnz, p.N, 64 * p.coarse_cols, 64 * p.coarse_rows, p.sparse_shared ? 1 : 0);
     } else {
         if (lds > 65536) err = hipFuncSetAttribute(reinterpret_cast<const void *>(dsd_rows64_f16_kernel<true>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (err != hipSuccess) return err;
         dsd_rows64_f16_kernel<true><<<grid, block, lds, st>>>(
-            slots, p.sched_wgs, p.batches, (const BlockDesc *)p.blocks, (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c,
-            p.offsets, 4 * p.coarse_nnz, p.N, 64 * p.coarse_cols, 64 * p.coarse_rows, p.sparse_shared ? 1 : 0);
+            (const half_t *)p.a, (const half_t *)p.b, (half_t *)p.c, (const BlockDesc *)p.blocks, p.offsets, slots,
+            p.sched_wgs, p.batches, 4 * p.coarse_nnz, p.N, 64 * p.coarse_cols, 64 * p.coarse_rows, p.sparse_shared ? 1 : 0);
     }
     return hipGetLastError();
 }

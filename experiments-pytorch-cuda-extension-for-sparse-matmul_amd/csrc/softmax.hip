@@ -486,8 +486,8 @@ __device__ __forceinline__ void softmax_fwd_sliced(const T *__restrict__ xb, T *
 // ---------------------------------------------------------------------------
 template <typename T, int CB, int CBS>
 __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void softmax_fwd_kernel(
-    const SchedEntry *__restrict__ sched, int batches, int nnz, const BlockDesc *__restrict__ blocks,
-    const T *__restrict__ x, T *__restrict__ y,
+    const T *__restrict__ x, T *__restrict__ y, const BlockDesc *__restrict__ blocks,
+    const SchedEntry *__restrict__ sched, int batches, int nnz,
     float scale2 /* scale * log2(e) */, int causal)
 {
     typedef Chunk<T> C;
@@ -808,8 +808,9 @@ __device__ __forceinline__ void softmax_bwd_sliced(const T *__restrict__ y, cons
 
 template <typename T, int CB, int CBS>
 __global__ __launch_bounds__(64 * SM_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void softmax_bwd_kernel(
-    const SchedEntry *__restrict__ sched, int batches, int nnz, const BlockDesc *__restrict__ blocks,
-    const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx, float scale)
+    const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx,
+    const BlockDesc *__restrict__ blocks, const SchedEntry *__restrict__ sched,
+    int batches, int nnz, float scale)
 {
     typedef Chunk<T> C;
     constexpr int NQ = C::NQ, EPC = C::EPC, LPR = C::LPR;
@@ -966,16 +967,16 @@ hipError_t launch_softmax_forward(int dtype, const SoftmaxArgs &p, hipStream_t s
     const float scale2 = p.scale * 1.4426950408889634f;
     if (dtype == BSA_F16)
         softmax_fwd_kernel<half_t, 4, 48><<<grid, block, 0, st>>>(
-            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, (const BlockDesc *)p.blocks,
-            (const half_t *)p.x, (half_t *)p.out, scale2, p.causal ? 1 : 0);
+            (const half_t *)p.x, (half_t *)p.out, (const BlockDesc *)p.blocks,
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
     else if (dtype == BSA_BF16)
         softmax_fwd_kernel<bf16_t, 4, 48><<<grid, block, 0, st>>>(
-            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, (const BlockDesc *)p.blocks,
-            (const bf16_t *)p.x, (bf16_t *)p.out, scale2, p.causal ? 1 : 0);
+            (const bf16_t *)p.x, (bf16_t *)p.out, (const BlockDesc *)p.blocks,
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
     else
         softmax_fwd_kernel<float, 2, 24><<<grid, block, 0, st>>>(
-            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, (const BlockDesc *)p.blocks,
-            (const float *)p.x, (float *)p.out, scale2, p.causal ? 1 : 0);
+            (const float *)p.x, (float *)p.out, (const BlockDesc *)p.blocks,
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, scale2, p.causal ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -984,16 +985,16 @@ hipError_t launch_softmax_backward(int dtype, const SoftmaxArgs &p, hipStream_t 
     dim3 grid((unsigned)p.sched_wgs * (unsigned)p.batches), block(64 * p.sched_waves);
     if (dtype == BSA_F16)
         softmax_bwd_kernel<half_t, 2, 24><<<grid, block, 0, st>>>(
-            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, (const BlockDesc *)p.blocks,
-            (const half_t *)p.x, (const half_t *)p.dy, (half_t *)p.out, p.scale);
+            (const half_t *)p.x, (const half_t *)p.dy, (half_t *)p.out, (const BlockDesc *)p.blocks,
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, p.scale);
     else if (dtype == BSA_BF16)
         softmax_bwd_kernel<bf16_t, 2, 24><<<grid, block, 0, st>>>(
-            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, (const BlockDesc *)p.blocks,
-            (const bf16_t *)p.x, (const bf16_t *)p.dy, (bf16_t *)p.out, p.scale);
+            (const bf16_t *)p.x, (const bf16_t *)p.dy, (bf16_t *)p.out, (const BlockDesc *)p.blocks,
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, p.scale);
     else
         softmax_bwd_kernel<float, 1, 24><<<grid, block, 0, st>>>(
-            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, (const BlockDesc *)p.blocks,
-            (const float *)p.x, (const float *)p.dy, (float *)p.out, p.scale);
+            (const float *)p.x, (const float *)p.dy, (float *)p.out, (const BlockDesc *)p.blocks,
+            (const SchedEntry *)p.sched + p.groups, p.batches, p.nnz, p.scale);
     return hipGetLastError();
 }
 

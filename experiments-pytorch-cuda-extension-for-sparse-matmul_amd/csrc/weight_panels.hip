@@ -64,8 +64,9 @@ __host__ __device__ constexpr int panel_list_length(int kblocks) { return (kbloc
 // ---------------------------------------------------------------------------
 template <int RT, bool S_KC, bool BF>
 __global__ __launch_bounds__(PANEL_THREADS, 3) void weight_panel_kernel(
-    const int *__restrict__ offsets, int row_tiles, int group_sets, const BlockDesc *__restrict__ blocks, int groups, int KT,
-    const half_t *__restrict__ dn, const half_t *__restrict__ sp, half_t *__restrict__ out, int nnz, int rows, int XT, int sp_shared)
+    const half_t *__restrict__ sp, const half_t *__restrict__ dn, half_t *__restrict__ out,
+    const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
+    int groups, int nnz, int rows, int KT, int XT, int sp_shared, int row_tiles, int group_sets)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int ROWS = 32 * RT, STAGES = panel_stages(RT), PANEL_BYTES = ROWS * 256;
@@ -356,9 +357,9 @@ constexpr int WG_STAGES = 4;
 
 template <bool BF>
 __global__ __launch_bounds__(512, 2) void weight_grad_kernel(
-    int shares, int sets_r, int sets_c, int steps_total, int R, int C, const int *__restrict__ offsets,
-    const BlockDesc *__restrict__ blocks, const half_t *__restrict__ a, const half_t *__restrict__ b, float *__restrict__ parts,
-    int nnz)
+    const half_t *__restrict__ a, const half_t *__restrict__ b, float *__restrict__ parts,
+    const BlockDesc *__restrict__ blocks, const int *__restrict__ offsets,
+    int R, int C, int nnz, int steps_total, int shares, int sets_r, int sets_c)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int item = xcd_contiguous(shares * sets_r * sets_c);
@@ -517,8 +518,8 @@ static hipError_t launch_panel(const WeightPanelArgs &p, hipStream_t st)
     }
     dim3 grid((unsigned)((tiles * sets + 7) / 8 * 8), (unsigned)p.batches);
     kernel<<<grid, 64 * (walkers + PANEL_FETCHERS), lds, st>>>(
-        p.offsets, tiles, sets, (const BlockDesc *)p.blocks, p.groups, p.KT, (const half_t *)p.dense, (const half_t *)p.sparse,
-        (half_t *)p.out, p.nnz, p.rows, BS * p.groups, p.sparse_shared ? 1 : 0);
+        (const half_t *)p.sparse, (const half_t *)p.dense, (half_t *)p.out, (const BlockDesc *)p.blocks, p.offsets, p.groups, p.nnz,
+        p.rows, p.KT, BS * p.groups, p.sparse_shared ? 1 : 0, tiles, sets);
     return hipGetLastError();
 }
 
@@ -585,8 +586,8 @@ hipError_t launch_weight_grad(int dtype, const WeightGradArgs &p, hipStream_t st
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return err;
     const unsigned grid = ((unsigned)p.shares * sets_r * sets_c + 7) / 8 * 8;
-    kernel<<<grid, 64 * WG_EDGE, lds, st>>>(p.shares, sets_r, sets_c, p.tokens / BS, p.mask_rows, p.mask_cols, p.offsets,
-                                            (const BlockDesc *)p.blocks, (const half_t *)p.a, (const half_t *)p.b, p.parts, p.nnz);
+    kernel<<<grid, 64 * WG_EDGE, lds, st>>>((const half_t *)p.a, (const half_t *)p.b, p.parts, (const BlockDesc *)p.blocks,
+                                            p.offsets, p.mask_rows, p.mask_cols, p.nnz, p.tokens / BS, p.shares, sets_r, sets_c);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     const size_t elements = (size_t)p.nnz * BS2;
