@@ -62,20 +62,22 @@ def test_multiple_batch_dims_and_many_batches(mode, ta, tb):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("mode,ta,tb", [("dsd", False, False), ("dsd", True, False), ("dds", False, False), ("dds", False, True)])
-def test_split_groups_reuse_their_workspace(mode, ta, tb, dtype):
+def test_split_groups_reuse_their_workspace(mode, ta, tb, dtype, monkeypatch):
     """Groups longer than one workgroup's span are cut into parts that meet in a workspace the
     library leaves zeroed: repeated calls, three 64-wide strips, several batches."""
     import sparse
     from sparse import _ops
-    old = _ops.SCHEDULE_GROUP_WALK, _ops.SCHEDULE_GROUP_WALK_LONG
-    try:
-        for sched in ((2, 2), (4, 8), (3, 1)):
-            _ops.SCHEDULE_GROUP_WALK = _ops.SCHEDULE_GROUP_WALK_LONG = sched
-            for name in ("long_row_5x40", "long_col_70x3"):
-                errs = [_run(mode, ZOO[name], 160, ta, tb, dtype, batch=(3,), seed=s) for s in range(3)]
-                assert max(errs) <= tol_of(dtype), (sched, name, errs)
-    finally:
-        _ops.SCHEDULE_GROUP_WALK, _ops.SCHEDULE_GROUP_WALK_LONG = old
+    used, walk = [], _ops._group_walk_schedule
+    monkeypatch.setattr(_ops, "_group_walk_schedule", lambda *args: used.append(walk(*args)) or used[-1])
+    for sched in ((2, 2), (4, 8), (3, 1)):
+        for name in ("SCHEDULE_GROUP_WALK", "SCHEDULE_GROUP_WALK_LONG", "SCHEDULE_GROUP_WALK_F32", "SCHEDULE_GROUP_WALK_F32_MIDDLE"):
+            monkeypatch.setattr(_ops, name, sched)
+        used.clear()
+        for name in ("long_row_5x40", "long_col_70x3"):
+            errs = [_run(mode, ZOO[name], 160, ta, tb, dtype, batch=(3,), seed=s) for s in range(3)]
+            assert max(errs) <= tol_of(dtype), (sched, name, errs)
+        split = [(s.cap, s.waves) for s in used if s.split_groups > 0]
+        assert len(split) >= 3 and set(split) == {sched}              # the table with the long group, in each call on it
 
 
 def test_split_result_is_deterministic():
