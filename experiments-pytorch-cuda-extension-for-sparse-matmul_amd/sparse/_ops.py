@@ -137,34 +137,33 @@ class Schedule:
         self._captured = {}
         self._spares = {}
         self._spaces = {}
-        self.last_key = None
 
     def workspace(self, mode: int, batches: int, size_m: int, size_n: int, stream: int):
         """Zeroed scratch for split groups, one per (shape, stream): launches on one stream run in
-        order and each leaves the buffer zero again; launches on different streams may overlap."""
+        order and each leaves the buffer zero again; launches on different streams may overlap.
+        Returns the buffer, its bytes and the key it is kept under (``None, 0, None`` where nothing is needed)."""
         if self.tile_slots == 0:
-            self.last_key = None
-            return None, 0
+            return None, 0, None
         need = _k.lib.bsa_matmul_workspace_bytes(mode, self.tile_slots, self.split_groups, batches, size_m, size_n)
-        self.last_key = (mode, batches, size_m, size_n, stream)
-        return self._zeroed(self.last_key, need)
+        return self._kept((mode, batches, size_m, size_n, stream), need)
 
     def attention_workspace(self, batches: int, head_dim: int, stream: int):
         """The same for the split rows of the fused attention forward."""
         if self.tile_slots == 0:
-            self.last_key = None
-            return None, 0
+            return None, 0, None
         need = _k.lib.bsa_attention_workspace_bytes(self.tile_slots, self.split_groups, batches, head_dim)
-        self.last_key = ("attention", batches, head_dim, stream)
-        return self._zeroed(self.last_key, need)
+        return self._kept(("attention", batches, head_dim, stream), need)
 
     def attention_backward_workspace(self, columns, batches: int, head_dim: int, stream: int):
         """The same for the backward walks: this schedule walks the rows, ``columns`` (or None) the columns."""
         ct, cg = (columns.tile_slots, columns.split_groups) if columns is not None else (0, 0)
         need = _k.lib.bsa_attention_backward_workspace_bytes(self.tile_slots, self.split_groups, ct, cg, batches,
                                                              head_dim)
-        self.last_key = ("attention_backward", id(columns), batches, head_dim, stream)
-        return self._zeroed(self.last_key, need)
+        return self._kept(("attention_backward", id(columns), batches, head_dim, stream), need)
+
+    def _kept(self, key, need):
+        ws, need = self._zeroed(key, need)
+        return ws, need, key if ws is not None else None
 
     def has_workspace(self, key):
         """Whether a launch that is being captured can be given the workspace of ``key`` (its last item is the stream): one
@@ -295,11 +294,11 @@ def _run_schedule(layout, batches, strips_n):
     return rs if rs.strips <= 4 * rs.waves and rs.pairs <= 64 * rs.waves else None
 
 
-def _launch(sched, status):
-    """Raise on a failed C-ABI call; the workspace the call was given is dropped first, because a launch
+def _launch(sched, key, status):
+    """Raise on a failed C-ABI call; the workspace the call was given, ``key`` (or None), is dropped first, because a launch
     that failed midway may have left its counters non-zero and every later call would sum stale parts."""
-    if status != 0 and sched is not None and sched.last_key is not None:
-        sched.discard(sched.last_key)
+    if status != 0 and key is not None:
+        sched.discard(key)
     _k.check(status)
 
 
@@ -587,8 +586,8 @@ def sparse_matmul(a, b, mode, row_layout, col_layout, trans_a=False, trans_b=Fal
                 dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(), layout[0].data_ptr(), layout[1].data_ptr(),
                 mask_rows, mask_cols, num_blocks, batches, sparse_batches, size_m, int(bool(trans_b)), stream))
         else:
-            ws, ws_bytes = sched.workspace(_k.MODES[mode], batches, size_m, size_n, stream)
-            _launch(sched, _k.lib.bsa_matmul(
+            ws, ws_bytes, key = sched.workspace(_k.MODES[mode], batches, size_m, size_n, stream)
+            _launch(sched, key, _k.lib.bsa_matmul(
                 _k.MODES[mode], dtype, a.data_ptr(), b.data_ptr(), c.data_ptr(),
                 layout[0].data_ptr(), layout[1].data_ptr(), layout[1].numel() - 1,
                 sched.table.data_ptr(), sched.workgroups, sched.waves, sched.tile_slots, sched.split_groups,
@@ -748,8 +747,8 @@ def sparse_attention_forward(q, k, v, row_blocks, row_table, scale=1.0, causal=F
         sched = _attention_schedule_for(row_layout, SCHEDULE_ATTENTION, batches)
         with _k.on_device(q.device):
             stream = _k.current_stream()
-            ws, ws_bytes = sched.attention_workspace(batches, head, stream)
-            _launch(sched, _k.lib.bsa_attention_forward(
+            ws, ws_bytes, key = sched.attention_workspace(batches, head, stream)
+            _launch(sched, key, _k.lib.bsa_attention_forward(
                 _DTYPES[q.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                 lse.data_ptr() if lse is not None else None,
                 row_blocks.data_ptr(), row_table.data_ptr(), sched.table.data_ptr(), sched.workgroups, sched.waves,
@@ -781,8 +780,8 @@ def sparse_attention_backward_scores(q, k, v, dout, out, lse, row_blocks, row_ta
         sched = _attention_schedule(row_layout, SCHEDULE_ATTENTION_BACKWARD, split=ATTENTION_SPLIT_ROWS)
         with _k.on_device(q.device):
             stream = _k.current_stream()
-            ws, ws_bytes = sched.attention_backward_workspace(None, batches, head, stream) if with_dq else (None, 0)
-            _launch(sched, _k.lib.bsa_attention_backward_scores(
+            ws, ws_bytes, key = sched.attention_backward_workspace(None, batches, head, stream) if with_dq else (None, 0, None)
+            _launch(sched, key, _k.lib.bsa_attention_backward_scores(
                 _DTYPES[q.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), out.data_ptr(),
                 lse.data_ptr(), p.data_ptr(), ds.data_ptr(), dq.data_ptr() if with_dq else None,
                 row_blocks.data_ptr(), row_table.data_ptr(),
@@ -827,8 +826,8 @@ def sparse_attention_backward(q, k, v, dout, out, lse, row_blocks, row_table, co
             else (None, 0, 0, 0, 0)
         with _k.on_device(q.device):
             stream = _k.current_stream()
-            ws, ws_bytes = rs.attention_backward_workspace(cs, batches, head, stream)
-            _launch(rs, _k.lib.bsa_attention_gradients(
+            ws, ws_bytes, key = rs.attention_backward_workspace(cs, batches, head, stream)
+            _launch(rs, key, _k.lib.bsa_attention_gradients(
                 _DTYPES[q.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), out.data_ptr(),
                 lse.data_ptr(), dq.data_ptr(), dk.data_ptr() if with_dkdv else None, dv.data_ptr() if with_dkdv else None,
                 delta.data_ptr(),
@@ -866,9 +865,8 @@ def _planned(make):
     return planned
 
 
-def _add(plans, op, flags, a, b, route, ints, tables, out=(), workspace=(None, 0), sched=None, aligned=False):
-    ws, ws_bytes = workspace
-    key = sched.last_key if ws is not None else None
+def _add(plans, op, flags, a, b, route, ints, tables, out=(), workspace=(None, 0, None), sched=None, aligned=False):
+    ws, ws_bytes, key = workspace
     _k.host_calls.add_plan(plans, op, flags, a, b, route, _DTYPES[a.dtype], aligned, ints, tables, out,
                            sched.plan_space(key, ws) if ws is not None else None, ws_bytes, _k.current_stream(), sched, key)
     return True

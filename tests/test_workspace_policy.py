@@ -124,3 +124,36 @@ def test_a_capture_takes_a_schedule_whose_workspace_it_can_have(sched, monkeypat
     assert chosen() is other                                          # the first would refuse: its graph is that of stream 2
     state["stream"] = 1
     assert chosen() is sched
+
+
+def test_a_plan_launches_with_the_workspace_of_its_own_stream(sched, monkeypatch):
+    """Two threads ask for a workspace, each on its stream, before either leaves its plan (filling one with zeros gives the
+    interpreter away): plans that launch with one buffer on two streams would add up each other's partial tiles."""
+    from sparse import _ops
+    state, added = {"stream": 1}, []
+    monkeypatch.setattr(_ops._k, "current_stream", lambda: state["stream"])
+    monkeypatch.setattr(_ops._k.host_calls, "new_space", lambda ws: ws)
+    monkeypatch.setattr(_ops._k.host_calls, "add_plan", lambda *args: added.append(args))
+    sched.tile_slots, sched.split_groups, sched._spaces = 4, 1, {}
+    a = torch.empty(2, 64, 64)
+    for ask in (lambda stream: sched.workspace(1, 2, 64, 64, stream), lambda stream: sched.attention_workspace(2, 64, stream),
+                lambda stream: sched.attention_backward_workspace(None, 2, 64, stream)):
+        added.clear()
+        asked = {stream: ask(stream) for stream in (1, 2)}
+        for stream, workspace in asked.items():
+            state["stream"] = stream
+            _ops._add(None, 0, 0, a, a, 0, (), (), workspace=workspace, sched=sched)
+        for (stream, workspace), args in zip(asked.items(), added):
+            space, nbytes, of_stream, schedule, key = args[-5:]
+            assert space.data_ptr() == workspace[0].data_ptr() == sched._workspaces[key].data_ptr()
+            assert nbytes == workspace[1] and of_stream == stream == key[-1] and schedule is sched
+    assert len(sched._workspaces) == 6
+
+
+def test_a_failed_launch_forgets_its_own_workspace(sched):
+    from sparse import _ops
+    sched.tile_slots, sched.split_groups, sched._spaces = 4, 1, {}
+    mine, other = (sched.workspace(1, 2, 64, 64, stream) for stream in (1, 2))
+    with pytest.raises(_ops._k.BsaError):
+        _ops._launch(sched, mine[2], 1)
+    assert [ws.data_ptr() for ws in sched._workspaces.values()] == [other[0].data_ptr()]
