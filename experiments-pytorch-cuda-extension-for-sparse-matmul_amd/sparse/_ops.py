@@ -6,6 +6,7 @@ signature (``native/sparse_ops.h:10-14``); the softmax entry points keep those o
 ``sparse_softmax.cu:208-210,233-236`` with ``scale`` / ``causal`` appended.
 """
 import functools
+import threading
 
 import torch
 
@@ -168,9 +169,11 @@ class Schedule:
     def has_workspace(self, key):
         """Whether a launch that is being captured can be given the workspace of ``key`` (its last item is the stream): one
         that the stream has, or a spare.  What a graph of another stream has is that graph's."""
-        return key in self._captured or key in self._workspaces or bool(self._spares.get(key[:-1]))
+        with self._lock:
+            return key in self._captured or key in self._workspaces or bool(self._spares.get(key[:-1]))
 
     _spaces = {}             # of a schedule that no plan launches by
+    _lock = threading.RLock()          # of what the schedules keep; none of the schedule's own, which is copied with its layout
     MAX_WORKSPACES = 16      # eager ones per schedule; the least recently used one goes first
 
     def _zeroed(self, key, need):
@@ -187,13 +190,22 @@ class Schedule:
         comes here again, where it is dropped and where a capture took the shape's spare."""
         if need == 0:
             return None, 0
+        gone = []
+        with self._lock:
+            ws = self._hand_out(key, need, gone)
+        for stream, _ in gone:
+            self._drain(stream)
+        return ws, need
+
+    def _hand_out(self, key, need, gone):
+        """``_zeroed`` under the lock: filling a buffer lets other threads in.  What is dropped goes to ``gone``, with its stream."""
         capturing = torch.cuda.is_current_stream_capturing()
         spares = self._spares.setdefault(key[:-1], [])
         ws = self._captured.get(key)
         if ws is not None:                              # the graph that owns it is being extended or re-captured
             if not capturing and not spares:
                 spares.append(torch.zeros(need, dtype=torch.uint8, device=self.table.device))
-            return ws, need
+            return ws
         ws = self._workspaces.pop(key, None)
         if ws is None:
             if capturing:
@@ -209,14 +221,13 @@ class Schedule:
             spares.append(torch.zeros(need, dtype=torch.uint8, device=self.table.device))
         if capturing:
             self._captured[key] = ws
-            return ws, need
+            return ws
         self._workspaces[key] = ws                      # most recently used last
         while len(self._workspaces) > self.MAX_WORKSPACES:
             old_key = next(iter(self._workspaces))
             self._forget_plans(old_key)
-            self._drain(old_key[-1])
-            self._workspaces.pop(old_key)
-        return ws, need
+            gone.append((old_key[-1], self._workspaces.pop(old_key)))
+        return ws
 
     def _drain(self, stream_handle):
         """Waits for the stream a workspace was used on before the workspace is given back to the allocator."""
@@ -224,9 +235,10 @@ class Schedule:
 
     def plan_space(self, key, ws):
         """What the plans that launch with the workspace ``ws`` of ``key`` share, and lose together."""
-        if key not in self._spaces:
-            self._spaces[key] = _k.host_calls.new_space(ws)
-        return self._spaces[key]
+        with self._lock:
+            if key not in self._spaces:
+                self._spaces[key] = _k.host_calls.new_space(ws)
+            return self._spaces[key]
 
     def _forget_plans(self, key):
         space = self._spaces.pop(key, None)
@@ -235,9 +247,10 @@ class Schedule:
 
     def discard(self, key):
         """Forget the workspace of ``key``: a launch that failed may have left its counters non-zero."""
-        self._forget_plans(key)
-        self._workspaces.pop(key, None)
-        self._captured.pop(key, None)
+        with self._lock:
+            self._forget_plans(key)
+            self._workspaces.pop(key, None)
+            self._captured.pop(key, None)
 
 
 class RunSchedule:

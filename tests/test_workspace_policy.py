@@ -2,6 +2,9 @@
 
 A captured graph holds the raw address of its workspace, so a buffer handed out under capture must
 never return to the allocator; an eager one may, once the stream it was used on has drained."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -157,3 +160,23 @@ def test_a_failed_launch_forgets_its_own_workspace(sched):
     with pytest.raises(_ops._k.BsaError):
         _ops._launch(sched, mine[2], 1)
     assert [ws.data_ptr() for ws in sched._workspaces.values()] == [other[0].data_ptr()]
+
+
+def test_threads_that_take_more_shapes_than_are_kept(sched):
+    """Filling a buffer and waiting for a stream give the interpreter away: another thread drops the same oldest buffer, or asks
+    for the one that is being dropped."""
+    sched._drain = lambda handle: time.sleep(0)
+    sched._spaces, errors = {}, []
+
+    def work(stream):
+        try:
+            for i in range(60):
+                ws, need = sched._zeroed(("dsd", i % (sched.MAX_WORKSPACES + 4), 64, 64, stream), 64)
+                assert need == ws.numel() == 64 and len(sched._workspaces) <= sched.MAX_WORKSPACES
+        except Exception as error:
+            errors.append(error)
+
+    threads = [threading.Thread(target=work, args=(stream,)) for stream in (1, 1, 2, 3)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert errors == []
