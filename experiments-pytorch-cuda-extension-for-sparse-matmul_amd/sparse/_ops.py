@@ -160,7 +160,7 @@ class Schedule:
         ct, cg = (columns.tile_slots, columns.split_groups) if columns is not None else (0, 0)
         need = _k.lib.bsa_attention_backward_workspace_bytes(self.tile_slots, self.split_groups, ct, cg, batches,
                                                              head_dim)
-        return self._kept(("attention_backward", id(columns), batches, head_dim, stream), need)
+        return self._kept(("attention_backward", ct, cg, batches, head_dim, stream), need)
 
     def _kept(self, key, need):
         ws, need = self._zeroed(key, need)

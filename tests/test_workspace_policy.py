@@ -180,3 +180,14 @@ def test_threads_that_take_more_shapes_than_are_kept(sched):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert errors == []
+
+
+def test_a_column_schedule_where_another_one_was(sched):
+    """An object that is gone leaves its id to the next: a backward workspace is as large as the columns it is asked for need."""
+    from types import SimpleNamespace
+    sched.tile_slots, sched.split_groups, sched._spaces = 4, 1, {}
+    columns = SimpleNamespace(tile_slots=2, split_groups=1)
+    small, few, _ = sched.attention_backward_workspace(columns, 2, 64, 1)
+    columns.tile_slots, columns.split_groups = 40, 3                  # the next one, at the same address
+    large, need, _ = sched.attention_backward_workspace(columns, 2, 64, 1)
+    assert small.numel() == few < need == large.numel()
