@@ -139,6 +139,12 @@ class Schedule:
         self._spares = {}
         self._spaces = {}
 
+    def __getstate__(self):
+        """A copy (of the layout) has no launches, graphs and plans yet: it gets the spares, which are always zero."""
+        with self._lock:
+            return {**self.__dict__, "_workspaces": {}, "_captured": {}, "_spaces": {},
+                    "_spares": {key: list(spares) for key, spares in self._spares.items()}}
+
     def workspace(self, mode: int, batches: int, size_m: int, size_n: int, stream: int):
         """Zeroed scratch for split groups, one per (shape, stream): launches on one stream run in
         order and each leaves the buffer zero again; launches on different streams may overlap.

@@ -319,3 +319,28 @@ def test_plans_are_bounded():
     for i, n in enumerate(list(range(1, 81)) + [1, 80, 2]):
         assert torch.equal(sparse.softmax(x[:n], L, 1.0, False), want[:n])
         assert len(kernel.host_calls.plan_workspaces(L._plans)) == min(i + 1, 64)
+
+
+@pytest.mark.parametrize("call", ["matmul", "attention"])
+def test_a_layout_with_plans_is_copied_and_saved(call):
+    """Split groups: the plans' workspaces stay with the layout they are of."""
+    import io
+    import sparse
+    L = _layout()
+    if call == "matmul":
+        args = [t.detach() for t in _product(L, "dds", False, False, 64, torch.float16)]
+        run = lambda layout: sparse.matmul(*args, "dds", layout)
+        offsets = L.col_layout[1]
+    else:
+        L = _layout("long_row_5x40")
+        args = [_randn(2, 32 * n, 64, dtype=torch.float16, seed=n) for n in (5, 40, 40)]
+        run = lambda layout: sparse.attention(*args, layout, 0.125)
+        offsets = L.row_layout[1]
+    want = run(L)
+    assert call == "attention" or any(s._spaces for s in offsets._bsa_schedules.values())
+    f = io.BytesIO()
+    torch.save(L, f)
+    f.seek(0)
+    for other in (copy.deepcopy(L), torch.load(f, weights_only=False)):
+        for _ in range(2):
+            assert torch.equal(run(other), want) and torch.equal(run(L), want)

@@ -2,6 +2,8 @@
 
 A captured graph holds the raw address of its workspace, so a buffer handed out under capture must
 never return to the allocator; an eager one may, once the stream it was used on has drained."""
+import copy
+import pickle
 import threading
 import time
 
@@ -191,3 +193,21 @@ def test_a_column_schedule_where_another_one_was(sched):
     columns.tile_slots, columns.split_groups = 40, 3                  # the next one, at the same address
     large, need, _ = sched.attention_backward_workspace(columns, 2, 64, 1)
     assert small.numel() == few < need == large.numel()
+
+
+def test_a_schedule_that_plans_launch_by_is_copied(sched):
+    """With its layout, by deepcopy and pickle: plans and buffers in use stay behind, the spares go along."""
+    from sparse import _ops
+    sched.tile_slots, sched.split_groups, sched._spaces = 4, 1, {}
+    ws, _, key = sched.workspace(1, 2, 64, 64, 1)
+    assert sched.plan_space(key, ws) is sched._spaces[key]
+    del sched._drain, sched.state, sched.drained                      # the fixture's own
+    ws.fill_(1)                                                       # as while a launch is under way
+    offsets = torch.zeros(3)
+    offsets._bsa_schedules = {"kind": sched}
+    for copied in (copy.deepcopy(offsets)._bsa_schedules["kind"], pickle.loads(pickle.dumps(sched))):
+        assert copied._workspaces == copied._captured == copied._spaces == {} and copied.tile_slots == 4
+        assert copied.has_workspace(key) and not copied._spares[key[:-1]][0].any()
+        again, _, _ = copied.workspace(1, 2, 64, 64, 1)
+        assert not again.any() and again.data_ptr() != ws.data_ptr()
+    assert list(sched._workspaces) == [key] and list(sched._spaces) == [key] and _ops.Schedule._spaces == {}
