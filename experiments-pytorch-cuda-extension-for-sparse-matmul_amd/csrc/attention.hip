@@ -447,9 +447,10 @@ __global__ __launch_bounds__(512, HD == 64 ? 3 : 2) void attention_bwd_rows_kern
 // and V 64, so a tile's operands are read four at a time instead of all at once).
 // us, both sides in turn on one box, two waves per SIMD (200 registers) -> three at 64: 48 heads of 8192 tokens 114.1 -> 105.8,
 // the training pass 275.2 -> 266.3; one (368 registers) -> two at 128, where a wave alone had nothing to wait beside: 16 heads of
-// 4096 tokens 63 -> 51, the training pass 133.1 -> 120.9 (left to the compiler two waves spill 53 registers: 183).  There a second
-// stage of tiles, requested a whole block ahead, took one wave 63.1 -> 66.1 us.  At 64 one workgroup per residency slot that walks several columns and requests the next one's
-// tiles early took 111 -> 129 us (its neighbours drift apart and leave the L2's working set), forward and rows likewise.
+// 4096 tokens 72 -> 58 under the profiler, the training pass 137.3 -> 128.4 (left to the compiler two waves spill 53 registers and
+// take nearly three times as long).  There a second stage of tiles, requested a whole block ahead, took one wave 63.1 -> 66.1 us.  At 64
+// one workgroup per residency slot that walks several columns and requests the next one's tiles early took 111 -> 129 us (its
+// neighbours drift apart and leave the L2's working set), forward and rows likewise.
 // Delta is scaled as it is read; with scale * delta in memory the whole backward pass takes 1 % less (48.4-49.0 against 49.3-50.1
 // us).  Starting the second product at delta, 184 registers, takes as long and is further from float64 (dk of fp16, causal:
 // 3.1957e-4 against 3.1949e-4, at head dim 128 3.4662e-4 against 3.4642e-4).

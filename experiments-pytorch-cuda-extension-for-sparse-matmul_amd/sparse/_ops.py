@@ -18,9 +18,11 @@ BLOCK = 32
 # Group walks (DSD, DDS).  A launch of few pairs is one generation of waves and lasts as long as its fullest SIMD: shorter chunks,
 # spread over more of them.  Counted are the pairs of all batch entries and 64-column strips.  A table whose longest group fits
 # the workgroup of a large launch is not cut by shorter chunks either (_group_walk_kinds): no launch needs a workspace that another
-# batch count of the same layout does not need.  us, median of a graph, chunks of 12 -> now (fp16 DSD): 592 pairs, rows of up to 6
-# 5.2 -> 4.6, 2024 (12) 7.1 -> 4.8, 4048 7.4 -> 5.7, 6072 7.5 -> 6.7, 12144 13.3 -> 10.3, 12240 (20) 9.9 -> 8.8; 18112 (9) would be 13.3 ->
-# 14.9.  Tables with longer groups gain nothing in fp16 (506 to 14664 pairs, chunks of 4 to 10 within 3 % below 5000, slower above).
+# batch count of the same layout does not need.  us, median of a graph of 20 launches, chunks of 12 -> now (fp16 DSD, longest row in
+# brackets): 506 pairs (12) 6.6 -> 4.4, 628 (5) 4.8 -> 4.3, 2024 (12) 6.8 -> 4.6, 4048 (12) 7.0 -> 5.3, 6072 (12) 7.1 -> 6.8,
+# 6120 (20) 6.9 -> 6.4, 9432 (12) 10.0 -> 8.4, 12144 (12) 13.0 -> 10.3, 12240 (20) 10.4 -> 8.7, 13344 (9) 11.8 -> 10.3; 16192 (12) would
+# be 14.1 -> 13.9, 17792 (9) 12.7 -> 13.0.  Tables with longer groups gain little in fp16 (columns of 64, chunks of 10 against 4 and 6:
+# 506 to 4048 pairs within 6 %, 8096 8.7 against 9.6 and 9.0, 12144 12.2 against 12.8 and 13.0; of 128: 6120 8.4 against 9.8 and 9.6).
 SCHEDULE_GROUP_WALK = (4, 4, True, -1, 2, True)          # groups of at most GROUP_WALK_LONG pairs (rows of attention masks)
 SCHEDULE_GROUP_WALK_MIDDLE = (6, 4, True, -1, 2, True)
 SCHEDULE_GROUP_WALK_LARGE = (12, 4, True, -1, 2, True)
@@ -29,7 +31,8 @@ GROUP_WALK_LONG = 24
 GROUP_WALK_SMALL_PAIRS, GROUP_WALK_MIDDLE_PAIRS = 4096, 14000
 SCHEDULE_SDD = (4, 2)
 # SDD of few blocks (of all batch entries, times 64-value pieces of the inner dimension): more waves of two blocks each.  fp16, us,
-# chunks of 4 -> 2: 592 blocks 3.9 -> 3.4, 2024 4.6 -> 4.1, 4048 4.8 -> 4.6, 7156 5.8 -> 5.6; 12240 would be 7.4 -> 7.6.  The same bits.
+# chunks of 4 -> 2: 506 blocks 3.5 -> 3.0, 2024 4.2 -> 3.7, 4048 4.5 -> 4.4, 6120 5.0 -> 4.9, 7084 5.9 -> 6.0; 8096 would be 5.6 -> 5.6,
+# 12240 7.2 -> 7.3.  The same bits.
 SCHEDULE_SDD_SMALL = (2, 2)
 SDD_SMALL_BLOCKS = 8000
 # fp32: a wave splits its row's operands into bf16 parts once, so chunks pay where the products are split: from as many blocks on as
@@ -40,11 +43,11 @@ SCHEDULE_SDD_F32 = (1, 4)
 SCHEDULE_SDD_F32_LARGE = (4, 2)
 SDD_F32_LARGE_BLOCKS = 3000            # of all batch entries together, at k = 64 and more
 # fp32: a pair keeps its SIMD's matrix pipe for 2048 clocks, so the chunks of the fullest SIMD are the launch.  us, chunks of 6 (10
-# in tables with longer groups) -> now: 592 pairs, rows of up to 6 11.5 -> 7.6, 2024 (12) 12.0 -> 8.2, (columns of 64) 17.9 -> 11.3;
-# 4048 (columns of 64) 19.5 -> 13.7, 6120 (rows of 20, columns of 128) 20.0 -> 15.5 and 21.8 -> 18.5, 8096 (12, 64) 20.3 -> 18.6 and 24.3 ->
-# 20.5, 10464
-# (rows of 7) 22.1 -> 21.5, 9776 (columns of 64) 24.5 -> 22.8; from 12000 pairs on chunks of 4 are ahead in some launches and behind in as
-# many (12144 29.2 -> 27.3, 13392 26.6 -> 27.1, 14664 26.9 -> 30.6).
+# in tables with longer groups) -> now.  Rows of up to 12: 506 pairs 11.0 -> 7.4, 2024 11.2 -> 7.8, 4048 11.6 -> 10.9, 8096 19.6 -> 18.3,
+# 10120 24.9 -> 21.2; of 5: 628 10.0 -> 7.4, 5024 13.8 -> 14.2; of 20 (chunks of 5 hold them): 6120 18.9 -> 16.3, 9180 23.3 -> 21.9.
+# Columns of 64: 506 17.1 -> 10.4, 2024 17.6 -> 11.0, 4048 18.0 -> 13.2, 8096 24.4 -> 20.9, 10120 25.8 -> 22.1; of 128: 6120 21.4 -> 17.9,
+# 9180 28.2 -> 22.5.  The line at 11000 lies where chunks of 4 stop being ahead for rows: 12144 pairs would be 25.4 -> 25.6 (12), 12240
+# 24.3 -> 23.3 (20); for columns they still would be at some sizes: 12144 28.7 -> 26.7 and 14674 34.7 -> 31.0 (64), 12240 26.1 -> 26.4 (128).
 SCHEDULE_GROUP_WALK_F32 = (3, 4, True, -1, 2, True)
 SCHEDULE_GROUP_WALK_F32_MIDDLE = (4, 4, True, -1, 2, True)
 SCHEDULE_GROUP_WALK_F32_LARGE = (6, 4, True, -1, 2, True)      # 73440 pairs, chunks of 12 -> 6: 114 -> 114
